@@ -69,7 +69,7 @@ __device__ __forceinline__ double wave_sum(double v)
     return v;
 }
 
-// Per-vertex offsets: P0 += dverts, and the projected vertices again (store_vertex's formula).
+// Per-vertex offsets: P0 += dverts, and the projected vertices again.
 __global__ void __launch_bounds__(256) k_add_offsets(int V, const FrameGPU* __restrict__ frames, int n,
                                                       const double* __restrict__ rt, const float* __restrict__ dverts,
                                                       double* __restrict__ P0, float4* __restrict__ vproj)
@@ -84,12 +84,8 @@ __global__ void __launch_bounds__(256) k_add_offsets(int V, const FrameGPU* __re
         p[a] = P0[3 * o + a] + (double)dverts[3 * o + a];
         P0[3 * o + a] = p[a];
     }
-    const FrameGPU fr = frames[f];
-    const double X = R[0] * p[0] + R[3] * p[1] + R[6] * p[2] + R[9];
-    const double Y = R[1] * p[0] + R[4] * p[1] + R[7] * p[2] + R[10];
-    const double Z = R[2] * p[0] + R[5] * p[1] + R[8] * p[2] + R[11];
-    vproj[o] = make_float4((float)((double)fr.phix * X / Z + (double)fr.cx), (float)((double)fr.phiy * Y / Z + (double)fr.cy),
-                           (float)Z, 0.f);
+    double q[3];
+    vproj[o] = project_vertex(FrameCam{frames[f].phix, frames[f].phiy, frames[f].cx, frames[f].cy}, R, p, q);
 }
 
 // Residuals of the visible pixels: the data loss (FP64, per frame) and dL/dB at the neighbours.

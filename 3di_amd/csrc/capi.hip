@@ -714,7 +714,7 @@ static int big_scratch(tdi_batch* b)
 // the normalised gradients read.
 // dverts (optional, device [fl.n][V][3]): per-vertex model-space offsets added after the synthesis
 // (all frames of the chunk listed, fl.act == nullptr).
-static int eval_render(tdi_batch* b, FrameList fl, const float* theta, int mixed, hipStream_t s,
+static int eval_render(tdi_batch* b, FrameList fl, const float* theta, hipStream_t s,
                        const Layout* Lp = nullptr, bool full_crop = false, const float* dverts = nullptr)
 {
     tdi_ctx* c = b->ctx;
@@ -723,8 +723,6 @@ static int eval_render(tdi_batch* b, FrameList fl, const float* theta, int mixed
     int rc;
     if (b->joint && L.nid && w.idshape)   // the identity stage's frames share alpha
         rc = launch_synthesize_shared_id(b->m, L, w.frames, fl, theta, w.rt, w.P0, nullptr, w.vproj, w.idshape, s);
-    else if (mixed & TDI_MIXED_SYNTH_MFMA)
-        rc = launch_synthesize_gemm(b->m, L, w.frames, fl, theta, w.rt, w.P0, nullptr, w.vproj, s);
     else
         rc = launch_synthesize(b->m, L, w.frames, fl, theta, w.rt, w.P0, nullptr, w.vproj, s);
     if (rc) return rc;
@@ -749,7 +747,7 @@ static int eval_render(tdi_batch* b, FrameList fl, const float* theta, int mixed
 // loop, model_fitter.cu:219-260): the same synthesis, raster and per-pixel terms as
 // eval_render, but shading and the objective work from the keys over the visible box, so
 // there is no visible list, no scatter and no per-pixel Jacobian records.
-static int eval_objective(tdi_batch* b, FrameList fl, const float* theta, int mixed, hipStream_t s,
+static int eval_objective(tdi_batch* b, FrameList fl, const float* theta, hipStream_t s,
                           const Layout* Lp = nullptr)
 {
     tdi_ctx* c = b->ctx;
@@ -758,8 +756,6 @@ static int eval_objective(tdi_batch* b, FrameList fl, const float* theta, int mi
     int rc;
     if (b->joint && L.nid && w.idshape)   // the identity stage's frames share alpha
         rc = launch_synthesize_shared_id(b->m, L, w.frames, fl, theta, w.rt, w.P0, nullptr, w.vproj, w.idshape, s);
-    else if (mixed & TDI_MIXED_SYNTH_MFMA)
-        rc = launch_synthesize_gemm(b->m, L, w.frames, fl, theta, w.rt, w.P0, nullptr, w.vproj, s);
     else
         rc = launch_synthesize(b->m, L, w.frames, fl, theta, w.rt, w.P0, nullptr, w.vproj, s);
     if (rc) return rc;
@@ -836,7 +832,7 @@ static int eval_jacobian(tdi_batch* b, FrameList fl, const float* theta, int mix
 static int eval_full(tdi_batch* b, FrameList fl, const float* theta, int mixed, hipStream_t s,
                      const Layout* Lp = nullptr)
 {
-    int rc = eval_render(b, fl, theta, mixed, s, Lp);
+    int rc = eval_render(b, fl, theta, s, Lp);
     if (rc) return rc;
     return eval_jacobian(b, fl, theta, mixed, s, Lp);
 }
@@ -915,7 +911,7 @@ int tdi_render(tdi_batch* b, const float* theta, float* img, float* blurred, flo
         if (rc) return rc;
         const long long off = b->hframes[i0].obs_off;
         const long long len = (i0 + n < b->n ? b->hframes[i0 + n].obs_off : b->total) - off;
-        if ((rc = eval_render(b, all_frames(n), theta + (size_t)i0 * K, 0, s, nullptr, true))) return rc;
+        if ((rc = eval_render(b, all_frames(n), theta + (size_t)i0 * K, s, nullptr, true))) return rc;
         if (img) TDI_HIP(hipMemcpyAsync(img + off, w.img, sizeof(float) * len, hipMemcpyDeviceToDevice, s));
         if (blurred) TDI_HIP(hipMemcpyAsync(blurred + off, w.blurred, sizeof(float) * len, hipMemcpyDeviceToDevice, s));
         if (obj && (rc = launch_misc_f64_to_f32(w.obj, obj + i0, n, s))) return rc;
@@ -959,7 +955,7 @@ int tdi_render_loss_grad(tdi_batch* b, const float* theta, const float* dverts, 
         const int n = std::min(w.C, b->n - i0);
         if ((rc = ws_load(b, i0, n, s))) break;
         const float* th = theta + (size_t)i0 * K;
-        if ((rc = eval_render(b, all_frames(n), th, 0, s, nullptr, false, dverts ? dverts + (size_t)i0 * V * 3 : nullptr)))
+        if ((rc = eval_render(b, all_frames(n), th, s, nullptr, false, dverts ? dverts + (size_t)i0 * V * 3 : nullptr)))
             break;
         rc = launch_adjoint(c->m, c->L, w.frames, n, th, w.P0, w.pvert, w.pbary, w.vis, w.npix, w.pixg, w.lmk, c->taps,
                             w.max_area, w.img, w.tmp, w.blurred, a, gloss ? gloss + i0 : nullptr,
@@ -1037,7 +1033,7 @@ static int joint_objective(tdi_batch* b, const float* dtheta, double* objs, hipS
     long long KJ;
     joint_sizes(b, Ks, KJ);
     b->joint = 1;
-    int rc = eval_objective(b, all_frames(b->n), dtheta, 0, s);
+    int rc = eval_objective(b, all_frames(b->n), dtheta, s);
     b->joint = 0;
     if (rc) return rc;
     return launch_shared_bounds(Ks, KJ, dtheta, c->m.lb, c->m.ub, 0, objs, nullptr, nullptr, s);
@@ -1614,6 +1610,7 @@ int tdi_landmark_slack_terms(tdi_batch* b, const float* theta, int32_t k_exp, co
 int tdi_fit_buffers(tdi_batch* b, const float* theta, int32_t mixed_flags, float* vproj, int32_t* nbr,
                     int32_t* npix, void* stream)
 {
+    (void)mixed_flags;   // the render is the same for all of them
     hipStream_t s = (hipStream_t)stream;
     Workspace& w = b->ws;
     const int K = b->ctx->L.K, V = b->ctx->m.V;
@@ -1623,7 +1620,7 @@ int tdi_fit_buffers(tdi_batch* b, const float* theta, int32_t mixed_flags, float
         if (rc) return rc;
         const long long off = b->hframes[i0].obs_off;
         const long long len = (i0 + n < b->n ? b->hframes[i0 + n].obs_off : b->total) - off;
-        if ((rc = eval_render(b, all_frames(n), theta + (size_t)i0 * K, mixed_flags, s))) return rc;
+        if ((rc = eval_render(b, all_frames(n), theta + (size_t)i0 * K, s))) return rc;
         if (vproj)
             TDI_HIP(hipMemcpyAsync(vproj + (size_t)i0 * V * 4, w.vproj, sizeof(float4) * (size_t)n * V,
                                    hipMemcpyDeviceToDevice, s));
@@ -1686,7 +1683,7 @@ int tdi_batch_autotune(tdi_batch* b, const float* theta, int32_t reps, int32_t* 
     const int n = std::min(w.C, b->n);
     const int mixed = c->opts.mixed_flags;
     int rc = ws_load(b, 0, n, s);
-    if (!rc) rc = eval_render(b, all_frames(n), theta, mixed, s);
+    if (!rc) rc = eval_render(b, all_frames(n), theta, s);
     if (rc) return rc;
     hipEvent_t e0, e1;
     TDI_HIP(hipEventCreate(&e0));
@@ -1768,10 +1765,7 @@ int tdi_stage_times(tdi_batch* b, const float* theta, int32_t mixed, int32_t rep
     double acc[7] = {0, 0, 0, 0, 0, 0, 0};
     for (int r = 0; r < reps; ++r) {
         TDI_HIP(hipEventRecord(ev[0], s));
-        if (mixed & TDI_MIXED_SYNTH_MFMA)
-            rc = launch_synthesize_gemm(b->m, c->L, w.frames, all_frames(n), theta, w.rt, w.P0, nullptr, w.vproj, s);
-        else
-            rc = launch_synthesize(b->m, c->L, w.frames, all_frames(n), theta, w.rt, w.P0, nullptr, w.vproj, s);
+        rc = launch_synthesize(b->m, c->L, w.frames, all_frames(n), theta, w.rt, w.P0, nullptr, w.vproj, s);
         if (rc) return rc;
         TDI_HIP(hipEventRecord(ev[1], s));
         if ((rc = launch_clear_keys_frames(w.frames, all_frames(n), w.keys, w.box, w.max_area, s))) return rc;
@@ -1872,7 +1866,7 @@ static int fit_plain(tdi_batch* b, float* theta_host, tdi_fit_report* reports)
                 for (int k = 0; k < K; ++k) tt[k] = (k >= hold0 && k < hold1) ? th[k] : th[k] + t * delta[k];
                 if (tt[off_tz] < 0.f) break;
                 TDI_HIP(hipMemcpyAsync(w.theta_try, tt.data(), sizeof(float) * K, hipMemcpyHostToDevice, s));
-                if ((rc = eval_objective(b, all_frames(1), w.theta_try, 0, s))) return rc;
+                if ((rc = eval_objective(b, all_frames(1), w.theta_try, s))) return rc;
                 double objt = 0, objb = 0;
                 int fok = 1;
                 TDI_HIP(hipMemcpyAsync(&objt, w.obj, sizeof(double), hipMemcpyDeviceToHost, s));
@@ -1892,7 +1886,7 @@ static int fit_plain(tdi_batch* b, float* theta_host, tdi_fit_report* reports)
             }
         }
         if (!terminate && !(rep.stop & (TDI_STOP_NAN | TDI_STOP_NOT_PD))) rep.stop |= TDI_STOP_MAXITER;
-        if ((rc = eval_objective(b, all_frames(1), w.theta, 0, s))) return rc;
+        if ((rc = eval_objective(b, all_frames(1), w.theta, s))) return rc;
         double fin = 0;
         TDI_HIP(hipMemcpyAsync(&fin, w.obj, sizeof(double), hipMemcpyDeviceToHost, s));
         TDI_HIP(hipStreamSynchronize(s));
@@ -2078,7 +2072,7 @@ static int light_fit(tdi_batch* b, const float* theta_host, float* lam_host, flo
             const FrameList fl{W.act_e, n};
             // the first evaluation renders every frame of the chunk; the light changes nothing else
             if (first) {
-                if ((rc = eval_render(b, fl, W.theta, 0, s, &Lx)) || (rc = eval_light_jacobian(b, fl, W.theta, s))) return rc;
+                if ((rc = eval_render(b, fl, W.theta, s, &Lx)) || (rc = eval_light_jacobian(b, fl, W.theta, s))) return rc;
             } else if ((rc = eval_light_full(b, fl, W.theta, s))) {
                 return rc;
             }
@@ -2237,7 +2231,7 @@ static int record_fit(tdi_batch* b, hipStream_t s)
         if ((rc = launch_split_fresh(n, w.st, w.mask_r, w.mask_u, s))) return rc;
         if ((rc = launch_compact_frames(n, w.mask_r, w.act_r, s))) return rc;
         if ((rc = launch_compact_frames(n, w.mask_u, w.act_u, s))) return rc;
-        if ((rc = eval_render(b, FrameList{w.act_r, w.C}, w.theta, o.mixed_flags, s))) return rc;
+        if ((rc = eval_render(b, FrameList{w.act_r, w.C}, w.theta, s))) return rc;
         if ((rc = eval_reused(b, FrameList{w.act_u, w.C}, w.theta, s))) return rc;
         if ((rc = eval_jacobian(b, FrameList{w.act_m, w.C}, w.theta, o.mixed_flags, s))) return rc;
         if ((rc = launch_cholesky(n, K, w.H, w.g, w.delta, w.status, (o.mixed_flags & TDI_MIXED_CHOL_F32) ? 1 : 0,
@@ -2249,7 +2243,7 @@ static int record_fit(tdi_batch* b, hipStream_t s)
                                         w.evalmask, hold0, hold1, s)))
                 return rc;
             if ((rc = launch_compact_frames(n, w.evalmask, w.act_e, s))) return rc;
-            if ((rc = eval_objective(b, FrameList{w.act_e, w.C}, w.theta_try, o.mixed_flags, s))) return rc;
+            if ((rc = eval_objective(b, FrameList{w.act_e, w.C}, w.theta_try, s))) return rc;
             if ((rc = launch_ls_decide(n, K, w.st, w.evalmask, w.searching, w.obj, w.objb, w.face_ok, w.theta,
                                        w.theta_try, o, s)))
                 return rc;
@@ -2309,7 +2303,7 @@ static int fit_batched(tdi_batch* b, float* theta, tdi_fit_report* reports, void
         if (reports) {
             // objective at the returned parameters
             if ((rc = set_mask_all(b, s))) return rc;
-            if ((rc = eval_render(b, all_frames(w.n_cur), w.theta, c->opts.mixed_flags, s))) return rc;
+            if ((rc = eval_render(b, all_frames(w.n_cur), w.theta, s))) return rc;
         }
         std::vector<double> hobj(w.C);
         std::vector<int> hnp(w.C);

@@ -256,6 +256,20 @@ __device__ inline void rodrigues_f64(const TU* uf, double* R)
         }
 }
 
+// Camera of a frame, and the projection every vertex path shares: q = R p + tau (rt: R column-major,
+// then tau) in FP64, image coordinates and depth rounded to FP32 once.
+struct FrameCam {
+    float phix, phiy, cx, cy;
+};
+__device__ __forceinline__ float4 project_vertex(const FrameCam& cam, const double* rt, const double* p, double* q)
+{
+#pragma unroll
+    for (int a = 0; a < 3; ++a) q[a] = rt[a] * p[0] + rt[3 + a] * p[1] + rt[6 + a] * p[2] + rt[9 + a];
+    const double iz = 1.0 / q[2];          // one FP64 division per vertex; x and y stay within 2 FP64 ulp
+    return make_float4((float)((double)cam.phix * q[0] * iz + (double)cam.cx),
+                       (float)((double)cam.phiy * q[1] * iz + (double)cam.cy), (float)q[2], 0.f);
+}
+
 // ------------------------------------------------------------------ host helpers
 void set_error(const char* fmt, ...);
 
@@ -304,8 +318,6 @@ int launch_synthesize_shared_id(const ModelGPU& m, const Layout& L, const FrameG
                                 hipStream_t s);
 // The per-frame vertex albedos of the listed frames (ModelGPU::alb) from their theta.
 int launch_albedo(const ModelGPU& m, const Layout& L, FrameList fl, const float* theta, float* alb, hipStream_t s);
-int launch_synthesize_gemm(const ModelGPU& m, const Layout& L, const FrameGPU* frames, FrameList fl,
-                           const float* theta, double* rt, double* P0, float* P, float4* vproj, hipStream_t s);
 
 // raster.hip
 int launch_clear_keys(uint64_t* keys, long long total, hipStream_t s);

@@ -5,43 +5,39 @@
 // view_transform_3d_pts_and_render_2d (funcs.cu:395-453): P = R P0 + tau,
 // xp = phix X/Z + cx, yp = phiy Y/Z + cy.
 //
-// Both forms accumulate the basis product, rotate, translate and project in FP64 and round
-// the results to FP32 once: the projected vertices then equal the correctly rounded values
-// (what an FP64 computation rounded to FP32 gives), so the FP32 coverage test downstream
-// sees the same inputs as an FP64 transcription would.  MI355X runs FP64 FMA and FP64 MFMA
-// at the same 78.6 TFLOP/s, so this costs little next to the rest of an iteration.
+// The basis product, rotation, translation and projection are FP64, rounded to FP32 once: the
+// projected vertices then equal the correctly rounded values (what an FP64 computation rounded to
+// FP32 gives), so the FP32 coverage test downstream sees the same inputs as an FP64 transcription
+// would.  MI355X runs FP64 FMA and FP64 MFMA at the same 78.6 TFLOP/s, so this costs little next
+// to the rest of an iteration.
 //
-//   k_synth_gemv   — one frame per grid row (the plain path): thread per vertex.
-//   k_synth_tile   — many frames: [3V x K] x [K x B] on v_mfma_f64_16x16x4f64; a workgroup
-//                    owns 16 vertices, stages their basis rows in LDS once and walks every
-//                    frame of the list; the epilogue fuses mean, rotation, translation and
-//                    projection from registers.
+//   k_synth_tile   — [3V x K] x [K x B] on v_mfma_f64_16x16x4f64; a workgroup owns 16 vertices,
+//                    stages their basis rows in LDS and walks every frame of the list; the
+//                    epilogue fuses mean, rotation, translation and projection from registers.
 #include "common.h"
 
 namespace tdi {
 
 namespace {
 
-constexpr int MAXK_LDS = 1024;
+constexpr int MAX_UNKNOWNS = 1024;
+constexpr int MAXK_LDS = 1024;          // identity coefficients that k_id_shape holds in LDS
 
-__device__ __forceinline__ void store_vertex(const FrameGPU& fr, const double* R, const double* tau, const double* p,
-                                             size_t o, double* P0, float* P, float4* vproj)
+__device__ __forceinline__ void store_vertex(const FrameCam& cam, const double* R, const double* p, size_t o, double* P0,
+                                             float* P, float4* vproj)
 {
     // model-space vertices stay FP64: the shading normal is the cross product of edges of
     // about a millimetre between coordinates of about 100 mm, which FP32 would round to 1e-5
     P0[3 * o + 0] = p[0];
     P0[3 * o + 1] = p[1];
     P0[3 * o + 2] = p[2];
-    const double X = R[0] * p[0] + R[3] * p[1] + R[6] * p[2] + tau[0];
-    const double Y = R[1] * p[0] + R[4] * p[1] + R[7] * p[2] + tau[1];
-    const double Z = R[2] * p[0] + R[5] * p[1] + R[8] * p[2] + tau[2];
+    double q[3];
+    vproj[o] = project_vertex(cam, R, p, q);
     if (P) {                               // camera-space vertices only when asked for
-        P[3 * o + 0] = (float)X;
-        P[3 * o + 1] = (float)Y;
-        P[3 * o + 2] = (float)Z;
+        P[3 * o + 0] = (float)q[0];
+        P[3 * o + 1] = (float)q[1];
+        P[3 * o + 2] = (float)q[2];
     }
-    vproj[o] = make_float4((float)((double)fr.phix * X / Z + (double)fr.cx), (float)((double)fr.phiy * Y / Z + (double)fr.cy),
-                           (float)Z, 0.f);
 }
 
 // FP64 rotation and translation of every listed frame, once per launch (the synthesis
@@ -60,42 +56,6 @@ __global__ void k_frame_rt(Layout L, const float* __restrict__ theta, const int*
     for (int a = 0; a < 3; ++a) o[9 + a] = tf[L.off_pose + a];
 }
 
-__global__ void __launch_bounds__(256) k_synth_gemv(ModelGPU m, Layout L, const FrameGPU* __restrict__ frames,
-                                                     const float* __restrict__ theta, const int* __restrict__ act,
-                                                     int n, const double* __restrict__ rt, double* __restrict__ P0,
-                                                     float* __restrict__ P, float4* __restrict__ vproj)
-{
-    __shared__ double R[12];
-    __shared__ float th[MAXK_LDS];
-    const double* tau = R + 9;
-    const int nact = fl_count(act, n);
-    for (int yi = blockIdx.y; yi < nact; yi += gridDim.y) {
-        const int f = fl_frame(act, yi);
-        const float* tf = theta + (size_t)f * L.K;
-        for (int i = threadIdx.x; i < L.K; i += blockDim.x) th[i] = tf[i];
-        if (threadIdx.x < 12) R[threadIdx.x] = rt[(size_t)f * 12 + threadIdx.x];
-        __syncthreads();
-        const int v = blockIdx.x * blockDim.x + threadIdx.x;
-        if (v < m.V) {
-            double p[3];
-#pragma unroll
-            for (int a = 0; a < 3; ++a) {
-                const int r = 3 * v + a;
-                double s = m.mean[r];
-                const float* e = m.exp_basis + (size_t)r * m.exp_ld;
-                for (int k = 0; k < L.nexp; ++k) s = fma((double)e[k], (double)th[L.off_exp + k], s);
-                if (L.nid) {
-                    const float* ib = m.id_basis + (size_t)r * m.id_ld;
-                    for (int k = 0; k < L.nid; ++k) s = fma((double)ib[k], (double)th[L.off_id + k], s);
-                }
-                p[a] = s;
-            }
-            store_vertex(frames[f], R, tau, p, (size_t)f * m.V + v, P0, P, vproj);
-        }
-        __syncthreads();
-    }
-}
-
 // FP64 MFMA operand layout, v_mfma_f64_16x16x4f64 (one double per lane for A and B):
 //   A[i][k]: lane = i + 16*k          B[k][j]: lane = j + 16*k
 // Accumulator: lane l, element r (0..3) holds C[l/16 + 4*r][l % 16] (measured on gfx950;
@@ -107,86 +67,169 @@ typedef double v4d __attribute__((ext_vector_type(4)));
 // accumulator per coordinate, whose tile row i is vertex i (A = that coordinate's basis rows of the
 // 16 vertices, B = the coefficients of 16 frames), so lane l, element r of the x, y and z
 // accumulators holds vertex l/16 + 4 r for frame l%16: every MFMA row is a vertex coordinate
-// (three MFMAs per k-step for 16 vertices).  The basis rows are staged in LDS (as FP64) once; then
-// each wavefront walks its own groups of 16 list entries with no further barrier.  A lane loads
-// the coefficients of its frame for its four k residues up front (one batch of independent loads),
-// and the epilogue (mean, FP64 rotation, translation, projection) runs from registers.
+// (three MFMAs per k-step for 16 vertices).  The columns of a k-step are free to choose: step
+// 4 t + s takes column 16 t + 4 kq + s from the lanes of residue kq = l/16, so that a lane's
+// entries of four steps are one aligned 16-byte piece of a basis row.
+//
+// Long lists: the basis rows are staged in LDS (as FP64), SY_KMAX columns at a time, identity
+// columns first.  With one such chunk (the per-frame fit: expression columns only) it is staged
+// once and each wavefront walks its own groups of 16 list entries with no further barrier; with
+// more, the workgroup stages every chunk for each four groups.
+//
+// One group (a list of up to 16 frames, such as the last line-search rounds of any batch): nothing
+// is reused from LDS and latency is all there is, so three wavefronts take a coordinate each
+// straight from memory and the four share the epilogue.  The sums run in the same order in both
+// forms, so a frame's vertices do not depend on the frames around it.
+//
+// Every caller takes this kernel, one frame too.  Single evaluations took a thread per vertex walking
+// its own three rows before: a sector per lane and load, and the whole basis again for every frame.
+// Measured at 53,361 vertices and 79 columns, that kernel against this one: 96 frames 2493 -> 104 us,
+// 48 frames 1258 -> 55 us, one frame 19.2 -> 21.7 us.  Bound by the FP64 matrix rate (31 us of the 104)
+// and the stores (40 B per vertex, 44 us).  The one-group form took the mean launch of a one-frame fit
+// from 10.2 to 6.9 us (its basis staging alone was 39 us of a launch: run-time divisors).
 constexpr int SY_VERTS = 16;               // vertices per workgroup
-constexpr int SY_KMAX = 80;                // expression coefficients held in LDS (K_exp <= 80)
+constexpr int SY_KMAX = 80;                // columns held in LDS at a time
 
-// Three wavefronts per SIMD (register budget 168) hide the coefficient loads of one behind the
-// MFMAs of the others.
+// this lane's B entries: columns 16 t + 4 kq + s of a chunk of kc, every load issued
+// unconditionally (clamped to a valid column) so the batch has no branches.  Nothing needs zeroing:
+// the A entries past the chunk's columns are zero, and an output column depends on its own frame's
+// B column only, so lanes without a live frame just skip the epilogue.
+__device__ __forceinline__ void synth_coefs(const float* __restrict__ tb, int kq, int kc, float* bv)
+{
+#pragma unroll
+    for (int q = 0; q < SY_KMAX / 4; ++q) bv[q] = tb[min(16 * (q >> 2) + 4 * kq + (q & 3), kc - 1)];
+}
+
+// Three wavefronts per SIMD (register budget 168): with four, 30 registers spill and 96 frames take
+// 148 us instead of 98.  ONE: a single chunk of columns.
+template <bool ONE>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
 k_synth_tile(ModelGPU m, Layout L, const FrameGPU* __restrict__ frames, const float* __restrict__ theta,
              const int* __restrict__ act, int n, const double* __restrict__ rt, const double* __restrict__ mean64,
              double* __restrict__ P0, float* __restrict__ P, float4* __restrict__ vproj)
 {
-    __shared__ double sA[3][SY_KMAX][16];              // [coordinate][k][vertex]
+    __shared__ double sA[3][SY_KMAX][16];              // [coordinate][column][vertex]
     __shared__ double smean[SY_VERTS * 3];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    if (fl_count(act, n) == 0) return;       // an emptied list: skip the basis staging
+    const int nact = fl_count(act, n);
+    if (nact == 0) return;                   // an emptied list
     const int v0 = blockIdx.x * SY_VERTS;
-    const int Ke = L.nexp, ke = m.exp_ld;
-    const int K4 = (Ke + 3) & ~3;
-    // basis rows of the workgroup's vertices, zero padded (k >= Ke, v >= V)
-    // (a fixed count of loads per thread, issued unconditionally from clamped indices and zeroed
-    // by a select, so that they are in flight together)
-    constexpr int NST = 3 * SY_KMAX * 16 / 256;
-    float av[NST];
-#pragma unroll
-    for (int q = 0; q < NST; ++q) {
-        const int e = tid + 256 * q;
-        const int k = e % K4, i = (e / K4) & 15, c = (e / K4) >> 4;
-        const int v = v0 + i;
-        av[q] = m.exp_basis[(size_t)(3 * min(v, m.V - 1) + min(c, 2)) * ke + min(k, Ke - 1)];
-    }
-#pragma unroll
-    for (int q = 0; q < NST; ++q) {
-        const int e = tid + 256 * q;
-        if (e < 3 * K4 * 16) {
-            const int k = e % K4, i = (e / K4) & 15, c = (e / K4) >> 4;
-            const int v = v0 + i;
-            sA[c][k][i] = (k < Ke && v < m.V) ? (double)av[q] : 0.0;
-        }
-    }
-    // the base shape: the model's mean, or a given FP64 shape (the identity stage's shared identity)
+    const int j = lane & 15, kq = lane >> 4;
+    // the base shape: the model's mean, or a given FP64 shape that holds the identity already (the
+    // identity stage's shared identity)
     for (int e = tid; e < SY_VERTS * 3; e += blockDim.x) {
         const int v = v0 + e / 3;
         smean[e] = v < m.V ? (mean64 ? mean64[3 * v0 + e] : (double)m.mean[3 * v0 + e]) : 0.0;
     }
-    __syncthreads();
-    const int nact = fl_count(act, n);
-    const int ngroups = Ke > 0 ? (nact + 15) >> 4 : 0;   // Ke == 0 is handled by k_synth_gemv
-    const int j = lane & 15, kq = lane >> 4;
-    for (int g = wave; g < ngroups; g += 4) {
+    if (ONE && nact <= 16) {
+        const bool live = j < nact;
+        const int f = fl_frame(act, live ? j : 0);
+        const FrameCam cam{frames[f].phix, frames[f].phiy, frames[f].cx, frames[f].cy};
+        double R[12];
+#pragma unroll
+        for (int q = 0; q < 12; ++q) R[q] = rt[(size_t)f * 12 + q];
+        double (*sacc)[64] = (double (*)[64]) & sA[0][0][0];   // [coordinate * 4 + element][lane]
+        if (wave < 3) {
+            const float* row = m.exp_basis + (3 * (size_t)min(v0 + j, m.V - 1) + wave) * m.exp_ld;
+            float4 A[SY_KMAX / 16];
+#pragma unroll
+            for (int t = 0; t < SY_KMAX / 16; ++t) {
+                A[t] = *(const float4*)(row + min(16 * t + 4 * kq, m.exp_ld - 4));
+                if (16 * t >= m.exp_ld) A[t] = make_float4(0.f, 0.f, 0.f, 0.f);
+            }
+            float bv[SY_KMAX / 4];
+            synth_coefs(theta + (size_t)f * L.K + L.off_exp, kq, L.nexp, bv);
+            v4d acc = (v4d){0, 0, 0, 0};
+#pragma unroll
+            for (int t = 0; t < SY_KMAX / 16; ++t) {
+                if (16 * t >= L.nexp) continue;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const float av = q == 0 ? A[t].x : q == 1 ? A[t].y : q == 2 ? A[t].z : A[t].w;
+                    acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)av, (double)bv[4 * t + q], acc, 0, 0, 0);
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) sacc[4 * wave + r][lane] = acc[r];
+        }
+        __syncthreads();
+        const int vl = kq + 4 * wave, v = v0 + vl;
+        if (live && v < m.V) {
+            double p[3];
+#pragma unroll
+            for (int a = 0; a < 3; ++a) p[a] = smean[3 * vl + a] + sacc[4 * a + wave][lane];
+            store_vertex(cam, R, p, (size_t)f * m.V + v, P0, P, vproj);
+        }
+        return;
+    }
+    const int nid = mean64 ? 0 : L.nid;
+    const int idc = (nid + SY_KMAX - 1) / SY_KMAX;                     // identity chunks
+    const int nch = ONE ? 1 : idc + (L.nexp + SY_KMAX - 1) / SY_KMAX;
+    if (nch == 0) __syncthreads();
+    const int ngroups = (nact + 15) >> 4;
+    for (int g0 = 0; g0 < ngroups; g0 += 4) {
+        const int g = g0 + wave;
         const int c = 16 * g + j;
         const bool live = c < nact;
         const int f = fl_frame(act, live ? c : 0);
-        // this lane's B entries: coefficient kq + 4 q of its frame, every load issued
-        // unconditionally (clamped to a valid column) so the batch has no branches.  Nothing
-        // needs zeroing: the A rows past K_exp are zero, and an output column depends on its
-        // own frame's B column only, so lanes without a live frame just skip the epilogue.
-        const float* tb = theta + (size_t)f * L.K + L.off_exp;
-        float bv[SY_KMAX / 4];
+        // the epilogue's camera and pose, loaded before the products that hide their latency
+        const FrameCam cam{frames[f].phix, frames[f].phiy, frames[f].cx, frames[f].cy};
+        double R[12];
 #pragma unroll
-        for (int q = 0; q < SY_KMAX / 4; ++q) bv[q] = tb[min(kq + 4 * q, Ke - 1)];
+        for (int q = 0; q < 12; ++q) R[q] = rt[(size_t)f * 12 + q];
         v4d acc[3];
 #pragma unroll
         for (int a = 0; a < 3; ++a) acc[a] = (v4d){0, 0, 0, 0};
+        for (int ch = 0; ch < nch; ++ch) {
+            const bool id = !ONE && ch < idc;
+            const int k0 = ONE ? 0 : SY_KMAX * (id ? ch : ch - idc);   // first column of the chunk in its basis
+            const int kc = ONE ? L.nexp : min(SY_KMAX, (id ? nid : L.nexp) - k0);
+            if (!ONE || g0 == 0) {
+                // basis rows of the workgroup's vertices: item = (coordinate, four columns, vertex),
+                // the 16 vertices on neighbouring lanes so that the LDS stores are contiguous; a
+                // fixed count of 16-byte loads per thread from clamped addresses, zeroed by a select,
+                // so that they are in flight together.  The rows are zero past their last column
+                // up to ld, a multiple of 16.
+                const float* basis = id ? m.id_basis : m.exp_basis;
+                const int ld = id ? m.id_ld : m.exp_ld;
+                constexpr int NC4 = SY_KMAX / 4, NIT = 3 * NC4 * 16, NST = (NIT + 255) / 256;
+                float4 av[NST];
 #pragma unroll
-        for (int q = 0; q < SY_KMAX / 4; ++q) {
-            if (4 * q < K4) {
+                for (int q = 0; q < NST; ++q) {
+                    const int e = min(tid + 256 * q, NIT - 1);
+                    const int i = e & 15, c4 = (e >> 4) % NC4, a = (e >> 4) / NC4;
+                    av[q] = *(const float4*)(basis + (size_t)(3 * min(v0 + i, m.V - 1) + a) * ld +
+                                             min(k0 + 4 * c4, ld - 4));
+                }
+                if (!ONE) __syncthreads();             // the previous chunk is no longer read
+#pragma unroll
+                for (int q = 0; q < NST; ++q) {
+                    const int e = tid + 256 * q;
+                    if (e < NIT) {
+                        const int i = e & 15, c4 = (e >> 4) % NC4, a = (e >> 4) / NC4;
+                        const bool in = k0 + 4 * c4 < ld && v0 + i < m.V;
+                        sA[a][4 * c4 + 0][i] = in ? (double)av[q].x : 0.0;
+                        sA[a][4 * c4 + 1][i] = in ? (double)av[q].y : 0.0;
+                        sA[a][4 * c4 + 2][i] = in ? (double)av[q].z : 0.0;
+                        sA[a][4 * c4 + 3][i] = in ? (double)av[q].w : 0.0;
+                    }
+                }
+                __syncthreads();
+            }
+            if (g >= ngroups) continue;
+            float bv[SY_KMAX / 4];
+            synth_coefs(theta + (size_t)f * L.K + (id ? L.off_id : L.off_exp) + k0, kq, kc, bv);
+#pragma unroll
+            for (int q = 0; q < SY_KMAX / 4; ++q) {
+                if (16 * (q >> 2) >= kc) continue;
                 const double b = (double)bv[q];
 #pragma unroll
                 for (int a = 0; a < 3; ++a)
-                    acc[a] = __builtin_amdgcn_mfma_f64_16x16x4f64(sA[a][4 * q + kq][j], b, acc[a], 0, 0, 0);
+                    acc[a] = __builtin_amdgcn_mfma_f64_16x16x4f64(sA[a][16 * (q >> 2) + 4 * kq + (q & 3)][j], b, acc[a],
+                                                                  0, 0, 0);
             }
         }
-        if (live) {
-            const FrameGPU fr = frames[f];
-            double R[12];
-#pragma unroll
-            for (int q = 0; q < 12; ++q) R[q] = rt[(size_t)f * 12 + q];
+        if (g < ngroups && live) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int vl = kq + 4 * r, v = v0 + vl;
@@ -194,7 +237,7 @@ k_synth_tile(ModelGPU m, Layout L, const FrameGPU* __restrict__ frames, const fl
                     double p[3];
 #pragma unroll
                     for (int a = 0; a < 3; ++a) p[a] = smean[3 * vl + a] + acc[a][r];
-                    store_vertex(fr, R, R + 9, p, (size_t)f * m.V + v, P0, P, vproj);
+                    store_vertex(cam, R, p, (size_t)f * m.V + v, P0, P, vproj);
                 }
             }
         }
@@ -211,20 +254,33 @@ static int launch_frame_rt(const Layout& L, FrameList fl, const float* theta, do
     return TDI_OK;
 }
 
+// The vertices of the listed frames, from the model's mean or (mean64) a base shape that already
+// holds the identity, then their albedos when the albedo is fitted.
+static int synthesize(const ModelGPU& m, const Layout& L, const FrameGPU* frames, FrameList fl, const float* theta,
+                      double* rt, const double* mean64, double* P0, float* P, float4* vproj, hipStream_t s)
+{
+    const dim3 grid((m.V + SY_VERTS - 1) / SY_VERTS);
+    if ((mean64 || L.nid == 0) && L.nexp > 0 && L.nexp <= SY_KMAX)
+        hipLaunchKernelGGL(k_synth_tile<true>, grid, dim3(256), 0, s, m, L, frames, theta, fl.act, fl.n, rt, mean64, P0,
+                           P, vproj);
+    else
+        hipLaunchKernelGGL(k_synth_tile<false>, grid, dim3(256), 0, s, m, L, frames, theta, fl.act, fl.n, rt, mean64, P0,
+                           P, vproj);
+    TDI_HIP(hipGetLastError());
+    if (m.alb && L.ntex) return launch_albedo(m, L, fl, theta, const_cast<float*>(m.alb), s);
+    return TDI_OK;
+}
+
 int launch_synthesize(const ModelGPU& m, const Layout& L, const FrameGPU* frames, FrameList fl, const float* theta,
                       double* rt, double* P0, float* P, float4* vproj, hipStream_t s)
 {
-    if (L.K > MAXK_LDS) {
-        set_error("synthesize: K=%d exceeds %d", L.K, MAXK_LDS);
+    if (L.K > MAX_UNKNOWNS) {
+        set_error("synthesize: K=%d exceeds %d", L.K, MAX_UNKNOWNS);
         return TDI_ERR_ARG;
     }
     int rc = launch_frame_rt(L, fl, theta, rt, s);
     if (rc) return rc;
-    dim3 grid((m.V + 255) / 256, grid_frames(fl.n, 64));
-    hipLaunchKernelGGL(k_synth_gemv, grid, dim3(256), 0, s, m, L, frames, theta, fl.act, fl.n, rt, P0, P, vproj);
-    TDI_HIP(hipGetLastError());
-    if (m.alb && L.ntex) return launch_albedo(m, L, fl, theta, const_cast<float*>(m.alb), s);
-    return TDI_OK;
+    return synthesize(m, L, frames, fl, theta, rt, nullptr, P0, P, vproj, s);
 }
 
 namespace {
@@ -284,21 +340,6 @@ int launch_albedo(const ModelGPU& m, const Layout& L, FrameList fl, const float*
     return TDI_OK;
 }
 
-int launch_synthesize_gemm(const ModelGPU& m, const Layout& L, const FrameGPU* frames, FrameList fl,
-                           const float* theta, double* rt, double* P0, float* P, float4* vproj, hipStream_t s)
-{
-    if (L.nid) return launch_synthesize(m, L, frames, fl, theta, rt, P0, P, vproj, s);
-    int rc = launch_frame_rt(L, fl, theta, rt, s);
-    if (rc) return rc;
-    if (L.nexp > SY_KMAX || L.nexp == 0) return launch_synthesize(m, L, frames, fl, theta, rt, P0, P, vproj, s);
-    const dim3 grid((m.V + SY_VERTS - 1) / SY_VERTS);
-    hipLaunchKernelGGL(k_synth_tile, grid, dim3(256), 0, s, m, L, frames, theta, fl.act, fl.n, rt,
-                       (const double*)nullptr, P0, P, vproj);
-    TDI_HIP(hipGetLastError());
-    if (m.alb && L.ntex) return launch_albedo(m, L, fl, theta, const_cast<float*>(m.alb), s);
-    return TDI_OK;
-}
-
 namespace {
 
 // mean + identity basis x alpha in FP64 for every vertex, alpha of the first listed frame (the
@@ -329,16 +370,12 @@ int launch_synthesize_shared_id(const ModelGPU& m, const Layout& L, const FrameG
                                 const float* theta, double* rt, double* P0, float* P, float4* vproj, double* idshape,
                                 hipStream_t s)
 {
-    if (L.nexp == 0 || L.nexp > SY_KMAX || L.nid > MAXK_LDS) return launch_synthesize(m, L, frames, fl, theta, rt, P0, P, vproj, s);
+    if (L.nid > MAXK_LDS) return launch_synthesize(m, L, frames, fl, theta, rt, P0, P, vproj, s);
     int rc = launch_frame_rt(L, fl, theta, rt, s);
     if (rc) return rc;
     hipLaunchKernelGGL(k_id_shape, dim3((m.V + 255) / 256), dim3(256), 0, s, m, L, fl.act, fl.n, theta, idshape);
-    const dim3 grid((m.V + SY_VERTS - 1) / SY_VERTS);
-    hipLaunchKernelGGL(k_synth_tile, grid, dim3(256), 0, s, m, L, frames, theta, fl.act, fl.n, rt,
-                       (const double*)idshape, P0, P, vproj);
     TDI_HIP(hipGetLastError());
-    if (m.alb && L.ntex) return launch_albedo(m, L, fl, theta, const_cast<float*>(m.alb), s);
-    return TDI_OK;
+    return synthesize(m, L, frames, fl, theta, rt, idshape, P0, P, vproj, s);
 }
 
 } // namespace tdi

@@ -121,7 +121,8 @@ typedef struct tdi_fit_options {
     float blur_sigma;           /* KERNEL_SIGMA config key (config.cu:53; cfg files use 0.75)      */
     float ref_face_size;        /* REF_FACE_SIZE; "face too large" if > 2x (renderer.cu:845-857), 0 = off */
     int32_t mixed_flags;        /* batched path arithmetic (no reference counterpart), bit set:
-                                   1 = FP64-MFMA basis GEMM over frames, 2 = BF16 hi/lo MFMA J^T J,
+                                   1 = FP64-MFMA basis GEMM over frames (every synthesis is
+                                   one, with or without the bit), 2 = BF16 hi/lo MFMA J^T J,
                                    4 = FP32 Cholesky + FP64 refinement, 8 = J^T r from the BF16
                                    MFMA tiles (else FP32; with 8 a NaN observed pixel contributes
                                    zero instead of stopping the frame on a NaN direction),
@@ -354,8 +355,7 @@ int tdi_landmark_joint_terms(tdi_batch* b, const float* theta, int32_t k_id, int
                              const double* z, double tau, double* H, double* g, double* obj);
 
 /* The integer buffers the fit itself computes, for bit-for-bit checks: a render at theta through
- * the same launches as a fit with these mixed_flags (TDI_MIXED_SYNTH_MFMA selects the FP64-MFMA
- * synthesis the batched fit uses), then
+ * the same launches as a fit (mixed_flags: none of the bits changes these buffers), then
  *   vproj [n][V][4] the projected vertices (x, y in image pixels, camera z, 0) the rasteriser
  *   reads -- view_transform_3d_pts_and_render_2d (funcs.cu:440-452);
  *   nbr   [sum W*H][4] per rendered pixel, in the frame's crop order from its crop offset, the
