@@ -176,64 +176,217 @@ __global__ void __launch_bounds__(256) k_barrier(ModelGPU m, Layout L, const Fra
 }
 
 // ------------------------------------------------------------------ batched Cholesky
-__device__ __forceinline__ int pk(int i, int j) { return i * (i + 1) / 2 + j; }   // i >= j
+// One workgroup of four wavefronts per matrix, the lower triangle in LDS as 16 x 16 blocks (padded
+// with the identity to a multiple of 16).  What bounds it is the chain of K dependent columns, so
+// the steps on that chain stay inside one wavefront, in registers, with no barrier:
+//   panel     wavefront 0 holds the panel's rows (lane l: rows l and l + 64 below the diagonal
+//             block's first), 16 columns each; pivots and column entries pass by lane reads;
+//   trailing  A22 -= L21 L21^T on the MFMA of the type (FP32 or FP64, four 16 x 16 x 4 steps per
+//             block), the blocks dealt to the four wavefronts; two barriers per panel;
+//   solves    wavefront 0, lane l holding entries l and l + 64, right-looking.
+// A barrier pair and an LDS round trip per column (what it replaces) took 283 us for one matrix of
+// 94 unknowns (mode 1 with the FP64 fallback) and 552 us for 448; this takes 66 and 132 us.
+constexpr int CMAXK = 112;
+constexpr int CHB = 16;                          // block edge
+constexpr int CHP = CHB + 1;                     // LDS row stride
+constexpr int CHN = CHB * CHP;                   // LDS elements per block
+constexpr int CHT = CMAXK / CHB;                 // most blocks per side
 
-template <typename T>
-__device__ bool chol_packed(T* A, int K, T* sflag)
+__device__ __forceinline__ int ch_block(int I, int J) { return (I * (I + 1) / 2 + J) * CHN; }   // I >= J
+
+__device__ __forceinline__ float lane_read(float v, int j)
 {
-    const int tid = threadIdx.x, nt = blockDim.x;
-    for (int j = 0; j < K; ++j) {
-        if (tid == 0) {
-            const T d = A[pk(j, j)];
-            if (!(d > T(0))) sflag[0] = T(1);
-            A[pk(j, j)] = sqrt(d);
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), j));
+}
+__device__ __forceinline__ double lane_read(double v, int j)
+{
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), j),
+                            __builtin_amdgcn_readlane(__double2loint(v), j));
+}
+
+typedef float ch_v4f __attribute__((ext_vector_type(4)));
+typedef double ch_v4d __attribute__((ext_vector_type(4)));
+// accumulator element r of lane l: row 4 (l / 16) + r for FP32, l / 16 + 4 r for FP64; column l % 16
+__device__ __forceinline__ ch_v4f ch_mma(float a, float b, ch_v4f c)
+{
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ ch_v4d ch_mma(double a, double b, ch_v4d c)
+{
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ int ch_row(float, int lane, int r) { return 4 * (lane >> 4) + r; }
+__device__ __forceinline__ int ch_row(double, int lane, int r) { return (lane >> 4) + 4 * r; }
+template <typename T> struct ChVec;
+template <> struct ChVec<float> { typedef ch_v4f type; };
+template <> struct ChVec<double> { typedef ch_v4d type; };
+
+// The lower blocks of H into LDS, scaled by sdinv on both sides when given; every load of the
+// thread (one entry of each block) is issued before the stores.
+template <typename T, typename TH>
+__device__ __forceinline__ void ch_load(T* A, const TH* __restrict__ Hf, int K, int nT, const float* sdinv)
+{
+    const int r = threadIdx.x >> 4, c = threadIdx.x & 15;
+    TH v[CHT * (CHT + 1) / 2];
+#pragma unroll
+    for (int I = 0; I < CHT; ++I)
+#pragma unroll
+        for (int J = 0; J <= I; ++J) {
+            if (I >= nT) continue;
+            v[I * (I + 1) / 2 + J] = Hf[(size_t)min(CHB * I + r, K - 1) * K + min(CHB * J + c, K - 1)];
+        }
+#pragma unroll
+    for (int I = 0; I < CHT; ++I)
+#pragma unroll
+        for (int J = 0; J <= I; ++J) {
+            if (I >= nT) continue;
+            const int i = CHB * I + r, j = CHB * J + c;
+            T x = (T)v[I * (I + 1) / 2 + J];
+            if (sdinv) x = x * (T)sdinv[i] * (T)sdinv[j];
+            if (i >= K || j >= K) x = i == j ? T(1) : T(0);
+            A[ch_block(I, J) + r * CHP + c] = x;
+        }
+}
+
+// s = sqrt(d) and 1 / s of a pivot, on the factorisation's critical path: the hardware's reciprocal
+// square root, with Newton steps to the type's last place in FP64 (its estimate holds about 24 bits:
+// two steps) and one correction of the root.
+__device__ __forceinline__ void ch_root(float d, float& s, float& inv)
+{
+    inv = __builtin_amdgcn_rsqf(d);
+    s = d * inv;
+    s = fmaf(0.5f * inv, fmaf(-s, s, d), s);
+}
+__device__ __forceinline__ void ch_root(double d, double& s, double& inv)
+{
+    double y = __builtin_amdgcn_rsq(d);
+    y = fma(0.5 * y, fma(-d * y, y, 1.0), y);
+    y = fma(0.5 * y, fma(-d * y, y, 1.0), y);
+    inv = y;
+    s = d * y;
+    s = fma(0.5 * y, fma(-s, s, d), s);
+}
+
+// A = L L^T in place; false (for every thread) at a pivot that is not positive.
+template <typename T>
+__device__ __forceinline__ bool ch_factor(T* A, int nT, int* sflag)
+{
+    typedef typename ChVec<T>::type V4;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l16 = lane & 15, kq = lane >> 4;
+    for (int p = 0; p < nT; ++p) {
+        if (wave == 0) {
+            const int rows = CHB * (nT - p);          // rows of the panel, the diagonal block first
+            const bool in0 = lane < rows, in1 = lane + 64 < rows;
+            T* r0 = A + ch_block(p + (in0 ? lane >> 4 : 0), p) + l16 * CHP;
+            T* r1 = A + ch_block(p + (in1 ? (lane + 64) >> 4 : 0), p) + l16 * CHP;
+            T x0[CHB], x1[CHB];
+#pragma unroll
+            for (int k = 0; k < CHB; ++k) {
+                x0[k] = r0[k];
+                x1[k] = r1[k];
+            }
+            bool bad = false;
+#pragma unroll
+            for (int k = 0; k < CHB; ++k) {
+                const T d = lane_read(x0[k], k);
+                bad = bad || !(d > T(0));
+                T s, inv;
+                ch_root(d, s, inv);
+                // rows above the pivot keep their entry (the block's unused upper triangle)
+                x0[k] = lane == k ? s : lane > k ? x0[k] * inv : x0[k];
+                x1[k] = x1[k] * inv;
+#pragma unroll
+                for (int j = k + 1; j < CHB; ++j) {
+                    const T ljk = lane_read(x0[k], j);
+                    x0[j] = fma(-x0[k], ljk, x0[j]);
+                    x1[j] = fma(-x1[k], ljk, x1[j]);
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < CHB; ++k) {
+                if (in0) r0[k] = x0[k];
+                if (in1) r1[k] = x1[k];
+            }
+            if (bad && lane == 0) *sflag = 1;
         }
         __syncthreads();
-        if (sflag[0] != T(0)) return false;
-        const T djj = A[pk(j, j)];
-        for (int i = j + 1 + tid; i < K; i += nt) A[pk(i, j)] /= djj;
-        __syncthreads();
-        const int m = K - j - 1;
-        const int npairs = m * (m + 1) / 2;
-        for (int e = tid; e < npairs; e += nt) {
-            // e -> (ii, kk) with 0 <= kk <= ii < m
-            int ii = (int)((sqrtf(8.f * e + 1.f) - 1.f) * 0.5f);
-            while ((ii + 1) * (ii + 2) / 2 <= e) ++ii;
-            while (ii * (ii + 1) / 2 > e) --ii;
-            const int kk = e - ii * (ii + 1) / 2;
-            const int i = j + 1 + ii, k = j + 1 + kk;
-            A[pk(i, k)] -= A[pk(i, j)] * A[pk(k, j)];
-        }
+        if (*sflag) return false;
+        int t = 0;
+        for (int I = p + 1; I < nT; ++I)
+            for (int J = p + 1; J <= I; ++J, ++t) {
+                if ((t & 3) != wave) continue;
+                T* C = A + ch_block(I, J) + l16;
+                const T* a = A + ch_block(I, p) + l16 * CHP + kq;
+                const T* b = A + ch_block(J, p) + l16 * CHP + kq;
+                V4 acc;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[r] = C[ch_row(T(0), lane, r) * CHP];
+#pragma unroll
+                for (int k = 0; k < CHB / 4; ++k) acc = ch_mma(-a[4 * k], b[4 * k], acc);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) C[ch_row(T(0), lane, r) * CHP] = acc[r];
+            }
         __syncthreads();
     }
     return true;
 }
 
-// Solve L L^T x = b in place (x overwrites b), b in shared memory.
-template <typename T>
-__device__ void chol_solve_packed(const T* A, int K, T* b)
+// L L^T x = b on one wavefront, in TB arithmetic: lane l holds entries l (b0) and l + 64 (b1).
+template <typename T, typename TB>
+__device__ __forceinline__ void ch_solve(const T* A, int nT, TB& b0, TB& b1)
 {
-    const int tid = threadIdx.x, nt = blockDim.x;
-    for (int i = 0; i < K; ++i) {
-        if (tid == 0) b[i] /= A[pk(i, i)];
-        __syncthreads();
-        const T yi = b[i];
-        for (int k = i + 1 + tid; k < K; k += nt) b[k] -= A[pk(k, i)] * yi;
-        __syncthreads();
+    const int lane = threadIdx.x & 63, l16 = lane & 15;
+    const int I0 = min(lane >> 4, nT - 1), I1 = min((lane + 64) >> 4, nT - 1);
+    const TB q0 = TB(1) / (TB)A[ch_block(I0, I0) + l16 * CHP + l16];
+    const TB q1 = TB(1) / (TB)A[ch_block(I1, I1) + l16 * CHP + l16];
+    for (int J = 0; J < nT; ++J) {
+        // column j of the rows below it (blocks above the diagonal are never used: masked)
+        const T* c0 = A + ch_block(max(I0, J), J) + l16 * CHP;
+        const T* c1 = A + ch_block(max(I1, J), J) + l16 * CHP;
+        T l0[CHB], l1[CHB];
+#pragma unroll
+        for (int c = 0; c < CHB; ++c) {
+            l0[c] = c0[c];
+            l1[c] = c1[c];
+        }
+#pragma unroll
+        for (int c = 0; c < CHB; ++c) {
+            const int j = CHB * J + c;
+            const TB y = j < 64 ? lane_read(b0 * q0, j & 63) : lane_read(b1 * q1, j & 63);
+            b0 = lane == j ? y : lane > j ? fma(-(TB)l0[c], y, b0) : b0;
+            b1 = lane + 64 == j ? y : lane + 64 > j ? fma(-(TB)l1[c], y, b1) : b1;
+        }
     }
-    for (int i = K - 1; i >= 0; --i) {
-        if (tid == 0) b[i] /= A[pk(i, i)];
-        __syncthreads();
-        const T xi = b[i];
-        for (int k = tid; k < i; k += nt) b[k] -= A[pk(i, k)] * xi;
-        __syncthreads();
+    for (int J = nT - 1; J >= 0; --J) {
+        // row j, of the entries before it
+        const T* c0 = A + ch_block(J, min(I0, J)) + l16;
+        const T* c1 = A + ch_block(J, min(I1, J)) + l16;
+        T l0[CHB], l1[CHB];
+#pragma unroll
+        for (int c = 0; c < CHB; ++c) {
+            l0[c] = c0[c * CHP];
+            l1[c] = c1[c * CHP];
+        }
+#pragma unroll
+        for (int c = CHB - 1; c >= 0; --c) {
+            const int j = CHB * J + c;
+            const TB x = j < 64 ? lane_read(b0 * q0, j & 63) : lane_read(b1 * q1, j & 63);
+            b0 = lane == j ? x : lane < j ? fma(-(TB)l0[c], x, b0) : b0;
+            b1 = lane + 64 == j ? x : lane + 64 < j ? fma(-(TB)l1[c], x, b1) : b1;
+        }
     }
 }
 
-constexpr int CMAXK = 112;
+__device__ __forceinline__ double ch_wave_sum(double v)
+{
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    return v;
+}
 
 // mode 0: FP64 factorisation and solve.  mode 1: FP32 factorisation of the equilibrated
-// matrix and solve, then one FP64 residual-refinement step (r = -g - H x computed in FP64,
+// matrix D^-1/2 H D^-1/2 (D = diag H, which removes the scale spread between pose and coefficient
+// columns) and solve, then one FP64 residual-refinement step (r = -g - H x computed in FP64,
 // correction solved with the FP32 factor); when the FP32 factorisation breaks down or the
 // correction exceeds 1e-3 of the solution (an ill-conditioned frame), the FP64 factorisation.
 template <typename TH>
@@ -244,113 +397,101 @@ __global__ void __launch_bounds__(256) k_cholesky(int K, const TH* __restrict__ 
     const int f = blockIdx.x;
     if (mask && !mask[f]) return;
     extern __shared__ double dsm[];
-    __shared__ double sflag[1];
-    __shared__ double sb[CMAXK];
-    __shared__ float sbf[CMAXK];
-    __shared__ float sflagf[1];
+    __shared__ int sflag;
+    __shared__ double sb[CMAXK];                 // the residual, then the verdict
+    __shared__ float sx[CMAXK];
     const TH* Hf = H + (size_t)f * K * K;
     const float* gf = g + (size_t)f * K;
-    const int tid = threadIdx.x;
-    const int np = K * (K + 1) / 2;
-    if (tid == 0) { sflag[0] = 0.0; sflagf[0] = 0.f; }
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int nT = (K + CHB - 1) / CHB;
+    const bool in0 = lane < K, in1 = lane + 64 < K;
+    if (tid == 0) sflag = 0;
     if (mode != 0) {
-        // FP32 factorisation of the equilibrated matrix D^-1/2 H D^-1/2 (D = diag H), which
-        // removes the scale spread between pose and coefficient columns, then one FP64
-        // residual-refinement step on the original system.  A frame whose scaled matrix is
-        // not positive definite in FP32 falls through to the FP64 factorisation below.
         float* A = (float*)dsm;
         __shared__ float sdinv[CMAXK];
-        for (int i = tid; i < K; i += blockDim.x) {
-            const float d = (float)Hf[(size_t)i * K + i];
+        for (int i = tid; i < CMAXK; i += blockDim.x) {
+            const float d = i < K ? (float)Hf[(size_t)i * K + i] : 1.f;
             sdinv[i] = d > 0.f ? rsqrtf(d) : 1.f;
         }
         __syncthreads();
-        for (int e = tid; e < np; e += blockDim.x) {
-            int i = (int)((sqrtf(8.f * e + 1.f) - 1.f) * 0.5f);
-            while ((i + 1) * (i + 2) / 2 <= e) ++i;
-            while (i * (i + 1) / 2 > e) --i;
-            const int j = e - i * (i + 1) / 2;
-            A[e] = (float)Hf[(size_t)i * K + j] * sdinv[i] * sdinv[j];
-        }
-        for (int i = tid; i < K; i += blockDim.x) sbf[i] = -gf[i] * sdinv[i];
+        ch_load<float, TH>(A, Hf, K, nT, sdinv);
         __syncthreads();
-        if (chol_packed<float>(A, K, sflagf)) {
-            chol_solve_packed<float>(A, K, sbf);
-            // x0 = D^-1/2 y
-            for (int i = tid; i < K; i += blockDim.x) sbf[i] *= sdinv[i];
-            __syncthreads();
-            // refinement: r = -g - H x0 in FP64, correction solved with the same scaled factor
-            for (int i = tid; i < K; i += blockDim.x) {
-                double r = -(double)gf[i];
-                for (int k = 0; k < K; ++k) r -= (double)Hf[(size_t)i * K + k] * (double)sbf[k];
-                sb[i] = r * (double)sdinv[i];
+        if (ch_factor<float>(A, nT, &sflag)) {
+            float x0 = 0.f, x1 = 0.f;            // wavefront 0: the FP32 solution
+            if (wave == 0) {
+                x0 = in0 ? -gf[lane] * sdinv[lane] : 0.f;
+                x1 = in1 ? -gf[lane + 64] * sdinv[lane + 64] : 0.f;
+                ch_solve<float, float>(A, nT, x0, x1);
+                x0 = in0 ? x0 * sdinv[lane] : 0.f;     // x = D^-1/2 y
+                x1 = in1 ? x1 * sdinv[lane + 64] : 0.f;
+                if (in0) sx[lane] = x0;
+                if (in1) sx[lane + 64] = x1;
             }
             __syncthreads();
-            for (int i = 0; i < K; ++i) {
-                if (tid == 0) sb[i] /= (double)A[pk(i, i)];
-                __syncthreads();
-                const double yi = sb[i];
-                for (int k = i + 1 + tid; k < K; k += blockDim.x) sb[k] -= (double)A[pk(k, i)] * yi;
-                __syncthreads();
+            // residual -g - H x in FP64, eight lanes per row
+            for (int i = tid >> 3; i < ((K + 31) & ~31); i += 32) {
+                const TH* row = Hf + (size_t)min(i, K - 1) * K;
+                double r = 0.0;
+                for (int k = tid & 7; k < K; k += 8) r = fma(-(double)row[k], (double)sx[k], r);
+                r += __shfl_xor(r, 1, 64);
+                r += __shfl_xor(r, 2, 64);
+                r += __shfl_xor(r, 4, 64);
+                if ((tid & 7) == 0 && i < K) sb[i] = (r - (double)gf[i]) * (double)sdinv[i];
             }
-            for (int i = K - 1; i >= 0; --i) {
-                if (tid == 0) sb[i] /= (double)A[pk(i, i)];
-                __syncthreads();
-                const double xi = sb[i];
-                for (int k = tid; k < i; k += blockDim.x) sb[k] -= (double)A[pk(i, k)] * xi;
-                __syncthreads();
-            }
-            // the correction measures the FP32 solution's error (about cond * 2^-24 of it); past
-            // 1e-3 of the solution one refinement step leaves more than ~1e-6, and the FP64
-            // factorisation below takes over
-            if (tid == 0) {
-                double cn = 0.0, xn = 0.0;
-                for (int i = 0; i < K; ++i) {
-                    const double c = sb[i] * (double)sdinv[i];
-                    cn += c * c;
-                    xn += (double)sbf[i] * (double)sbf[i];
+            __syncthreads();
+            if (wave == 0) {
+                double c0 = in0 ? sb[lane] : 0.0, c1 = in1 ? sb[lane + 64] : 0.0;
+                ch_solve<float, double>(A, nT, c0, c1);
+                c0 = in0 ? c0 * (double)sdinv[lane] : 0.0;
+                c1 = in1 ? c1 * (double)sdinv[lane + 64] : 0.0;
+                // the correction measures the FP32 solution's error (about cond * 2^-24 of it); past
+                // 1e-3 of the solution one refinement step leaves more than ~1e-6, and the FP64
+                // factorisation below takes over
+                const double cn = ch_wave_sum(c0 * c0 + c1 * c1);
+                const double xn = ch_wave_sum((double)x0 * x0 + (double)x1 * x1);
+                const bool good = cn <= 1e-6 * xn;
+                if (good) {
+                    if (in0) delta[(size_t)f * K + lane] = (float)((double)x0 + c0);
+                    if (in1) delta[(size_t)f * K + lane + 64] = (float)((double)x1 + c1);
+                    if (lane == 0) status[f] = TDI_OK;
                 }
-                sflag[0] = (cn <= 1e-6 * xn) ? 0.0 : 1.0;
+                if (lane == 0) sflag = good ? 2 : 0;
             }
-            __syncthreads();
-            if (sflag[0] == 0.0) {
-                for (int i = tid; i < K; i += blockDim.x)
-                    delta[(size_t)f * K + i] = (float)((double)sbf[i] + sb[i] * (double)sdinv[i]);
-                if (tid == 0) status[f] = TDI_OK;
-                return;
-            }
-            __syncthreads();
-            if (tid == 0) sflag[0] = 0.0;
+        } else if (tid == 0) {
+            sflag = 0;                            // read by every thread before (ch_factor's barrier)
         }
+        __syncthreads();
+        if (sflag == 2) return;
         __syncthreads();
     }
     // FP64 factorisation and solve (mode 0, and the fallback of mode 1)
     double* A = dsm;
-    for (int e = tid; e < np; e += blockDim.x) {
-        int i = (int)((sqrtf(8.f * e + 1.f) - 1.f) * 0.5f);
-        while ((i + 1) * (i + 2) / 2 <= e) ++i;
-        while (i * (i + 1) / 2 > e) --i;
-        const int j = e - i * (i + 1) / 2;
-        A[e] = (double)Hf[(size_t)i * K + j];
-    }
-    for (int i = tid; i < K; i += blockDim.x) sb[i] = -(double)gf[i];
+    ch_load<double, TH>(A, Hf, K, nT, nullptr);
     __syncthreads();
-    if (!chol_packed<double>(A, K, sflag)) {
+    if (!ch_factor<double>(A, nT, &sflag)) {
         if (tid == 0) status[f] = TDI_NOT_PD;
         return;
     }
-    chol_solve_packed<double>(A, K, sb);
-    for (int i = tid; i < K; i += blockDim.x) delta[(size_t)f * K + i] = (float)sb[i];
-    if (tid == 0) status[f] = TDI_OK;
+    if (wave == 0) {
+        double x0 = in0 ? -(double)gf[lane] : 0.0, x1 = in1 ? -(double)gf[lane + 64] : 0.0;
+        ch_solve<double, double>(A, nT, x0, x1);
+        if (in0) delta[(size_t)f * K + lane] = (float)x0;
+        if (in1) delta[(size_t)f * K + lane + 64] = (float)x1;
+        if (lane == 0) status[f] = TDI_OK;
+    }
 }
 
 // ------------------------------------------------------------------ line-search state machine
-__global__ void k_ls_init(int n, int K, FitState* __restrict__ st, const int* __restrict__ chol_status,
-                          const float* __restrict__ delta, const float* __restrict__ g, const double* __restrict__ obj,
-                          int* __restrict__ searching)
+// One wavefront per frame (delta . g is a sum over its lanes in a fixed order).
+__global__ void __launch_bounds__(64) k_ls_init(int n, int K, FitState* __restrict__ st, const int* __restrict__ chol_status,
+                                                 const float* __restrict__ delta, const float* __restrict__ g,
+                                                 const double* __restrict__ obj, int* __restrict__ searching)
 {
-    const int f = blockIdx.x * blockDim.x + threadIdx.x;
-    if (f >= n) return;
+    const int f = blockIdx.x, lane = threadIdx.x;
+    double dg = 0.0;
+    for (int k = lane; k < K; k += 64) dg += (double)delta[(size_t)f * K + k] * (double)g[(size_t)f * K + k];
+    dg = ch_wave_sum(dg);
+    if (lane != 0) return;
     FitState s = st[f];
     searching[f] = 0;
     if (!s.active) return;
@@ -365,8 +506,6 @@ __global__ void k_ls_init(int n, int K, FitState* __restrict__ st, const int* __
         s.stop |= TDI_STOP_NAN;
         s.status = TDI_NAN;
     } else {
-        double dg = 0.0;
-        for (int k = 0; k < K; ++k) dg += (double)delta[(size_t)f * K + k] * (double)g[(size_t)f * K + k];
         s.dg = (float)dg;
         s.obj0 = obj[f];
         s.t = 1.f;
@@ -713,7 +852,8 @@ static int launch_cholesky_t(int n, int K, const TH* H, const float* g, float* d
         set_error("cholesky: K=%d > %d", K, CMAXK);
         return TDI_ERR_ARG;
     }
-    const size_t lds = (size_t)K * (K + 1) / 2 * sizeof(double);   // FP64 fallback of mode 1 included
+    const int nT = (K + CHB - 1) / CHB;
+    const size_t lds = (size_t)nT * (nT + 1) / 2 * CHN * sizeof(double);   // FP64 fallback of mode 1 included
     hipLaunchKernelGGL(k_cholesky<TH>, dim3(n), dim3(256), lds, s, K, H, g, delta, status, mask, mode);
     TDI_HIP(hipGetLastError());
     return TDI_OK;
@@ -736,7 +876,7 @@ int launch_cholesky(int n, int K, const double* H, const float* g, float* delta,
 int launch_ls_init(int n, int K, FitState* st, const int* chol_status, const float* delta, const float* g,
                    const double* obj, int* searching, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_ls_init, dim3((n + 255) / 256), dim3(256), 0, s, n, K, st, chol_status, delta, g, obj,
+    hipLaunchKernelGGL(k_ls_init, dim3(n), dim3(64), 0, s, n, K, st, chol_status, delta, g, obj,
                        searching);
     TDI_HIP(hipGetLastError());
     return TDI_OK;
