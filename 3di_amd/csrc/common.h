@@ -265,9 +265,8 @@ __device__ __forceinline__ float4 project_vertex(const FrameCam& cam, const doub
 {
 #pragma unroll
     for (int a = 0; a < 3; ++a) q[a] = rt[a] * p[0] + rt[3 + a] * p[1] + rt[6 + a] * p[2] + rt[9 + a];
-    const double iz = 1.0 / q[2];          // one FP64 division per vertex; x and y stay within 2 FP64 ulp
-    return make_float4((float)((double)cam.phix * q[0] * iz + (double)cam.cx),
-                       (float)((double)cam.phiy * q[1] * iz + (double)cam.cy), (float)q[2], 0.f);
+    return make_float4((float)((double)cam.phix * q[0] / q[2] + (double)cam.cx),
+                       (float)((double)cam.phiy * q[1] / q[2] + (double)cam.cy), (float)q[2], 0.f);
 }
 
 // ------------------------------------------------------------------ host helpers

@@ -67,9 +67,7 @@ typedef double v4d __attribute__((ext_vector_type(4)));
 // accumulator per coordinate, whose tile row i is vertex i (A = that coordinate's basis rows of the
 // 16 vertices, B = the coefficients of 16 frames), so lane l, element r of the x, y and z
 // accumulators holds vertex l/16 + 4 r for frame l%16: every MFMA row is a vertex coordinate
-// (three MFMAs per k-step for 16 vertices).  The columns of a k-step are free to choose: step
-// 4 t + s takes column 16 t + 4 kq + s from the lanes of residue kq = l/16, so that a lane's
-// entries of four steps are one aligned 16-byte piece of a basis row.
+// (three MFMAs per k-step for 16 vertices); step q takes columns 4 q .. 4 q + 3, in that order.
 //
 // Long lists: the basis rows are staged in LDS (as FP64), SY_KMAX columns at a time, identity
 // columns first.  With one such chunk (the per-frame fit: expression columns only) it is staged
@@ -90,14 +88,30 @@ typedef double v4d __attribute__((ext_vector_type(4)));
 constexpr int SY_VERTS = 16;               // vertices per workgroup
 constexpr int SY_KMAX = 80;                // columns held in LDS at a time
 
-// this lane's B entries: columns 16 t + 4 kq + s of a chunk of kc, every load issued
+// this lane's B entries: columns kq + 4 q of a chunk of kc, every load issued
 // unconditionally (clamped to a valid column) so the batch has no branches.  Nothing needs zeroing:
 // the A entries past the chunk's columns are zero, and an output column depends on its own frame's
 // B column only, so lanes without a live frame just skip the epilogue.
 __device__ __forceinline__ void synth_coefs(const float* __restrict__ tb, int kq, int kc, float* bv)
 {
 #pragma unroll
-    for (int q = 0; q < SY_KMAX / 4; ++q) bv[q] = tb[min(16 * (q >> 2) + 4 * kq + (q & 3), kc - 1)];
+    for (int q = 0; q < SY_KMAX / 4; ++q) bv[q] = tb[min(kq + 4 * q, kc - 1)];
+}
+
+// y[q] on the lanes of residue kq (lane / 16) = element kq of the lanes of residue q: a 4 x 4
+// transpose over the four 16-lane rows of a wavefront.
+__device__ __forceinline__ void transpose_residues(float4 x, float* y)
+{
+    unsigned a0 = __float_as_uint(x.x), a1 = __float_as_uint(x.y), a2 = __float_as_uint(x.z), a3 = __float_as_uint(x.w);
+    // the upper half of the first with the lower half of the second, then the odd rows with the even
+    const auto s02 = __builtin_amdgcn_permlane32_swap(a0, a2, false, false);
+    const auto s13 = __builtin_amdgcn_permlane32_swap(a1, a3, false, false);
+    const auto s01 = __builtin_amdgcn_permlane16_swap(s02[0], s13[0], false, false);
+    const auto s23 = __builtin_amdgcn_permlane16_swap(s02[1], s13[1], false, false);
+    y[0] = __uint_as_float(s01[0]);
+    y[1] = __uint_as_float(s01[1]);
+    y[2] = __uint_as_float(s23[0]);
+    y[3] = __uint_as_float(s23[1]);
 }
 
 // Three wavefronts per SIMD (register budget 168): with four, 30 registers spill and 96 frames take
@@ -131,23 +145,20 @@ k_synth_tile(ModelGPU m, Layout L, const FrameGPU* __restrict__ frames, const fl
         double (*sacc)[64] = (double (*)[64]) & sA[0][0][0];   // [coordinate * 4 + element][lane]
         if (wave < 3) {
             const float* row = m.exp_basis + (3 * (size_t)min(v0 + j, m.V - 1) + wave) * m.exp_ld;
-            float4 A[SY_KMAX / 16];
+            // columns 16 t + 4 kq .. + 3 in one load, then transposed over the four residues into
+            // columns 16 t + 4 q + kq (one load per column took 34.6 us of a one-frame launch)
+            float A[SY_KMAX / 4], bv[SY_KMAX / 4];
+            float4 ld4[SY_KMAX / 16];
 #pragma unroll
-            for (int t = 0; t < SY_KMAX / 16; ++t) {
-                A[t] = *(const float4*)(row + min(16 * t + 4 * kq, m.exp_ld - 4));
-                if (16 * t >= m.exp_ld) A[t] = make_float4(0.f, 0.f, 0.f, 0.f);
-            }
-            float bv[SY_KMAX / 4];
+            for (int t = 0; t < SY_KMAX / 16; ++t) ld4[t] = *(const float4*)(row + min(16 * t + 4 * kq, m.exp_ld - 4));
+#pragma unroll
+            for (int t = 0; t < SY_KMAX / 16; ++t) transpose_residues(ld4[t], A + 4 * t);
             synth_coefs(theta + (size_t)f * L.K + L.off_exp, kq, L.nexp, bv);
             v4d acc = (v4d){0, 0, 0, 0};
 #pragma unroll
-            for (int t = 0; t < SY_KMAX / 16; ++t) {
-                if (16 * t >= L.nexp) continue;
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const float av = q == 0 ? A[t].x : q == 1 ? A[t].y : q == 2 ? A[t].z : A[t].w;
-                    acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)av, (double)bv[4 * t + q], acc, 0, 0, 0);
-                }
+            for (int q = 0; q < SY_KMAX / 4; ++q) {
+                if (4 * q >= L.nexp) continue;         // within ld: zero past the last column
+                acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)A[q], (double)bv[q], acc, 0, 0, 0);
             }
 #pragma unroll
             for (int r = 0; r < 4; ++r) sacc[4 * wave + r][lane] = acc[r];
@@ -221,12 +232,11 @@ k_synth_tile(ModelGPU m, Layout L, const FrameGPU* __restrict__ frames, const fl
             synth_coefs(theta + (size_t)f * L.K + (id ? L.off_id : L.off_exp) + k0, kq, kc, bv);
 #pragma unroll
             for (int q = 0; q < SY_KMAX / 4; ++q) {
-                if (16 * (q >> 2) >= kc) continue;
+                if (4 * q >= kc) continue;
                 const double b = (double)bv[q];
 #pragma unroll
                 for (int a = 0; a < 3; ++a)
-                    acc[a] = __builtin_amdgcn_mfma_f64_16x16x4f64(sA[a][16 * (q >> 2) + 4 * kq + (q & 3)][j], b, acc[a],
-                                                                  0, 0, 0);
+                    acc[a] = __builtin_amdgcn_mfma_f64_16x16x4f64(sA[a][4 * q + kq][j], b, acc[a], 0, 0, 0);
             }
         }
         if (g < ngroups && live) {

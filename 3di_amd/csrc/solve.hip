@@ -185,7 +185,8 @@ __global__ void __launch_bounds__(256) k_barrier(ModelGPU m, Layout L, const Fra
 //             block), the blocks dealt to the four wavefronts; two barriers per panel;
 //   solves    wavefront 0, lane l holding entries l and l + 64, right-looking.
 // A barrier pair and an LDS round trip per column (what it replaces) took 283 us for one matrix of
-// 94 unknowns (mode 1 with the FP64 fallback) and 552 us for 448; this takes 66 and 132 us.
+// 94 unknowns (mode 1 with the FP64 fallback) and 552 us for 448; this takes 71 and 135 us, and gives the
+// same bits (each entry takes its products in the same order; an MFMA step is four FMAs in order).
 constexpr int CMAXK = 112;
 constexpr int CHB = 16;                          // block edge
 constexpr int CHP = CHB + 1;                     // LDS row stride
@@ -248,23 +249,32 @@ __device__ __forceinline__ void ch_load(T* A, const TH* __restrict__ Hf, int K, 
         }
 }
 
-// s = sqrt(d) and 1 / s of a pivot, on the factorisation's critical path: the hardware's reciprocal
-// square root, with Newton steps to the type's last place in FP64 (its estimate holds about 24 bits:
-// two steps) and one correction of the root.
-__device__ __forceinline__ void ch_root(float d, float& s, float& inv)
+// The factorisation's divisions and roots sit on its critical path, so they are a few FMAs around the
+// hardware's reciprocal square root instead of the compiler's full sequences, rounded as IEEE's all
+// the same (Markstein, "Computation of elementary functions on the IBM RISC System/6000 processor",
+// 1990): with y the rounded reciprocal of b, q = a y and one fma(a - b q, y, q) give the rounded a / b.
+template <typename T>
+__device__ __forceinline__ T ch_div(T a, T b, T y)
 {
-    inv = __builtin_amdgcn_rsqf(d);
-    s = d * inv;
-    s = fmaf(0.5f * inv, fmaf(-s, s, d), s);
+    const T q = a * y;
+    return fma(fma(-b, q, a), y, q);
 }
-__device__ __forceinline__ void ch_root(double d, double& s, double& inv)
+// s = sqrt(d) and y = 1 / s
+__device__ __forceinline__ void ch_root(float d, float& s, float& y)
 {
-    double y = __builtin_amdgcn_rsq(d);
+    y = __builtin_amdgcn_rsqf(d);
+    s = d * y;
+    s = fmaf(0.5f * y, fmaf(-s, s, d), s);
+    y = fmaf(fmaf(-s, y, 1.f), y, y);
+}
+__device__ __forceinline__ void ch_root(double d, double& s, double& y)
+{
+    y = __builtin_amdgcn_rsq(d);               // about 24 bits: two Newton steps
     y = fma(0.5 * y, fma(-d * y, y, 1.0), y);
     y = fma(0.5 * y, fma(-d * y, y, 1.0), y);
-    inv = y;
     s = d * y;
     s = fma(0.5 * y, fma(-s, s, d), s);
+    y = fma(fma(-s, y, 1.0), y, y);
 }
 
 // A = L L^T in place; false (for every thread) at a pivot that is not positive.
@@ -294,8 +304,8 @@ __device__ __forceinline__ bool ch_factor(T* A, int nT, int* sflag)
                 T s, inv;
                 ch_root(d, s, inv);
                 // rows above the pivot keep their entry (the block's unused upper triangle)
-                x0[k] = lane == k ? s : lane > k ? x0[k] * inv : x0[k];
-                x1[k] = x1[k] * inv;
+                x0[k] = lane == k ? s : lane > k ? ch_div(x0[k], s, inv) : x0[k];
+                x1[k] = ch_div(x1[k], s, inv);
 #pragma unroll
                 for (int j = k + 1; j < CHB; ++j) {
                     const T ljk = lane_read(x0[k], j);
@@ -338,8 +348,8 @@ __device__ __forceinline__ void ch_solve(const T* A, int nT, TB& b0, TB& b1)
 {
     const int lane = threadIdx.x & 63, l16 = lane & 15;
     const int I0 = min(lane >> 4, nT - 1), I1 = min((lane + 64) >> 4, nT - 1);
-    const TB q0 = TB(1) / (TB)A[ch_block(I0, I0) + l16 * CHP + l16];
-    const TB q1 = TB(1) / (TB)A[ch_block(I1, I1) + l16 * CHP + l16];
+    const TB d0 = A[ch_block(I0, I0) + l16 * CHP + l16], d1 = A[ch_block(I1, I1) + l16 * CHP + l16];
+    const TB q0 = TB(1) / d0, q1 = TB(1) / d1;
     for (int J = 0; J < nT; ++J) {
         // column j of the rows below it (blocks above the diagonal are never used: masked)
         const T* c0 = A + ch_block(max(I0, J), J) + l16 * CHP;
@@ -353,7 +363,7 @@ __device__ __forceinline__ void ch_solve(const T* A, int nT, TB& b0, TB& b1)
 #pragma unroll
         for (int c = 0; c < CHB; ++c) {
             const int j = CHB * J + c;
-            const TB y = j < 64 ? lane_read(b0 * q0, j & 63) : lane_read(b1 * q1, j & 63);
+            const TB y = j < 64 ? lane_read(ch_div(b0, d0, q0), j & 63) : lane_read(ch_div(b1, d1, q1), j & 63);
             b0 = lane == j ? y : lane > j ? fma(-(TB)l0[c], y, b0) : b0;
             b1 = lane + 64 == j ? y : lane + 64 > j ? fma(-(TB)l1[c], y, b1) : b1;
         }
@@ -371,7 +381,7 @@ __device__ __forceinline__ void ch_solve(const T* A, int nT, TB& b0, TB& b1)
 #pragma unroll
         for (int c = CHB - 1; c >= 0; --c) {
             const int j = CHB * J + c;
-            const TB x = j < 64 ? lane_read(b0 * q0, j & 63) : lane_read(b1 * q1, j & 63);
+            const TB x = j < 64 ? lane_read(ch_div(b0, d0, q0), j & 63) : lane_read(ch_div(b1, d1, q1), j & 63);
             b0 = lane == j ? x : lane < j ? fma(-(TB)l0[c], x, b0) : b0;
             b1 = lane + 64 == j ? x : lane + 64 < j ? fma(-(TB)l1[c], x, b1) : b1;
         }
@@ -428,16 +438,32 @@ __global__ void __launch_bounds__(256) k_cholesky(int K, const TH* __restrict__ 
                 if (in1) sx[lane + 64] = x1;
             }
             __syncthreads();
-            // residual -g - H x in FP64, eight lanes per row
-            for (int i = tid >> 3; i < ((K + 31) & ~31); i += 32) {
-                const TH* row = Hf + (size_t)min(i, K - 1) * K;
-                double r = 0.0;
-                for (int k = tid & 7; k < K; k += 8) r = fma(-(double)row[k], (double)sx[k], r);
-                r += __shfl_xor(r, 1, 64);
-                r += __shfl_xor(r, 2, 64);
-                r += __shfl_xor(r, 4, 64);
-                if ((tid & 7) == 0 && i < K) sb[i] = (r - (double)gf[i]) * (double)sdinv[i];
+            // residual -g - H x in FP64, a thread per row over the columns in order; the rows go
+            // through LDS 16 columns at a time so that they are read in whole sectors
+            double* sH = (double*)((float*)dsm + nT * (nT + 1) / 2 * CHN);
+            const int hr = tid >> 4, hc = tid & 15;
+            TH hv[CHT];
+            auto fetch = [&](int J) {
+#pragma unroll
+                for (int I = 0; I < CHT; ++I)
+                    if (I < nT) hv[I] = Hf[(size_t)min(CHB * I + hr, K - 1) * K + min(CHB * J + hc, K - 1)];
+            };
+            double r = tid < K ? -(double)gf[tid] : 0.0;
+            fetch(0);
+            for (int J = 0; J < nT; ++J) {
+#pragma unroll
+                for (int I = 0; I < CHT; ++I)
+                    if (I < nT) sH[(CHB * I + hr) * CHP + hc] = (double)hv[I];
+                __syncthreads();
+                if (J + 1 < nT) fetch(J + 1);
+                if (tid < K) {
+#pragma unroll
+                    for (int c = 0; c < CHB; ++c)
+                        if (CHB * J + c < K) r = fma(-sH[tid * CHP + c], (double)sx[CHB * J + c], r);
+                }
+                __syncthreads();
             }
+            if (tid < K) sb[tid] = r * (double)sdinv[tid];
             __syncthreads();
             if (wave == 0) {
                 double c0 = in0 ? sb[lane] : 0.0, c1 = in1 ? sb[lane + 64] : 0.0;
@@ -853,7 +879,9 @@ static int launch_cholesky_t(int n, int K, const TH* H, const float* g, float* d
         return TDI_ERR_ARG;
     }
     const int nT = (K + CHB - 1) / CHB;
-    const size_t lds = (size_t)nT * (nT + 1) / 2 * CHN * sizeof(double);   // FP64 fallback of mode 1 included
+    // the FP64 blocks, or mode 1's FP32 blocks and 16 columns of H in FP64
+    const size_t nb = (size_t)nT * (nT + 1) / 2 * CHN;
+    const size_t lds = std::max(nb * sizeof(double), nb * sizeof(float) + (size_t)nT * CHN * sizeof(double));
     hipLaunchKernelGGL(k_cholesky<TH>, dim3(n), dim3(256), lds, s, K, H, g, delta, status, mask, mode);
     TDI_HIP(hipGetLastError());
     return TDI_OK;
