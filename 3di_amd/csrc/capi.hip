@@ -7,6 +7,8 @@
 //               workspace sized for a chunk of frames.  No allocation happens inside a fit.
 #include "common.h"
 
+#include <atomic>
+#include <chrono>
 #include <cmath>
 #include <cstdarg>
 #include <cstring>
@@ -72,13 +74,43 @@ using namespace tdi;
 struct DevPool {
     std::mutex mu;
     std::multimap<size_t, void*> blocks;
+    std::vector<int*> host;          // free pinned blocks of HOST_INTS ints (one per batch in use)
     size_t cached = 0, limit = 0;
+    static constexpr size_t HOST_INTS = 16, HOST_KEEP = 64;
     DevPool()
     {
         size_t fb = 0, tb = 0;
         limit = hipMemGetInfo(&fb, &tb) == hipSuccess ? tb / 4 : 0;
     }
-    ~DevPool() { trim(); }
+    ~DevPool()
+    {
+        trim();
+        for (int* p : host) (void)hipHostFree(p);
+    }
+    int* take_host()
+    {
+        {
+            std::lock_guard<std::mutex> lock(mu);
+            if (!host.empty()) {
+                int* p = host.back();
+                host.pop_back();
+                return p;
+            }
+        }
+        int* p = nullptr;
+        if (hipHostMalloc((void**)&p, sizeof(int) * HOST_INTS, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        return p;
+    }
+    // the device no longer writes p
+    void put_host(int* p)
+    {
+        std::lock_guard<std::mutex> lock(mu);
+        if (host.size() < HOST_KEEP) host.push_back(p);
+        else (void)hipHostFree(p);
+    }
     void* take(size_t bytes)
     {
         std::lock_guard<std::mutex> lock(mu);
@@ -186,8 +218,8 @@ struct Workspace {
     int *npix = nullptr, *status = nullptr, *face_ok = nullptr, *mask = nullptr, *searching = nullptr,
         *evalmask = nullptr;
     int *act_m = nullptr, *act_e = nullptr;   // frame lists of mask / evalmask ([0] = count)
-    int *mask_r = nullptr, *mask_u = nullptr;  // active frames with a stale / reusable render
-    int *act_r = nullptr, *act_u = nullptr;    // their frame lists
+    int *act_r = nullptr, *act_u = nullptr;    // active frames with a stale / reusable render
+    int* seq = nullptr;                        // number of the line search's last report to the host
     int* tcount = nullptr;                     // [C][tmax] resolve tile counts
     int tmax = 0;
     double* rt = nullptr;                      // [C][12] FP64 rotation (column-major) + translation
@@ -208,6 +240,11 @@ struct Workspace {
     int max_area = 0;
 };
 
+// The pieces a batched fit is launched in (record_piece): the full evaluation up to the first
+// line-search round, with the renders that its frames need, one further round, and the evaluation at
+// the result.
+enum FitPiece { PIECE_HEAD_STALE, PIECE_HEAD_FRESH, PIECE_HEAD_BOTH, PIECE_ROUND, PIECE_RESULT, FIT_PIECES };
+
 struct tdi_batch {
     tdi_ctx* ctx = nullptr;
     ModelGPU m{};                     // the context's model with this batch's vertex albedos (alb)
@@ -219,8 +256,8 @@ struct tdi_batch {
     float* lmk = nullptr;             // [n][6][51]
     Workspace ws;
     Alloc mem;
-    hipGraphExec_t graph = nullptr;
-    hipGraphExec_t graph_fine = nullptr;   // the finetune fit's schedule
+    hipGraphExec_t graph[2][FIT_PIECES] = {};   // the fit's captured pieces, and the finetune fit's
+    int* status = nullptr;                 // pinned host memory: the line search's reports (k_ls_status)
     int finetune = 0;                      // set while a finetune fit runs: bounds and pose hold
     int joint = 0;                         // set while the identity stage's joint fit evaluates
     // scratch of the normal equations above 111 unknowns (allocated on first use): the Jacobian
@@ -432,8 +469,7 @@ static int ws_alloc(tdi_batch* b, int C, long long cap)
     w.status = A.get<int>(C);
     w.face_ok = A.get<int>(C);
     w.mask = A.get<int>(C);
-    w.mask_r = A.get<int>(C);
-    w.mask_u = A.get<int>(C);
+    w.seq = A.get<int>(1);
     w.act_r = A.get<int>(C + 1);
     w.act_u = A.get<int>(C + 1);
     w.searching = A.get<int>(C);
@@ -641,9 +677,12 @@ extern "C" int tdi_batch_create(tdi_ctx* c, int32_t n, const tdi_frame_desc* fd,
             b->ws.di_area = it->second.di_area;
         }
     }
+    b->status = c->pool->take_host();
+    if (!b->status) { b->mem.release(); delete b; set_error("pinned host allocation failed"); return TDI_ERR_NOMEM; }
     if (hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess ||
         hipEventCreateWithFlags(&b->ev_in, hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&b->ev_out, hipEventDisableTiming) != hipSuccess) {
+        c->pool->put_host(b->status);
         b->mem.release();
         delete b;
         set_error("stream/event creation failed");
@@ -653,19 +692,28 @@ extern "C" int tdi_batch_create(tdi_ctx* c, int32_t n, const tdi_frame_desc* fd,
     return TDI_OK;
 }
 
+static void drop_graphs(tdi_batch* b)
+{
+    for (auto& kind : b->graph)
+        for (hipGraphExec_t& g : kind) {
+            if (g) (void)hipGraphExecDestroy(g);
+            g = nullptr;
+        }
+}
+
 extern "C" int tdi_batch_destroy(tdi_batch* b)
 {
     if (!b) return TDI_OK;
     (void)hipSetDevice(b->ctx->device);
-    if (b->graph) (void)hipGraphExecDestroy(b->graph);
-    if (b->graph_fine) (void)hipGraphExecDestroy(b->graph_fine);
+    drop_graphs(b);
     if (b->stream) (void)hipStreamDestroy(b->stream);
     if (b->ev_in) (void)hipEventDestroy(b->ev_in);
     if (b->ev_out) (void)hipEventDestroy(b->ev_out);
     (void)hipFree(b->big_U);
     (void)hipFree(b->big_partials);
     (void)hipFree(b->big_D);
-    b->mem.release();
+    b->mem.release();                      // waits for the device
+    if (b->status) b->mem.pool->put_host(b->status);
     delete b;
     return TDI_OK;
 }
@@ -708,6 +756,15 @@ static int big_scratch(tdi_batch* b)
     return TDI_OK;
 }
 
+// The barrier's value and the face check, after a synthesis at theta.
+static int barrier_objective(tdi_batch* b, const Layout& L, FrameList fl, const float* theta, hipStream_t s)
+{
+    const tdi_ctx* c = b->ctx;
+    Workspace& w = b->ws;
+    return launch_barrier_obj(bounds_model(b), L, w.frames, fl, theta, w.rt, w.P0, w.vproj, lmk_arrays(w),
+                              c->opts.use_landmarks, c->opts.ref_face_size, w.obj, w.objb, w.face_ok, s);
+}
+
 // Objective at theta for the frames in `mask`: synthesis, face check, raster, resolve,
 // barrier objective, shading, blur, gradients (Renderer::render + evaluate_objective_function).
 // full_crop: blur the whole crops (the rendered image is an output), else only the region
@@ -727,13 +784,11 @@ static int eval_render(tdi_batch* b, FrameList fl, const float* theta, hipStream
         rc = launch_synthesize(b->m, L, w.frames, fl, theta, w.rt, w.P0, nullptr, w.vproj, s);
     if (rc) return rc;
     if (dverts && (rc = launch_add_offsets(c->m.V, w.frames, fl.n, w.rt, dverts, w.P0, w.vproj, s))) return rc;
-    if ((rc = launch_face_check(c->m.V, c->m.lmk_ids, w.vproj, c->opts.ref_face_size, fl, w.face_ok, s))) return rc;
     if ((rc = launch_clear_keys_frames(w.frames, fl, w.keys, w.box, w.max_area, s))) return rc;
     if ((rc = launch_raster(c->m, w.frames, fl, w.vproj, c->opts.ntmp_cap, w.keys, w.box, s))) return rc;
     if ((rc = launch_resolve(c->m, w.frames, fl, w.vproj, w.keys, w.cum, w.vis, w.npix, nullptr, w.pvert, w.pbary, w.max_area, w.tcount, w.tmax, w.box, s)))
         return rc;
-    if ((rc = launch_barrier(bounds_model(b), L, w.frames, fl, theta, lmk_arrays(w), c->opts.use_landmarks, 0, w.obj,
-                             w.objb, w.H, w.g, s)))
+    if ((rc = barrier_objective(b, L, fl, theta, s)))
         return rc;
     if ((rc = launch_shade(b->m, L, w.frames, fl, theta, w.P0, w.pvert, w.pbary, w.npix,
                            full_crop ? nullptr : w.box, w.img, w.max_area, s)))
@@ -746,9 +801,10 @@ static int eval_render(tdi_batch* b, FrameList fl, const float* theta, hipStream
 // Objective only, for the line search (the F(theta + t delta) of fit_3DMM_shape_rigid's Armijo
 // loop, model_fitter.cu:219-260): the same synthesis, raster and per-pixel terms as
 // eval_render, but shading and the objective work from the keys over the visible box, so
-// there is no visible list, no scatter and no per-pixel Jacobian records.
+// there is no visible list, no scatter and no per-pixel Jacobian records.  trial (a batched fit's
+// line-search round): the rotations are in w.rt already and the partials are left to k_ls_decide.
 static int eval_objective(tdi_batch* b, FrameList fl, const float* theta, hipStream_t s,
-                          const Layout* Lp = nullptr)
+                          const Layout* Lp = nullptr, bool trial = false)
 {
     tdi_ctx* c = b->ctx;
     const Layout& L = Lp ? *Lp : c->L;
@@ -757,18 +813,17 @@ static int eval_objective(tdi_batch* b, FrameList fl, const float* theta, hipStr
     if (b->joint && L.nid && w.idshape)   // the identity stage's frames share alpha
         rc = launch_synthesize_shared_id(b->m, L, w.frames, fl, theta, w.rt, w.P0, nullptr, w.vproj, w.idshape, s);
     else
-        rc = launch_synthesize(b->m, L, w.frames, fl, theta, w.rt, w.P0, nullptr, w.vproj, s);
+        rc = launch_synthesize(b->m, L, w.frames, fl, theta, w.rt, w.P0, nullptr, w.vproj, s, trial);
     if (rc) return rc;
-    if ((rc = launch_face_check(c->m.V, c->m.lmk_ids, w.vproj, c->opts.ref_face_size, fl, w.face_ok, s))) return rc;
     if ((rc = launch_clear_keys_frames(w.frames, fl, w.keys, w.box, w.max_area, s))) return rc;
     if ((rc = launch_raster(c->m, w.frames, fl, w.vproj, c->opts.ntmp_cap, w.keys, w.box, s))) return rc;
     if ((rc = launch_visible_box(w.frames, fl, w.keys, w.max_area, w.tcount, w.tmax, w.box, s))) return rc;
-    if ((rc = launch_barrier(bounds_model(b), L, w.frames, fl, theta, lmk_arrays(w), c->opts.use_landmarks, 0, w.obj,
-                             w.objb, w.H, w.g, s)))
+    if ((rc = barrier_objective(b, L, fl, theta, s)))
         return rc;
     if ((rc = launch_shade_keys(b->m, L, w.frames, fl, theta, w.P0, w.vproj, w.keys, w.box, w.img, s))) return rc;
     if ((rc = launch_blur(w.frames, fl, c->taps, w.box, w.img, w.tmp, w.blurred, w.max_area, s))) return rc;
-    return launch_objective(w.frames, fl, w.keys, w.box, w.blurred, b->obs_g, c->opts.data_weight, w.objp, w.obj, s);
+    return launch_objective(w.frames, fl, w.keys, w.box, w.blurred, b->obs_g, c->opts.data_weight, w.objp,
+                            trial ? nullptr : w.obj, s);
 }
 
 static int launch_normal_eq(tdi_batch* b, FrameList fl, int mixed, hipStream_t s, const Layout* Lp = nullptr)
@@ -795,8 +850,7 @@ static int eval_reused(tdi_batch* b, FrameList fl, const float* theta, hipStream
     if ((rc = launch_resolve(c->m, w.frames, fl, w.vproj, w.keys, w.cum, w.vis, w.npix, nullptr, w.pvert, w.pbary,
                              w.max_area, w.tcount, w.tmax, w.box, s)))
         return rc;
-    if ((rc = launch_barrier(bounds_model(b), L, w.frames, fl, theta, lmk_arrays(w), c->opts.use_landmarks, 0, w.obj,
-                             w.objb, w.H, w.g, s)))
+    if ((rc = barrier_objective(b, L, fl, theta, s)))
         return rc;
     return launch_grads(w.frames, fl, w.vis, w.npix, w.cum, w.blurred, b->obs_g, c->opts.data_weight, w.pixg, w.pnb,
                         w.pcoef, w.objp, w.obj, w.max_area, s);
@@ -820,12 +874,12 @@ static int eval_jacobian(tdi_batch* b, FrameList fl, const float* theta, int mix
         if ((rc = launch_jtj_big(L, w.frames, fl, w.npix, w.pnb, w.pcoef, w.pixg, w.dI, c->opts.data_weight, w.H, w.g,
                                  b->big_U, b->big_partials, b->big_S, w.max_area, s)))
             return rc;
-        return launch_barrier_big(bounds_model(b), L, w.frames, fl, theta, lmk_arrays(w), c->opts.use_landmarks,
-                                  b->big_D, w.H, w.g, s);
+        return launch_barrier_big(bounds_model(b), L, w.frames, fl, theta, w.rt, w.P0, lmk_arrays(w),
+                                  c->opts.use_landmarks, b->big_D, w.H, w.g, s);
     }
     if ((rc = launch_normal_eq(b, fl, mixed, s, &L))) return rc;
-    return launch_barrier(bounds_model(b), L, w.frames, fl, theta, lmk_arrays(w), c->opts.use_landmarks, 1, w.obj,
-                          w.objb, w.H, w.g, s);
+    return launch_barrier(bounds_model(b), L, w.frames, fl, theta, w.rt, w.P0, lmk_arrays(w),
+                          c->opts.use_landmarks, w.H, w.g, s);
 }
 
 // Objective, gradient and Gauss-Newton matrix at theta (get_obj_hessian_and_gradient_multiframe).
@@ -1642,13 +1696,13 @@ int tdi_barrier_terms(tdi_batch* b, const float* theta, double* H, double* g, do
         int rc = ws_load(b, i0, n, s);
         if (rc) return rc;
         const float* th = theta + (size_t)i0 * K;
+        if ((rc = launch_synthesize(b->m, c->L, w.frames, all_frames(n), th, w.rt, w.P0, nullptr, w.vproj, s))) return rc;
         TDI_HIP(hipMemsetAsync(w.H, 0, sizeof(double) * (size_t)n * K * K, s));
         TDI_HIP(hipMemsetAsync(w.g, 0, sizeof(float) * (size_t)n * K, s));
-        if ((rc = launch_barrier(c->m, c->L, w.frames, all_frames(n), th, lmk_arrays(w), c->opts.use_landmarks, 0,
-                                 w.obj, w.objb, w.H, w.g, s)))
+        if ((rc = barrier_objective(b, c->L, all_frames(n), th, s)))
             return rc;
-        if ((rc = launch_barrier(c->m, c->L, w.frames, all_frames(n), th, lmk_arrays(w), c->opts.use_landmarks, 1,
-                                 w.obj, w.objb, w.H, w.g, s)))
+        if ((rc = launch_barrier(c->m, c->L, w.frames, all_frames(n), th, w.rt, w.P0, lmk_arrays(w),
+                                 c->opts.use_landmarks, w.H, w.g, s)))
             return rc;
         if (H) TDI_HIP(hipMemcpyAsync(H + (size_t)i0 * K * K, w.H, sizeof(double) * (size_t)n * K * K,
                                       hipMemcpyDeviceToDevice, s));
@@ -1731,8 +1785,7 @@ int tdi_batch_autotune(tdi_batch* b, const float* theta, int32_t reps, int32_t* 
     if (rc) { w.S = S0; return rc; }
     w.S = best_S;
     w.di_area = best_area;
-    if (b->graph) { (void)hipGraphExecDestroy(b->graph); b->graph = nullptr; }
-    if (b->graph_fine) { (void)hipGraphExecDestroy(b->graph_fine); b->graph_fine = nullptr; }
+    drop_graphs(b);
     {
         std::lock_guard<std::mutex> lock(g_tune_mu);
         g_tuned[TuneKey(c->L.K, w.C, w.cap, b->max_area, mixed)] = TuneChoice{best_S, best_area};
@@ -1781,8 +1834,7 @@ int tdi_stage_times(tdi_batch* b, const float* theta, int32_t mixed, int32_t rep
                                w.pnb, w.pcoef, w.objp, w.obj, w.max_area, s)))
             return rc;
         TDI_HIP(hipEventRecord(ev[3], s));
-        if ((rc = launch_barrier(c->m, c->L, w.frames, all_frames(n), theta, lmk_arrays(w), c->opts.use_landmarks, 0, w.obj,
-                                 w.objb, w.H, w.g, s)))
+        if ((rc = barrier_objective(b, c->L, all_frames(n), theta, s)))
             return rc;
         TDI_HIP(hipEventRecord(ev[4], s));
         if ((rc = launch_dI(b->m, c->L, w.frames, all_frames(n), theta, w.P0, w.pvert, w.pbary, w.npix, w.pixg, w.dI,
@@ -1790,8 +1842,8 @@ int tdi_stage_times(tdi_batch* b, const float* theta, int32_t mixed, int32_t rep
             return rc;
         TDI_HIP(hipEventRecord(ev[5], s));
         if ((rc = launch_normal_eq(b, all_frames(n), mixed, s))) return rc;
-        if ((rc = launch_barrier(c->m, c->L, w.frames, all_frames(n), theta, lmk_arrays(w), c->opts.use_landmarks, 1, w.obj,
-                                 w.objb, w.H, w.g, s)))
+        if ((rc = launch_barrier(c->m, c->L, w.frames, all_frames(n), theta, w.rt, w.P0, lmk_arrays(w),
+                                 c->opts.use_landmarks, w.H, w.g, s)))
             return rc;
         TDI_HIP(hipEventRecord(ev[6], s));
         if ((rc = launch_cholesky(n, c->L.K, w.H, w.g, w.delta, w.status, (mixed & TDI_MIXED_CHOL_F32) ? 1 : 0, nullptr, s)))
@@ -2208,49 +2260,118 @@ int tdi_fit_lintensity(tdi_batch* b, const float* theta, float* lam, float* Lint
 } // extern "C"
 
 // ---------------------------------------------------------------------------- batched fit
-// One GN iteration for every frame of the workspace, all decisions on the device.
-static int record_fit(tdi_batch* b, hipStream_t s)
+// Line-search rounds of an iteration: steps t = beta^k >= t_min, capped by max_ls.
+static int ls_rounds(const tdi_fit_options& o)
+{
+    int rounds = 0;
+    for (double t = 1.0; t >= o.t_min && rounds < o.max_ls; t *= o.armijo_beta) ++rounds;
+    return rounds;
+}
+
+// One piece of the fit for every frame of the workspace (see fit_batched), all decisions on the device.
+static int record_piece(tdi_batch* b, FitPiece piece, hipStream_t s)
 {
     tdi_ctx* c = b->ctx;
     const tdi_fit_options& o = c->opts;
     Workspace& w = b->ws;
-    const int n = w.C, K = c->L.K, off_tz = c->L.off_pose + 2;
+    const int n = w.C, K = c->L.K;
     // the finetune fit's trials keep the pose (model_fitter.cu:502)
     const int hold0 = b->finetune ? c->L.off_pose : 0, hold1 = b->finetune ? c->L.off_pose + 6 : 0;
-    // evaluation rounds of the line search: steps t = beta^k >= t_min, capped by max_ls
-    int rounds = 0;
-    for (double t = 1.0; t >= o.t_min && rounds < o.max_ls; t *= o.armijo_beta) ++rounds;
+    const bool head = piece == PIECE_HEAD_STALE || piece == PIECE_HEAD_FRESH || piece == PIECE_HEAD_BOTH;
+    auto propose = [&]() -> int {
+        const int rc = launch_ls_propose(n, c->L, o.t_min, w.st, w.theta, w.delta, w.theta_try, w.rt, w.searching,
+                                         w.evalmask, hold0, hold1, s);
+        return rc ? rc : launch_ls_status(n, w.st, w.evalmask, w.act_e, w.seq, b->status, s);
+    };
     int rc;
-    for (int it = 0; it < o.max_iters; ++it) {
-        if ((rc = launch_copy_mask(n, w.st, w.mask, s))) return rc;
-        if ((rc = launch_compact_frames(n, w.mask, w.act_m, s))) return rc;
+    if (head || piece == PIECE_RESULT) {
         // A frame whose last line-search evaluation was accepted has the render of its new theta
         // in its own workspace slots (later rounds render only the frames still searching): its
         // synthesis, keys, visible box, shaded and blurred images are reused.  The others (the
         // first iteration, a search that ended on tz < 0 or on the round cap) are rendered.
-        if ((rc = launch_split_fresh(n, w.st, w.mask_r, w.mask_u, s))) return rc;
-        if ((rc = launch_compact_frames(n, w.mask_r, w.act_r, s))) return rc;
-        if ((rc = launch_compact_frames(n, w.mask_u, w.act_u, s))) return rc;
-        if ((rc = eval_render(b, FrameList{w.act_r, w.C}, w.theta, s))) return rc;
-        if ((rc = eval_reused(b, FrameList{w.act_u, w.C}, w.theta, s))) return rc;
+        if ((rc = launch_iter_lists(n, w.st, piece == PIECE_RESULT, w.mask, w.act_m, w.act_r, w.act_u, s))) return rc;
+        if (piece != PIECE_HEAD_FRESH && (rc = eval_render(b, FrameList{w.act_r, w.C}, w.theta, s))) return rc;
+        if (piece != PIECE_HEAD_STALE && (rc = eval_reused(b, FrameList{w.act_u, w.C}, w.theta, s))) return rc;
+        if (piece == PIECE_RESULT) return TDI_OK;
         if ((rc = eval_jacobian(b, FrameList{w.act_m, w.C}, w.theta, o.mixed_flags, s))) return rc;
         if ((rc = launch_cholesky(n, K, w.H, w.g, w.delta, w.status, (o.mixed_flags & TDI_MIXED_CHOL_F32) ? 1 : 0,
                                   w.mask, s)))
             return rc;
         if ((rc = launch_ls_init(n, K, w.st, w.status, w.delta, w.g, w.obj, w.searching, s))) return rc;
-        for (int r = 0; r < rounds; ++r) {
-            if ((rc = launch_ls_propose(n, K, off_tz, o.t_min, w.st, w.theta, w.delta, w.theta_try, w.searching,
-                                        w.evalmask, hold0, hold1, s)))
-                return rc;
-            if ((rc = launch_compact_frames(n, w.evalmask, w.act_e, s))) return rc;
-            if ((rc = eval_objective(b, FrameList{w.act_e, w.C}, w.theta_try, s))) return rc;
-            if ((rc = launch_ls_decide(n, K, w.st, w.evalmask, w.searching, w.obj, w.objb, w.face_ok, w.theta,
-                                       w.theta_try, o, s)))
-                return rc;
+        if ((rc = propose())) return rc;
+        if (ls_rounds(o) == 0) return TDI_OK;
+    }
+    // k_ls_propose left the trials' rotations; k_ls_decide sums their objectives
+    if ((rc = eval_objective(b, FrameList{w.act_e, w.C}, w.theta_try, s, nullptr, true))) return rc;
+    if ((rc = launch_ls_decide(n, K, w.st, w.act_e, w.evalmask, w.searching, w.obj, w.objb, w.objp, w.face_ok, w.theta,
+                               w.theta_try, o, s)))
+        return rc;
+    return propose();
+}
+
+// Launches a piece, as a captured graph unless TDI_NO_GRAPH is set.
+static int run_piece(tdi_batch* b, FitPiece piece, bool use_graph, hipStream_t s)
+{
+    if (!use_graph) return record_piece(b, piece, s);
+    // the finetune fit's bounds and pose hold differ
+    hipGraphExec_t& ge = b->graph[b->finetune ? 1 : 0][piece];
+    if (!ge) {
+        hipGraph_t g;
+        TDI_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
+        const int rc = record_piece(b, piece, s);
+        const hipError_t ec = hipStreamEndCapture(s, &g);
+        if (rc) return rc;
+        if (ec != hipSuccess) { set_error("graph capture failed: %s", hipGetErrorString(ec)); return TDI_ERR_HIP; }
+        TDI_HIP(hipGraphInstantiate(&ge, g, nullptr, nullptr, 0));
+        (void)hipGraphDestroy(g);
+    }
+    TDI_HIP(hipGraphLaunch(ge, s));
+    return TDI_OK;
+}
+
+// Waits for report `number` of the line search: a short spin on the pinned block, which sees a report
+// a few microseconds after the kernel wrote it, then a wait on the stream.
+static int wait_status(tdi_batch* b, int number, hipStream_t s)
+{
+    volatile int* seq = b->status;
+    const auto start = std::chrono::steady_clock::now();
+    for (int i = 0;; ++i) {
+        if (*seq == number) {
+            std::atomic_thread_fence(std::memory_order_acquire);
+            return TDI_OK;
         }
-        if ((rc = launch_ls_propose(n, K, off_tz, o.t_min, w.st, w.theta, w.delta, w.theta_try, w.searching, w.evalmask,
-                                    hold0, hold1, s)))
+        if ((i & 63) == 63 && std::chrono::steady_clock::now() - start > std::chrono::microseconds(300)) break;
+    }
+    TDI_HIP(hipStreamSynchronize(s));
+    if (*seq != number) { set_error("line search: report %d missing (%d)", number, *seq); return TDI_ERR_HIP; }
+    return TDI_OK;
+}
+
+// The iterations of a chunk.  The host launches piece by piece and learns from k_ls_status how many
+// frames still search and whether any stays active, so that the rounds and iterations that no frame
+// needs are not launched: the fixed schedule of 12 iterations x 12 rounds was about 2,400 launches of
+// 2 to 4 us each, most of them over empty lists (one frame: 9.1 ms, with the reports 6.6 ms; a report
+// and the next launch cost about 25 us against 65 us for an empty round).
+static int fit_chunk(tdi_batch* b, bool use_graph, hipStream_t s)
+{
+    const tdi_fit_options& o = b->ctx->opts;
+    const int rounds = ls_rounds(o);
+    b->status[0] = 0;
+    TDI_HIP(hipMemsetAsync(b->ws.seq, 0, sizeof(int), s));
+    int rc, number = 0;
+    bool stale = true, fresh = false;
+    for (int it = 0; it < o.max_iters; ++it) {
+        if ((rc = run_piece(b, stale && fresh ? PIECE_HEAD_BOTH : stale ? PIECE_HEAD_STALE : PIECE_HEAD_FRESH, use_graph, s)))
             return rc;
+        number += rounds > 0 ? 2 : 1;
+        if ((rc = wait_status(b, number, s))) return rc;
+        for (int r = 1; r < rounds && b->status[1] > 0; ++r) {
+            if ((rc = run_piece(b, PIECE_ROUND, use_graph, s))) return rc;
+            if ((rc = wait_status(b, ++number, s))) return rc;
+        }
+        if (b->status[2] == 0) break;
+        stale = b->status[3] > 0;
+        fresh = b->status[2] > b->status[3];
     }
     return TDI_OK;
 }
@@ -2276,34 +2397,17 @@ static int fit_batched(tdi_batch* b, float* theta, tdi_fit_report* reports, void
         if (rc) return rc;
         for (int i = 0; i < w.C; ++i) {
             FitState f{};
-            f.active = i < n;
+            f.active = f.real = i < n;
             hst[i] = f;
         }
         TDI_HIP(hipMemcpyAsync(w.st, hst.data(), sizeof(FitState) * w.C, hipMemcpyHostToDevice, s));
         TDI_HIP(hipMemcpyAsync(w.theta, theta + (size_t)i0 * K, sizeof(float) * n * K, hipMemcpyDeviceToDevice, s));
-        if (use_graph) {
-            // one captured schedule per kind of fit (the finetune fit's bounds and pose hold differ)
-            hipGraphExec_t& ge = b->finetune ? b->graph_fine : b->graph;
-            if (!ge) {
-                hipGraph_t g;
-                TDI_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-                rc = record_fit(b, s);
-                hipError_t ec = hipStreamEndCapture(s, &g);
-                if (rc) return rc;
-                if (ec != hipSuccess) { set_error("graph capture failed: %s", hipGetErrorString(ec)); return TDI_ERR_HIP; }
-                TDI_HIP(hipGraphInstantiate(&ge, g, nullptr, nullptr, 0));
-                (void)hipGraphDestroy(g);
-            }
-            TDI_HIP(hipGraphLaunch(ge, s));
-        } else {
-            if ((rc = record_fit(b, s))) return rc;
-        }
+        if ((rc = fit_chunk(b, use_graph, s))) return rc;
         TDI_HIP(hipMemcpyAsync(theta + (size_t)i0 * K, w.theta, sizeof(float) * n * K, hipMemcpyDeviceToDevice, s));
         TDI_HIP(hipMemcpyAsync(hst.data(), w.st, sizeof(FitState) * w.C, hipMemcpyDeviceToHost, s));
         if (reports) {
-            // objective at the returned parameters
-            if ((rc = set_mask_all(b, s))) return rc;
-            if ((rc = eval_render(b, all_frames(w.n_cur), w.theta, s))) return rc;
+            // objective and pixel count at the returned parameters
+            if ((rc = run_piece(b, PIECE_RESULT, use_graph, s))) return rc;
         }
         std::vector<double> hobj(w.C);
         std::vector<int> hnp(w.C);

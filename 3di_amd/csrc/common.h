@@ -77,6 +77,7 @@ struct FitState {
     int status;              // tdi_status
     int iters, outer, ls_evals, inner;
     int fresh;               // 1 when the frame's render in the workspace is that of its theta
+    int real;                // 0 for the padding slots of a chunk
     float t;                 // current step
     float dg;                // delta . g
     double obj0;             // F(theta) of the current iteration
@@ -166,6 +167,17 @@ __device__ inline int4 pixel_nbrs(const int* __restrict__ cum, int k, long long 
     int kr = cum[base + kright] - 1;
     if (kr < 0) kr = 0;
     return make_int4(kl, kr, pos - 1, pos + 1);
+}
+
+// Division on a critical path: a few FMAs around a reciprocal instead of the compiler's full sequence,
+// rounded as IEEE's all the same (Markstein, "Computation of elementary functions on the IBM RISC
+// System/6000 processor", 1990): with y the rounded reciprocal of b, q = a y and one
+// fma(a - b q, y, q) give the rounded a / b.
+template <typename T>
+__device__ __forceinline__ T ch_div(T a, T b, T y)
+{
+    const T q = a * y;
+    return fma(fma(-b, q, a), y, q);
 }
 
 // Rodrigues rotation and its derivatives in FP32 (fill_theta_etc, rotation_header.cu:46-149).
@@ -269,6 +281,36 @@ __device__ __forceinline__ float4 project_vertex(const FrameCam& cam, const doub
                        (float)((double)cam.phiy * q[1] / q[2] + (double)cam.cy), (float)q[2], 0.f);
 }
 
+// Workgroups per frame of the objective kernels: each writes its partial sum into its own
+// slot of a [frames][OBJ_PARTS] buffer.
+constexpr int OBJ_PARTS = 256;
+
+// The sum of a frame's np partials by one wavefront (the result on every lane).
+__device__ __forceinline__ double obj_partials(const double* __restrict__ p, int np)
+{
+    double s = 0.0;
+    for (int b = threadIdx.x & 63; b < np; b += 64) s += p[b];
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    return s;
+}
+
+// Column kernels (shade.hip): workgroups of four wavefronts, one column per wavefront at a time; 8
+// workgroups per slot of the list capacity for large batches, up to 128 for few frames; the
+// per-frame split is then chosen on the device from the list's length.
+constexpr int COL_MIN = 8, COL_MAX = 128;
+__device__ __forceinline__ int col_fpb(int nb, int nact)
+{
+    const int fpb = nact > 0 ? nb / nact : COL_MAX;
+    return fpb < COL_MIN ? COL_MIN : (fpb > COL_MAX ? COL_MAX : fpb);
+}
+
+inline int col_blocks(int n)
+{
+    int bx = n > 0 ? 4096 / n : COL_MAX;
+    bx = bx < COL_MIN ? COL_MIN : (bx > COL_MAX ? COL_MAX : bx);
+    return bx * (n > 0 ? n : 1);
+}
+
 // ------------------------------------------------------------------ host helpers
 void set_error(const char* fmt, ...);
 
@@ -288,7 +330,7 @@ void set_error(const char* fmt, ...);
 // Landmarks per frame, [n][6][51]: x, y (image pixels), box lx, ux, ly, uy (face-size units).
 // The frames a per-frame launch works on: every workspace slot 0..n-1 (act == nullptr), or
 // the compacted list act[1 .. act[0]] of slot indices built on the device from a mask
-// (launch_compact_frames).  Per-frame kernels walk the list with a grid-stride loop over
+// (launch_iter_lists, launch_ls_status).  Per-frame kernels walk the list with a grid-stride loop over
 // blockIdx.y (or blockIdx.x), so a launch over few frames costs little even though a
 // captured graph fixes its grid.
 struct FrameList {
@@ -308,8 +350,9 @@ struct LmkArrays {
 // geometry.hip
 // rt: [slots][12] scratch for the per-frame FP64 rotation (column-major) and translation;
 // P (camera-space vertices) may be null: the fit itself only needs P0 and the projections
+// (rt_ready: rt already holds them for theta)
 int launch_synthesize(const ModelGPU& m, const Layout& L, const FrameGPU* frames, FrameList fl, const float* theta,
-                      double* rt, double* P0, float* P, float4* vproj, hipStream_t s);
+                      double* rt, double* P0, float* P, float4* vproj, hipStream_t s, bool rt_ready = false);
 // Synthesis of frames that share their identity coefficients (the identity stage's evaluations):
 // the identity shape once (FP64, idshape [V][3]), then the expression MFMA tiles on it.
 int launch_synthesize_shared_id(const ModelGPU& m, const Layout& L, const FrameGPU* frames, FrameList fl,
@@ -347,6 +390,7 @@ int launch_shade_keys(const ModelGPU& m, const Layout& L, const FrameGPU* frames
                       const double* P0, const float4* vproj, const uint64_t* keys, const int4* box, float* img,
                       hipStream_t s);
 // objp: [frames][256] per-workgroup partials of the data objective (reduced in order into obj)
+// (obj null: the caller reduces them, with col_blocks(fl.n) as their count)
 int launch_obj_from_barrier(FrameList fl, const double* objb, double* obj, hipStream_t s);
 int launch_objective(const FrameGPU* frames, FrameList fl, const uint64_t* keys, const int4* box,
                      const float* blurred, const float2* obs_g, float w, double* objp, double* obj, hipStream_t s);
@@ -392,12 +436,17 @@ int launch_jtj_mfma(const Layout& L, const FrameGPU* frames, FrameList fl, const
                     float* partials, int S, int g_on_mfma, int two_term, hipStream_t s);
 
 // solve.hip
-int launch_barrier(const ModelGPU& m, const Layout& L, const FrameGPU* frames, FrameList fl,
-                   const float* theta, const LmkArrays& lm, int use_landmarks, int mode, double* obj, double* objb,
-                   double* H, float* g, hipStream_t s);
-// The barrier's derivative terms (mode 1) at any K: D is [n][2][NLMK][K] doubles of scratch.
+// rt, P0 and vproj: of a synthesis at theta
+int launch_barrier_obj(const ModelGPU& m, const Layout& L, const FrameGPU* frames, FrameList fl, const float* theta,
+                       const double* rt, const double* P0, const float4* vproj, const LmkArrays& lm, int use_landmarks,
+                       float ref_face_size, double* obj, double* objb, int* face_ok, hipStream_t s);
+// the derivative terms, K <= 112, and at any K (D is [n][2][NLMK][K] doubles of scratch)
+int launch_barrier(const ModelGPU& m, const Layout& L, const FrameGPU* frames, FrameList fl, const float* theta,
+                   const double* rt, const double* P0, const LmkArrays& lm, int use_landmarks, double* H, float* g,
+                   hipStream_t s);
 int launch_barrier_big(const ModelGPU& m, const Layout& L, const FrameGPU* frames, FrameList fl, const float* theta,
-                       const LmkArrays& lm, int use_landmarks, double* D, double* H, float* g, hipStream_t s);
+                       const double* rt, const double* P0, const LmkArrays& lm, int use_landmarks, double* D, double* H,
+                       float* g, hipStream_t s);
 // cholesky_big.hip: FP64 blocked Cholesky solve for K above what one workgroup holds in LDS
 constexpr int CHOL_BIG_MAXK = 4096;
 int launch_cholesky_big(int n, int K, const float* H, const float* g, float* delta, int* status, hipStream_t s);
@@ -453,17 +502,18 @@ int launch_cholesky(int n, int K, const double* H, const float* g, float* delta,
                     hipStream_t s);
 int launch_ls_init(int n, int K, FitState* st, const int* chol_status, const float* delta, const float* g,
                    const double* obj, int* searching, hipStream_t s);
-// unknowns [hold0, hold1) keep theta's values in the trials (hold0 == hold1: none)
-int launch_ls_propose(int n, int K, int off_tz, float t_min, FitState* st, const float* theta, const float* delta,
-                      float* theta_try, int* searching, int* evalmask, int hold0, int hold1, hipStream_t s);
-int launch_ls_decide(int n, int K, FitState* st, const int* evalmask, int* searching, const double* obj,
-                     const double* objb, const int* face_ok, float* theta, const float* theta_try,
+// unknowns [hold0, hold1) keep theta's values in the trials (hold0 == hold1: none); rt: the trials'
+// rotations and translations
+int launch_ls_propose(int n, const Layout& L, float t_min, FitState* st, const float* theta, const float* delta,
+                      float* theta_try, double* rt, int* searching, int* evalmask, int hold0, int hold1, hipStream_t s);
+// obj: written from the barrier's value and the objective's partials (of the list act's evaluation)
+int launch_ls_decide(int n, int K, FitState* st, const int* act, const int* evalmask, int* searching, double* obj,
+                     const double* objb, const double* objp, const int* face_ok, float* theta, const float* theta_try,
                      const tdi_fit_options& o, hipStream_t s);
-int launch_face_check(int V, const int* lmk_ids, const float4* vproj, float ref_face_size, FrameList fl,
-                      int* face_ok, hipStream_t s);
-int launch_copy_mask(int n, const FitState* st, int* mask, hipStream_t s);
-int launch_split_fresh(int n, const FitState* st, int* mask_r, int* mask_u, hipStream_t s);
-// act[0] = number of set entries of mask[0..n-1], act[1..] = their indices in increasing order
-int launch_compact_frames(int n, const int* mask, int* act, hipStream_t s);
+// the frame lists of one evaluation (mask, act_m: active; act_r, act_u: of these the frames with a
+// stale and with a reusable render; all: every real frame as active) and the line search's list with its
+// report to the host (status, pinned memory; seq, its device counter)
+int launch_iter_lists(int n, const FitState* st, int all, int* mask, int* act_m, int* act_r, int* act_u, hipStream_t s);
+int launch_ls_status(int n, const FitState* st, const int* evalmask, int* act_e, int* seq, int* status, hipStream_t s);
 
 } // namespace tdi

@@ -282,13 +282,13 @@ static int synthesize(const ModelGPU& m, const Layout& L, const FrameGPU* frames
 }
 
 int launch_synthesize(const ModelGPU& m, const Layout& L, const FrameGPU* frames, FrameList fl, const float* theta,
-                      double* rt, double* P0, float* P, float4* vproj, hipStream_t s)
+                      double* rt, double* P0, float* P, float4* vproj, hipStream_t s, bool rt_ready)
 {
     if (L.K > MAX_UNKNOWNS) {
         set_error("synthesize: K=%d exceeds %d", L.K, MAX_UNKNOWNS);
         return TDI_ERR_ARG;
     }
-    int rc = launch_frame_rt(L, fl, theta, rt, s);
+    const int rc = rt_ready ? TDI_OK : launch_frame_rt(L, fl, theta, rt, s);
     if (rc) return rc;
     return synthesize(m, L, frames, fl, theta, rt, nullptr, P0, P, vproj, s);
 }

@@ -21,10 +21,6 @@ struct Taps {
     float t[15];
 };
 
-// Workgroups per frame of the objective kernels: each writes its partial sum into its own
-// slot of a [frames][OBJ_PARTS] buffer, reduced in order by k_obj_reduce.
-constexpr int OBJ_PARTS = 256;
-
 namespace {
 
 // Region of a crop a pass has to cover, half-open [X0, X1) x [Y0, Y1).  Without a box (or
@@ -56,17 +52,9 @@ __device__ __forceinline__ bool crop_region(const FrameGPU& fr, const int4* box,
 // (one column per wavefront) when it is short, so that the last line-search rounds, whose
 // lists hold few frames, spread each frame over more wavefronts.  Slots of fpb consecutive
 // workgroups walk the list.
-constexpr int COL_MIN = 8, COL_MAX = 128;
-
 struct ColMap {
     int fpb, nslots, slot, sub;
 };
-
-__device__ __forceinline__ int col_fpb(int nb, int nact)
-{
-    const int fpb = nact > 0 ? nb / nact : COL_MAX;
-    return fpb < COL_MIN ? COL_MIN : (fpb > COL_MAX ? COL_MAX : fpb);
-}
 
 __device__ __forceinline__ ColMap col_map(int nact)
 {
@@ -348,13 +336,22 @@ __global__ void __launch_bounds__(256) k_blur_tiles(const FrameGPU* __restrict__
         float* dst = out + fr.pix_off;
         for (int t = cm.sub; t < ntx * nty; t += cm.fpb) {
             const int x0 = rg.X0 + (t % ntx) * BT_X, y0 = rg.Y0 + (t / ntx) * BT_Y;
-            // input tile: columns x0-7 .. x0+BT_X+6, rows y0-7 .. y0+BT_Y+6, zero outside the crop
-            for (int c = wave; c < BT_IX; c += 4) {
-                const int x = x0 - 7 + c;
-                for (int r = lane; r < BT_IY; r += 64) {
-                    const int y = y0 - 7 + r;
-                    simg[c][r] = (x >= rs.X0 && x < rs.X1 && y >= rs.Y0 && y < rs.Y1) ? src[(size_t)x * H + y] : 0.f;
-                }
+            // input tile: columns x0-7 .. x0+BT_X+6, rows y0-7 .. y0+BT_Y+6, zero outside the crop; every
+            // load of the thread is issued before the LDS stores (one at a time, the loads' latency took
+            // 11 of the 13 us of a one-frame launch)
+            constexpr int NLD = (BT_IX * BT_IY + 255) / 256;
+            float v[NLD];
+#pragma unroll
+            for (int q = 0; q < NLD; ++q) {
+                const int e = threadIdx.x + 256 * q, c = e / BT_IY, r = e - c * BT_IY;
+                const int x = x0 - 7 + c, y = y0 - 7 + r;
+                const bool in = x >= rs.X0 && x < rs.X1 && y >= rs.Y0 && y < rs.Y1 && c < BT_IX;
+                v[q] = in ? src[(size_t)x * H + y] : 0.f;
+            }
+#pragma unroll
+            for (int q = 0; q < NLD; ++q) {
+                const int e = threadIdx.x + 256 * q, c = e / BT_IY, r = e - c * BT_IY;
+                if (c < BT_IX) simg[c][r] = v[q];
             }
             __syncthreads();
             // along y, for the rows of the tile over all its input columns (zero outside the crop)
@@ -478,21 +475,19 @@ __global__ void __launch_bounds__(256) k_objective(const FrameGPU* __restrict__ 
     }
 }
 
-// obj[f] += the workgroup partials of the data objective, summed in workgroup order, so that
-// the objective of a frame does not depend on the order in which workgroups finish.
+// obj[f] += the workgroup partials of the data objective, in a fixed order (obj_partials), so that
+// the objective of a frame does not depend on the order in which workgroups finish.  A wavefront per
+// frame: one thread walking 128 partials took 9.4 us of a one-frame evaluation.
 // nparts: partials per frame; col_nb > 0: a column kernel of col_nb workgroups wrote them (as
 // many per frame as col_map gave it).
-__global__ void k_obj_reduce(const int* __restrict__ act, int n, int nparts, int col_nb,
-                             const double* __restrict__ objp, double* __restrict__ obj)
+__global__ void __launch_bounds__(64) k_obj_reduce(const int* __restrict__ act, int n, int nparts, int col_nb,
+                                                    const double* __restrict__ objp, double* __restrict__ obj)
 {
     const int nact = fl_count(act, n);
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nact) return;
-    const int f = fl_frame(act, i);
-    const int np = col_nb > 0 ? col_fpb(col_nb, nact) : nparts;
-    double s = 0.0;
-    for (int b = 0; b < np; ++b) s += objp[(size_t)f * OBJ_PARTS + b];
-    obj[f] += s;
+    if ((int)blockIdx.x >= nact) return;
+    const int f = fl_frame(act, blockIdx.x);
+    const double s = obj_partials(objp + (size_t)f * OBJ_PARTS, col_nb > 0 ? col_fpb(col_nb, nact) : nparts);
+    if (threadIdx.x == 0) obj[f] += s;
 }
 
 // obj[f] = objb[f] for the listed frames: the objective restarted from the barrier value that the
@@ -522,16 +517,6 @@ __global__ void __launch_bounds__(256) k_obs_grad(const FrameGPU* __restrict__ f
             obs_g[fr.obs_off + k] = make_float2(2.f * sx / hs, 2.f * sy / hs);
         }
     }
-}
-
-// Column kernels: workgroups of four wavefronts, one column per wavefront at a time; 8
-// workgroups per slot of the list capacity for large batches, up to 128 for few frames (the
-// per-frame split is then chosen on the device, see col_map).
-inline dim3 col_grid(int n)
-{
-    int bx = n > 0 ? 4096 / n : COL_MAX;
-    bx = bx < COL_MIN ? COL_MIN : (bx > COL_MAX ? COL_MAX : bx);
-    return dim3(bx * (n > 0 ? n : 1));
 }
 
 // Visible-list kernels: workgroups of 256 threads over a frame's visible list (the ones past
@@ -564,7 +549,7 @@ int launch_shade(const ModelGPU& m, const Layout& L, const FrameGPU* frames, Fra
         set_error("shade: k_tex %d > 512", L.ntex);
         return TDI_ERR_ARG;
     }
-    hipLaunchKernelGGL(k_clear_crops, col_grid(fl.n), dim3(256), 0, s, frames, fl.act, fl.n, box, img);
+    hipLaunchKernelGGL(k_clear_crops, dim3(col_blocks(fl.n)), dim3(256), 0, s, frames, fl.act, fl.n, box, img);
     hipLaunchKernelGGL(k_shade, list_grid(max_area, fl.n), dim3(256), 0, s, m, L, frames, fl.act, fl.n, theta, P0,
                        pvert, pbary, npix, img);
     TDI_HIP(hipGetLastError());
@@ -579,7 +564,7 @@ int launch_shade_keys(const ModelGPU& m, const Layout& L, const FrameGPU* frames
         set_error("shade: k_tex %d > 512", L.ntex);
         return TDI_ERR_ARG;
     }
-    hipLaunchKernelGGL(k_shade_keys, col_grid(fl.n), dim3(256), 0, s, m, L, frames, fl.act, fl.n, theta, P0, vproj,
+    hipLaunchKernelGGL(k_shade_keys, dim3(col_blocks(fl.n)), dim3(256), 0, s, m, L, frames, fl.act, fl.n, theta, P0, vproj,
                        (const unsigned long long*)keys, box, img);
     TDI_HIP(hipGetLastError());
     return TDI_OK;
@@ -588,10 +573,11 @@ int launch_shade_keys(const ModelGPU& m, const Layout& L, const FrameGPU* frames
 int launch_objective(const FrameGPU* frames, FrameList fl, const uint64_t* keys, const int4* box,
                      const float* blurred, const float2* obs_g, float w, double* objp, double* obj, hipStream_t s)
 {
-    const dim3 grid = col_grid(fl.n);
+    const dim3 grid = dim3(col_blocks(fl.n));
     hipLaunchKernelGGL(k_objective, grid, dim3(256), 0, s, frames, fl.act, fl.n,
                        (const unsigned long long*)keys, box, blurred, obs_g, w, objp);
-    hipLaunchKernelGGL(k_obj_reduce, dim3((fl.n + 255) / 256), dim3(256), 0, s, fl.act, fl.n, 0, (int)grid.x, objp, obj);
+    if (obj)
+        hipLaunchKernelGGL(k_obj_reduce, dim3(std::max(1, fl.n)), dim3(64), 0, s, fl.act, fl.n, 0, (int)grid.x, objp, obj);
     TDI_HIP(hipGetLastError());
     return TDI_OK;
 }
@@ -609,7 +595,7 @@ int launch_blur(const FrameGPU* frames, FrameList fl, const float* taps, const i
     Taps t;
     for (int i = 0; i < 15; ++i) t.t[i] = taps[i];
     (void)tmp;   // the fused kernel keeps the intermediate in LDS
-    hipLaunchKernelGGL(k_blur_tiles, col_grid(fl.n), dim3(256), 0, s, frames, fl.act, fl.n, box, t, in, out);
+    hipLaunchKernelGGL(k_blur_tiles, dim3(col_blocks(fl.n)), dim3(256), 0, s, frames, fl.act, fl.n, box, t, in, out);
     TDI_HIP(hipGetLastError());
     return TDI_OK;
 }
@@ -621,7 +607,7 @@ int launch_grads(const FrameGPU* frames, FrameList fl, const int* vis_list, cons
     const dim3 grid = list_grid(max_area, fl.n);
     hipLaunchKernelGGL(k_grads, grid, dim3(256), 0, s, frames, fl.act, fl.n, vis_list, npix, cum,
                        blurred, obs_g, w, pixg, pnb, pcoef, objp);
-    hipLaunchKernelGGL(k_obj_reduce, dim3((fl.n + 255) / 256), dim3(256), 0, s, fl.act, fl.n, (int)grid.x, 0, objp, obj);
+    hipLaunchKernelGGL(k_obj_reduce, dim3(std::max(1, fl.n)), dim3(64), 0, s, fl.act, fl.n, (int)grid.x, 0, objp, obj);
     TDI_HIP(hipGetLastError());
     return TDI_OK;
 }

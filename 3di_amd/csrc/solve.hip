@@ -24,153 +24,338 @@ namespace {
 
 constexpr int BMAXK = 112;
 
-// mode 0: objective only -> obj[f] = objb[f] = barrier value
-// mode 1: derivatives only -> H[f] += barrier Hessian, g[f] += barrier gradient
-// Everything is FP64 (rotation and its derivatives, landmark positions, constraint values,
-// weights, projected-landmark derivatives, sums, H); the FP32 g receives one rounding.
-// Dynamic LDS: the projected-landmark derivatives dx, dy as double [51][K] each, scaled by the
-// square roots of the Gauss-Newton weights, so that the landmark block is sum_i ex ex^T + ey ey^T.
-__global__ void __launch_bounds__(256) k_barrier(ModelGPU m, Layout L, const FrameGPU* __restrict__ frames,
-                                                  const int* __restrict__ act, int n, const float* __restrict__ theta,
-                                                  LmkArrays lm, int use_lmk, int mode, double* __restrict__ obj,
-                                                  double* __restrict__ objb, double* __restrict__ H,
-                                                  float* __restrict__ g)
+// The log barrier of one frame per workgroup, FP64 throughout (rotation and its derivatives, landmark
+// positions, constraint values, weights, projected-landmark derivatives, sums, H); the FP32 g receives
+// one rounding per term.  It is a few thousand operations, so latency bounds it: the rotation and the
+// landmark vertices are the synthesis's (rt, P0) instead of a serial sin/cos and 79-term sums, every
+// logarithm has a thread, and gathers are issued in batches.  One frame of 94 unknowns: 129
+// objectives and 24 derivative launches took 4552 us, now 592 and 1002 us.
+
+struct LmkBox {              // constraint values of one landmark (compute_Gs)
+    double vx, vy, vz, Gxm, Gym, Gxp, Gyp;
+};
+
+__device__ __forceinline__ LmkBox landmark_box(const FrameGPU& fr, const double* rt, const double* p, const float* L6,
+                                               int i)
+{
+    LmkBox o;
+    o.vx = rt[0] * p[0] + rt[3] * p[1] + rt[6] * p[2] + rt[9];
+    o.vy = rt[1] * p[0] + rt[4] * p[1] + rt[7] * p[2] + rt[10];
+    o.vz = rt[2] * p[0] + rt[5] * p[1] + rt[8] * p[2] + rt[11];
+    const double xproj = fr.phix * o.vx / o.vz + fr.cx;
+    const double yproj = fr.phiy * o.vy / o.vz + fr.cy;
+    const double lx = L6[i], ly = L6[NLMK + i];
+    const double blx = L6[2 * NLMK + i], bux = L6[3 * NLMK + i];
+    const double bly = L6[4 * NLMK + i], buy = L6[5 * NLMK + i];
+    const double fs = fr.face_size;
+    o.Gxm = xproj - (lx + blx * fs);
+    o.Gym = yproj - (ly + bly * fs);
+    o.Gxp = (lx + bux * fs) - xproj;
+    o.Gyp = (ly + buy * fs) - yproj;
+    return o;
+}
+
+// Objective: obj[f] = objb[f] = the barrier's value; face_ok (when given): the "face too large" test
+// of compute_nonrigid_shape2 (renderer.cu:836-857) on projected landmark vertices 0, 9 and 40.
+__global__ void __launch_bounds__(256) k_barrier_obj(ModelGPU m, Layout L, const FrameGPU* __restrict__ frames,
+                                                      const int* __restrict__ act, int n,
+                                                      const float* __restrict__ theta, const double* __restrict__ rt,
+                                                      const double* __restrict__ P0, const float4* __restrict__ vproj,
+                                                      LmkArrays lm, int use_lmk, float ref_face_size,
+                                                      double* __restrict__ obj, double* __restrict__ objb,
+                                                      int* __restrict__ face_ok)
+{
+    if ((int)blockIdx.x >= fl_count(act, n)) return;
+    const int f = fl_frame(act, blockIdx.x);
+    const FrameGPU fr = frames[f];
+    const float* tf = theta + (size_t)f * L.K;
+    __shared__ double sred[4];
+    const int tid = threadIdx.x;
+    if (face_ok && tid == 255) {
+        int ok = 1;
+        if (ref_face_size > 0.f) {
+            const float4* vp = vproj + (size_t)f * m.V;
+            const float4 a = vp[m.lmk_ids[0]], b = vp[m.lmk_ids[9]], c = vp[m.lmk_ids[40]];
+            const float iod = fabsf(b.x - a.x), lem = fabsf(a.y - c.y), rem = fabsf(b.y - c.y);
+            const float lim = 2.f * ref_face_size;
+            ok = !(iod > lim || lem > lim || rem > lim);
+        }
+        face_ok[f] = ok;
+    }
+    double acc = 0.0;
+    if (use_lmk && tid < 4 * NLMK) {              // one side of one landmark's box per thread
+        const int i = tid >> 2, side = tid & 3;
+        double R[12], p[3];
+        const double* pl = P0 + ((size_t)f * m.V + m.lmk_ids[i]) * 3;
+        for (int q = 0; q < 12; ++q) R[q] = rt[(size_t)f * 12 + q];
+        for (int a = 0; a < 3; ++a) p[a] = pl[a];
+        const LmkBox o = landmark_box(fr, R, p, lm.base + (size_t)f * 6 * NLMK, i);
+        acc = -log(side == 0 ? o.Gxm : side == 1 ? o.Gym : side == 2 ? o.Gxp : o.Gyp);
+    }
+    for (int e = 255 - tid; e < 2 * L.K; e += blockDim.x) {   // coefficient bounds (only finite ones)
+        const int j = e >> 1;
+        const float lb = m.lb[j], ub = m.ub[j];
+        if (!(ub < INFINITY) || !(lb > -INFINITY)) continue;
+        const double x = tf[j];
+        acc += -log(e & 1 ? x - (double)lb : (double)ub - x);
+    }
+    for (int o = 32; o > 0; o >>= 1) acc += __shfl_down(acc, o, 64);
+    if ((tid & 63) == 0) sred[tid >> 6] = acc;
+    __syncthreads();
+    if (tid == 0) {
+        const double s = sred[0] + sred[1] + sred[2] + sred[3];
+        obj[f] = s;
+        objb[f] = s;
+    }
+}
+
+// What the derivative terms of one frame start from, in LDS.
+struct BarrierFrame {
+    double rt[12], dR[27];
+    double p[NLMK][3], v[NLMK][3];
+    double zz[NLMK], izz[NLMK];                      // depth squared and its reciprocal
+    double rx[NLMK], ry[NLMK], gx[NLMK], gy[NLMK];   // square roots of the Gauss-Newton weights, gradient weights
+    int id[NLMK];
+};
+
+// Fills it (every thread of the workgroup; ends with a barrier).
+__device__ __forceinline__ void barrier_frame(const ModelGPU& m, const Layout& L, const FrameGPU& fr, int f,
+                                              const float* __restrict__ tf, const double* __restrict__ rt,
+                                              const double* __restrict__ P0, const float* __restrict__ L6, BarrierFrame& B)
+{
+    const int tid = threadIdx.x;
+    if (tid < 12) B.rt[tid] = rt[(size_t)f * 12 + tid];
+    if (tid >= 64 && tid < 64 + 3 * NLMK) {
+        const int e = tid - 64, i = e / 3, a = e - 3 * i, id = m.lmk_ids[i];
+        if (a == 0) B.id[i] = id;
+        B.p[i][a] = P0[((size_t)f * m.V + id) * 3 + a];
+    }
+    __syncthreads();
+    if (tid < 27) {
+        // entry (row r, column c) of dR/du_i, as rodrigues_f64_d forms it
+        const int i = tid / 9, c = (tid % 9) / 3, r = tid % 3;
+        double u[3], e[3], w[3], Rc[3];
+        for (int a = 0; a < 3; ++a) {
+            u[a] = tf[L.off_pose + 3 + a];
+            e[a] = -B.rt[i * 3 + a] + (i == a);
+            Rc[a] = B.rt[c * 3 + a];
+        }
+        const double th = sqrt(u[0] * u[0] + u[1] * u[1] + u[2] * u[2]);
+        const double inv = 1.0 / (th * th);
+        w[0] = u[1] * e[2] - u[2] * e[1];
+        w[1] = u[2] * e[0] - u[0] * e[2];
+        w[2] = u[0] * e[1] - u[1] * e[0];
+        // row r of u_i [u]x + [w]x: zero at column r, -x2 or +x1 ... around it
+        const double ui = i == 0 ? u[0] : i == 1 ? u[1] : u[2];
+        double acc = 0.0;
+        for (int k = 0; k < 3; ++k) {
+            if (k == r) continue;
+            const int o = 3 - r - k;                              // the third axis
+            const double sg = (k - r == 1 || k - r == -2) ? -1.0 : 1.0;
+            const double uo = o == 0 ? u[0] : o == 1 ? u[1] : u[2], wo = o == 0 ? w[0] : o == 1 ? w[1] : w[2];
+            acc += (ui * (sg * uo) + sg * wo) * Rc[k];
+        }
+        B.dR[tid] = acc * inv;
+    }
+    if (tid >= 64 && tid < 64 + NLMK) {
+        const int i = tid - 64;
+        const LmkBox o = landmark_box(fr, B.rt, B.p[i], L6, i);
+        B.v[i][0] = o.vx; B.v[i][1] = o.vy; B.v[i][2] = o.vz;
+        B.zz[i] = o.vz * o.vz;
+        B.izz[i] = 1.0 / B.zz[i];
+        B.rx[i] = sqrt(1.0 / (o.Gxm * o.Gxm) + 1.0 / (o.Gxp * o.Gxp));
+        B.ry[i] = sqrt(1.0 / (o.Gym * o.Gym) + 1.0 / (o.Gyp * o.Gyp));
+        B.gx[i] = -1.0 / o.Gxm + 1.0 / o.Gxp;
+        B.gy[i] = -1.0 / o.Gym + 1.0 / o.Gyp;
+    }
+    __syncthreads();
+}
+
+// d(projected landmark i)/d(direction dv) as (dx, dy)
+__device__ __forceinline__ void landmark_dxy(const FrameGPU& fr, const BarrierFrame& B, int i, const double* dv,
+                                             double& dx, double& dy)
+{
+    const double vx = B.v[i][0], vy = B.v[i][1], vz = B.v[i][2];
+    dx = ch_div(fr.phix * (dv[0] * vz - dv[2] * vx), B.zz[i], B.izz[i]);
+    dy = ch_div(fr.phiy * (dv[1] * vz - dv[2] * vy), B.zz[i], B.izz[i]);
+}
+
+// Rows of the projected-landmark derivatives: dx of landmark i to column j at D[dxrow(i)][j], dy at
+// D[dyrow(i)][j], for the geometric unknowns; the other columns are left as they are.
+template <typename Store>
+__device__ __forceinline__ void barrier_rows(const ModelGPU& m, const Layout& L, const FrameGPU& fr,
+                                             const BarrierFrame& B, Store store)
+{
+    const int tid = threadIdx.x;
+    // basis columns: the gathers of BATCH entries per thread are issued before the arithmetic
+    constexpr int BATCH = 8;
+    for (int blk = 0; blk < 2; ++blk) {
+        const int nc = blk ? L.nexp : L.nid, off = blk ? L.off_exp : L.off_id, ld = blk ? m.exp_ld : m.id_ld;
+        const float* basis = blk ? m.exp_basis : m.id_basis;
+        for (int e0 = 0; e0 < NLMK * nc; e0 += 256 * BATCH) {
+            float b[BATCH][3];
+#pragma unroll
+            for (int q = 0; q < BATCH; ++q) {
+                const int e = min(e0 + 256 * q + tid, NLMK * nc - 1), i = e / nc, c = e - i * nc;
+#pragma unroll
+                for (int a = 0; a < 3; ++a) b[q][a] = basis[(size_t)(3 * B.id[i] + a) * ld + c];
+            }
+#pragma unroll
+            for (int q = 0; q < BATCH; ++q) {
+                const int e = e0 + 256 * q + tid, i = e / nc, c = e - i * nc;
+                if (e >= NLMK * nc) continue;
+                double dv[3], dx, dy;
+#pragma unroll
+                for (int a = 0; a < 3; ++a)
+                    dv[a] = B.rt[a] * (double)b[q][0] + B.rt[3 + a] * (double)b[q][1] + B.rt[6 + a] * (double)b[q][2];
+                landmark_dxy(fr, B, i, dv, dx, dy);
+                store(i, off + c, dx, dy);
+            }
+        }
+    }
+    for (int e = tid; e < NLMK * 6; e += blockDim.x) {
+        const int i = e / 6, c = e - 6 * i;
+        double dv[3] = {0.0, 0.0, 0.0}, dx, dy;
+        if (c < 3) {
+            dv[0] = c == 0; dv[1] = c == 1; dv[2] = c == 2;
+        } else {
+            const double* d = B.dR + 9 * (c - 3);
+            for (int a = 0; a < 3; ++a) dv[a] = d[a] * B.p[i][0] + d[3 + a] * B.p[i][1] + d[6 + a] * B.p[i][2];
+        }
+        landmark_dxy(fr, B, i, dv, dx, dy);
+        store(i, L.off_pose + c, dx, dy);
+    }
+}
+
+// Gradient and Hessian diagonal of the bounds of unknown j (zero where it has none).
+__device__ __forceinline__ void bound_terms(const ModelGPU& m, const float* tf, int j, float& g, double& h)
+{
+    g = 0.f;
+    h = 0.0;
+    const float lbf = m.lb[j], ubf = m.ub[j];
+    if (!(ubf < INFINITY) || !(lbf > -INFINITY)) return;
+    const double x = tf[j], lb = lbf, ub = ubf;
+    const double fub = x - ub, flb = lb - x;
+    g = (float)(-1.0 / fub + 1.0 / flb);
+    const double a = -1.0 / (fub + 1e-12), b = 1.0 / (flb + 1e-12);
+    h = a * a + b * b;
+}
+
+constexpr int BAR_THREADS = 512;
+constexpr int BAR_PARTS = BAR_THREADS / 128, BAR_LMK = (NLMK + BAR_PARTS - 1) / BAR_PARTS;   // landmarks per part
+
+// Derivatives: H[f] += barrier Hessian, g[f] += barrier gradient, for K <= BMAXK.  A thread owns a
+// column j and a part of the landmarks: projected-landmark derivatives, the gradient's partial sum, and
+// the derivatives scaled by the square roots of the Gauss-Newton weights into dynamic LDS
+// [2 NLMK][KS], KS = K padded to 4; then the landmark block sum_i ex ex^T + ey ey^T, four rows of a
+// column per thread (lanes along the columns: conflict-free reads, the four rows' as broadcasts).
+__global__ void __launch_bounds__(BAR_THREADS) k_barrier(ModelGPU m, Layout L, const FrameGPU* __restrict__ frames,
+                                                          const int* __restrict__ act, int n,
+                                                          const float* __restrict__ theta, const double* __restrict__ rt,
+                                                          const double* __restrict__ P0, LmkArrays lm, int use_lmk,
+                                                          double* __restrict__ H,
+                                                          float* __restrict__ g)
 {
     // one workgroup per listed frame (the grid has a workgroup per slot)
     if ((int)blockIdx.x >= fl_count(act, n)) return;
     const int f = fl_frame(act, blockIdx.x);
-    const int K = L.K;
+    const int K = L.K, KS = (K + 3) & ~3;
     const FrameGPU fr = frames[f];
     const float* tf = theta + (size_t)f * K;
     extern __shared__ double sdyn[];
-    double* sdx = sdyn;                    // [NLMK][K], sqrt(wx_i) dx_i/dtheta
-    double* sdy = sdyn + (size_t)NLMK * K; // [NLMK][K]
-    __shared__ double sR[9], sdR[27];
-    __shared__ double sv[NLMK][3], sp[NLMK][3];
-    __shared__ double swx[NLMK], swy[NLMK], sgx[NLMK], sgy[NLMK];
-    __shared__ double sred[4];
+    __shared__ BarrierFrame B;
+    __shared__ double sbound[BMAXK];
+    __shared__ double sg[BAR_PARTS][128];
     const int tid = threadIdx.x;
-    if (tid == 0) rodrigues_f64_d(tf + L.off_pose + 3, sR, sdR);
-    __syncthreads();
-    double acc = 0.0;
-    // coefficient bounds (only finite bounds take part)
-    for (int j = tid; j < K; j += blockDim.x) {
-        const float lbf = m.lb[j], ubf = m.ub[j];
-        if (!(ubf < INFINITY) || !(lbf > -INFINITY)) continue;
-        const double x = tf[j], lb = lbf, ub = ubf;
-        const double fub = x - ub, flb = lb - x;
-        if (mode == 0) {
-            acc += -log(-fub) - log(-flb);
-        } else {
-            g[(size_t)f * K + j] += (float)(-1.0 / fub + 1.0 / flb);
-            const double a = -1.0 / (fub + 1e-12), b = 1.0 / (flb + 1e-12);
-            H[(size_t)f * K * K + (size_t)j * K + j] += a * a + b * b;
+    double* Hf = H + (size_t)f * K * K;
+    float gb = 0.f;
+    if (tid < K) {                                   // K <= BMAXK < BAR_THREADS
+        double hb;
+        bound_terms(m, tf, tid, gb, hb);
+        if (use_lmk) sbound[tid] = hb;
+        else {
+            g[(size_t)f * K + tid] += gb;
+            Hf[(size_t)tid * K + tid] += hb;
         }
     }
-    if (use_lmk) {
-        // the model-space landmark positions, one thread per coordinate
-        if (tid < 3 * NLMK) {
-            const int i = tid / 3, a = tid - 3 * i, r = 3 * m.lmk_ids[i] + a;
-            double s = m.mean[r];
-            for (int k = 0; k < L.nexp; ++k) s = fma((double)m.exp_basis[(size_t)r * m.exp_ld + k], (double)tf[L.off_exp + k], s);
-            for (int k = 0; k < L.nid; ++k) s = fma((double)m.id_basis[(size_t)r * m.id_ld + k], (double)tf[L.off_id + k], s);
-            sp[i][a] = s;
+    if (!use_lmk) return;
+    barrier_frame(m, L, fr, f, tf, rt, P0, lm.base + (size_t)f * 6 * NLMK, B);
+    {
+        const int j = tid & 127, part = tid >> 7;
+        const bool exp = j >= L.off_exp && j < L.off_pose, id = j >= L.off_id && j < L.off_exp;
+        const bool trans = j >= L.off_pose && j < L.off_pose + 3, rot = j >= L.off_pose + 3 && j < L.off_light;
+        const float* col = exp ? m.exp_basis + (j - L.off_exp) : m.id_basis + (j - L.off_id);
+        const int ld = exp ? m.exp_ld : m.id_ld;
+        float e[BAR_LMK][3];
+#pragma unroll
+        for (int q = 0; q < BAR_LMK; ++q) {
+            const int i = min(part * BAR_LMK + q, NLMK - 1);
+#pragma unroll
+            for (int a = 0; a < 3; ++a) e[q][a] = exp || id ? col[(size_t)(3 * B.id[i] + a) * ld] : 0.f;
         }
-        __syncthreads();
-        if (tid < NLMK) {
-            const int i = tid;
-            const double p[3] = {sp[i][0], sp[i][1], sp[i][2]};
-            const double vx = sR[0] * p[0] + sR[3] * p[1] + sR[6] * p[2] + tf[L.off_pose + 0];
-            const double vy = sR[1] * p[0] + sR[4] * p[1] + sR[7] * p[2] + tf[L.off_pose + 1];
-            const double vz = sR[2] * p[0] + sR[5] * p[1] + sR[8] * p[2] + tf[L.off_pose + 2];
-            sv[i][0] = vx; sv[i][1] = vy; sv[i][2] = vz;
-            const double xproj = fr.phix * vx / vz + fr.cx;
-            const double yproj = fr.phiy * vy / vz + fr.cy;
-            const float* L6 = lm.base + (size_t)f * 6 * NLMK;
-            const double lx = L6[i], ly = L6[NLMK + i];
-            const double blx = L6[2 * NLMK + i], bux = L6[3 * NLMK + i];
-            const double bly = L6[4 * NLMK + i], buy = L6[5 * NLMK + i];
-            const double fs = fr.face_size;
-            const double Gxm = xproj - (lx + blx * fs);
-            const double Gym = yproj - (ly + bly * fs);
-            const double Gxp = (lx + bux * fs) - xproj;
-            const double Gyp = (ly + buy * fs) - yproj;
-            if (mode == 0) {
-                acc += -log(Gxm) - log(Gym) - log(Gxp) - log(Gyp);
+        double s = 0.0;
+#pragma unroll
+        for (int q = 0; q < BAR_LMK; ++q) {
+            const int i = part * BAR_LMK + q;
+            if (i >= NLMK) continue;
+            double dv[3], dx, dy;
+            if (exp || id) {
+#pragma unroll
+                for (int a = 0; a < 3; ++a)
+                    dv[a] = B.rt[a] * (double)e[q][0] + B.rt[3 + a] * (double)e[q][1] + B.rt[6 + a] * (double)e[q][2];
+            } else if (rot) {
+                const double* d = B.dR + 9 * (j - L.off_pose - 3);
+#pragma unroll
+                for (int a = 0; a < 3; ++a) dv[a] = d[a] * B.p[i][0] + d[3 + a] * B.p[i][1] + d[6 + a] * B.p[i][2];
             } else {
-                swx[i] = 1.0 / (Gxm * Gxm) + 1.0 / (Gxp * Gxp);
-                swy[i] = 1.0 / (Gym * Gym) + 1.0 / (Gyp * Gyp);
-                sgx[i] = -1.0 / Gxm + 1.0 / Gxp;
-                sgy[i] = -1.0 / Gym + 1.0 / Gyp;
+#pragma unroll
+                for (int a = 0; a < 3; ++a) dv[a] = trans && j - L.off_pose == a ? 1.0 : 0.0;
+            }
+            landmark_dxy(fr, B, i, dv, dx, dy);
+            s += B.gx[i] * dx + B.gy[i] * dy;
+            if (j < KS) {
+                sdyn[(2 * i) * KS + j] = dx * B.rx[i];
+                sdyn[(2 * i + 1) * KS + j] = dy * B.ry[i];
             }
         }
-        __syncthreads();
-        if (mode == 1) {
-            // projected-landmark gradients dx[i][j], dy[i][j]
-            for (int e = tid; e < NLMK * K; e += blockDim.x) {
-                const int i = e / K, j = e - i * K;
-                double dv[3] = {0.0, 0.0, 0.0};
-                bool geo = true;
-                if (j >= L.off_pose && j < L.off_pose + 3) {
-                    dv[j - L.off_pose] = 1.0;
-                } else if (j >= L.off_pose + 3 && j < L.off_light) {
-                    const double* d = sdR + 9 * (j - L.off_pose - 3);
-                    for (int a = 0; a < 3; ++a) dv[a] = d[a] * sp[i][0] + d[3 + a] * sp[i][1] + d[6 + a] * sp[i][2];
-                } else if (j >= L.off_exp && j < L.off_pose) {
-                    const int v = m.lmk_ids[i], c = j - L.off_exp;
-                    double e3[3];
-                    for (int a = 0; a < 3; ++a) e3[a] = m.exp_basis[(size_t)(3 * v + a) * m.exp_ld + c];
-                    for (int a = 0; a < 3; ++a) dv[a] = sR[a] * e3[0] + sR[3 + a] * e3[1] + sR[6 + a] * e3[2];
-                } else if (j >= L.off_id && j < L.off_exp) {
-                    const int v = m.lmk_ids[i], c = j - L.off_id;
-                    double e3[3];
-                    for (int a = 0; a < 3; ++a) e3[a] = m.id_basis[(size_t)(3 * v + a) * m.id_ld + c];
-                    for (int a = 0; a < 3; ++a) dv[a] = sR[a] * e3[0] + sR[3 + a] * e3[1] + sR[6 + a] * e3[2];
-                } else {
-                    geo = false;
-                }
-                double dxj = 0.0, dyj = 0.0;
-                if (geo) {
-                    const double vx = sv[i][0], vy = sv[i][1], vz = sv[i][2];
-                    dxj = fr.phix * (dv[0] * vz - dv[2] * vx) / (vz * vz);
-                    dyj = fr.phiy * (dv[1] * vz - dv[2] * vy) / (vz * vz);
-                }
-                // gradient: sum_i gx_i dx_i; the Hessian uses sqrt(w) dx
-                sdx[(size_t)i * K + j] = dxj;
-                sdy[(size_t)i * K + j] = dyj;
-            }
-            __syncthreads();
-            for (int j = tid; j < K; j += blockDim.x) {
-                double s = 0.0;
-                for (int i = 0; i < NLMK; ++i) s += sgx[i] * sdx[(size_t)i * K + j] + sgy[i] * sdy[(size_t)i * K + j];
-                g[(size_t)f * K + j] += (float)s;
-            }
-            __syncthreads();
-            for (int e = tid; e < NLMK * K; e += blockDim.x) {
-                const int i = e / K;
-                sdx[e] *= sqrt(swx[i]);
-                sdy[e] *= sqrt(swy[i]);
-            }
-            __syncthreads();
-            for (int e = tid; e < K * K; e += blockDim.x) {
-                const int a = e / K, b = e - a * K;
-                if (b < a) continue;
-                double s = 0.0;
-                for (int i = 0; i < NLMK; ++i)
-                    s += sdx[(size_t)i * K + a] * sdx[(size_t)i * K + b] + sdy[(size_t)i * K + a] * sdy[(size_t)i * K + b];
-                H[(size_t)f * K * K + e] += s;
-                if (b != a) H[(size_t)f * K * K + (size_t)b * K + a] += s;
-            }
-        }
+        sg[part][j] = s;
     }
-    if (mode == 0) {
-        for (int o = 32; o > 0; o >>= 1) acc += __shfl_down(acc, o, 64);
-        if ((tid & 63) == 0) sred[tid >> 6] = acc;
-        __syncthreads();
-        if (tid == 0) {
-            const double s = sred[0] + sred[1] + sred[2] + sred[3];
-            obj[f] = s;
-            objb[f] = s;
+    __syncthreads();
+    if (tid < K) {
+        double s = sg[0][tid];
+#pragma unroll
+        for (int p = 1; p < BAR_PARTS; ++p) s += sg[p][tid];
+        g[(size_t)f * K + tid] = g[(size_t)f * K + tid] + gb + (float)s;
+    }
+    // task t: row group I (rows 4 I .. 4 I + 3) and column b of the upper triangle
+    const int T = KS / 4;
+    for (int t = tid;; t += BAR_THREADS) {
+        int I = 0, b = t;
+        while (I < T && b >= K - 4 * I) { b -= K - 4 * I; ++I; }
+        if (I >= T) break;
+        b += 4 * I;
+        // both triangles are read: the data term's mirrored entries differ in the last places
+        double hv[4], hl[4], s[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int a = min(4 * I + r, K - 1);
+            hv[r] = Hf[(size_t)a * K + b];
+            hl[r] = Hf[(size_t)b * K + a];
+        }
+#pragma unroll 3
+        for (int i = 0; i < NLMK; ++i) {
+            const double* dx = sdyn + (2 * i) * KS;
+            const double* dy = dx + KS;
+            const double xb = dx[b], yb = dy[b];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) s[r] += dx[4 * I + r] * xb + dy[4 * I + r] * yb;
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int a = 4 * I + r;
+            if (a > b) continue;
+            Hf[(size_t)a * K + b] = a == b ? hv[r] + sbound[a] + s[r] : hv[r] + s[r];
+            if (a != b) Hf[(size_t)b * K + a] = hl[r] + s[r];
         }
     }
 }
@@ -249,17 +434,7 @@ __device__ __forceinline__ void ch_load(T* A, const TH* __restrict__ Hf, int K, 
         }
 }
 
-// The factorisation's divisions and roots sit on its critical path, so they are a few FMAs around the
-// hardware's reciprocal square root instead of the compiler's full sequences, rounded as IEEE's all
-// the same (Markstein, "Computation of elementary functions on the IBM RISC System/6000 processor",
-// 1990): with y the rounded reciprocal of b, q = a y and one fma(a - b q, y, q) give the rounded a / b.
-template <typename T>
-__device__ __forceinline__ T ch_div(T a, T b, T y)
-{
-    const T q = a * y;
-    return fma(fma(-b, q, a), y, q);
-}
-// s = sqrt(d) and y = 1 / s
+// s = sqrt(d) and y = 1 / s, on the factorisation's critical path (see ch_div)
 __device__ __forceinline__ void ch_root(float d, float& s, float& y)
 {
     y = __builtin_amdgcn_rsqf(d);
@@ -544,12 +719,12 @@ __global__ void __launch_bounds__(64) k_ls_init(int n, int K, FitState* __restri
 
 // Trials theta + t delta; unknowns [hold0, hold1) keep theta's value (the finetune fit's pose,
 // model_fitter.cu:502).
-__global__ void k_ls_propose(int n, int K, int off_tz, float t_min, FitState* __restrict__ st,
+__global__ void k_ls_propose(int n, int K, int off_pose, float t_min, FitState* __restrict__ st,
                              const float* __restrict__ theta, const float* __restrict__ delta,
-                             float* __restrict__ theta_try, int* __restrict__ searching, int* __restrict__ evalmask,
-                             int hold0, int hold1)
+                             float* __restrict__ theta_try, double* __restrict__ rt, int* __restrict__ searching,
+                             int* __restrict__ evalmask, int hold0, int hold1)
 {
-    const int f = blockIdx.x;
+    const int f = blockIdx.x, off_tz = off_pose + 2;
     if (f >= n) return;
     __shared__ int go;
     if (threadIdx.x == 0) {
@@ -579,20 +754,37 @@ __global__ void k_ls_propose(int n, int K, int off_tz, float t_min, FitState* __
     __syncthreads();
     if (!go) return;
     const float t = st[f].t;
-    for (int k = threadIdx.x; k < K; k += blockDim.x)
-        theta_try[(size_t)f * K + k] = (k >= hold0 && k < hold1) ? theta[(size_t)f * K + k]
-                                                                 : theta[(size_t)f * K + k] + t * delta[(size_t)f * K + k];
+    __shared__ float pose[6];
+    for (int k = threadIdx.x; k < K; k += blockDim.x) {
+        const float x = (k >= hold0 && k < hold1) ? theta[(size_t)f * K + k]
+                                                  : theta[(size_t)f * K + k] + t * delta[(size_t)f * K + k];
+        theta_try[(size_t)f * K + k] = x;
+        if (k >= off_pose && k < off_pose + 6) pose[k - off_pose] = x;
+    }
+    __syncthreads();
+    // the trial's rotation and translation for the synthesis that follows
+    if (threadIdx.x == 0) {
+        double R[9];
+        rodrigues_f64(pose + 3, R);
+        for (int k = 0; k < 9; ++k) rt[(size_t)f * 12 + k] = R[k];
+        for (int a = 0; a < 3; ++a) rt[(size_t)f * 12 + 9 + a] = pose[a];
+    }
 }
 
-__global__ void k_ls_decide(int n, int K, FitState* __restrict__ st, const int* __restrict__ evalmask,
-                            int* __restrict__ searching, const double* __restrict__ obj, const double* __restrict__ objb,
+// One wavefront per frame; it also sums the frame's objective from the evaluation's partials.
+__global__ void __launch_bounds__(64) k_ls_decide(int n, int K, FitState* __restrict__ st, const int* __restrict__ act,
+                            const int* __restrict__ evalmask, int* __restrict__ searching, double* __restrict__ obj,
+                            const double* __restrict__ objb, const double* __restrict__ objp, int col_nb,
                             const int* __restrict__ face_ok, float* __restrict__ theta,
                             const float* __restrict__ theta_try, tdi_fit_options o)
 {
     const int f = blockIdx.x;
     if (f >= n || !evalmask[f]) return;
     __shared__ int accept;
+    const double data = obj_partials(objp + (size_t)f * OBJ_PARTS, col_fpb(col_nb, act[0]));
     if (threadIdx.x == 0) {
+        const double F = objb[f] + data;
+        obj[f] = F;
         FitState s = st[f];
         int acc = 0;
         if (!face_ok[f] || isnan(objb[f])) {
@@ -604,7 +796,7 @@ __global__ void k_ls_decide(int n, int K, FitState* __restrict__ st, const int* 
                 s.active = 0;
                 s.searching = 0;
                 s.stop |= TDI_STOP_DECREMENT;
-            } else if (obj[f] < s.obj0 + (double)(o.armijo_alpha * s.t * s.dg)) {
+            } else if (F < s.obj0 + (double)(o.armijo_alpha * s.t * s.dg)) {
                 acc = 1;
                 s.searching = 0;
             } else {
@@ -622,69 +814,86 @@ __global__ void k_ls_decide(int n, int K, FitState* __restrict__ st, const int* 
     for (int k = threadIdx.x; k < K; k += blockDim.x) theta[(size_t)f * K + k] = theta_try[(size_t)f * K + k];
 }
 
-// "Face too large" test of compute_nonrigid_shape2 (renderer.cu:836-857) on projected
-// landmark vertices 0, 9 and 40.
-__global__ void k_face_check(int V, const int* __restrict__ lmk_ids, const float4* __restrict__ vproj,
-                             float ref_face_size, const int* __restrict__ act, int n, int* __restrict__ face_ok)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= fl_count(act, n)) return;
-    const int f = fl_frame(act, i);
-    if (ref_face_size <= 0.f) { face_ok[f] = 1; return; }
-    const float4* vp = vproj + (size_t)f * V;
-    const float4 a = vp[lmk_ids[0]], b = vp[lmk_ids[9]], c = vp[lmk_ids[40]];
-    const float iod = fabsf(b.x - a.x), lem = fabsf(a.y - c.y), rem = fabsf(b.y - c.y);
-    const float lim = 2.f * ref_face_size;
-    face_ok[f] = !(iod > lim || lem > lim || rem > lim);
-}
-
-__global__ void k_copy_mask(int n, const FitState* __restrict__ st, int* __restrict__ mask)
-{
-    const int f = blockIdx.x * blockDim.x + threadIdx.x;
-    if (f < n) mask[f] = st[f].active;
-}
-
-// Active frames whose workspace render is stale (mask_r) or that of their theta (mask_u).
-__global__ void k_split_fresh(int n, const FitState* __restrict__ st, int* __restrict__ mask_r,
-                              int* __restrict__ mask_u)
-{
-    const int f = blockIdx.x * blockDim.x + threadIdx.x;
-    if (f >= n) return;
-    const FitState s = st[f];
-    mask_r[f] = s.active && !s.fresh;
-    mask_u[f] = s.active && s.fresh;
-}
-
-// Stream compaction of a mask into a frame list, one 1024-thread workgroup: per 1024-entry
-// tile a wavefront ballot and popcount give each set entry its rank within the wave, the
-// wave totals in LDS give the wave offsets, and a running count carries across tiles.
+// Frame lists, built by one workgroup: per 1024-entry tile a wavefront ballot and popcount give each
+// set entry its rank within the wave, the wave totals in LDS give the wave offsets, and a running
+// count carries across tiles.
 constexpr int CMP_THREADS = 1024;
+constexpr int CMP_WAVES = CMP_THREADS / 64;
 
-__global__ void __launch_bounds__(CMP_THREADS) k_compact_frames(int n, const int* __restrict__ mask,
-                                                                  int* __restrict__ act)
-{
-    constexpr int NW = CMP_THREADS / 64;
-    __shared__ int swave[NW];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const unsigned long long lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+struct ListBuilder {
     int running = 0;
-    for (int t0 = 0; t0 < n; t0 += CMP_THREADS) {
-        const int f = t0 + tid;
-        const int set = (f < n) && mask[f];
+    // every thread of the workgroup calls it, with its entry and whether it is set (act null: count only)
+    __device__ __forceinline__ void add(int f, bool set, int* __restrict__ act, int* swave)
+    {
+        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+        const unsigned long long lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
         const unsigned long long b = __ballot(set);
         if (lane == 0) swave[wave] = __popcll(b);
         __syncthreads();
         int off = 0, total = 0;
 #pragma unroll
-        for (int w = 0; w < NW; ++w) {
+        for (int w = 0; w < CMP_WAVES; ++w) {
             off += (w < wave) ? swave[w] : 0;
             total += swave[w];
         }
-        if (set) act[1 + running + off + __popcll(b & lt)] = f;
+        if (set && act) act[1 + running + off + __popcll(b & lt)] = f;
         running += total;
         __syncthreads();
     }
-    if (tid == 0) act[0] = running;
+};
+
+// The lists of one evaluation: act_m the active frames, of these act_r with a stale and act_u with a
+// reusable render in the workspace; mask the active frames.  all: every real frame counts as active.
+__global__ void __launch_bounds__(CMP_THREADS) k_iter_lists(int n, const FitState* __restrict__ st, int all,
+                                                              int* __restrict__ mask, int* __restrict__ act_m,
+                                                              int* __restrict__ act_r, int* __restrict__ act_u)
+{
+    __shared__ int swave[CMP_WAVES];
+    ListBuilder lm, lr, lu;
+    for (int t0 = 0; t0 < n; t0 += CMP_THREADS) {
+        const int f = t0 + threadIdx.x;
+        const bool in = f < n;
+        const int active = in && (all ? st[f].real : st[f].active), fresh = in && st[f].fresh;
+        if (in) mask[f] = active;
+        lm.add(f, active, act_m, swave);
+        lr.add(f, active && !fresh, act_r, swave);
+        lu.add(f, active && fresh, act_u, swave);
+    }
+    if (threadIdx.x == 0) {
+        act_m[0] = lm.running;
+        act_r[0] = lr.running;
+        act_u[0] = lu.running;
+    }
+}
+
+// act_e from evalmask, and what the host decides the next launches from, in its own memory: status[1]
+// frames to evaluate, [2] active frames, [3] active frames with a stale render; then status[0], the
+// number of this report (counted in *seq), which the host waits for.
+__global__ void __launch_bounds__(CMP_THREADS) k_ls_status(int n, const FitState* __restrict__ st,
+                                                             const int* __restrict__ evalmask, int* __restrict__ act_e,
+                                                             int* __restrict__ seq, int* status)
+{
+    __shared__ int swave[CMP_WAVES];
+    ListBuilder le, la, ls;
+    for (int t0 = 0; t0 < n; t0 += CMP_THREADS) {
+        const int f = t0 + threadIdx.x;
+        const bool in = f < n;
+        const int active = in && st[f].active, fresh = in && st[f].fresh;
+        le.add(f, in && evalmask[f], act_e, swave);
+        la.add(f, active, nullptr, swave);
+        ls.add(f, active && !fresh, nullptr, swave);
+    }
+    if (threadIdx.x == 0) {
+        act_e[0] = le.running;
+        const int k = *seq + 1;
+        *seq = k;
+        volatile int* out = status;
+        out[1] = le.running;
+        out[2] = la.running;
+        out[3] = ls.running;
+        __threadfence_system();
+        __hip_atomic_store(status, k, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
 }
 
 // The barrier's derivative terms (k_barrier mode 1) for frames with more unknowns than the
@@ -693,6 +902,7 @@ __global__ void __launch_bounds__(CMP_THREADS) k_compact_frames(int n, const int
 // Same formulas, FP64 throughout.
 __global__ void __launch_bounds__(256) k_barrier_rows(ModelGPU m, Layout L, const FrameGPU* __restrict__ frames,
                                                        const int* __restrict__ act, int n, const float* __restrict__ theta,
+                                                       const double* __restrict__ rt, const double* __restrict__ P0,
                                                        LmkArrays lm, int use_lmk, double* __restrict__ D,
                                                        double* __restrict__ H, float* __restrict__ g)
 {
@@ -703,96 +913,38 @@ __global__ void __launch_bounds__(256) k_barrier_rows(ModelGPU m, Layout L, cons
     const float* tf = theta + (size_t)f * K;
     double* sdx = D + (size_t)f * 2 * NLMK * K;
     double* sdy = sdx + (size_t)NLMK * K;
-    __shared__ double sR[9], sdR[27];
-    __shared__ double sv[NLMK][3], sp[NLMK][3];
-    __shared__ double swx[NLMK], swy[NLMK], sgx[NLMK], sgy[NLMK];
+    __shared__ BarrierFrame B;
     const int tid = threadIdx.x;
-    if (tid == 0) rodrigues_f64_d(tf + L.off_pose + 3, sR, sdR);
-    __syncthreads();
     for (int j = tid; j < K; j += blockDim.x) {
-        const float lbf = m.lb[j], ubf = m.ub[j];
-        if (!(ubf < INFINITY) || !(lbf > -INFINITY)) continue;
-        const double x = tf[j], lb = lbf, ub = ubf;
-        const double fub = x - ub, flb = lb - x;
-        g[(size_t)f * K + j] += (float)(-1.0 / fub + 1.0 / flb);
-        const double a = -1.0 / (fub + 1e-12), b = 1.0 / (flb + 1e-12);
-        H[(size_t)f * K * K + (size_t)j * K + j] += a * a + b * b;
+        float gb;
+        double hb;
+        bound_terms(m, tf, j, gb, hb);
+        g[(size_t)f * K + j] += gb;
+        H[(size_t)f * K * K + (size_t)j * K + j] += hb;
     }
     if (!use_lmk) return;
-    if (tid < 3 * NLMK) {
-        const int i = tid / 3, a = tid - 3 * i, r = 3 * m.lmk_ids[i] + a;
-        double sacc = m.mean[r];
-        for (int k = 0; k < L.nexp; ++k) sacc = fma((double)m.exp_basis[(size_t)r * m.exp_ld + k], (double)tf[L.off_exp + k], sacc);
-        for (int k = 0; k < L.nid; ++k) sacc = fma((double)m.id_basis[(size_t)r * m.id_ld + k], (double)tf[L.off_id + k], sacc);
-        sp[i][a] = sacc;
+    barrier_frame(m, L, fr, f, tf, rt, P0, lm.base + (size_t)f * 6 * NLMK, B);
+    // the columns without geometry (albedo, light) are zero
+    const int ng = L.off_light - L.off_id;
+    for (int e = tid; e < NLMK * (K - ng); e += blockDim.x) {
+        const int i = e / (K - ng), c = e - i * (K - ng), j = c < L.off_id ? c : c + ng;
+        sdx[(size_t)i * K + j] = sdy[(size_t)i * K + j] = 0.0;
     }
-    __syncthreads();
-    if (tid < NLMK) {
-        const int i = tid;
-        const double p[3] = {sp[i][0], sp[i][1], sp[i][2]};
-        const double vx = sR[0] * p[0] + sR[3] * p[1] + sR[6] * p[2] + tf[L.off_pose + 0];
-        const double vy = sR[1] * p[0] + sR[4] * p[1] + sR[7] * p[2] + tf[L.off_pose + 1];
-        const double vz = sR[2] * p[0] + sR[5] * p[1] + sR[8] * p[2] + tf[L.off_pose + 2];
-        sv[i][0] = vx; sv[i][1] = vy; sv[i][2] = vz;
-        const double xproj = fr.phix * vx / vz + fr.cx;
-        const double yproj = fr.phiy * vy / vz + fr.cy;
-        const float* L6 = lm.base + (size_t)f * 6 * NLMK;
-        const double lx = L6[i], ly = L6[NLMK + i];
-        const double blx = L6[2 * NLMK + i], bux = L6[3 * NLMK + i];
-        const double bly = L6[4 * NLMK + i], buy = L6[5 * NLMK + i];
-        const double fs = fr.face_size;
-        const double Gxm = xproj - (lx + blx * fs);
-        const double Gym = yproj - (ly + bly * fs);
-        const double Gxp = (lx + bux * fs) - xproj;
-        const double Gyp = (ly + buy * fs) - yproj;
-        swx[i] = 1.0 / (Gxm * Gxm) + 1.0 / (Gxp * Gxp);
-        swy[i] = 1.0 / (Gym * Gym) + 1.0 / (Gyp * Gyp);
-        sgx[i] = -1.0 / Gxm + 1.0 / Gxp;
-        sgy[i] = -1.0 / Gym + 1.0 / Gyp;
-    }
-    __syncthreads();
-    for (int e = tid; e < NLMK * K; e += blockDim.x) {
-        const int i = e / K, j = e - i * K;
-        double dv[3] = {0.0, 0.0, 0.0};
-        bool geo = true;
-        if (j >= L.off_pose && j < L.off_pose + 3) {
-            dv[j - L.off_pose] = 1.0;
-        } else if (j >= L.off_pose + 3 && j < L.off_light) {
-            const double* d = sdR + 9 * (j - L.off_pose - 3);
-            for (int a = 0; a < 3; ++a) dv[a] = d[a] * sp[i][0] + d[3 + a] * sp[i][1] + d[6 + a] * sp[i][2];
-        } else if (j >= L.off_exp && j < L.off_pose) {
-            const int v = m.lmk_ids[i], c = j - L.off_exp;
-            double e3[3];
-            for (int a = 0; a < 3; ++a) e3[a] = m.exp_basis[(size_t)(3 * v + a) * m.exp_ld + c];
-            for (int a = 0; a < 3; ++a) dv[a] = sR[a] * e3[0] + sR[3 + a] * e3[1] + sR[6 + a] * e3[2];
-        } else if (j >= L.off_id && j < L.off_exp) {
-            const int v = m.lmk_ids[i], c = j - L.off_id;
-            double e3[3];
-            for (int a = 0; a < 3; ++a) e3[a] = m.id_basis[(size_t)(3 * v + a) * m.id_ld + c];
-            for (int a = 0; a < 3; ++a) dv[a] = sR[a] * e3[0] + sR[3 + a] * e3[1] + sR[6 + a] * e3[2];
-        } else {
-            geo = false;
-        }
-        double dxj = 0.0, dyj = 0.0;
-        if (geo) {
-            const double vx = sv[i][0], vy = sv[i][1], vz = sv[i][2];
-            dxj = fr.phix * (dv[0] * vz - dv[2] * vx) / (vz * vz);
-            dyj = fr.phiy * (dv[1] * vz - dv[2] * vy) / (vz * vz);
-        }
-        sdx[(size_t)i * K + j] = dxj;
-        sdy[(size_t)i * K + j] = dyj;
-    }
+    barrier_rows(m, L, fr, B, [&](int i, int j, double dx, double dy) {
+        sdx[(size_t)i * K + j] = dx;
+        sdy[(size_t)i * K + j] = dy;
+    });
     __syncthreads();
     for (int j = tid; j < K; j += blockDim.x) {
-        double sacc = 0.0;
-        for (int i = 0; i < NLMK; ++i) sacc += sgx[i] * sdx[(size_t)i * K + j] + sgy[i] * sdy[(size_t)i * K + j];
-        g[(size_t)f * K + j] += (float)sacc;
-    }
-    __syncthreads();
-    for (int e = tid; e < NLMK * K; e += blockDim.x) {
-        const int i = e / K;
-        sdx[e] *= sqrt(swx[i]);
-        sdy[e] *= sqrt(swy[i]);
+        double s = 0.0;
+#pragma unroll 8
+        for (int i = 0; i < NLMK; ++i) {
+            const double dx = sdx[(size_t)i * K + j], dy = sdy[(size_t)i * K + j];
+            s += B.gx[i] * dx + B.gy[i] * dy;
+            sdx[(size_t)i * K + j] = dx * B.rx[i];
+            sdy[(size_t)i * K + j] = dy * B.ry[i];
+        }
+        g[(size_t)f * K + j] += (float)s;
     }
 }
 
@@ -834,10 +986,11 @@ __global__ void __launch_bounds__(256) k_barrier_hess(int K, const int* __restri
 } // namespace
 
 int launch_barrier_big(const ModelGPU& m, const Layout& L, const FrameGPU* frames, FrameList fl, const float* theta,
-                       const LmkArrays& lm, int use_landmarks, double* D, double* H, float* g, hipStream_t s)
+                       const double* rt, const double* P0, const LmkArrays& lm, int use_landmarks, double* D, double* H, float* g,
+                       hipStream_t s)
 {
     hipLaunchKernelGGL(k_barrier_rows, dim3(fl.n > 0 ? fl.n : 1), dim3(256), 0, s, m, L, frames, fl.act, fl.n, theta,
-                       lm, use_landmarks, D, H, g);
+                       rt, P0, lm, use_landmarks, D, H, g);
     if (use_landmarks) {
         const int T = (L.K + BH_T - 1) / BH_T;
         hipLaunchKernelGGL(k_barrier_hess, dim3(T * (T + 1) / 2, grid_frames(fl.n, 1 << 16)), dim3(256), 0, s, L.K,
@@ -847,25 +1000,34 @@ int launch_barrier_big(const ModelGPU& m, const Layout& L, const FrameGPU* frame
     return TDI_OK;
 }
 
-int launch_barrier(const ModelGPU& m, const Layout& L, const FrameGPU* frames, FrameList fl,
-                   const float* theta, const LmkArrays& lm, int use_landmarks, int mode, double* obj, double* objb,
-                   double* H, float* g, hipStream_t s)
+int launch_barrier_obj(const ModelGPU& m, const Layout& L, const FrameGPU* frames, FrameList fl, const float* theta,
+                       const double* rt, const double* P0, const float4* vproj, const LmkArrays& lm, int use_landmarks,
+                       float ref_face_size, double* obj, double* objb, int* face_ok, hipStream_t s)
 {
-    // the objective needs no LDS rows; the derivative terms above BMAXK go through launch_barrier_big
-    if (L.K > BMAXK && mode == 1 && use_landmarks) {
+    hipLaunchKernelGGL(k_barrier_obj, dim3(fl.n > 0 ? fl.n : 1), dim3(256), 0, s, m, L, frames, fl.act, fl.n, theta, rt,
+                       P0, vproj, lm, use_landmarks, ref_face_size, obj, objb, face_ok);
+    TDI_HIP(hipGetLastError());
+    return TDI_OK;
+}
+
+int launch_barrier(const ModelGPU& m, const Layout& L, const FrameGPU* frames, FrameList fl, const float* theta,
+                   const double* rt, const double* P0, const LmkArrays& lm, int use_landmarks, double* H, float* g, hipStream_t s)
+{
+    if (L.K > BMAXK) {
         set_error("barrier: K=%d > %d (derivative terms: launch_barrier_big)", L.K, BMAXK);
         return TDI_ERR_ARG;
     }
-    const size_t lds = mode == 1 && use_landmarks ? 2 * sizeof(double) * NLMK * L.K : 0;
-    if (lds > 64 * 1024) {
-        // above the default dynamic-LDS limit: allow up to what K <= BMAXK needs (91 KB), once per process
+    const size_t lds = use_landmarks ? sizeof(double) * 2 * NLMK * ((L.K + 3) & ~3) : 0;
+    if (lds > 56 * 1024) {
+        // with the static part above the default limit: allow up to what K <= BMAXK needs (91 KB), once
+        // per process
         static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(k_barrier),
                                                            hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                           (int)(2 * sizeof(double) * NLMK * BMAXK));
+                                                           (int)(sizeof(double) * 2 * NLMK * BMAXK));
         TDI_HIP(attr);
     }
-    hipLaunchKernelGGL(k_barrier, dim3(fl.n > 0 ? fl.n : 1), dim3(256), lds, s, m, L, frames, fl.act, fl.n, theta, lm,
-                       use_landmarks, mode, obj, objb, H, g);
+    hipLaunchKernelGGL(k_barrier, dim3(fl.n > 0 ? fl.n : 1), dim3(BAR_THREADS), lds, s, m, L, frames, fl.act, fl.n, theta,
+                       rt, P0, lm, use_landmarks, H, g);
     TDI_HIP(hipGetLastError());
     return TDI_OK;
 }
@@ -910,51 +1072,35 @@ int launch_ls_init(int n, int K, FitState* st, const int* chol_status, const flo
     return TDI_OK;
 }
 
-int launch_ls_propose(int n, int K, int off_tz, float t_min, FitState* st, const float* theta, const float* delta,
-                      float* theta_try, int* searching, int* evalmask, int hold0, int hold1, hipStream_t s)
+int launch_ls_propose(int n, const Layout& L, float t_min, FitState* st, const float* theta, const float* delta,
+                      float* theta_try, double* rt, int* searching, int* evalmask, int hold0, int hold1, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_ls_propose, dim3(n), dim3(64), 0, s, n, K, off_tz, t_min, st, theta, delta, theta_try,
-                       searching, evalmask, hold0, hold1);
+    hipLaunchKernelGGL(k_ls_propose, dim3(n), dim3(64), 0, s, n, L.K, L.off_pose, t_min, st, theta, delta, theta_try,
+                       rt, searching, evalmask, hold0, hold1);
     TDI_HIP(hipGetLastError());
     return TDI_OK;
 }
 
-int launch_ls_decide(int n, int K, FitState* st, const int* evalmask, int* searching, const double* obj,
-                     const double* objb, const int* face_ok, float* theta, const float* theta_try,
+int launch_ls_decide(int n, int K, FitState* st, const int* act, const int* evalmask, int* searching, double* obj,
+                     const double* objb, const double* objp, const int* face_ok, float* theta, const float* theta_try,
                      const tdi_fit_options& o, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_ls_decide, dim3(n), dim3(64), 0, s, n, K, st, evalmask, searching, obj, objb, face_ok, theta,
-                       theta_try, o);
+    hipLaunchKernelGGL(k_ls_decide, dim3(n), dim3(64), 0, s, n, K, st, act, evalmask, searching, obj, objb, objp,
+                       col_blocks(n), face_ok, theta, theta_try, o);
     TDI_HIP(hipGetLastError());
     return TDI_OK;
 }
 
-int launch_face_check(int V, const int* lmk_ids, const float4* vproj, float ref_face_size, FrameList fl,
-                      int* face_ok, hipStream_t s)
+int launch_iter_lists(int n, const FitState* st, int all, int* mask, int* act_m, int* act_r, int* act_u, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_face_check, dim3((fl.n + 255) / 256 > 0 ? (fl.n + 255) / 256 : 1), dim3(256), 0, s, V,
-                       lmk_ids, vproj, ref_face_size, fl.act, fl.n, face_ok);
+    hipLaunchKernelGGL(k_iter_lists, dim3(1), dim3(CMP_THREADS), 0, s, n, st, all, mask, act_m, act_r, act_u);
     TDI_HIP(hipGetLastError());
     return TDI_OK;
 }
 
-int launch_copy_mask(int n, const FitState* st, int* mask, hipStream_t s)
+int launch_ls_status(int n, const FitState* st, const int* evalmask, int* act_e, int* seq, int* status, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_copy_mask, dim3((n + 255) / 256), dim3(256), 0, s, n, st, mask);
-    TDI_HIP(hipGetLastError());
-    return TDI_OK;
-}
-
-int launch_split_fresh(int n, const FitState* st, int* mask_r, int* mask_u, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_split_fresh, dim3((n + 255) / 256), dim3(256), 0, s, n, st, mask_r, mask_u);
-    TDI_HIP(hipGetLastError());
-    return TDI_OK;
-}
-
-int launch_compact_frames(int n, const int* mask, int* act, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_compact_frames, dim3(1), dim3(CMP_THREADS), 0, s, n, mask, act);
+    hipLaunchKernelGGL(k_ls_status, dim3(1), dim3(CMP_THREADS), 0, s, n, st, evalmask, act_e, seq, status);
     TDI_HIP(hipGetLastError());
     return TDI_OK;
 }
