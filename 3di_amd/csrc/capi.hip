@@ -210,7 +210,11 @@ struct Workspace {
     float* pcoef = nullptr;
     int4* pvert = nullptr;       // per visible position: vertices of its triangle, crop index
     float2* pbary = nullptr;     // per visible position: (alpha, beta)
-    float* dI = nullptr;
+    float4* pq = nullptr;        // per visible position, from the pixel pass of the Jacobian (JacScratch)
+    float2* pshade = nullptr;
+    uint2 *ptri = nullptr, *plist = nullptr;
+    int* pstart = nullptr;
+    float* dI = nullptr;         // [cap][dI_stride(K)]
     float *theta = nullptr, *theta_try = nullptr, *delta = nullptr, *g = nullptr;
     double* H = nullptr;       // [C][K][K] normal matrices (FP64)
     double *obj = nullptr, *objb = nullptr;
@@ -269,6 +273,69 @@ struct tdi_batch {
     hipStream_t stream = nullptr;     // capture-capable stream owned by the batch (default priority)
     hipEvent_t ev_in = nullptr, ev_out = nullptr;
 };
+
+// Groups of triangles over at most PATCH_VERTS vertices each, grown breadth first from triangle to
+// triangle over shared vertices so that a patch is compact on the mesh (few vertices are in two patches);
+// a patch whose surroundings are used up goes on from the first triangle left.
+struct MeshPatches {
+    std::vector<int> off, vert;
+    std::vector<uint2> tri;
+};
+
+static MeshPatches mesh_patches(int V, int NT, const int32_t* tris)
+{
+    MeshPatches P;
+    std::vector<int> start(V + 1, 0), list(3 * (size_t)NT), place(V, -1), queue;
+    for (size_t e = 0; e < 3 * (size_t)NT; ++e) start[tris[e] + 1]++;
+    for (int v = 0; v < V; ++v) start[v + 1] += start[v];
+    {
+        std::vector<int> at(start.begin(), start.end() - 1);
+        for (int t = 0; t < NT; ++t)
+            for (int c = 0; c < 3; ++c) list[at[tris[3 * (size_t)t + c]]++] = t;
+    }
+    P.tri.assign(NT, uint2{0xffffffffu, 0});
+    P.off.push_back(0);
+    int next = 0, left = NT;                       // first triangle that may be unassigned
+    size_t first = 0;                              // this patch's vertices start here in vert
+    auto count = [&] { return (int)(P.vert.size() - first); };
+    auto add = [&](int t) -> bool {
+        const int32_t* v = tris + 3 * (size_t)t;
+        int fresh = 0;
+        for (int c = 0; c < 3; ++c)
+            fresh += place[v[c]] < 0 && (c == 0 || v[c] != v[0]) && (c < 2 || v[c] != v[1]);
+        if (count() + fresh > PATCH_VERTS) return false;
+        unsigned ids = 0;
+        for (int c = 0; c < 3; ++c) {
+            if (place[v[c]] < 0) {
+                place[v[c]] = count();
+                P.vert.push_back(v[c]);
+                queue.push_back(v[c]);
+            }
+            ids |= (unsigned)place[v[c]] << (8 * c);
+        }
+        P.tri[t] = uint2{(unsigned)(P.off.size() - 1), ids};
+        --left;
+        return true;
+    };
+    while (left > 0) {
+        queue.clear();
+        size_t head = 0;
+        for (;;) {
+            if (head == queue.size()) {            // surroundings used up (or a new patch)
+                while (next < NT && P.tri[next].x != 0xffffffffu) ++next;
+                if (next == NT || !add(next)) break;
+                continue;
+            }
+            const int v = queue[head++];
+            for (int e = start[v]; e < start[v + 1]; ++e)
+                if (P.tri[list[e]].x == 0xffffffffu) add(list[e]);
+        }
+        for (size_t e = first; e < P.vert.size(); ++e) place[P.vert[e]] = -1;
+        first = P.vert.size();
+        P.off.push_back((int)first);
+    }
+    return P;
+}
 
 extern "C" {
 
@@ -367,6 +434,13 @@ int tdi_ctx_create(const tdi_model_desc* md, const tdi_fit_options* opts, int de
     m.tex_basis = md->k_tex ? up_rows(md->tex_basis, (size_t)V, md->k_tex, m.tex_ld) : nullptr;
     m.tris = (const int*)up(md->triangles, sizeof(int) * 3 * (size_t)NT);
     m.lmk_ids = (const int*)up(md->landmark_ids, sizeof(int) * NLMK);
+    const MeshPatches patches = mesh_patches(V, NT, md->triangles);
+    if ((int)patches.off.size() - 1 <= PATCH_MAX) {
+        m.np = (int)patches.off.size() - 1;
+        m.patch_off = (const int*)up(patches.off.data(), sizeof(int) * patches.off.size());
+        m.patch_vert = (const int*)up(patches.vert.data(), sizeof(int) * patches.vert.size());
+        m.tri_patch = (const uint2*)up(patches.tri.data(), sizeof(uint2) * NT);
+    }
     const Layout& L = c->L;
     c->Lx = L;
     if (!L.nlight) {
@@ -456,7 +530,12 @@ static int ws_alloc(tdi_batch* b, int C, long long cap)
     w.pcoef = A.get<float>(cap);
     w.pvert = A.get<int4>(cap);
     w.pbary = A.get<float2>(cap);
-    w.dI = A.get<float>((size_t)cap * K);
+    w.pq = A.get<float4>(cap);
+    w.pshade = c->L.ntex ? A.get<float2>(cap) : nullptr;
+    w.ptri = c->m.np ? A.get<uint2>(cap) : nullptr;
+    w.plist = c->m.np ? A.get<uint2>(cap) : nullptr;
+    w.pstart = c->m.np ? A.get<int>((size_t)C * (c->m.np + 1)) : nullptr;
+    w.dI = A.get<float>((size_t)cap * dI_stride(K));
     w.theta = A.get<float>((size_t)C * K);
     w.theta_try = A.get<float>((size_t)C * K);
     w.delta = A.get<float>((size_t)C * K);
@@ -533,6 +612,11 @@ static int mean_crop(const Workspace& w)
 static int dI_area(const Workspace& w)
 {
     return w.di_area > 0 ? w.di_area : mean_crop(w);
+}
+
+static JacScratch jac_scratch(const Workspace& w)
+{
+    return JacScratch{w.pq, w.pshade, w.ptri, w.plist, w.pstart};
 }
 
 static LmkArrays lmk_arrays(const Workspace& w)
@@ -648,8 +732,8 @@ extern "C" int tdi_batch_create(tdi_ctx* c, int32_t n, const tdi_frame_desc* fd,
         if (hipMemGetInfo(&fb, &tb) == hipSuccess && fb > 0) budget_gb = 0.5 * (double)(fb + c->pool->cached_bytes()) / 1e9;
     }
     const int V = c->m.V, K = c->Lx.K;
-    const double per_frame = (double)V * 40 + 64.0 * K * K + 8.0 * resolve_tiles(maxA);
-    const double per_pixel = 108.0 + 4.0 * K;
+    const double per_frame = (double)V * 40 + 64.0 * K * K + 8.0 * resolve_tiles(maxA) + 4.0 * c->m.np;
+    const double per_pixel = 108.0 + (c->m.np ? 40.0 : 24.0) + 4.0 * dI_stride(K);
     auto chunk_cap = [&](int Cc) {
         long long best = 0;
         for (int i0 = 0; i0 < n; i0 += Cc) {
@@ -786,7 +870,7 @@ static int eval_render(tdi_batch* b, FrameList fl, const float* theta, hipStream
     if (dverts && (rc = launch_add_offsets(c->m.V, w.frames, fl.n, w.rt, dverts, w.P0, w.vproj, s))) return rc;
     if ((rc = launch_clear_keys_frames(w.frames, fl, w.keys, w.box, w.max_area, s))) return rc;
     if ((rc = launch_raster(c->m, w.frames, fl, w.vproj, c->opts.ntmp_cap, w.keys, w.box, s))) return rc;
-    if ((rc = launch_resolve(c->m, w.frames, fl, w.vproj, w.keys, w.cum, w.vis, w.npix, nullptr, w.pvert, w.pbary, w.max_area, w.tcount, w.tmax, w.box, s)))
+    if ((rc = launch_resolve(c->m, w.frames, fl, w.vproj, w.keys, w.cum, w.vis, w.npix, nullptr, w.pvert, w.pbary, w.ptri, w.max_area, w.tcount, w.tmax, w.box, s)))
         return rc;
     if ((rc = barrier_objective(b, L, fl, theta, s)))
         return rc;
@@ -848,7 +932,7 @@ static int eval_reused(tdi_batch* b, FrameList fl, const float* theta, hipStream
     Workspace& w = b->ws;
     int rc;
     if ((rc = launch_resolve(c->m, w.frames, fl, w.vproj, w.keys, w.cum, w.vis, w.npix, nullptr, w.pvert, w.pbary,
-                             w.max_area, w.tcount, w.tmax, w.box, s)))
+                             w.ptri, w.max_area, w.tcount, w.tmax, w.box, s)))
         return rc;
     if ((rc = barrier_objective(b, L, fl, theta, s)))
         return rc;
@@ -864,8 +948,8 @@ static int eval_jacobian(tdi_batch* b, FrameList fl, const float* theta, int mix
     const Layout& L = Lp ? *Lp : c->L;
     Workspace& w = b->ws;
     int rc;
-    if ((rc = launch_dI(b->m, L, w.frames, fl, theta, w.P0, w.pvert, w.pbary, w.npix, w.pixg, w.dI,
-                        dI_area(w), s)))
+    if ((rc = launch_dI(b->m, L, w.frames, fl, theta, w.P0, w.pvert, w.pbary, w.npix, w.pixg, jac_scratch(w), w.dI,
+                        dI_area(w), w.max_area, s)))
         return rc;
     if (L.K > SMALL_JTJ_MAXK) {
         // hundreds of unknowns (the identity stage): J^T J on FP64 MFMA over 64 x 64 tiles and
@@ -945,7 +1029,7 @@ int tdi_rasterize(tdi_batch* b, const float* xyz, const float* xyp, uint64_t* ke
         if ((rc = launch_clear_keys(w.keys, len, s))) return rc;
         if ((rc = launch_misc_fill_f32(w.bary, 2 * len, 0.f, s))) return rc;
         if ((rc = launch_raster(c->m, w.frames, all_frames(n), w.vproj, c->opts.ntmp_cap, w.keys, w.box, s))) return rc;
-        if ((rc = launch_resolve(c->m, w.frames, all_frames(n), w.vproj, w.keys, w.cum, w.vis, w.npix, w.bary, w.pvert, w.pbary, w.max_area, w.tcount, w.tmax, w.box, s)))
+        if ((rc = launch_resolve(c->m, w.frames, all_frames(n), w.vproj, w.keys, w.cum, w.vis, w.npix, w.bary, w.pvert, w.pbary, w.ptri, w.max_area, w.tcount, w.tmax, w.box, s)))
             return rc;
         if (keys) TDI_HIP(hipMemcpyAsync(keys + off, w.keys, sizeof(uint64_t) * len, hipMemcpyDeviceToDevice, s));
         if (bary) TDI_HIP(hipMemcpyAsync(bary + 2 * off, w.bary, sizeof(float) * 2 * len, hipMemcpyDeviceToDevice, s));
@@ -1766,7 +1850,7 @@ int tdi_batch_autotune(tdi_batch* b, const float* theta, int32_t reps, int32_t* 
     float best = 1e30f;
     for (int i = 0; i < 4 && !rc; ++i) {
         rc = timed([&] { return launch_dI(b->m, c->L, w.frames, all_frames(n), theta, w.P0, w.pvert, w.pbary, w.npix,
-                                          w.pixg, w.dI, areas[i], s); },
+                                          w.pixg, jac_scratch(w), w.dI, areas[i], w.max_area, s); },
                    rep[i]);
         if (!rc && rep[i] < best) { best = rep[i]; best_area = areas[i]; }
     }
@@ -1823,7 +1907,7 @@ int tdi_stage_times(tdi_batch* b, const float* theta, int32_t mixed, int32_t rep
         TDI_HIP(hipEventRecord(ev[1], s));
         if ((rc = launch_clear_keys_frames(w.frames, all_frames(n), w.keys, w.box, w.max_area, s))) return rc;
         if ((rc = launch_raster(c->m, w.frames, all_frames(n), w.vproj, c->opts.ntmp_cap, w.keys, w.box, s))) return rc;
-        if ((rc = launch_resolve(c->m, w.frames, all_frames(n), w.vproj, w.keys, w.cum, w.vis, w.npix, nullptr, w.pvert, w.pbary, w.max_area, w.tcount, w.tmax, w.box, s)))
+        if ((rc = launch_resolve(c->m, w.frames, all_frames(n), w.vproj, w.keys, w.cum, w.vis, w.npix, nullptr, w.pvert, w.pbary, w.ptri, w.max_area, w.tcount, w.tmax, w.box, s)))
             return rc;
         TDI_HIP(hipEventRecord(ev[2], s));
         if ((rc = launch_shade(b->m, c->L, w.frames, all_frames(n), theta, w.P0, w.pvert, w.pbary, w.npix, w.box, w.img,
@@ -1837,8 +1921,8 @@ int tdi_stage_times(tdi_batch* b, const float* theta, int32_t mixed, int32_t rep
         if ((rc = barrier_objective(b, c->L, all_frames(n), theta, s)))
             return rc;
         TDI_HIP(hipEventRecord(ev[4], s));
-        if ((rc = launch_dI(b->m, c->L, w.frames, all_frames(n), theta, w.P0, w.pvert, w.pbary, w.npix, w.pixg, w.dI,
-                            dI_area(w), s)))
+        if ((rc = launch_dI(b->m, c->L, w.frames, all_frames(n), theta, w.P0, w.pvert, w.pbary, w.npix, w.pixg,
+                            jac_scratch(w), w.dI, dI_area(w), w.max_area, s)))
             return rc;
         TDI_HIP(hipEventRecord(ev[5], s));
         if ((rc = launch_normal_eq(b, all_frames(n), mixed, s))) return rc;

@@ -55,7 +55,14 @@ struct ModelGPU {
     // the order the shading sums them), when the albedo is fitted: the shading and the Jacobian
     // then read them instead of summing the basis at every pixel (NULL: they sum it)
     const float* alb = nullptr;
+    // Mesh patches: groups of triangles over at most PATCH_VERTS vertices (ctx creation), for kernels that
+    // keep a patch's basis rows in LDS.  np = 0: none (a mesh of more than PATCH_MAX patches).
+    int np = 0;
+    const int* patch_off = nullptr;    // [np + 1] into patch_vert
+    const int* patch_vert = nullptr;   // vertex ids
+    const uint2* tri_patch = nullptr;  // [NT] patch, corners' places in it (8 bits each, tris' order)
 };
+constexpr int PATCH_VERTS = 128, PATCH_MAX = 4096;
 
 // One frame of a batch, device-resident.
 struct FrameGPU {
@@ -372,10 +379,10 @@ int launch_box_full(const FrameGPU* frames, int n, int4* box, hipStream_t s);
 // tcount: [slots][tmax] tile counts, tmax >= resolve_tiles(largest crop)
 int resolve_tiles(int max_area);
 // pvert/pbary: per visible position (vb, vc, va, crop index k) and (alpha, beta), so that the
-// per-pixel kernels after resolve reach the vertices in one load
+// per-pixel kernels after resolve reach the vertices in one load; ptri: its triangle's patch entry
 int launch_resolve(const ModelGPU& m, const FrameGPU* frames, FrameList fl, const float4* vproj,
                    const uint64_t* keys, int* cum, int* vis_list, int* npix, float* bary, int4* pvert,
-                   float2* pbary, int max_area, int* tcount, int tmax, int4* box, hipStream_t s);
+                   float2* pbary, uint2* ptri, int max_area, int* tcount, int tmax, int4* box, hipStream_t s);
 
 // visible box (and tile counts) only, for the passes that work from the keys
 int launch_visible_box(const FrameGPU* frames, FrameList fl, const uint64_t* keys, int max_area, int* tcount,
@@ -408,9 +415,20 @@ int launch_obs_prepare(const FrameGPU* frames, int n, const float* taps, const f
 int launch_ortho_init(const ModelGPU& m, int n, const float* lmk, const float* cams, float* x_orth, float* pose,
                       float* angles, int* info, hipStream_t s);
 
+// row stride of dI: K padded so that rows start on 16 bytes
+inline __host__ __device__ int dI_stride(int K) { return (K + 3) & ~3; }
+// per visible position: q (dI of a model-space direction e is q . e); Id and S of the shading (fitted
+// albedo only); patch and corners of its triangle; per frame the positions sorted by patch
+struct JacScratch {
+    float4* pq;
+    float2* pshade;
+    const uint2* ptri;
+    uint2* plist;
+    int* pstart;           // [slots][np + 1]
+};
 int launch_dI(const ModelGPU& m, const Layout& L, const FrameGPU* frames, FrameList fl, const float* theta,
               const double* P0, const int4* pvert, const float2* pbary, const int* npix, const float4* pixg,
-              float* dI, int mean_area, hipStream_t s);
+              const JacScratch& js, float* dI, int mean_area, int max_area, hipStream_t s);
 // the light columns alone ([pixel][4]: lambda, Lintensity) of the four appended light unknowns
 int launch_dI_light(const ModelGPU& m, const Layout& L, const FrameGPU* frames, FrameList fl, const float* theta,
                     const double* P0, const int4* pvert, const float2* pbary, const int* npix, float* dIl, int max_area,

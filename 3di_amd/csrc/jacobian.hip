@@ -14,9 +14,9 @@
 //   cublasSgemm (derivative_computer.cu:159-164): H += w (Jx^T Jx + Jy^T Jy),
 //   g -= w (Jx^T g^s_x + Jy^T g^s_y).
 //
-// k_dI          : four pixels per wavefront, 16 lanes over the K columns of each, so four
-//                 independent gather chains (triangle -> vertices -> basis rows) are in flight
-//                 per wave; basis rows are read with unit stride across the 16 lanes.
+// k_dI_px       : a thread per visible pixel: pose and light columns and what the other columns need.
+// k_dI_patch    : the expression and identity columns of many frames from mesh patches in LDS.
+// k_dI          : the same by gathers (few frames), and the albedo columns.
 // k_jtj_f32     : FP32 J^T J / J^T r from LDS-staged J rows, 4x4 register tiles (plain path).
 // k_jtj_lds     : one row u = c |d| s per pixel (the reference's two rows are parallel), formed
 //                 from branch-free gathers of dI, split into BF16 parts (hi/mid/lo) in LDS in
@@ -58,22 +58,164 @@ __device__ inline void load_frame_rot(const Layout& L, const FrameGPU& fr, const
     for (int k = 0; k < 5; ++k) s.sh[k] = L.nlight == 9 ? tf[L.off_light + 4 + k] : 0.f;
 }
 
-constexpr int DI_PX_PER_WG = 256;   // pixels per workgroup and frame in k_dI
-constexpr int DI_PASSES = 4;        // strip passes of k_dI (its grid's z)
+// The per-pixel part of the Jacobian, a thread per visible pixel: q (dI of a model-space direction e
+// is q . e), the pose and light columns, and with a fitted albedo Id and S for its columns.  Inside the
+// column kernel these ran once per 16 lanes, FP64 normal and divisions included, and took more of its
+// time than the gathers.  The columns (at most 15 per pixel) leave through LDS so that a row's are
+// stored together.
+constexpr int PX_COLS = 15;
 
-// Four wavefronts per SIMD (register budget 128): more pixels' gathers in flight per CU.
-// IDTEX: the layout has identity or albedo columns (the identity stage); the per-frame fit's
-// instantiation carries none of their code, which would cost it registers.
-template <bool IDTEX>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k_dI(ModelGPU m, Layout L, const FrameGPU* __restrict__ frames,
-                                             const int* __restrict__ act, int n, const float* __restrict__ theta,
-                                             const double* __restrict__ P0, const int4* __restrict__ pvert,
-                                             const float2* __restrict__ pbary, const int* __restrict__ npix,
-                                             const float4* __restrict__ pixg, float* __restrict__ dI)
+__global__ void __launch_bounds__(256) k_dI_px(ModelGPU m, Layout L, const FrameGPU* __restrict__ frames,
+                                                const int* __restrict__ act, int n, const float* __restrict__ theta,
+                                                const double* __restrict__ P0, const int4* __restrict__ pvert,
+                                                const float2* __restrict__ pbary, const int* __restrict__ npix,
+                                                const float4* __restrict__ pixg, float4* __restrict__ pq,
+                                                float2* __restrict__ pshade, float* __restrict__ dI)
 {
     __shared__ FrameRot sr;
     __shared__ float stex[512];
+    __shared__ float scol[4][64][PX_COLS + 2];
     const int nact = fl_count(act, n);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int K = L.K, ldI = dI_stride(K), ncol = K - L.off_pose;
+    for (int yi = blockIdx.y; yi < nact; yi += gridDim.y) {
+        const int f = fl_frame(act, yi);
+        const int N = npix[f];
+        if ((int)blockIdx.x * 256 >= N) continue;
+        const FrameGPU fr = frames[f];
+        const float* tf = theta + (size_t)f * K;
+        if (threadIdx.x == 0) load_frame_rot(L, fr, tf, sr);
+        for (int q = threadIdx.x; q < L.ntex; q += blockDim.x) stex[q] = tf[L.off_tex + q];
+        __syncthreads();
+        const long long base = fr.pix_off;
+        const double* P0f = P0 + (size_t)f * m.V * 3;
+        for (int p0 = blockIdx.x * 256; p0 < N; p0 += gridDim.x * 256) {
+            const int pos = min(p0 + (int)threadIdx.x, N - 1);
+            const int4 pv = pvert[base + pos];
+            const float2 ab = pbary[base + pos];
+            const float al = ab.x, be = ab.y, ga = gamma_rn(al, be);
+            const int vb = pv.x, vc = pv.y, va = pv.z;
+            float v[3], p0v[3];
+            double p0d[3];
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+                p0d[a] = (double)al * P0f[3 * vb + a] + (double)be * P0f[3 * vc + a] + (double)ga * P0f[3 * va + a];
+                p0v[a] = (float)p0d[a];
+            }
+            // camera-space surface point R p0 + tau (R column-major)
+#pragma unroll
+            for (int a = 0; a < 3; ++a)
+                v[a] = sr.R[a] * p0v[0] + sr.R[3 + a] * p0v[1] + sr.R[6 + a] * p0v[2] + sr.tau[a];
+            const float4 gg = pixg[base + pos];
+            const float iz = 1.f / v[2];
+            // dI = c . dv with c = (-gx phix / vz, -gy phiy / vz, (gx phix vx + gy phiy vy) / vz^2)
+            const float c0 = -gg.x * fr.phix * iz;
+            const float c1 = -gg.y * fr.phiy * iz;
+            const float c2 = (gg.x * fr.phix * v[0] + gg.y * fr.phiy * v[1]) * iz * iz;
+            // q = R^T c, so that dI for a model-space direction e is q . e
+            const float q0 = sr.R[0] * c0 + sr.R[1] * c1 + sr.R[2] * c2;
+            const float q1 = sr.R[3] * c0 + sr.R[4] * c1 + sr.R[5] * c2;
+            const float q2 = sr.R[6] * c0 + sr.R[7] * c1 + sr.R[8] * c2;
+            float* col = scol[wave][lane];
+            col[0] = c0;
+            col[1] = c1;
+            col[2] = c2;
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                const float* d = sr.dR + 9 * i;
+                const float dvx = d[0] * p0v[0] + d[3] * p0v[1] + d[6] * p0v[2];
+                const float dvy = d[1] * p0v[0] + d[4] * p0v[1] + d[7] * p0v[2];
+                const float dvz = d[2] * p0v[0] + d[5] * p0v[1] + d[8] * p0v[2];
+                col[3 + i] = c0 * dvx + c1 * dvy + c2 * dvz;
+            }
+            // shading quantities for albedo and light columns
+            if (L.ntex || L.nlight) {
+                // normal and Id in FP64 from the FP64 corners (edges of about a millimetre)
+                const double* B0 = P0f + 3 * vb;
+                const double* C0 = P0f + 3 * vc;
+                const double* A0 = P0f + 3 * va;
+                const double e1x = B0[0] - A0[0], e1y = B0[1] - A0[1], e1z = B0[2] - A0[2];
+                const double e2x = C0[0] - A0[0], e2y = C0[1] - A0[1], e2z = C0[2] - A0[2];
+                double ndx = e1y * e2z - e1z * e2y, ndy = e1z * e2x - e1x * e2z, ndz = e1x * e2y - e1y * e2x;
+                const double inv = 1.0 / sqrt(ndx * ndx + ndy * ndy + ndz * ndz);
+                ndx *= inv; ndy *= inv; ndz *= inv;
+                const double d0 = (double)sr.lam[0] - sr.tau[0], d1 = (double)sr.lam[1] - sr.tau[1],
+                             d2 = (double)sr.lam[2] - sr.tau[2];
+                const double lx = sr.R[0] * d0 + sr.R[1] * d1 + sr.R[2] * d2;
+                const double ly = sr.R[3] * d0 + sr.R[4] * d1 + sr.R[5] * d2;
+                const double lz = sr.R[6] * d0 + sr.R[7] * d1 + sr.R[8] * d2;
+                const float Id = (float)(ndx * lx + ndy * ly + ndz * lz - (ndx * p0d[0] + ndy * p0d[1] + ndz * p0d[2]));
+                const float nx = (float)ndx, ny = (float)ndy, nz = (float)ndz;
+                const float* rsrc = m.alb ? m.alb + (size_t)f * m.V : m.tex_mean;
+                float rb = rsrc[vb], rc = rsrc[vc], ra = rsrc[va];
+                for (int q = 0; !m.alb && q < L.ntex; ++q) {
+                    rb = fmaf(m.tex_basis[(size_t)vb * m.tex_ld + q], stex[q], rb);
+                    rc = fmaf(m.tex_basis[(size_t)vc * m.tex_ld + q], stex[q], rc);
+                    ra = fmaf(m.tex_basis[(size_t)va * m.tex_ld + q], stex[q], ra);
+                }
+                const float rho = al * rb + be * rc + ga * ra;
+                float rn[3], Y[5] = {0.f, 0.f, 0.f, 0.f, 0.f}, S = 0.f;
+                rn[0] = sr.R[0] * nx + sr.R[3] * ny + sr.R[6] * nz;
+                rn[1] = sr.R[1] * nx + sr.R[4] * ny + sr.R[7] * nz;
+                rn[2] = sr.R[2] * nx + sr.R[5] * ny + sr.R[8] * nz;
+                if (L.nlight == 9) {
+                    sh2_terms(rn, Y);
+                    S = rn[0] * sr.a[0] + rn[1] * sr.a[1] + rn[2] * sr.a[2];
+#pragma unroll
+                    for (int k = 0; k < 5; ++k) S += sr.sh[k] * Y[k];
+                }
+                if (L.nlight) {
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) col[6 + c] = (L.nlight == 9 ? rho : sr.L * rho) * rn[c];
+                    col[9] = rho * Id;
+                    if (L.nlight == 9) {
+#pragma unroll
+                        for (int k = 0; k < 5; ++k) col[10 + k] = rho * Y[k];
+                    }
+                }
+                if (L.ntex && p0 + (int)threadIdx.x < N) pshade[base + pos] = make_float2(Id, S);
+            }
+            if (p0 + (int)threadIdx.x < N) pq[base + pos] = make_float4(q0, q1, q2, 0.f);
+            // this wavefront's 64 rows, four at a time
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            const int w0 = p0 + 64 * wave, l16 = lane & 15;
+            float* out = dI + (size_t)(base + w0) * ldI + L.off_pose + l16;
+#pragma unroll 4
+            for (int r = lane >> 4; r < 64; r += 4)
+                if (w0 + r < N && l16 < ncol) out[(size_t)r * ldI] = scol[wave][r][l16];
+            __builtin_amdgcn_wave_barrier();
+        }
+        __syncthreads();   // sr and stex are rewritten by the next iteration
+    }
+}
+
+constexpr int DI_PX_PER_WG = 256;   // pixels per workgroup and frame in k_dI
+constexpr int DI_PASSES = 4;        // strip passes of k_dI (its grid's z)
+
+// One column value of a geometric block: q . (al e_b + be e_c + ga e_a), one order of roundings for every
+// kernel that forms it.
+__device__ __forceinline__ float dI_value(float q0, float q1, float q2, float al, float be, float ga, float bx, float by,
+                                          float bz, float cx, float cy, float cz, float ax, float ay, float az)
+{
+    const float ex = fmaf(ga, ax, fmaf(al, bx, be * cx));
+    const float ey = fmaf(ga, ay, fmaf(al, by, be * cy));
+    const float ez = fmaf(ga, az, fmaf(al, bz, be * cz));
+    return fmaf(q2, ez, fmaf(q1, ey, q0 * ex));
+}
+
+// The basis columns by gathers from the bases, four pixels per wavefront and 16 lanes over the columns
+// of each, so four independent gather chains are in flight per wave; basis rows are read with unit
+// stride across the 16 lanes.  geo: the expression and identity columns (else only the albedo's).
+__global__ void __launch_bounds__(256) k_dI(ModelGPU m, Layout L, const FrameGPU* __restrict__ frames,
+                                             const int* __restrict__ act, int n, const float* __restrict__ theta,
+                                             const int4* __restrict__ pvert, const float2* __restrict__ pbary,
+                                             const int* __restrict__ npix, const float4* __restrict__ pq,
+                                             const float2* __restrict__ pshade, int geo, float* __restrict__ dI)
+{
+    const int nact = fl_count(act, n);
+    const int ldI = dI_stride(L.K);
     for (int yi = blockIdx.y; yi < nact; yi += gridDim.y) {
     const int f = fl_frame(act, yi);
     const int N = npix[f];
@@ -82,7 +224,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
     // dispatcher places on one XCD (workgroups are dealt round-robin to the 8 XCDs and gridDim.x
     // is a multiple of 8): each XCD's L2 then holds the basis rows of one strip of the mesh.
     // A strip is shared by as many workgroups as give each about DI_PX_PER_WG pixels; the
-    // others leave before the frame set-up.
+    // others leave at once.
     // With gridDim.z passes the frame is cut into 8 gridDim.z strips: pass z takes strips
     // 8 z .. 8 z + 7 of every frame, and the dispatcher issues pass 0's workgroups (all frames)
     // before pass 1's, so an XCD's L2 holds the rows of a narrower strip at a time.
@@ -90,17 +232,12 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
     const int strip = (blockIdx.x & 7) + 8 * (int)blockIdx.z, sb = blockIdx.x >> 3;
     const int nsb = max(1, min((int)(gridDim.x >> 3), (N + nst * DI_PX_PER_WG - 1) / (nst * DI_PX_PER_WG)));
     if (sb >= nsb) continue;
-    const FrameGPU fr = frames[f];
-    const float* tf = theta + (size_t)f * L.K;
-    if (threadIdx.x == 0) load_frame_rot(L, fr, tf, sr);
-    for (int q = threadIdx.x; q < L.ntex; q += blockDim.x) stex[q] = tf[L.off_tex + q];
-    __syncthreads();
-    const long long base = fr.pix_off;
+    const long long base = frames[f].pix_off;
     const int lane = threadIdx.x & 63;
     const int wave = uniform(threadIdx.x >> 6);
     const int sub = lane >> 4, l16 = lane & 15;      // four pixels per wavefront, 16 lanes each
-    const double* P0f = P0 + (size_t)f * m.V * 3;
-    const int K = L.K;
+    const float* tf = theta + (size_t)f * L.K;
+    const float Li = L.nlight ? tf[L.off_light + 3] : frames[f].Lint;
     const int q0 = (int)((long long)N * strip / nst), q1 = (int)((long long)N * (strip + 1) / nst);
     for (int pos0 = q0 + (sb * 4 + wave) * 4; pos0 < q1; pos0 += nsb * 16) {
         const int pos = pos0 + sub;
@@ -109,123 +246,42 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
         const float2 ab = pbary[base + pos];
         const float al = ab.x, be = ab.y, ga = gamma_rn(al, be);
         const int vb = pv.x, vc = pv.y, va = pv.z;
-        float v[3], p0[3];
-        double p0d[3];
+        float* out = dI + (size_t)(base + pos) * ldI;
+        if (geo) {
+            const float4 q = pq[base + pos];
+            // 80 columns per group: every basis gather of the group is issued before the arithmetic
+            // (clamped columns, masked stores), so the group costs one round trip
+            for (int blk = 0; blk < 2; ++blk) {
+                const int nc = blk ? L.nid : L.nexp, off = blk ? L.off_id : L.off_exp, ld = blk ? m.id_ld : m.exp_ld;
+                const float* basis = blk ? m.id_basis : m.exp_basis;
+                const float* Eb = basis + (size_t)(3 * vb) * ld;   // rows 3v, 3v+1, 3v+2
+                const float* Ec = basis + (size_t)(3 * vc) * ld;
+                const float* Ea = basis + (size_t)(3 * va) * ld;
+                for (int c0 = 0; c0 < nc; c0 += 80) {
+                    float eb[5][3], ec[5][3], ea[5][3];
 #pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            p0d[a] = (double)al * P0f[3 * vb + a] + (double)be * P0f[3 * vc + a] + (double)ga * P0f[3 * va + a];
-            p0[a] = (float)p0d[a];
-        }
-        // camera-space surface point R p0 + tau (R column-major)
+                    for (int i = 0; i < 5; ++i) {
+                        const int c = min(c0 + 16 * i + l16, nc - 1);
 #pragma unroll
-        for (int a = 0; a < 3; ++a) v[a] = sr.R[a] * p0[0] + sr.R[3 + a] * p0[1] + sr.R[6 + a] * p0[2] + sr.tau[a];
-        const float4 gg = pixg[base + pos];
-        const float iz = 1.f / v[2];
-        // dI = c . dv with c = (-gx phix / vz, -gy phiy / vz, (gx phix vx + gy phiy vy) / vz^2)
-        const float c0 = -gg.x * fr.phix * iz;
-        const float c1 = -gg.y * fr.phiy * iz;
-        const float c2 = (gg.x * fr.phix * v[0] + gg.y * fr.phiy * v[1]) * iz * iz;
-        // q = R^T c, so that dI for a model-space direction e is q . e
-        const float q0 = sr.R[0] * c0 + sr.R[1] * c1 + sr.R[2] * c2;
-        const float q1 = sr.R[3] * c0 + sr.R[4] * c1 + sr.R[5] * c2;
-        const float q2 = sr.R[6] * c0 + sr.R[7] * c1 + sr.R[8] * c2;
-        // shading quantities for albedo and light columns
-        float rho = 0.f, Id = 0.f, rn[3] = {0.f, 0.f, 0.f}, Y[5] = {0.f, 0.f, 0.f, 0.f, 0.f}, S = 0.f;
-        if (L.ntex || L.nlight) {
-            // normal and Id in FP64 from the FP64 corners (edges of about a millimetre)
-            const double* B0 = P0f + 3 * vb;
-            const double* C0 = P0f + 3 * vc;
-            const double* A0 = P0f + 3 * va;
-            const double e1x = B0[0] - A0[0], e1y = B0[1] - A0[1], e1z = B0[2] - A0[2];
-            const double e2x = C0[0] - A0[0], e2y = C0[1] - A0[1], e2z = C0[2] - A0[2];
-            double ndx = e1y * e2z - e1z * e2y, ndy = e1z * e2x - e1x * e2z, ndz = e1x * e2y - e1y * e2x;
-            const double inv = 1.0 / sqrt(ndx * ndx + ndy * ndy + ndz * ndz);
-            ndx *= inv; ndy *= inv; ndz *= inv;
-            const double d0 = (double)sr.lam[0] - sr.tau[0], d1 = (double)sr.lam[1] - sr.tau[1],
-                         d2 = (double)sr.lam[2] - sr.tau[2];
-            const double lx = sr.R[0] * d0 + sr.R[1] * d1 + sr.R[2] * d2;
-            const double ly = sr.R[3] * d0 + sr.R[4] * d1 + sr.R[5] * d2;
-            const double lz = sr.R[6] * d0 + sr.R[7] * d1 + sr.R[8] * d2;
-            Id = (float)(ndx * lx + ndy * ly + ndz * lz - (ndx * p0d[0] + ndy * p0d[1] + ndz * p0d[2]));
-            const float nx = (float)ndx, ny = (float)ndy, nz = (float)ndz;
-            const float* rsrc = m.alb ? m.alb + (size_t)f * m.V : m.tex_mean;
-            float rb = rsrc[vb], rc = rsrc[vc], ra = rsrc[va];
-            for (int q = 0; !m.alb && q < L.ntex; ++q) {
-                rb = fmaf(m.tex_basis[(size_t)vb * m.tex_ld + q], stex[q], rb);
-                rc = fmaf(m.tex_basis[(size_t)vc * m.tex_ld + q], stex[q], rc);
-                ra = fmaf(m.tex_basis[(size_t)va * m.tex_ld + q], stex[q], ra);
-            }
-            rho = al * rb + be * rc + ga * ra;
-            rn[0] = sr.R[0] * nx + sr.R[3] * ny + sr.R[6] * nz;
-            rn[1] = sr.R[1] * nx + sr.R[4] * ny + sr.R[7] * nz;
-            rn[2] = sr.R[2] * nx + sr.R[5] * ny + sr.R[8] * nz;
-            if (L.nlight == 9) {
-                sh2_terms(rn, Y);
-                S = rn[0] * sr.a[0] + rn[1] * sr.a[1] + rn[2] * sr.a[2];
-#pragma unroll
-                for (int k = 0; k < 5; ++k) S += sr.sh[k] * Y[k];
-            }
-        }
-        float* out = dI + (size_t)(base + pos) * K;
-        // expression columns, 80 per group: every basis gather of the group is issued before
-        // the arithmetic (clamped columns, masked stores), so the group costs one round trip
-        if (L.nexp) {
-            const int ke = m.exp_ld;
-            const float* Eb = m.exp_basis + (size_t)(3 * vb) * ke;   // rows 3v, 3v+1, 3v+2
-            const float* Ec = m.exp_basis + (size_t)(3 * vc) * ke;
-            const float* Ea = m.exp_basis + (size_t)(3 * va) * ke;
-            for (int c0 = 0; c0 < L.nexp; c0 += 80) {
-                float eb[5][3], ec[5][3], ea[5][3];
-#pragma unroll
-                for (int i = 0; i < 5; ++i) {
-                    const int c = min(c0 + 16 * i + l16, L.nexp - 1);
-#pragma unroll
-                    for (int a = 0; a < 3; ++a) {
-                        eb[i][a] = Eb[(size_t)a * ke + c];
-                        ec[i][a] = Ec[(size_t)a * ke + c];
-                        ea[i][a] = Ea[(size_t)a * ke + c];
+                        for (int a = 0; a < 3; ++a) {
+                            eb[i][a] = Eb[(size_t)a * ld + c];
+                            ec[i][a] = Ec[(size_t)a * ld + c];
+                            ea[i][a] = Ea[(size_t)a * ld + c];
+                        }
                     }
-                }
 #pragma unroll
-                for (int i = 0; i < 5; ++i) {
-                    const int c = c0 + 16 * i + l16;
-                    const float ex = al * eb[i][0] + be * ec[i][0] + ga * ea[i][0];
-                    const float ey = al * eb[i][1] + be * ec[i][1] + ga * ea[i][1];
-                    const float ez = al * eb[i][2] + be * ec[i][2] + ga * ea[i][2];
-                    if (c < L.nexp) out[L.off_exp + c] = q0 * ex + q1 * ey + q2 * ez;
-                }
-            }
-        }
-        // identity columns (the identity stage), 80 per group as the expression columns
-        if (IDTEX && L.nid) {
-            const int ki = m.id_ld;
-            const float* Ib = m.id_basis + (size_t)(3 * vb) * ki;
-            const float* Ic = m.id_basis + (size_t)(3 * vc) * ki;
-            const float* Ia = m.id_basis + (size_t)(3 * va) * ki;
-            for (int c0 = 0; c0 < L.nid; c0 += 80) {
-                float eb[5][3], ec[5][3], ea[5][3];
-#pragma unroll
-                for (int i = 0; i < 5; ++i) {
-                    const int c = min(c0 + 16 * i + l16, L.nid - 1);
-#pragma unroll
-                    for (int a = 0; a < 3; ++a) {
-                        eb[i][a] = Ib[(size_t)a * ki + c];
-                        ec[i][a] = Ic[(size_t)a * ki + c];
-                        ea[i][a] = Ia[(size_t)a * ki + c];
+                    for (int i = 0; i < 5; ++i) {
+                        const int c = c0 + 16 * i + l16;
+                        const float val = dI_value(q.x, q.y, q.z, al, be, ga, eb[i][0], eb[i][1], eb[i][2], ec[i][0],
+                                                   ec[i][1], ec[i][2], ea[i][0], ea[i][1], ea[i][2]);
+                        if (c < nc) out[off + c] = val;
                     }
-                }
-#pragma unroll
-                for (int i = 0; i < 5; ++i) {
-                    const int c = c0 + 16 * i + l16;
-                    const float ex = al * eb[i][0] + be * ec[i][0] + ga * ea[i][0];
-                    const float ey = al * eb[i][1] + be * ec[i][1] + ga * ea[i][1];
-                    const float ez = al * eb[i][2] + be * ec[i][2] + ga * ea[i][2];
-                    if (c < L.nid) out[L.off_id + c] = q0 * ex + q1 * ey + q2 * ez;
                 }
             }
         }
         // albedo columns (the identity stage), 80 per group
-        if (IDTEX && L.ntex) {
+        if (L.ntex) {
+            const float2 sh = pshade[base + pos];
             const int kt = m.tex_ld;
             const float* Tb = m.tex_basis + (size_t)vb * kt;
             const float* Tc = m.tex_basis + (size_t)vc * kt;
@@ -243,29 +299,176 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
                 for (int i = 0; i < 5; ++i) {
                     const int c = c0 + 16 * i + l16;
                     const float tt = al * tb[i] + be * tc[i] + ga * ta[i];
-                    if (c < L.ntex) out[L.off_tex + c] = tt + sr.L * Id * tt + S * tt;
+                    if (c < L.ntex) out[L.off_tex + c] = tt + Li * sh.x * tt + sh.y * tt;
                 }
             }
         }
-        // the other columns: pose and light
-        for (int j = L.off_pose + l16; j < K; j += 16) {
-            float val;
-            if (j < L.off_pose + 3) {
-                val = (j == L.off_pose) ? c0 : (j == L.off_pose + 1) ? c1 : c2;
-            } else if (j < L.off_light) {
-                const float* d = sr.dR + 9 * (j - L.off_pose - 3);
-                const float dvx = d[0] * p0[0] + d[3] * p0[1] + d[6] * p0[2];
-                const float dvy = d[1] * p0[0] + d[4] * p0[1] + d[7] * p0[2];
-                const float dvz = d[2] * p0[0] + d[5] * p0[1] + d[8] * p0[2];
-                val = c0 * dvx + c1 * dvy + c2 * dvz;
-            } else {
-                const int c = j - L.off_light;
-                val = (c < 3) ? (L.nlight == 9 ? rho : sr.L * rho) * rn[c] : (c == 3) ? rho * Id : rho * Y[min(c - 4, 4)];
+    }
+    }
+}
+
+// The visible positions of a frame sorted by the mesh patch of their triangle: a count, a prefix sum and
+// a scatter by one workgroup per frame, the patches' counts in LDS.  plist: (position, corners' places).
+constexpr int BIN_THREADS = 1024;
+
+__global__ void __launch_bounds__(BIN_THREADS) k_patch_bin(const FrameGPU* __restrict__ frames, const int* __restrict__ act,
+                                                            int n, const int* __restrict__ npix, int np,
+                                                            const uint2* __restrict__ ptri, uint2* __restrict__ plist,
+                                                            int* __restrict__ pstart)
+{
+    __shared__ int hist[PATCH_MAX];
+    __shared__ int swave[BIN_THREADS / 64];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int nact = fl_count(act, n);
+    for (int yi = blockIdx.x; yi < nact; yi += gridDim.x) {
+        const int f = fl_frame(act, yi);
+        const long long base = frames[f].pix_off;
+        const int N = npix[f];
+        for (int p = tid; p < np; p += BIN_THREADS) hist[p] = 0;
+        __syncthreads();
+#pragma unroll 4
+        for (int pos = tid; pos < N; pos += BIN_THREADS) atomicAdd(&hist[ptri[base + pos].x], 1);
+        __syncthreads();
+        // exclusive prefix sum, PATCH_MAX / BIN_THREADS consecutive patches per thread
+        constexpr int PER = PATCH_MAX / BIN_THREADS;
+        int c[PER], sum = 0;
+#pragma unroll
+        for (int k = 0; k < PER; ++k) {
+            const int p = tid * PER + k;
+            c[k] = p < np ? hist[p] : 0;
+            sum += c[k];
+        }
+        int run = sum;
+        for (int o = 1; o < 64; o <<= 1) {
+            const int x = __shfl_up(run, o, 64);
+            if (lane >= o) run += x;
+        }
+        if (lane == 63) swave[wave] = run;
+        __syncthreads();
+        int at = run - sum;
+#pragma unroll
+        for (int w = 0; w < BIN_THREADS / 64; ++w) at += w < wave ? swave[w] : 0;
+        int* ps = pstart + (size_t)f * (np + 1);
+#pragma unroll
+        for (int k = 0; k < PER; ++k) {
+            const int p = tid * PER + k;
+            if (p < np) {
+                ps[p] = at;
+                hist[p] = at;
             }
-            out[j] = val;
+            at += c[k];
+        }
+        if (tid == 0) ps[np] = N;
+        __syncthreads();
+#pragma unroll 4
+        for (int pos = tid; pos < N; pos += BIN_THREADS) {
+            const uint2 t = ptri[base + pos];
+            plist[base + atomicAdd(&hist[t.x], 1)] = make_uint2((unsigned)pos, t.y);
+        }
+        __syncthreads();   // hist and swave are rewritten for the next frame
+    }
+}
+
+// One chunk of up to 80 geometric columns from mesh patches.  A visible pixel's columns need three
+// vertices' basis rows, 2880 bytes at 80 columns: gathered per pixel that is 8 times the row it writes,
+// through L2 and beyond (159 GB of HBM traffic for 4096 frames, 7.7 TB/s, 25.8 ms).  Here a workgroup
+// holds the rows of one patch (PATCH_VERTS vertices, 120 KB of LDS) and walks the pixels that all its
+// frames have on it, so a basis row leaves HBM once per slice of the list.  A wavefront takes a
+// frame's pixels 64 at a time: their records into its own part of LDS, then four pixels per step, 16
+// lanes over the columns of each (columns 4 l .. 4 l + 3 and 64 + l of lane l).
+constexpr int PT_THREADS = 1024, PT_WAVES = PT_THREADS / 64, PT_COLS = 80;
+constexpr size_t PT_LDS = sizeof(float) * PATCH_VERTS * 3 * PT_COLS + sizeof(float4) * 2 * 64 * PT_WAVES;
+
+__global__ void __launch_bounds__(PT_THREADS) k_dI_patch(ModelGPU m, const float* __restrict__ basis, int ld, int k0,
+                                                          int nc, int off, int ldI, const FrameGPU* __restrict__ frames,
+                                                          const int* __restrict__ act, int n,
+                                                          const uint2* __restrict__ plist, const int* __restrict__ pstart,
+                                                          const float4* __restrict__ pq, const float2* __restrict__ pbary,
+                                                          float* __restrict__ dI)
+{
+    extern __shared__ float4 spt[];
+    float* sE = (float*)spt;                                            // [vertex][axis][PT_COLS]
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = uniform(tid >> 6);
+    float4* rec = spt + PATCH_VERTS * 3 * PT_COLS / 4 + 2 * 64 * wave;  // [64]: (q, al), (be, ga, position, places)
+    const int nact = fl_count(act, n);
+    const int p = blockIdx.x;
+    const int y0 = (int)((long long)nact * blockIdx.y / gridDim.y), y1 = (int)((long long)nact * (blockIdx.y + 1) / gridDim.y);
+    if (y0 == y1) return;
+    {
+        const int* pv = m.patch_vert + m.patch_off[p];
+        const int nv = m.patch_off[p + 1] - m.patch_off[p];
+        for (int e = tid; e < nv * 3 * (PT_COLS / 4); e += PT_THREADS) {
+            const int r = e / (PT_COLS / 4), c4 = e - r * (PT_COLS / 4);
+            const int v = pv[r / 3], a = r % 3;
+            float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (k0 + 4 * c4 < ld) x = *(const float4*)(basis + (size_t)(3 * v + a) * ld + k0 + 4 * c4);
+            spt[e] = x;
         }
     }
-    __syncthreads();   // sr and stex are rewritten by the next iteration
+    __syncthreads();
+    const int sub = lane >> 4, l16 = lane & 15;
+    const bool vec = ((off + k0) & 3) == 0;
+    for (int yi = y0 + wave; yi < y1; yi += PT_WAVES) {
+        const int f = fl_frame(act, yi);
+        const long long base = frames[f].pix_off;
+        const int* ps = pstart + (size_t)f * (m.np + 1) + p;
+        const int e1 = ps[1];
+        for (int e0 = ps[0]; e0 < e1; e0 += 64) {
+            const int cnt = min(64, e1 - e0);
+            if (lane < cnt) {
+                const uint2 t = plist[base + e0 + lane];
+                const float4 q = pq[base + t.x];
+                const float2 ab = pbary[base + t.x];
+                rec[2 * lane] = make_float4(q.x, q.y, q.z, ab.x);
+                rec[2 * lane + 1] = make_float4(ab.y, gamma_rn(ab.x, ab.y), __uint_as_float(t.x), __uint_as_float(t.y));
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            for (int r = sub; r < cnt; r += 4) {
+                const float4 A = rec[2 * r], C = rec[2 * r + 1];
+                const float al = A.w, be = C.x, ga = C.y;
+                const unsigned ids = __float_as_uint(C.w);
+                const float* Eb = sE + (ids & 255) * (3 * PT_COLS);
+                const float* Ec = sE + ((ids >> 8) & 255) * (3 * PT_COLS);
+                const float* Ea = sE + ((ids >> 16) & 255) * (3 * PT_COLS);
+                float4 b4[3], c4[3], a4[3];
+                float b1[3], c1[3], a1[3];
+#pragma unroll
+                for (int a = 0; a < 3; ++a) {
+                    b4[a] = *(const float4*)(Eb + a * PT_COLS + 4 * l16);
+                    c4[a] = *(const float4*)(Ec + a * PT_COLS + 4 * l16);
+                    a4[a] = *(const float4*)(Ea + a * PT_COLS + 4 * l16);
+                    b1[a] = Eb[a * PT_COLS + 64 + l16];
+                    c1[a] = Ec[a * PT_COLS + 64 + l16];
+                    a1[a] = Ea[a * PT_COLS + 64 + l16];
+                }
+                float4 v;
+                v.x = dI_value(A.x, A.y, A.z, al, be, ga, b4[0].x, b4[1].x, b4[2].x, c4[0].x, c4[1].x, c4[2].x, a4[0].x,
+                               a4[1].x, a4[2].x);
+                v.y = dI_value(A.x, A.y, A.z, al, be, ga, b4[0].y, b4[1].y, b4[2].y, c4[0].y, c4[1].y, c4[2].y, a4[0].y,
+                               a4[1].y, a4[2].y);
+                v.z = dI_value(A.x, A.y, A.z, al, be, ga, b4[0].z, b4[1].z, b4[2].z, c4[0].z, c4[1].z, c4[2].z, a4[0].z,
+                               a4[1].z, a4[2].z);
+                v.w = dI_value(A.x, A.y, A.z, al, be, ga, b4[0].w, b4[1].w, b4[2].w, c4[0].w, c4[1].w, c4[2].w, a4[0].w,
+                               a4[1].w, a4[2].w);
+                const float v1 = dI_value(A.x, A.y, A.z, al, be, ga, b1[0], b1[1], b1[2], c1[0], c1[1], c1[2], a1[0], a1[1],
+                                          a1[2]);
+                float* out = dI + (size_t)(base + __float_as_uint(C.z)) * ldI + off + k0;
+                const int c = 4 * l16;
+                if (vec && c + 3 < nc) {
+                    *(float4*)(out + c) = v;
+                } else {
+                    if (c < nc) out[c] = v.x;
+                    if (c + 1 < nc) out[c + 1] = v.y;
+                    if (c + 2 < nc) out[c + 2] = v.z;
+                    if (c + 3 < nc) out[c + 3] = v.w;
+                }
+                if (64 + l16 < nc) out[64 + l16] = v1;
+            }
+            __builtin_amdgcn_wave_barrier();   // the next batch rewrites the records
+        }
     }
 }
 
@@ -402,7 +605,8 @@ __global__ void __launch_bounds__(256) k_jtj_f32(Layout L, const FrameGPU* __res
     const int T = KP / 4;
     const int ntiles = T * (T + 1) / 2;
     const int p0 = (int)((long long)N * s / S), p1 = (int)((long long)N * (s + 1) / S);
-    const float* dIf = dI + (size_t)fr.pix_off * K;
+    const int ldI = dI_stride(K);
+    const float* dIf = dI + (size_t)fr.pix_off * ldI;
     const int tid = threadIdx.x;
     float acc[2][16];
     int tI[2], tJ[2];
@@ -428,7 +632,7 @@ __global__ void __launch_bounds__(256) k_jtj_f32(Layout L, const FrameGPU* __res
         for (int e = tid; e < F32_CH * KP; e += 256) {
             const int p = e / KP, j = e - p * KP;
             float jx = 0.f, jy = 0.f;
-            if (spc[p].valid && j < K) jrow(spc[p], dIf, K, j, jx, jy);
+            if (spc[p].valid && j < K) jrow(spc[p], dIf, ldI, j, jx, jy);
             sJ[2 * p][j] = jx;
             sJ[2 * p + 1][j] = jy;
         }
@@ -739,8 +943,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(T >= 7
         const FrameGPU fr = frames[f];
         const int N = npix[f];
         const int K = L.K;
+        const int ldI = dI_stride(K);
         const int p0 = (int)((long long)N * s / S), p1 = (int)((long long)N * (s + 1) / S);
-        const float* dIf = dI + (size_t)fr.pix_off * K;
+        const float* dIf = dI + (size_t)fr.pix_off * ldI;
         v4f acc[MT];
 #pragma unroll
         for (int t = 0; t < MT; ++t) acc[t] = (v4f){0.f, 0.f, 0.f, 0.f};
@@ -786,10 +991,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(T >= 7
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
                     const int4 nb = snb[4 * pq + q];
-                    ld[r][4 * q + 0] = dIf[(size_t)nb.x * K + jj];
-                    ld[r][4 * q + 1] = dIf[(size_t)nb.y * K + jj];
-                    ld[r][4 * q + 2] = dIf[(size_t)nb.z * K + jj];
-                    ld[r][4 * q + 3] = dIf[(size_t)nb.w * K + jj];
+                    ld[r][4 * q + 0] = dIf[(size_t)nb.x * ldI + jj];
+                    ld[r][4 * q + 1] = dIf[(size_t)nb.y * ldI + jj];
+                    ld[r][4 * q + 2] = dIf[(size_t)nb.z * ldI + jj];
+                    ld[r][4 * q + 3] = dIf[(size_t)nb.w * ldI + jj];
                 }
             }
 #pragma unroll
@@ -899,7 +1104,8 @@ __global__ void __launch_bounds__(256) k_urows(int K, int KP, const FrameGPU* __
         const int f = fl_frame(act, yi);
         const FrameGPU fr = frames[f];
         const int N = npix[f];
-        const float* dIf = dI + (size_t)fr.pix_off * K;
+        const int ldI = dI_stride(K);
+        const float* dIf = dI + (size_t)fr.pix_off * ldI;
         for (int p0 = pb0 * UR_PX; p0 < N; p0 += npb * UR_PX) {
             const int pe = min(N, p0 + UR_PX);
             for (int p = p0; p < pe; ++p) {
@@ -912,8 +1118,8 @@ __global__ void __launch_bounds__(256) k_urows(int K, int KP, const FrameGPU* __
                 const float dn = sqrtf(dx * dx + dy * dy);
                 float u = 0.f;
                 if (j < K) {
-                    const float dh = dIf[(size_t)nb.y * K + j] - dIf[(size_t)nb.x * K + j];
-                    const float dv = dIf[(size_t)nb.w * K + j] - dIf[(size_t)nb.z * K + j];
+                    const float dh = dIf[(size_t)nb.y * ldI + j] - dIf[(size_t)nb.x * ldI + j];
+                    const float dv = dIf[(size_t)nb.w * ldI + j] - dIf[(size_t)nb.z * ldI + j];
                     const float wgt = c * dn;
                     u = wgt * dy * dh - wgt * dx * dv;
                 } else if (j == K) {
@@ -1094,27 +1300,50 @@ int jtj_splits(int n, int per_frame_pixels_hint)
     return S;
 }
 
+// From this many listed frames on, the geometric columns go through mesh patches.
+constexpr int PATCH_MIN_FRAMES = 8;
+
 int launch_dI(const ModelGPU& m, const Layout& L, const FrameGPU* frames, FrameList fl, const float* theta,
               const double* P0, const int4* pvert, const float2* pbary, const int* npix, const float4* pixg,
-              float* dI, int mean_area, hipStream_t s)
+              const JacScratch& js, float* dI, int mean_area, int max_area, hipStream_t s)
 {
     if (L.ntex > 512) {
         set_error("dI: k_tex %d > 512", L.ntex);
         return TDI_ERR_ARG;
     }
-    // 8 DI_PASSES strips per frame, each shared by up to nsb workgroups; one frame per grid row
-    // (sized for a quarter-visible mean crop: larger frames loop, and few workgroups of a grid
-    // row find no pixels)
-    int nsb = (mean_area / 4 + 8 * DI_PASSES * DI_PX_PER_WG - 1) / (8 * DI_PASSES * DI_PX_PER_WG);
-    if (nsb > 64) nsb = 64;
-    if (nsb < 1) nsb = 1;
-    const dim3 grid(8 * nsb, grid_frames(fl.n, 1 << 16), DI_PASSES);
-    if (L.nid || L.ntex)
-        hipLaunchKernelGGL(k_dI<true>, grid, dim3(256), 0, s, m, L, frames, fl.act, fl.n, theta, P0, pvert, pbary, npix,
-                           pixg, dI);
-    else
-        hipLaunchKernelGGL(k_dI<false>, grid, dim3(256), 0, s, m, L, frames, fl.act, fl.n, theta, P0, pvert, pbary, npix,
-                           pixg, dI);
+    const int gy = grid_frames(fl.n, 1 << 16);
+    // the pixel pass: sized for a half-visible largest crop, at most 64 workgroups per frame when many
+    const int px = std::max(1, std::min((max_area / 2 + 255) / 256, std::max(16, std::min(256, 8192 / std::max(1, fl.n)))));
+    hipLaunchKernelGGL(k_dI_px, dim3(px, gy), dim3(256), 0, s, m, L, frames, fl.act, fl.n, theta, P0, pvert, pbary, npix,
+                       pixg, js.pq, js.pshade, dI);
+    const bool patch = m.np > 0 && fl.n >= PATCH_MIN_FRAMES && L.nexp + L.nid > 0;
+    if (patch) {
+        // 155 KB of dynamic LDS, allowed once per process
+        static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(k_dI_patch),
+                                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)PT_LDS);
+        TDI_HIP(attr);
+        hipLaunchKernelGGL(k_patch_bin, dim3(gy), dim3(BIN_THREADS), 0, s, frames, fl.act, fl.n, npix, m.np, js.ptri,
+                           js.plist, js.pstart);
+        // about 64 frames per workgroup, four per wavefront: its patch is loaded once for them
+        const int slices = std::max(1, std::min(64, fl.n / 64));
+        for (int blk = 0; blk < 2; ++blk) {
+            const int nc = blk ? L.nid : L.nexp, off = blk ? L.off_id : L.off_exp, ld = blk ? m.id_ld : m.exp_ld;
+            for (int k0 = 0; k0 < nc; k0 += PT_COLS)
+                hipLaunchKernelGGL(k_dI_patch, dim3(m.np, slices), dim3(PT_THREADS), PT_LDS, s, m,
+                                   blk ? m.id_basis : m.exp_basis, ld, k0, std::min(PT_COLS, nc - k0), off, dI_stride(L.K),
+                                   frames, fl.act, fl.n, js.plist, js.pstart, js.pq, pbary, dI);
+        }
+    }
+    if (!patch || L.ntex) {
+        // 8 DI_PASSES strips per frame, each shared by up to nsb workgroups; one frame per grid row
+        // (sized for a quarter-visible mean crop: larger frames loop, and few workgroups of a grid
+        // row find no pixels)
+        int nsb = (mean_area / 4 + 8 * DI_PASSES * DI_PX_PER_WG - 1) / (8 * DI_PASSES * DI_PX_PER_WG);
+        if (nsb > 64) nsb = 64;
+        if (nsb < 1) nsb = 1;
+        hipLaunchKernelGGL(k_dI, dim3(8 * nsb, gy, DI_PASSES), dim3(256), 0, s, m, L, frames, fl.act, fl.n, theta, pvert,
+                           pbary, npix, js.pq, js.pshade, patch ? 0 : 1, dI);
+    }
     TDI_HIP(hipGetLastError());
     return TDI_OK;
 }

@@ -268,7 +268,9 @@ __global__ void __launch_bounds__(RES_THREADS) k_resolve_write(const int* __rest
                                                                 const int4* __restrict__ box,
                                                                 int* __restrict__ cum, int* __restrict__ vis,
                                                                 int* __restrict__ npix, float2* __restrict__ bary,
-                                                                int4* __restrict__ pvert, float2* __restrict__ pbary)
+                                                                int4* __restrict__ pvert, float2* __restrict__ pbary,
+                                                                const uint2* __restrict__ tri_patch,
+                                                                uint2* __restrict__ ptri)
 {
     __shared__ int swave[RES_NW];
     __shared__ int soff[RES_NW];
@@ -322,6 +324,7 @@ __global__ void __launch_bounds__(RES_THREADS) k_resolve_write(const int* __rest
             // so that they are in flight together; then the coverage arithmetic and the stores
             int tv[RES_PER_THREAD][3];
             float4 tB[RES_PER_THREAD], tC[RES_PER_THREAD], tA[RES_PER_THREAD];
+            uint2 tp[RES_PER_THREAD];
 #pragma unroll
             for (int q = 0; q < RES_PER_THREAD; ++q) {
                 tv[q][0] = tv[q][1] = tv[q][2] = 0;
@@ -330,6 +333,7 @@ __global__ void __launch_bounds__(RES_THREADS) k_resolve_write(const int* __rest
                     tv[q][0] = tris[3 * t];
                     tv[q][1] = tris[3 * t + 1];
                     tv[q][2] = tris[3 * t + 2];
+                    if (tri_patch) tp[q] = tri_patch[t];
                 }
             }
 #pragma unroll
@@ -353,6 +357,7 @@ __global__ void __launch_bounds__(RES_THREADS) k_resolve_write(const int* __rest
                     if (bary) bary[base + k] = make_float2(al, be);
                     pvert[base + pos] = make_int4(tv[q][0], tv[q][1], tv[q][2], k);
                     pbary[base + pos] = make_float2(al, be);
+                    if (tri_patch) ptri[base + pos] = tp[q];
                     ++pos;
                 }
             }
@@ -453,7 +458,7 @@ int launch_visible_box(const FrameGPU* frames, FrameList fl, const uint64_t* key
 
 int launch_resolve(const ModelGPU& m, const FrameGPU* frames, FrameList fl, const float4* vproj,
                    const uint64_t* keys, int* cum, int* vis_list, int* npix, float* bary, int4* pvert,
-                   float2* pbary, int max_area, int* tcount, int tmax, int4* box, hipStream_t s)
+                   float2* pbary, uint2* ptri, int max_area, int* tcount, int tmax, int4* box, hipStream_t s)
 {
     int bx = resolve_tiles(max_area);
     if (bx > tmax) {
@@ -466,7 +471,7 @@ int launch_resolve(const ModelGPU& m, const FrameGPU* frames, FrameList fl, cons
                        (const unsigned long long*)keys, tcount, tmax, box);
     hipLaunchKernelGGL(k_resolve_write, grid, dim3(RES_THREADS), 0, s, m.tris, m.V, frames, fl.act, fl.n, vproj,
                        (const unsigned long long*)keys, tcount, tmax, box, cum, vis_list, npix, (float2*)bary,
-                       pvert, pbary);
+                       pvert, pbary, ptri ? m.tri_patch : nullptr, ptri);
     TDI_HIP(hipGetLastError());
     return TDI_OK;
 }
