@@ -918,7 +918,7 @@ static int launch_normal_eq(tdi_batch* b, FrameList fl, int mixed, hipStream_t s
     if (mixed & TDI_MIXED_JTJ_BF16)
         return launch_jtj_mfma(L, w.frames, fl, w.npix, w.pnb, w.pcoef, w.pixg, w.dI, c->opts.data_weight, w.H,
                                w.g, w.partials, w.S, (mixed & TDI_MIXED_JTR_BF16) ? 1 : 0,
-                               (mixed & TDI_MIXED_TWO_TERM) ? 1 : 0, s);
+                               (mixed & TDI_MIXED_TWO_TERM) ? 1 : 0, w.max_area, s);
     return launch_jtj_f32(L, w.frames, fl, w.npix, w.pnb, w.pcoef, w.pixg, w.dI, c->opts.data_weight, w.H, w.g,
                           w.partials, w.S, s);
 }

@@ -451,7 +451,7 @@ int launch_jtj_f32(const Layout& L, const FrameGPU* frames, FrameList fl, const 
                    float* partials, int S, hipStream_t s);
 int launch_jtj_mfma(const Layout& L, const FrameGPU* frames, FrameList fl, const int* npix, const int4* pnb,
                     const float* pcoef, const float4* pixg, const float* dI, float w, double* H, float* g,
-                    float* partials, int S, int g_on_mfma, int two_term, hipStream_t s);
+                    float* partials, int S, int g_on_mfma, int two_term, int max_area, hipStream_t s);
 
 // solve.hip
 // rt, P0 and vproj: of a synthesis at theta

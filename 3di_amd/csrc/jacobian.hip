@@ -387,6 +387,7 @@ __global__ void __launch_bounds__(PT_THREADS) k_dI_patch(ModelGPU m, const float
                                                           float* __restrict__ dI)
 {
     extern __shared__ float4 spt[];
+    __shared__ int snext;
     float* sE = (float*)spt;                                            // [vertex][axis][PT_COLS]
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = uniform(tid >> 6);
@@ -395,6 +396,7 @@ __global__ void __launch_bounds__(PT_THREADS) k_dI_patch(ModelGPU m, const float
     const int p = blockIdx.x;
     const int y0 = (int)((long long)nact * blockIdx.y / gridDim.y), y1 = (int)((long long)nact * (blockIdx.y + 1) / gridDim.y);
     if (y0 == y1) return;
+    if (tid == 0) snext = y0;
     {
         const int* pv = m.patch_vert + m.patch_off[p];
         const int nv = m.patch_off[p + 1] - m.patch_off[p];
@@ -409,7 +411,12 @@ __global__ void __launch_bounds__(PT_THREADS) k_dI_patch(ModelGPU m, const float
     __syncthreads();
     const int sub = lane >> 4, l16 = lane & 15;
     const bool vec = ((off + k0) & 3) == 0;
-    for (int yi = y0 + wave; yi < y1; yi += PT_WAVES) {
+    // frames differ in their pixels on the patch: each wavefront takes the next one left
+    for (;;) {
+        int yi = 0;
+        if (lane == 0) yi = atomicAdd(&snext, 1);
+        yi = uniform(yi);
+        if (yi >= y1) break;
         const int f = fl_frame(act, yi);
         const long long base = frames[f].pix_off;
         const int* ps = pstart + (size_t)f * (m.np + 1) + p;
@@ -672,8 +679,12 @@ __global__ void __launch_bounds__(256) k_jtj_f32(Layout L, const FrameGPU* __res
 }
 
 // Sum the S partials in FP64 into the FP64 normal matrix; tiles are 4x4 (f32 kernel) or 16x16
-// (MFMA kernel), upper triangle.
-__global__ void __launch_bounds__(256) k_jtj_reduce(const int* __restrict__ act, int n, int K, int KP, int TS, int S,
+// (MFMA kernel), upper triangle.  A thread per tile element, so that every partial is read once and in
+// order (a thread per matrix entry read each twice, the lower triangle's a line per lane: 357 us for
+// 448 frames of 64 splits, now 96 us); the element goes to both triangles, those of a diagonal tile to
+// their own place.
+template <int TS>
+__global__ void __launch_bounds__(256) k_jtj_reduce(const int* __restrict__ act, int n, int K, int KP, int S,
                                                      const float* __restrict__ Hp, const float* __restrict__ gp,
                                                      float w, double* __restrict__ H, float* __restrict__ g,
                                                      int g_from_tiles)
@@ -683,26 +694,30 @@ __global__ void __launch_bounds__(256) k_jtj_reduce(const int* __restrict__ act,
     const int f = fl_frame(act, yi);
     const int T = KP / TS;
     const int ntiles = T * (T + 1) / 2;
-    for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < K * K + K; e += gridDim.x * blockDim.x) {
-        if (e < K * K) {
-            int a = e / K, b = e - (e / K) * K;
-            if (a / TS > b / TS) { const int t = a; a = b; b = t; }
-            const int tile = tri_index(a / TS, b / TS, T);
-            const int off = (a % TS) * TS + (b % TS);
+    const int ne = ntiles * TS * TS;
+    for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < ne + K; e += gridDim.x * blockDim.x) {
+        if (e < ne) {
+            int tile = e / (TS * TS), I = 0;
+            const int off = e - tile * (TS * TS);
+            while (tile >= T - I) { tile -= T - I; ++I; }
+            const int a = I * TS + off / TS, b = (I + tile) * TS + off % TS;
+            // column K carries J^T r: entry (a, K)
+            if (a >= K || b > K || (b == K && !g_from_tiles)) continue;
+            const float* h = Hp + (size_t)f * S * ne + e;
             double sum = 0.0;
-            for (int s = 0; s < S; ++s) sum += Hp[(((size_t)f * S + s) * ntiles + tile) * TS * TS + off];
-            H[(size_t)f * K * K + e] = (double)w * sum;
-        } else {
-            const int j = e - K * K;
-            double sum = 0.0;
-            if (g_from_tiles) {
-                // J^T r lives in column K of the augmented product: entry (j, K)
-                const int tile = tri_index(j / TS, K / TS, T);
-                const int off = (j % TS) * TS + (K % TS);
-                for (int s = 0; s < S; ++s) sum += Hp[(((size_t)f * S + s) * ntiles + tile) * TS * TS + off];
-            } else {
-                for (int s = 0; s < S; ++s) sum += gp[((size_t)f * S + s) * KP + j];
+#pragma unroll 8
+            for (int s = 0; s < S; ++s) sum += h[(size_t)s * ne];
+            if (b == K) {
+                g[(size_t)f * K + a] = (float)(-w * sum);
+                continue;
             }
+            H[(size_t)f * K * K + (size_t)a * K + b] = (double)w * sum;
+            if (tile != 0) H[(size_t)f * K * K + (size_t)b * K + a] = (double)w * sum;
+        } else if (!g_from_tiles) {
+            const int j = e - ne;
+            double sum = 0.0;
+#pragma unroll 8
+            for (int s = 0; s < S; ++s) sum += gp[((size_t)f * S + s) * KP + j];
             g[(size_t)f * K + j] = (float)(-w * sum);
         }
     }
@@ -917,7 +932,10 @@ __device__ __forceinline__ void jl_store(const v4f* acc, float* __restrict__ Hou
     jl_store_rows<T, W, 0>(acc, Hout, lane >> 4, lane & 15);
 }
 
-template <int T>
+// FAR: a frame's rows may lie 2^32 bytes or more apart; else the neighbour positions are kept as 32-bit
+// byte offsets, which the gathers add to a uniform base (with a 64-bit
+// multiply per gather: 1239 us for 448 frames, 10 registers spilled; now 1210 us, 2 spilled).
+template <int T, bool FAR>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(T >= 7 ? 2 : 4))) k_jtj_lds(Layout L, const FrameGPU* __restrict__ frames,
                                                   const int* __restrict__ act, int n, const int* __restrict__ npix,
                                                   const int4* __restrict__ pnb, const float* __restrict__ pcoef,
@@ -976,6 +994,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(T >= 7
                     // search direction
                     if (!(rk == rk)) rk = 0.f;
                 }
+                if (!FAR) {
+                    nb.x *= 4 * ldI; nb.y *= 4 * ldI; nb.z *= 4 * ldI; nb.w *= 4 * ldI;
+                }
                 snb[tid] = nb;
                 scf[tid] = cf;
                 srk[tid] = rk;
@@ -991,10 +1012,14 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(T >= 7
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
                     const int4 nb = snb[4 * pq + q];
-                    ld[r][4 * q + 0] = dIf[(size_t)nb.x * ldI + jj];
-                    ld[r][4 * q + 1] = dIf[(size_t)nb.y * ldI + jj];
-                    ld[r][4 * q + 2] = dIf[(size_t)nb.z * ldI + jj];
-                    ld[r][4 * q + 3] = dIf[(size_t)nb.w * ldI + jj];
+                    auto row = [&](int o) {
+                        return FAR ? dIf[(size_t)o * ldI + jj]
+                                   : *(const float*)((const char*)dIf + ((unsigned)o + 4u * (unsigned)jj));
+                    };
+                    ld[r][4 * q + 0] = row(nb.x);
+                    ld[r][4 * q + 1] = row(nb.y);
+                    ld[r][4 * q + 2] = row(nb.z);
+                    ld[r][4 * q + 3] = row(nb.w);
                 }
             }
 #pragma unroll
@@ -1300,7 +1325,10 @@ int jtj_splits(int n, int per_frame_pixels_hint)
     return S;
 }
 
-// From this many listed frames on, the geometric columns go through mesh patches.
+// From this many listed frames on, the geometric columns go through mesh patches: below, too few pixels
+// share a patch to pay for loading it and for the sorting.  The whole stage by gathers against patches,
+// crops of 96 to 384 pixels: 1 frame 26 against 35 us, 4 frames 89 / 84, 8 frames 94 / 92, 12 frames
+// 93 / 71, 48 frames 418 / 219 us.
 constexpr int PATCH_MIN_FRAMES = 8;
 
 int launch_dI(const ModelGPU& m, const Layout& L, const FrameGPU* frames, FrameList fl, const float* theta,
@@ -1324,8 +1352,8 @@ int launch_dI(const ModelGPU& m, const Layout& L, const FrameGPU* frames, FrameL
         TDI_HIP(attr);
         hipLaunchKernelGGL(k_patch_bin, dim3(gy), dim3(BIN_THREADS), 0, s, frames, fl.act, fl.n, npix, m.np, js.ptri,
                            js.plist, js.pstart);
-        // about 64 frames per workgroup, four per wavefront: its patch is loaded once for them
-        const int slices = std::max(1, std::min(64, fl.n / 64));
+        // about 128 frames per workgroup, eight per wavefront: its patch is loaded once for them
+        const int slices = std::max(1, std::min(64, fl.n / 128));
         for (int blk = 0; blk < 2; ++blk) {
             const int nc = blk ? L.nid : L.nexp, off = blk ? L.off_id : L.off_exp, ld = blk ? m.id_ld : m.exp_ld;
             for (int k0 = 0; k0 < nc; k0 += PT_COLS)
@@ -1404,15 +1432,15 @@ int launch_jtj_f32(const Layout& L, const FrameGPU* frames, FrameList fl, const 
     const int gy = grid_frames(n, 1 << 16);
     hipLaunchKernelGGL(k_jtj_f32, dim3(S, gy), dim3(256), 0, s, L, frames, fl.act, n, npix, pnb, pcoef, pixg, dI, S,
                        KP, Hp, gp);
-    int bx = (K * K + K + 255) / 256;
-    hipLaunchKernelGGL(k_jtj_reduce, dim3(bx, gy), dim3(256), 0, s, fl.act, n, K, KP, 4, S, Hp, gp, w, H, g, 0);
+    const int bx = (T * (T + 1) / 2 * 16 + K + 255) / 256;
+    hipLaunchKernelGGL(k_jtj_reduce<4>, dim3(bx, gy), dim3(256), 0, s, fl.act, n, K, KP, S, Hp, gp, w, H, g, 0);
     TDI_HIP(hipGetLastError());
     return TDI_OK;
 }
 
 int launch_jtj_mfma(const Layout& L, const FrameGPU* frames, FrameList fl, const int* npix, const int4* pnb,
                     const float* pcoef, const float4* pixg, const float* dI, float w, double* H, float* g,
-                    float* partials, int S, int g_on_mfma, int two_term, hipStream_t s)
+                    float* partials, int S, int g_on_mfma, int two_term, int max_area, hipStream_t s)
 {
     const int K = L.K;
     const int KP = ((K + 1 + 15) / 16) * 16;
@@ -1427,17 +1455,22 @@ int launch_jtj_mfma(const Layout& L, const FrameGPU* frames, FrameList fl, const
     const int gy = grid_frames(n, 1 << 16);
     const dim3 grid(S, gy);
     const int* act = fl.act;
+    const bool far = (double)max_area * dI_stride(K) * 4.0 >= 4294967296.0;
+    auto launch = [&](auto near_kernel, auto far_kernel) {
+        hipLaunchKernelGGL(far ? far_kernel : near_kernel, grid, dim3(256), 0, s, L, frames, act, n, npix, pnb, pcoef, pixg,
+                           dI, S, nsplit, partials, gp);
+    };
     switch (T) {
-    case 1: hipLaunchKernelGGL(k_jtj_lds<1>, grid, dim3(256), 0, s, L, frames, act, n, npix, pnb, pcoef, pixg, dI, S, nsplit, partials, gp); break;
-    case 2: hipLaunchKernelGGL(k_jtj_lds<2>, grid, dim3(256), 0, s, L, frames, act, n, npix, pnb, pcoef, pixg, dI, S, nsplit, partials, gp); break;
-    case 3: hipLaunchKernelGGL(k_jtj_lds<3>, grid, dim3(256), 0, s, L, frames, act, n, npix, pnb, pcoef, pixg, dI, S, nsplit, partials, gp); break;
-    case 4: hipLaunchKernelGGL(k_jtj_lds<4>, grid, dim3(256), 0, s, L, frames, act, n, npix, pnb, pcoef, pixg, dI, S, nsplit, partials, gp); break;
-    case 5: hipLaunchKernelGGL(k_jtj_lds<5>, grid, dim3(256), 0, s, L, frames, act, n, npix, pnb, pcoef, pixg, dI, S, nsplit, partials, gp); break;
-    case 6: hipLaunchKernelGGL(k_jtj_lds<6>, grid, dim3(256), 0, s, L, frames, act, n, npix, pnb, pcoef, pixg, dI, S, nsplit, partials, gp); break;
-    default: hipLaunchKernelGGL(k_jtj_lds<7>, grid, dim3(256), 0, s, L, frames, act, n, npix, pnb, pcoef, pixg, dI, S, nsplit, partials, gp); break;
+    case 1: launch(k_jtj_lds<1, false>, k_jtj_lds<1, true>); break;
+    case 2: launch(k_jtj_lds<2, false>, k_jtj_lds<2, true>); break;
+    case 3: launch(k_jtj_lds<3, false>, k_jtj_lds<3, true>); break;
+    case 4: launch(k_jtj_lds<4, false>, k_jtj_lds<4, true>); break;
+    case 5: launch(k_jtj_lds<5, false>, k_jtj_lds<5, true>); break;
+    case 6: launch(k_jtj_lds<6, false>, k_jtj_lds<6, true>); break;
+    default: launch(k_jtj_lds<7, false>, k_jtj_lds<7, true>); break;
     }
-    int bx = (K * K + K + 255) / 256;
-    hipLaunchKernelGGL(k_jtj_reduce, dim3(bx, gy), dim3(256), 0, s, act, n, K, KP, 16, S, partials, gp, w, H, g,
+    const int bx = (T * (T + 1) / 2 * 256 + K + 255) / 256;
+    hipLaunchKernelGGL(k_jtj_reduce<16>, dim3(bx, gy), dim3(256), 0, s, act, n, K, KP, S, partials, gp, w, H, g,
                        g_on_mfma);
     TDI_HIP(hipGetLastError());
     return TDI_OK;
