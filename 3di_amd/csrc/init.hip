@@ -11,10 +11,13 @@
 // (logbarrier_initializer.cu:1862-1914) refits from the mirrored pose when sigma_x < 0 and
 // seeds the perspective pose with initialize_kernel (logbarrier_initializer.cu:31-46).
 //
-// Here a frame is a wavefront: lane i holds landmark i, and the 28 + 7 + 1 sums of J^T J,
-// J^T e and e.e are wavefront reductions whose lane-0 result is broadcast, so every lane takes
-// the same decisions.  The reference runs each frame as a chain of cuBLAS calls and host
-// copies; batching every frame into one launch is the point of this kernel.
+// Here a frame is a wavefront, alone in its workgroup: lane i holds landmark i, and the 28 + 7 + 1
+// sums of J^T J, J^T e and e.e are taken together (wave_sums) and read back by every lane, so every
+// lane takes the same decisions.  The reference runs each frame as a chain of cuBLAS calls and host
+// copies; batching every frame into one launch is the point of this kernel.  A frame's chain of steps
+// bounds it: with a reduction per sum and a division per entry of the 7 x 7 solve, 264 us for 512
+// frames; with one division per pivot and a workgroup for each frame, 131 us.
+#include "chol.h"
 #include "common.h"
 
 namespace tdi {
@@ -23,7 +26,6 @@ namespace {
 
 constexpr int OI_MAXITER = 100;
 constexpr int OI_MAXINNER = 1000;
-constexpr int OI_WAVES = 4;   // frames per workgroup
 
 // Sum over the wavefront; every lane gets lane 0's result.
 __device__ __forceinline__ double wave_sum(double v)
@@ -32,14 +34,48 @@ __device__ __forceinline__ double wave_sum(double v)
     return __shfl(v, 0, 64);
 }
 
+// The sums over the wavefront of N values, each lane's in v, with wave_sum's rounding: at every step a
+// lane hands on half of the values it still holds and keeps the other half, so the lot takes N + 2 or
+// so exchanges instead of 6 N.  Then sum k is v[0] of lane sums_lane(k).
+template <int N>
+__device__ __forceinline__ void wave_sums(double (&v)[N])
+{
+    const int lane = threadIdx.x & 63;
+    int n = N;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        const int h = (n + 1) / 2;
+        const bool up = lane & o;
+#pragma unroll
+        for (int k = 0; k < h; ++k) {
+            const double b = k + h < n ? v[k + h] : 0.0;
+            v[k] = (up ? b : v[k]) + __shfl_xor(up ? v[k] : b, o, 64);
+        }
+        n = h;
+    }
+}
+template <int N>
+constexpr int sums_lane(int k)
+{
+    int lane = 0;
+    for (int o = 32, n = N; o > 0; o >>= 1) {
+        const int h = (n + 1) / 2;
+        if (k >= h) { lane |= o; k -= h; }
+        n = h;
+    }
+    return lane;
+}
+
 // R = I + sin(th) [n]x + (1 - cos th) [n]x^2 and, if dR, dR/du_i = (u_i [u]x + [u x (I - R) e_i]x) R / th^2
 // (rotation_header.cu:46-149), column-major, FP64.
 __device__ void rot64(const double* u, double* R, double* dR)
 {
     const double th = sqrt(u[0] * u[0] + u[1] * u[1] + u[2] * u[2]);
-    const double n0 = u[0] / th, n1 = u[1] / th, n2 = u[2] / th;
+    const double iu = 1.0 / th, n0 = ch_div(u[0], th, iu), n1 = ch_div(u[1], th, iu), n2 = ch_div(u[2], th, iu);
     const double N[9] = {0, n2, -n1, -n2, 0, n0, n1, -n0, 0};
-    const double s = sin(th), c1 = 1.0 - cos(th);
+    double s, c;
+    sincos(th, &s, &c);
+    const double c1 = 1.0 - c;
     for (int c = 0; c < 3; ++c)
         for (int r = 0; r < 3; ++r) {
             double acc = 0.0;
@@ -68,7 +104,7 @@ __device__ void rot64(const double* u, double* R, double* dR)
 // Delta = -H^-1 g for the 7x7 normal matrix held as its upper triangle (row by row).
 __device__ bool chol7(const double* Hu, const double* g, double* d)
 {
-    double Lm[7][7];
+    double Lm[7][7], inv[7];
     int k = 0;
     for (int a = 0; a < 7; ++a)
         for (int b = a; b < 7; ++b, ++k) Lm[b][a] = Hu[k];
@@ -76,24 +112,24 @@ __device__ bool chol7(const double* Hu, const double* g, double* d)
         double dj = Lm[j][j];
         for (int q = 0; q < j; ++q) dj -= Lm[j][q] * Lm[j][q];
         if (!(dj > 0.0)) return false;
-        dj = sqrt(dj);
+        ch_root(dj, dj, inv[j], [](int) {});
         Lm[j][j] = dj;
         for (int i = j + 1; i < 7; ++i) {
             double s = Lm[i][j];
             for (int q = 0; q < j; ++q) s -= Lm[i][q] * Lm[j][q];
-            Lm[i][j] = s / dj;
+            Lm[i][j] = ch_div(s, dj, inv[j]);
         }
     }
     double y[7];
     for (int i = 0; i < 7; ++i) {
         double s = -g[i];
         for (int q = 0; q < i; ++q) s -= Lm[i][q] * y[q];
-        y[i] = s / Lm[i][i];
+        y[i] = ch_div(s, Lm[i][i], inv[i]);
     }
     for (int i = 6; i >= 0; --i) {
         double s = y[i];
         for (int q = i + 1; q < 7; ++q) s -= Lm[q][i] * d[q];
-        d[i] = s / Lm[i][i];
+        d[i] = ch_div(s, Lm[i][i], inv[i]);
     }
     return true;
 }
@@ -133,12 +169,18 @@ __device__ int ortho_fit(double* x, const double* p, double xlb, double ylb, boo
         }
         if (!on)
             for (int a = 0; a < 7; ++a) jx[a] = jy[a] = 0.0;
-        double Hu[28], g[7];
+        double v[36], Hu[28], g[7];
         int k = 0;
         for (int a = 0; a < 7; ++a)
-            for (int b = a; b < 7; ++b, ++k) Hu[k] = wave_sum(jx[a] * jx[b] + jy[a] * jy[b]);
-        for (int a = 0; a < 7; ++a) g[a] = wave_sum(jx[a] * ex + jy[a] * ey);
-        const double obj = wave_sum(ex * ex + ey * ey);
+            for (int b = a; b < 7; ++b, ++k) v[k] = jx[a] * jx[b] + jy[a] * jy[b];
+        for (int a = 0; a < 7; ++a) v[28 + a] = jx[a] * ex + jy[a] * ey;
+        v[35] = ex * ex + ey * ey;
+        wave_sums<36>(v);
+#pragma unroll
+        for (int q = 0; q < 28; ++q) Hu[q] = lane_read(v[0], sums_lane<36>(q));
+#pragma unroll
+        for (int a = 0; a < 7; ++a) g[a] = lane_read(v[0], sums_lane<36>(28 + a));
+        const double obj = lane_read(v[0], sums_lane<36>(35));
         double d[7];
         if (!chol7(Hu, g, d)) {
             // the reference goes on with whatever potrs returns after a failed potrf; the frame stops
@@ -216,16 +258,15 @@ __device__ void rotvec_euler(const double* e, double* r)
     r[0] = v[0] * f; r[1] = v[1] * f; r[2] = v[2] * f;
 }
 
-__global__ void __launch_bounds__(64 * OI_WAVES) k_ortho_init(const float* __restrict__ mean,
-                                                               const int* __restrict__ lmk_ids, int n,
+__global__ void __launch_bounds__(64) k_ortho_init(const float* __restrict__ mean,
+                                                               const int* __restrict__ lmk_ids,
                                                                const float* __restrict__ lmk,
                                                                const float* __restrict__ cams,
                                                                float* __restrict__ x_orth, float* __restrict__ pose,
                                                                float* __restrict__ angles, int* __restrict__ info)
 {
-    const int lane = threadIdx.x & 63;
-    const int f = blockIdx.x * OI_WAVES + (threadIdx.x >> 6);
-    if (f >= n) return;   // whole wavefronts leave together
+    const int lane = threadIdx.x;
+    const int f = blockIdx.x;
     const bool on = lane < NLMK;
     const int li = on ? lane : 0;
     const int vid = lmk_ids[li];
@@ -278,8 +319,7 @@ int launch_ortho_init(const ModelGPU& m, int n, const float* lmk, const float* c
                       float* angles, int* info, hipStream_t s)
 {
     if (n <= 0) return TDI_OK;
-    hipLaunchKernelGGL(k_ortho_init, dim3((n + OI_WAVES - 1) / OI_WAVES), dim3(64 * OI_WAVES), 0, s, m.mean, m.lmk_ids,
-                       n, lmk, cams, x_orth, pose, angles, info);
+    hipLaunchKernelGGL(k_ortho_init, dim3(n), dim3(64), 0, s, m.mean, m.lmk_ids, lmk, cams, x_orth, pose, angles, info);
     TDI_HIP(hipGetLastError());
     return TDI_OK;
 }

@@ -16,6 +16,7 @@
 // The batched state machine keeps every per-frame decision of the reference but runs it
 // for all frames of a batch with masks, so the whole fit is a fixed launch sequence
 // (graph-capturable): frames that have accepted a step or stopped sit out later rounds.
+#include "chol.h"
 #include "common.h"
 
 namespace tdi {
@@ -372,197 +373,6 @@ __global__ void __launch_bounds__(BAR_THREADS) k_barrier(ModelGPU m, Layout L, c
 // A barrier pair and an LDS round trip per column (what it replaces) took 283 us for one matrix of
 // 94 unknowns (mode 1 with the FP64 fallback) and 552 us for 448; this takes 71 and 135 us, and gives the
 // same bits (each entry takes its products in the same order; an MFMA step is four FMAs in order).
-constexpr int CMAXK = 112;
-constexpr int CHB = 16;                          // block edge
-constexpr int CHP = CHB + 1;                     // LDS row stride
-constexpr int CHN = CHB * CHP;                   // LDS elements per block
-constexpr int CHT = CMAXK / CHB;                 // most blocks per side
-
-__device__ __forceinline__ int ch_block(int I, int J) { return (I * (I + 1) / 2 + J) * CHN; }   // I >= J
-
-__device__ __forceinline__ float lane_read(float v, int j)
-{
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), j));
-}
-__device__ __forceinline__ double lane_read(double v, int j)
-{
-    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), j),
-                            __builtin_amdgcn_readlane(__double2loint(v), j));
-}
-
-typedef float ch_v4f __attribute__((ext_vector_type(4)));
-typedef double ch_v4d __attribute__((ext_vector_type(4)));
-// accumulator element r of lane l: row 4 (l / 16) + r for FP32, l / 16 + 4 r for FP64; column l % 16
-__device__ __forceinline__ ch_v4f ch_mma(float a, float b, ch_v4f c)
-{
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ ch_v4d ch_mma(double a, double b, ch_v4d c)
-{
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ int ch_row(float, int lane, int r) { return 4 * (lane >> 4) + r; }
-__device__ __forceinline__ int ch_row(double, int lane, int r) { return (lane >> 4) + 4 * r; }
-template <typename T> struct ChVec;
-template <> struct ChVec<float> { typedef ch_v4f type; };
-template <> struct ChVec<double> { typedef ch_v4d type; };
-
-// The lower blocks of H into LDS, scaled by sdinv on both sides when given; every load of the
-// thread (one entry of each block) is issued before the stores.
-template <typename T, typename TH>
-__device__ __forceinline__ void ch_load(T* A, const TH* __restrict__ Hf, int K, int nT, const float* sdinv)
-{
-    const int r = threadIdx.x >> 4, c = threadIdx.x & 15;
-    TH v[CHT * (CHT + 1) / 2];
-#pragma unroll
-    for (int I = 0; I < CHT; ++I)
-#pragma unroll
-        for (int J = 0; J <= I; ++J) {
-            if (I >= nT) continue;
-            v[I * (I + 1) / 2 + J] = Hf[(size_t)min(CHB * I + r, K - 1) * K + min(CHB * J + c, K - 1)];
-        }
-#pragma unroll
-    for (int I = 0; I < CHT; ++I)
-#pragma unroll
-        for (int J = 0; J <= I; ++J) {
-            if (I >= nT) continue;
-            const int i = CHB * I + r, j = CHB * J + c;
-            T x = (T)v[I * (I + 1) / 2 + J];
-            if (sdinv) x = x * (T)sdinv[i] * (T)sdinv[j];
-            if (i >= K || j >= K) x = i == j ? T(1) : T(0);
-            A[ch_block(I, J) + r * CHP + c] = x;
-        }
-}
-
-// s = sqrt(d) and y = 1 / s, on the factorisation's critical path (see ch_div)
-__device__ __forceinline__ void ch_root(float d, float& s, float& y)
-{
-    y = __builtin_amdgcn_rsqf(d);
-    s = d * y;
-    s = fmaf(0.5f * y, fmaf(-s, s, d), s);
-    y = fmaf(fmaf(-s, y, 1.f), y, y);
-}
-__device__ __forceinline__ void ch_root(double d, double& s, double& y)
-{
-    y = __builtin_amdgcn_rsq(d);               // about 24 bits: two Newton steps
-    y = fma(0.5 * y, fma(-d * y, y, 1.0), y);
-    y = fma(0.5 * y, fma(-d * y, y, 1.0), y);
-    s = d * y;
-    s = fma(0.5 * y, fma(-s, s, d), s);
-    y = fma(fma(-s, y, 1.0), y, y);
-}
-
-// A = L L^T in place; false (for every thread) at a pivot that is not positive.
-template <typename T>
-__device__ __forceinline__ bool ch_factor(T* A, int nT, int* sflag)
-{
-    typedef typename ChVec<T>::type V4;
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int l16 = lane & 15, kq = lane >> 4;
-    for (int p = 0; p < nT; ++p) {
-        if (wave == 0) {
-            const int rows = CHB * (nT - p);          // rows of the panel, the diagonal block first
-            const bool in0 = lane < rows, in1 = lane + 64 < rows;
-            T* r0 = A + ch_block(p + (in0 ? lane >> 4 : 0), p) + l16 * CHP;
-            T* r1 = A + ch_block(p + (in1 ? (lane + 64) >> 4 : 0), p) + l16 * CHP;
-            T x0[CHB], x1[CHB];
-#pragma unroll
-            for (int k = 0; k < CHB; ++k) {
-                x0[k] = r0[k];
-                x1[k] = r1[k];
-            }
-            bool bad = false;
-#pragma unroll
-            for (int k = 0; k < CHB; ++k) {
-                const T d = lane_read(x0[k], k);
-                bad = bad || !(d > T(0));
-                T s, inv;
-                ch_root(d, s, inv);
-                // rows above the pivot keep their entry (the block's unused upper triangle)
-                x0[k] = lane == k ? s : lane > k ? ch_div(x0[k], s, inv) : x0[k];
-                x1[k] = ch_div(x1[k], s, inv);
-#pragma unroll
-                for (int j = k + 1; j < CHB; ++j) {
-                    const T ljk = lane_read(x0[k], j);
-                    x0[j] = fma(-x0[k], ljk, x0[j]);
-                    x1[j] = fma(-x1[k], ljk, x1[j]);
-                }
-            }
-#pragma unroll
-            for (int k = 0; k < CHB; ++k) {
-                if (in0) r0[k] = x0[k];
-                if (in1) r1[k] = x1[k];
-            }
-            if (bad && lane == 0) *sflag = 1;
-        }
-        __syncthreads();
-        if (*sflag) return false;
-        int t = 0;
-        for (int I = p + 1; I < nT; ++I)
-            for (int J = p + 1; J <= I; ++J, ++t) {
-                if ((t & 3) != wave) continue;
-                T* C = A + ch_block(I, J) + l16;
-                const T* a = A + ch_block(I, p) + l16 * CHP + kq;
-                const T* b = A + ch_block(J, p) + l16 * CHP + kq;
-                V4 acc;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) acc[r] = C[ch_row(T(0), lane, r) * CHP];
-#pragma unroll
-                for (int k = 0; k < CHB / 4; ++k) acc = ch_mma(-a[4 * k], b[4 * k], acc);
-#pragma unroll
-                for (int r = 0; r < 4; ++r) C[ch_row(T(0), lane, r) * CHP] = acc[r];
-            }
-        __syncthreads();
-    }
-    return true;
-}
-
-// L L^T x = b on one wavefront, in TB arithmetic: lane l holds entries l (b0) and l + 64 (b1).
-template <typename T, typename TB>
-__device__ __forceinline__ void ch_solve(const T* A, int nT, TB& b0, TB& b1)
-{
-    const int lane = threadIdx.x & 63, l16 = lane & 15;
-    const int I0 = min(lane >> 4, nT - 1), I1 = min((lane + 64) >> 4, nT - 1);
-    const TB d0 = A[ch_block(I0, I0) + l16 * CHP + l16], d1 = A[ch_block(I1, I1) + l16 * CHP + l16];
-    const TB q0 = TB(1) / d0, q1 = TB(1) / d1;
-    for (int J = 0; J < nT; ++J) {
-        // column j of the rows below it (blocks above the diagonal are never used: masked)
-        const T* c0 = A + ch_block(max(I0, J), J) + l16 * CHP;
-        const T* c1 = A + ch_block(max(I1, J), J) + l16 * CHP;
-        T l0[CHB], l1[CHB];
-#pragma unroll
-        for (int c = 0; c < CHB; ++c) {
-            l0[c] = c0[c];
-            l1[c] = c1[c];
-        }
-#pragma unroll
-        for (int c = 0; c < CHB; ++c) {
-            const int j = CHB * J + c;
-            const TB y = j < 64 ? lane_read(ch_div(b0, d0, q0), j & 63) : lane_read(ch_div(b1, d1, q1), j & 63);
-            b0 = lane == j ? y : lane > j ? fma(-(TB)l0[c], y, b0) : b0;
-            b1 = lane + 64 == j ? y : lane + 64 > j ? fma(-(TB)l1[c], y, b1) : b1;
-        }
-    }
-    for (int J = nT - 1; J >= 0; --J) {
-        // row j, of the entries before it
-        const T* c0 = A + ch_block(J, min(I0, J)) + l16;
-        const T* c1 = A + ch_block(J, min(I1, J)) + l16;
-        T l0[CHB], l1[CHB];
-#pragma unroll
-        for (int c = 0; c < CHB; ++c) {
-            l0[c] = c0[c * CHP];
-            l1[c] = c1[c * CHP];
-        }
-#pragma unroll
-        for (int c = CHB - 1; c >= 0; --c) {
-            const int j = CHB * J + c;
-            const TB x = j < 64 ? lane_read(ch_div(b0, d0, q0), j & 63) : lane_read(ch_div(b1, d1, q1), j & 63);
-            b0 = lane == j ? x : lane < j ? fma(-(TB)l0[c], x, b0) : b0;
-            b1 = lane + 64 == j ? x : lane + 64 < j ? fma(-(TB)l1[c], x, b1) : b1;
-        }
-    }
-}
-
 __device__ __forceinline__ double ch_wave_sum(double v)
 {
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
