@@ -4,17 +4,20 @@
 // matrix, copyMatsFloatToDouble / copyVectorDoubleToFloatNegated, solver.cu:11-81) for the
 // joint identity-stage system (K up to a few thousand: 199 + 199 + 94 per frame).  Blocked
 // right-looking factorisation in place on an FP64 copy in HBM, 32-column panels:
-//   k_chol_diag    one wavefront per matrix: the 32x32 diagonal block factored in registers,
-//                  lane i holding row i, the column entries passed by lane reads;
-//   k_chol_offdiag a grid of 64-row blocks per matrix: the panel below it, L21 = A21 L11^-T
-//                  (one row per thread in registers, L11 and its reciprocal diagonal in LDS);
+//   k_chol_first   the first 32x32 diagonal block, factored by one wavefront per matrix, and -g put
+//                  into the matrix's unused upper triangle as one more row below the last;
+//   k_chol_offdiag a grid of 64-row blocks per matrix: the panel below the diagonal block, L21 =
+//                  A21 L11^-T (one row per thread in registers, L11 and its reciprocal diagonal in
+//                  LDS); the row of -g with it, which leaves L^-1 (-g) behind;
 //   k_chol_update  a grid of 32x32 tiles of the trailing lower triangle per matrix:
-//                  A22 -= L21 L21^T, both 32-row slices of the panel staged in LDS;
-//   k_chol_trsv    one workgroup per matrix: L y = -g, then L^T delta = y, by 32-row panels,
-//                  right-looking (the solution and the panel's diagonal block in LDS; each
-//                  panel's triangle on one wavefront from registers, then every later entry
-//                  updated by all threads with coalesced reads of the panel's rows or columns).
+//                  A22 -= L21 L21^T, both 32-row slices of the panel staged in LDS; the workgroup
+//                  of the next diagonal block factors it at once;
+//   k_chol_back    one workgroup per matrix: L^T delta = L^-1 (-g) by 32-row panels, right-looking.
+// The chain of K dependent columns bounds it, at two launches a panel: one matrix of 1338 unknowns
+// took 2976 us with the diagonal block in a launch of its own (15 us each), rows solved entry by
+// entry (29 us), and the forward solve after the factorisation (about half of 747 us); now 1386 us.
 // A non-positive (or NaN) pivot marks the matrix TDI_NOT_PD; its later launches do nothing.
+#include "chol.h"
 #include "common.h"
 
 namespace tdi {
@@ -29,54 +32,68 @@ __global__ void __launch_bounds__(256) k_f32_to_f64(size_t n, const float* __res
         out[i] = in[i];
 }
 
-// lane j's value of v (j uniform)
-__device__ __forceinline__ double lane_value(double v, int j)
-{
-    const int lo = __builtin_amdgcn_readlane(__double2loint(v), j);
-    const int hi = __builtin_amdgcn_readlane(__double2hiint(v), j);
-    return __hiloint2double(hi, lo);
-}
+// Where entry j of the row of -g (then of L^-1 (-g)) is kept: the strict upper triangle of row 0, and for
+// the last entry of row 1 (K >= 3).
+__device__ __forceinline__ size_t rhs_at(int K, int j) { return j < K - 1 ? (size_t)j + 1 : (size_t)2 * K - 1; }
 
-// The 32 x 32 diagonal block of the panel at k0, factored on one wavefront and written back:
-// lane i holds row i (entries j <= i; rows and columns past the matrix padded with the identity).
-__global__ void __launch_bounds__(64) k_chol_diag(int K, int k0, double* __restrict__ A, int* __restrict__ status)
+// The diagonal block of the panel at k0, in r (lane i: row i, entries j <= i; rows and columns past nb
+// the identity's), factored by one wavefront and written.  In a step the root and the division of a
+// column are independent of the update by the column before, which fills their gaps.
+__device__ __forceinline__ void chol_diag(int K, int k0, int nb, double* __restrict__ M, double (&r)[CB],
+                                          int* __restrict__ status)
 {
-    const int mtx = blockIdx.x;
-    if (status[mtx] != TDI_OK) return;
-    double* M = A + (size_t)mtx * K * K;
-    const int nb = min(CB, K - k0), lane = threadIdx.x;
-    const bool row = lane < nb;
-    const double* Mr = M + (size_t)(k0 + (row ? lane : 0)) * K + k0;
-    double r[CB];
-#pragma unroll
-    for (int j = 0; j < CB; ++j) r[j] = (row && j < nb && j <= lane) ? Mr[min(j, nb - 1)] : (lane == j ? 1.0 : 0.0);
-    // column k: pivot from lane k, the rows below scaled, then the trailing rows updated
+    const int lane = threadIdx.x & 63;
+    bool bad = false;
+    double dg = 0.0;
 #pragma unroll
     for (int k = 0; k < CB; ++k) {
-        const double d = lane_value(r[k], k);
-        if (!(d > 0.0)) {
-            if (lane == 0) status[mtx] = TDI_NOT_PD;
-            return;
-        }
+        const double d = lane_read(r[k], k);
+        bad = bad || !(d > 0.0);
         const double dk = sqrt(d), inv = 1.0 / dk;
-        r[k] = lane == k ? dk : (lane > k ? r[k] * inv : r[k]);
+        dg = lane == k ? dk : dg;
+        r[k] *= inv;
+        if (k > 0) {
 #pragma unroll
-        for (int j = k + 1; j < CB; ++j) {
-            const double ljk = lane_value(r[k], j);
-            if (lane >= j) r[j] = fma(-r[k], ljk, r[j]);
+            for (int j = k + 1; j < CB; ++j) r[j] = fma(-r[k - 1], lane_read(r[k - 1], j), r[j]);
         }
+        if (k + 1 < CB) r[k + 1] = fma(-r[k], lane_read(r[k], k + 1), r[k + 1]);
+        __builtin_amdgcn_sched_barrier(0);
     }
-    if (row) {
+    if (bad) {
+        if (lane == 0) *status = TDI_NOT_PD;
+        return;
+    }
+    if (lane < nb) {
         double* Mw = M + (size_t)(k0 + lane) * K + k0;
 #pragma unroll
         for (int j = 0; j < CB; ++j)
-            if (j < nb && j <= lane) Mw[j] = r[j];
+            if (j < lane) Mw[j] = r[j];
+        Mw[lane] = dg;
     }
 }
 
-// The panel below the diagonal block: row r of A21 solves x L11^T = a (forward substitution over
-// the panel's columns), 64 rows per workgroup (a grid over the rows), each row in its thread's
-// registers, L11 and the reciprocals of its diagonal in LDS (read as broadcasts).
+template <typename TG>
+__global__ void __launch_bounds__(64) k_chol_first(int K, double* __restrict__ A, const TG* __restrict__ g,
+                                                    int* __restrict__ status)
+{
+    const int mtx = blockIdx.x, lane = threadIdx.x, nb = min(CB, K);
+    if (status[mtx] != TDI_OK) return;
+    double* M = A + (size_t)mtx * K * K;
+    const double* Mr = M + (size_t)min(lane, nb - 1) * K;
+    double r[CB];
+#pragma unroll
+    for (int j = 0; j < CB; ++j) {
+        const double x = Mr[min(j, nb - 1)];
+        r[j] = (lane < nb && j < nb && j <= lane) ? x : (lane == j ? 1.0 : 0.0);
+    }
+    for (int j = lane; j < K; j += 64) M[rhs_at(K, j)] = -(double)g[(size_t)mtx * K + j];
+    chol_diag(K, 0, nb, M, r, status + mtx);
+}
+
+// The panel below the diagonal block: row r of A21 (row K: -g) solves x L11^T = a, 64 rows per workgroup
+// (a grid over the rows), each row in its thread's registers, L11 by columns and the reciprocals of its
+// diagonal in LDS (read as broadcasts).  An entry that is done leaves every later one at once (the same
+// products in the same order as entry by entry, but a chain of 64 operations instead of 528).
 __global__ void __launch_bounds__(64) k_chol_offdiag(int K, int k0, double* __restrict__ A,
                                                       const int* __restrict__ status)
 {
@@ -85,49 +102,64 @@ __global__ void __launch_bounds__(64) k_chol_offdiag(int K, int k0, double* __re
     double* M = A + (size_t)mtx * K * K;
     const int nb = min(CB, K - k0), tid = threadIdx.x;
     const int r0 = k0 + nb + blockIdx.x * 64;
-    if (r0 >= K) return;
-    __shared__ double D[CB][CB];
+    __shared__ double2 D2[CB][CB / 2];      // D[j][i] = L11[i][j]
     __shared__ double sinv[CB];
+    double* D = reinterpret_cast<double*>(D2);
+    const int gr = r0 + tid;
+    const bool in = gr <= K, last = gr >= K;
+    double* Mr = M + (size_t)min(gr, K - 1) * K + k0;
+    double p[CB];
     {
-        // every load of the block issued before the LDS stores (64 threads, 16 entries each)
+        // every load issued before the LDS stores (64 threads, 16 entries of L11 each)
         double v[CB * CB / 64];
 #pragma unroll
         for (int q = 0; q < CB * CB / 64; ++q) {
             const int e = tid + 64 * q, i = e / CB, j = e - i * CB;
-            const bool in = i < nb && j < nb && j <= i;
             const double x = M[(size_t)(k0 + min(i, nb - 1)) * K + k0 + min(j, nb - 1)];
-            v[q] = in ? x : (i == j ? 1.0 : 0.0);
+            v[q] = (i < nb && j < nb && j <= i) ? x : (i == j ? 1.0 : 0.0);
+        }
+#pragma unroll
+        for (int j = 0; j < CB; ++j) {
+            const int c = min(j, nb - 1);
+            const double x = last ? M[rhs_at(K, k0 + c)] : Mr[c];
+            p[j] = j < nb ? x : 0.0;
         }
 #pragma unroll
         for (int q = 0; q < CB * CB / 64; ++q) {
-            const int e = tid + 64 * q;
-            D[e / CB][e % CB] = v[q];
+            const int e = tid + 64 * q, i = e / CB, j = e - i * CB;
+            D[j * CB + i] = v[q];
+            if (i == j) sinv[j] = 1.0 / v[q];
         }
     }
     __syncthreads();
-    if (tid < CB) sinv[tid] = 1.0 / D[tid][tid];
-    __syncthreads();
-    const int gr = r0 + tid;
-    if (gr >= K) return;
-    double* Mr = M + (size_t)gr * K + k0;
-    double p[CB];
+    double2 l[CB / 2], ln[CB / 2];
 #pragma unroll
-    for (int j = 0; j < CB; ++j) p[j] = j < nb ? Mr[min(j, nb - 1)] : 0.0;
+    for (int q = 0; q < CB / 2; ++q) l[q] = D2[0][q];
 #pragma unroll
     for (int j = 0; j < CB; ++j) {
-        double sacc = p[j];
 #pragma unroll
-        for (int q = 0; q < j; ++q) sacc = fma(-p[q], D[j][q], sacc);
-        p[j] = sacc * sinv[j];
+        for (int q = (j + 2) / 2; q < CB / 2; ++q) ln[q] = D2[min(j + 1, CB - 1)][q];
+        p[j] *= sinv[j];
+#pragma unroll
+        for (int q = j + 1; q < CB; ++q) p[q] = fma(-p[j], (q & 1) ? l[q / 2].y : l[q / 2].x, p[q]);
+        // the updates stay here: put off, they would keep every column's entries in registers
+#pragma unroll
+        for (int q = j + 1; q < CB; ++q) asm volatile("" : "+v"(p[q]) :: "memory");
+#pragma unroll
+        for (int q = 0; q < CB / 2; ++q) l[q] = ln[q];
     }
+    if (!in) return;
 #pragma unroll
     for (int j = 0; j < CB; ++j)
-        if (j < nb) Mr[j] = p[j];
+        if (j < nb) {
+            if (last) M[rhs_at(K, k0 + j)] = p[j];
+            else Mr[j] = p[j];
+        }
 }
 
 // Tile (ti, tj), ti >= tj, of the trailing matrix below/right of the panel at k0.
 __global__ void __launch_bounds__(256) k_chol_update(int K, int k0, double* __restrict__ A,
-                                                      const int* __restrict__ status)
+                                                      int* __restrict__ status)
 {
     const int mtx = blockIdx.y;
     if (status[mtx] != TDI_OK) return;
@@ -171,27 +203,47 @@ __global__ void __launch_bounds__(256) k_chol_update(int K, int k0, double* __re
         for (int q = 0; q < 4; ++q) acc[q] = fma(li, Lj[b4 + q][c], acc[q]);
     }
     const int gi = r0 + ti * CB + a;
-    if (gi >= K) return;
+    if (ti != 0) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const int gj = r0 + tj * CB + b4 + q;
-        if (gj < K && gj <= gi) M[(size_t)gi * K + gj] -= acc[q];
+        for (int q = 0; q < 4; ++q) {
+            const int gj = r0 + tj * CB + b4 + q;
+            if (gi < K && gj < K && gj <= gi) M[(size_t)gi * K + gj] -= acc[q];
+        }
     }
+    if (ti == tj && tid < CB && r0 + tj * CB + tid < K) {       // the row of -g, at the tile's columns
+        double* y = M + rhs_at(K, r0 + tj * CB + tid);
+        double s[CB / 4];                    // sums of four in order, then by pairs
+#pragma unroll
+        for (int c = 0; c < CB; ++c)         // L is 0 past nb
+            s[c / 4] = fma(Lj[tid][c], M[rhs_at(K, k0 + min(c, nb - 1))], c % 4 ? s[c / 4] : 0.0);
+        *y -= ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
+    }
+    if (ti != 0) return;
+    // the next panel's diagonal block
+    double v[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) v[q] = M[(size_t)min(gi, K - 1) * K + min(r0 + b4 + q, K - 1)] - acc[q];
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        Li[a][b4 + q] = (gi < K && r0 + b4 + q <= gi) ? v[q] : (a == b4 + q ? 1.0 : 0.0);
+    __syncthreads();
+    if (tid >= 64) return;
+    double r[CB];
+#pragma unroll
+    for (int j = 0; j < CB; ++j) r[j] = tid < CB ? Li[tid & (CB - 1)][j] : 0.0;
+    chol_diag(K, r0, min(CB, K - r0), M, r, status + mtx);
 }
 
-// L y = -g, then L^T delta = y, one workgroup per matrix, by 32-row panels with the solution in
-// LDS (K <= CHOL_BIG_MAXK), right-looking: each panel's 32 x 32 diagonal block staged in LDS by all
-// threads, its triangle solved on wavefront 0 (lane i holding row i, forward, or column i,
-// backward, in registers, the solved entries passed by lane reads), then every entry not yet
-// solved updated with the panel's solution by all threads: forward, eight lanes per later row,
-// each reading four consecutive entries of the panel's columns (a row's 32 entries in one
-// coalesced read) and the eight partial sums combined by lane shuffles; backward, one earlier
-// column per thread, the panel's rows read coalesced across the threads.
-constexpr int TRSV_THREADS = 1024;
+// L^T delta = y (left by the factorisation), one workgroup per matrix, by 32-row panels from the last,
+// with the solution in LDS (K <= CHOL_BIG_MAXK), right-looking.  The panels' serial parts bound it, so
+// wavefront 0 solves a panel's triangle (lane i holding column i, the solved entries passed by lane
+// reads) while the others already load the panel's rows, a column each, and all the next panel's
+// diagonal block.
+constexpr int BACK_THREADS = 768, BACK_COLS = BACK_THREADS - 64;   // three wavefronts a SIMD: 32 rows fit in registers
 
-template <typename TG, typename TD>
-__global__ void __launch_bounds__(TRSV_THREADS) k_chol_trsv(int K, const double* __restrict__ A,
-                                                             const TG* __restrict__ g, TD* __restrict__ delta,
+template <typename TD>
+__global__ void __launch_bounds__(BACK_THREADS) k_chol_back(int K, const double* __restrict__ A, TD* __restrict__ delta,
                                                              const int* __restrict__ status)
 {
     const int mtx = blockIdx.x;
@@ -200,89 +252,60 @@ __global__ void __launch_bounds__(TRSV_THREADS) k_chol_trsv(int K, const double*
     __shared__ double sy[CHOL_BIG_MAXK];
     __shared__ double sD[CB][CB + 1];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    for (int i = tid; i < K; i += blockDim.x) sy[i] = -(double)g[(size_t)mtx * K + i];
-    // the diagonal block of the panel at p0 (zero past the matrix), one entry per thread
-    auto stage = [&](int p0, int nb) {
-        const int i = tid >> 5, j = tid & 31;
-        const double x = L[(size_t)(p0 + min(i, nb - 1)) * K + p0 + min(j, nb - 1)];
-        sD[i][j] = (i < nb && j < nb) ? x : 0.0;
+    for (int i = tid; i < K; i += blockDim.x) sy[i] = L[rhs_at(K, i)];
+    // entry e of the diagonal block at p0 (the identity past the matrix); a thread has two at most
+    auto entry = [&](int p0, int e) {
+        const int nb = min(CB, K - p0), di = (e >> 5) & (CB - 1), dj = e & (CB - 1);
+        const double x = L[(size_t)(p0 + min(di, nb - 1)) * K + p0 + min(dj, nb - 1)];
+        return di < nb && dj < nb ? x : di == dj ? 1.0 : 0.0;
     };
-    // forward: y_p = L_pp^-1 b_p, then b_i -= L_ip y_p for the rows below
-    for (int p0 = 0; p0 < K; p0 += CB) {
-        const int nb = min(CB, K - p0);
-        stage(p0, nb);
-        __syncthreads();
-        if (wave == 0) {
-            const bool in = lane < nb;
-            const int r0 = in ? lane : 0;
-            double lr[CB];
-#pragma unroll
-            for (int j = 0; j < CB; ++j) lr[j] = (in && j < lane) ? sD[r0][j] : 0.0;
-            const double rinv = in ? 1.0 / sD[r0][r0] : 1.0;
-            double r = in ? sy[p0 + r0] : 0.0;
-#pragma unroll
-            for (int j = 0; j < CB; ++j) {
-                if (lane == j) r *= rinv;
-                const double yj = lane_value(r, j);
-                if (lane > j) r = fma(-lr[j], yj, r);
-            }
-            if (in) sy[p0 + lane] = r;
-        }
-        __syncthreads();
-        {
-            const int sub = tid & 7, c0 = 4 * sub;
-            double yv[4];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) yv[q] = c0 + q < nb ? sy[p0 + c0 + q] : 0.0;
-            for (int i0 = p0 + nb; i0 < K; i0 += TRSV_THREADS / 8) {
-                const int i = i0 + (tid >> 3);
-                const int ic = min(i, K - 1);
-                const double* Lr = L + (size_t)ic * K + p0;
-                double acc = 0.0;
-#pragma unroll
-                for (int q = 0; q < 4; ++q) acc = fma(Lr[min(c0 + q, nb - 1)], yv[q], acc);
-                acc += __shfl_xor(acc, 1, 64);
-                acc += __shfl_xor(acc, 2, 64);
-                acc += __shfl_xor(acc, 4, 64);
-                if (sub == 0 && i < K) sy[i] -= acc;
-            }
-        }
-        __syncthreads();
-    }
-    // backward: x_p = L_pp^-T y_p, then y_i -= L_pi x_p for the entries before the panel
     const int last = ((K - 1) / CB) * CB;
+    auto store = [&](double a, double b) {
+        sD[tid >> 5][tid & (CB - 1)] = a;
+        if (tid + BACK_THREADS < CB * CB) sD[(tid + BACK_THREADS) >> 5][tid & (CB - 1)] = b;
+    };
+    store(entry(last, tid), entry(last, tid + BACK_THREADS));
+    __syncthreads();
     for (int p0 = last; p0 >= 0; p0 -= CB) {
-        const int nb = min(CB, K - p0);
-        stage(p0, nb);
-        __syncthreads();
+        const int nb = min(CB, K - p0), col = tid - 64;
+        const int pn = max(p0 - CB, 0);
+        const double na = entry(pn, tid), nc = entry(pn, tid + BACK_THREADS);
+        double lv[CB];
         if (wave == 0) {
-            const bool in = lane < nb;
-            const int c = in ? lane : 0;
+            int c = lane & (CB - 1);
+            asm volatile("" : "+v"(c));        // the comparisons are made here, not kept over the panels
             double lc[CB];
 #pragma unroll
-            for (int j = 0; j < CB; ++j) lc[j] = (in && j > lane) ? sD[j][c] : 0.0;
-            const double rinv = in ? 1.0 / sD[c][c] : 1.0;
-            double r = in ? sy[p0 + c] : 0.0;
+            for (int j = 0; j < CB; ++j) lc[j] = j > c ? sD[j][c] : 0.0;
+            const double dd = sD[c][c], rinv = 1.0 / dd;
+            double r = c < nb ? sy[p0 + c] : 0.0;
 #pragma unroll
-            for (int j = CB - 1; j >= 0; --j) {
-                if (lane == j) r *= rinv;
-                const double xj = lane_value(r, j);
-                if (lane < j) r = fma(-lc[j], xj, r);
-            }
-            if (in) sy[p0 + lane] = r;
+            for (int j = CB - 1; j >= 0; --j) r = fma(-lc[j], lane_read(ch_div(r, dd, rinv), j), r);
+            if (lane < nb) sy[p0 + lane] = ch_div(r, dd, rinv);
+        } else {
+            const double* Lc = L + (size_t)p0 * K + min(col, max(p0 - 1, 0));
+#pragma unroll
+            for (int j = 0; j < CB; ++j) lv[j] = Lc[(size_t)min(j, nb - 1) * K];
         }
         __syncthreads();
-        for (int i = tid; i < p0; i += blockDim.x) {
-            const double* Lc = L + (size_t)p0 * K + i;
+        if (wave > 0 && col < p0) {
             double acc = 0.0;
 #pragma unroll
-            for (int j = 0; j < CB; ++j) {
-                const int jj = min(j, nb - 1);
-                const double l = Lc[(size_t)jj * K];
-                acc = fma(j < nb ? l : 0.0, sy[p0 + jj], acc);
+            for (int j = 0; j < CB; ++j)
+                if (j < nb) acc = fma(lv[j], sy[p0 + j], acc);
+            sy[col] -= acc;
+            for (int i = col + BACK_COLS; i < p0; i += BACK_COLS) {
+                const double* Lc = L + (size_t)p0 * K + i;
+                acc = 0.0;
+#pragma unroll
+                for (int j = 0; j < CB; ++j) {
+                    const double l = Lc[(size_t)min(j, nb - 1) * K];
+                    acc = fma(j < nb ? l : 0.0, sy[p0 + min(j, nb - 1)], acc);
+                }
+                sy[i] -= acc;
             }
-            sy[i] -= acc;
         }
+        store(na, nc);
         __syncthreads();
     }
     for (int i = tid; i < K; i += blockDim.x) delta[(size_t)mtx * K + i] = (TD)sy[i];
@@ -294,16 +317,15 @@ __global__ void __launch_bounds__(TRSV_THREADS) k_chol_trsv(int K, const double*
 template <typename TG, typename TD>
 static int chol_big_run(int n, int K, double* A, const TG* g, TD* delta, int* status, hipStream_t s)
 {
+    hipLaunchKernelGGL(k_chol_first<TG>, dim3(n), dim3(64), 0, s, K, A, g, status);
     for (int k0 = 0; k0 < K; k0 += CB) {
-        hipLaunchKernelGGL(k_chol_diag, dim3(n), dim3(64), 0, s, K, k0, A, status);
-        const int below = K - k0 - CB;
-        if (below > 0)
-            hipLaunchKernelGGL(k_chol_offdiag, dim3((below + 63) / 64, n), dim3(64), 0, s, K, k0, A, status);
-        const int T = (K - k0 - CB + CB - 1) / CB;
+        const int below = std::max(0, K - k0 - CB);
+        hipLaunchKernelGGL(k_chol_offdiag, dim3((below + 64) / 64, n), dim3(64), 0, s, K, k0, A, status);
+        const int T = (below + CB - 1) / CB;
         if (T > 0) hipLaunchKernelGGL(k_chol_update, dim3(T * (T + 1) / 2, n), dim3(256), 0, s, K, k0, A, status);
         if (hipGetLastError() != hipSuccess) return TDI_ERR_HIP;
     }
-    hipLaunchKernelGGL((k_chol_trsv<TG, TD>), dim3(n), dim3(TRSV_THREADS), 0, s, K, A, g, delta, status);
+    hipLaunchKernelGGL(k_chol_back<TD>, dim3(n), dim3(BACK_THREADS), 0, s, K, A, delta, status);
     return hipGetLastError() != hipSuccess ? TDI_ERR_HIP : TDI_OK;
 }
 
