@@ -9,14 +9,15 @@
 // The adjoint runs backwards through the forward's stages with the visibility (triangle of each
 // pixel) held fixed; the rasterisation is recomputed from theta rather than stored:
 //   k_adj_dB     residuals -> dL/dg (through the normalisation g^ = 2 g / h, h = 1e-16 + 2|g|)
-//                -> dL/dB scattered to the four neighbours of each visible pixel (FP64 atomics);
+//                of each visible pixel;
+//   k_adj_dI     dL/dB, gathered from the four neighbours' dL/dg;
 //   blur         dL/dI = K^T dL/dB = K dL/dB (the 15 taps are symmetric, zero outside the crop);
 //   k_adj_shade  per visible pixel, dL/dI through the shading I = rho (1 + L Id + S) into the
 //                triangle's model-space corners (normal, surface point, and the barycentrics of the
 //                pixel centre in the projected triangle), the pose (projection and shading) and
 //                the light; FP64, corners accumulated with FP64 atomics;
 //   k_adj_lmk    the landmark term;
-//   k_adj_basis  dL/d(expression, identity) = basis^T dL/dP0, per frame;
+//   k_adj_basis  dL/d(expression, identity) = basis^T dL/dP0, 16 frames at a time;
 //   k_adj_out    gradients in the unknowns' layout (pose, expression, identity, light; albedo 0),
 //                scaled by the upstream gradient of each frame's loss.
 // The shading derivative matches newfuncs.cu:18-167's forward; it is the exact derivative of the
@@ -88,10 +89,24 @@ __global__ void __launch_bounds__(256) k_add_offsets(int V, const FrameGPU* __re
     vproj[o] = project_vertex(FrameCam{frames[f].phix, frames[f].phiy, frames[f].cx, frames[f].cy}, R, p, q);
 }
 
-// Residuals of the visible pixels: the data loss (FP64, per frame) and dL/dB at the neighbours.
+// A workgroup's sum of v (256 threads), on thread 0: one atomic a workgroup, as those on one address
+// follow each other.
+__device__ __forceinline__ double block_sum(double v, double* red)
+{
+    v = wave_sum(v);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    __syncthreads();
+    return red[0] + red[1] + red[2] + red[3];
+}
+
+// Residuals of the visible pixels: the data loss (FP64, per frame) and dL/dg, whose neighbours gather it
+// (k_adj_dI).  At the crop's edge the gradient takes pixel 0 for the missing neighbour: its share of
+// dL/dB goes to edge.  With dL/dB scattered to the neighbours and a loss sum per wavefront it took 63 us
+// for 48 frames (and 9 to round dL/dB), now 19 (and 23 to gather it).
 __global__ void __launch_bounds__(256) k_adj_dB(const FrameGPU* __restrict__ frames, int n, const int* __restrict__ vis,
                                                  const int* __restrict__ npix, const float4* __restrict__ pixg,
-                                                 double* __restrict__ dB, double* __restrict__ loss, int want_grad)
+                                                 double2* __restrict__ dg, double* __restrict__ edge, double* __restrict__ loss,
+                                                 int want_grad)
 {
     const int f = blockIdx.y;
     if (f >= n) return;
@@ -114,32 +129,45 @@ __global__ void __launch_bounds__(256) k_adj_dB(const FrameGPU* __restrict__ fra
         const double dgy = 2.0 * ay / h - 4.0 * ag * gy / (gn * h * h);
         const int k = vis[base + pos];
         const int x = k / fr.H, y = k - x * fr.H;
-        const int kr = (x < fr.W - 1) ? k + fr.H : 0, kl = (x > 0) ? k - fr.H : 0;
-        const int ka = (y > 0) ? k - 1 : 0, kb = (y < fr.H - 1) ? k + 1 : 0;
-        atomicAdd(dB + base + kr, 0.5 * dgx);
-        atomicAdd(dB + base + kl, -0.5 * dgx);
-        atomicAdd(dB + base + kb, 0.5 * dgy);
-        atomicAdd(dB + base + ka, -0.5 * dgy);
+        dg[base + k] = make_double2(dgx, dgy);
+        double e = 0.0;
+        if (x == fr.W - 1) e += 0.5 * dgx;
+        if (x == 0) e -= 0.5 * dgx;
+        if (y == fr.H - 1) e += 0.5 * dgy;
+        if (y == 0) e -= 0.5 * dgy;
+        if (e != 0.0) atomicAdd(edge + f, e);
     }
-    acc = wave_sum(acc);
-    if ((threadIdx.x & 63) == 0) atomicAdd(loss + f, acc);
+    __shared__ double red[4];
+    acc = block_sum(acc, red);
+    if (threadIdx.x == 0 && acc != 0.0) atomicAdd(loss + f, acc);
 }
 
-__global__ void __launch_bounds__(256) k_d2f(const FrameGPU* __restrict__ frames, int n, const double* __restrict__ in,
-                                              float* __restrict__ out)
+// dL/dB of every pixel of the crop, rounded, from dL/dg of its neighbours (zero where none is visible).
+__global__ void __launch_bounds__(256) k_adj_dI(const FrameGPU* __restrict__ frames, int n, const double2* __restrict__ dg,
+                                                 const double* __restrict__ edge, float* __restrict__ out)
 {
     const int f = blockIdx.y;
     if (f >= n) return;
     const FrameGPU fr = frames[f];
     const int A = fr.W * fr.H;
-    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < A; k += gridDim.x * blockDim.x)
-        out[fr.pix_off + k] = (float)in[fr.pix_off + k];
+    const double2* d = dg + fr.pix_off;
+    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < A; k += gridDim.x * blockDim.x) {
+        const int x = k / fr.H, y = k - x * fr.H;
+        double v = k == 0 ? edge[f] : 0.0;
+        if (x > 0) v += 0.5 * d[k - fr.H].x;
+        if (x < fr.W - 1) v -= 0.5 * d[k + fr.H].x;
+        if (y > 0) v += 0.5 * d[k - 1].y;
+        if (y < fr.H - 1) v -= 0.5 * d[k + 1].y;
+        out[fr.pix_off + k] = (float)v;
+    }
 }
 
 constexpr int ADJ_G = 15;   // per-frame accumulators: pose 6, light 9
 
-// dL/dI of the visible pixels through the shading, the barycentrics and the projection.
-__global__ void __launch_bounds__(256) k_adj_shade(ModelGPU m, Layout L, const FrameGPU* __restrict__ frames, int n,
+// dL/dI of the visible pixels through the shading, the barycentrics and the projection.  The atomics on
+// the vertices bound it; those on a frame's pose and light sums are one a workgroup and sum (one a
+// wavefront: 433 us for 48 frames, now 327).
+__global__ void __launch_bounds__(256, 2) k_adj_shade(ModelGPU m, Layout L, const FrameGPU* __restrict__ frames, int n,
                                                     const float* __restrict__ theta, const double* __restrict__ P0,
                                                     const int4* __restrict__ pvert, const float2* __restrict__ pbary,
                                                     const int* __restrict__ npix, const float* __restrict__ gI,
@@ -268,9 +296,17 @@ __global__ void __launch_bounds__(256) k_adj_shade(ModelGPU m, Layout L, const F
         for (int c = 0; c < 3; ++c)
             for (int a = 0; a < 3; ++a) atomicAdd(dPf + 3 * vv[c] + a, gC[c][a]);
     }
+    __shared__ double red[4][ADJ_G];
+#pragma unroll
     for (int j = 0; j < ADJ_G; ++j) {
         const double s = wave_sum(acc[j]);
-        if ((threadIdx.x & 63) == 0 && s != 0.0) atomicAdd(gpl + (size_t)f * ADJ_G + j, s);
+        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6][j] = s;
+    }
+    __syncthreads();
+    if (threadIdx.x < ADJ_G) {
+        const int j = threadIdx.x;
+        const double s = red[0][j] + red[1][j] + red[2][j] + red[3][j];
+        if (s != 0.0) atomicAdd(gpl + (size_t)f * ADJ_G + j, s);
     }
 }
 
@@ -321,43 +357,60 @@ __global__ void __launch_bounds__(64) k_adj_lmk(ModelGPU m, Layout L, const Fram
     }
 }
 
-// out[f][k] += sum_r basis[r][k] dP0[f][r] over the 3V rows, k < nk; rows split over gridDim.x.
-constexpr int BAS_COLS = 128;
+// out[f][k] += sum_r basis[r][k] dP0[f][r] over the 3V rows, k < nk: a product of dP0 (16 frames of
+// blockIdx.y) and the basis (80 columns of blockIdx.z) on the FP64 MFMA, the rows split over gridDim.x and
+// the wavefronts.  Reading the basis and dP0 bounds it, so a frame tile reads the basis once (a pass
+// over the basis per frame took 756 us for 48 frames and 79 columns, this 49).
+constexpr int BAS_TILES = 5;
+
+typedef double adj_v4d __attribute__((ext_vector_type(4)));
 
 __global__ void __launch_bounds__(256) k_adj_basis(int V, const float* __restrict__ basis, int ld, int nk, int n,
                                                     const double* __restrict__ dP0, double* __restrict__ out)
 {
-    __shared__ double red[4][BAS_COLS];
-    const int f = blockIdx.y;
-    if (f >= n) return;
-    const int rows = 3 * V;
-    const int r0 = (int)((long long)rows * blockIdx.x / gridDim.x), r1 = (int)((long long)rows * (blockIdx.x + 1) / gridDim.x);
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const double* d = dP0 + (size_t)f * rows;
-    for (int c0 = 0; c0 < nk; c0 += BAS_COLS) {
-        double s0 = 0.0, s1 = 0.0;
-        const int k0 = c0 + lane, k1 = c0 + 64 + lane;
-        for (int r = r0 + wave; r < r1; r += 4) {
-            const double dv = d[r];
-            if (dv == 0.0) continue;
-            const float* b = basis + (size_t)r * ld;
-            if (k0 < nk) s0 = fma((double)b[k0], dv, s0);
-            if (k1 < nk) s1 = fma((double)b[k1], dv, s1);
+    __shared__ double red[4][BAS_TILES][16][17];
+    const int rows = 3 * V, f0 = 16 * blockIdx.y, c0 = 16 * BAS_TILES * blockIdx.z;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, l16 = lane & 15, kq = lane >> 4;
+    // 16 rows a step: rows 4 kq + j of it are lane group kq's, for product j
+    const int steps = (rows + 15) / 16, parts = 4 * gridDim.x, part = 4 * blockIdx.x + wave;
+    const int s0 = (int)((long long)steps * part / parts), s1 = (int)((long long)steps * (part + 1) / parts);
+    const double* d = dP0 + (size_t)min(f0 + l16, n - 1) * rows;
+    int col[BAS_TILES];
+    adj_v4d acc[BAS_TILES];
+#pragma unroll
+    for (int t = 0; t < BAS_TILES; ++t) {
+        col[t] = min(c0 + 16 * t + l16, nk - 1);
+        acc[t] = adj_v4d{0.0, 0.0, 0.0, 0.0};
+    }
+#pragma unroll 2
+    for (int s = s0; s < s1; ++s) {
+        double a[4];
+        float b[4][BAS_TILES];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int r = 16 * s + 4 * kq + j, rc = min(r, rows - 1);
+            const double x = d[rc];
+            a[j] = r < rows ? x : 0.0;
+#pragma unroll
+            for (int t = 0; t < BAS_TILES; ++t) b[j][t] = basis[(size_t)rc * ld + col[t]];
         }
-        red[wave][lane] = s0;
-        red[wave][64 + lane] = s1;
-        __syncthreads();
-        if (wave == 0) {
-            for (int h = 0; h < 2; ++h) {
-                const int k = c0 + 64 * h + lane;
-                if (k < nk) {
-                    const double s = red[0][64 * h + lane] + red[1][64 * h + lane] + red[2][64 * h + lane] +
-                                     red[3][64 * h + lane];
-                    if (s != 0.0) atomicAdd(out + (size_t)f * nk + k, s);
-                }
-            }
-        }
-        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int t = 0; t < BAS_TILES; ++t)
+                acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[j], (double)b[j][t], acc[t], 0, 0, 0);
+    }
+    // element r of lane l: frame l / 16 + 4 r, column l % 16
+#pragma unroll
+    for (int t = 0; t < BAS_TILES; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) red[wave][t][kq + 4 * r][l16] = acc[t][r];
+    __syncthreads();
+    for (int e = threadIdx.x; e < BAS_TILES * 256; e += 256) {
+        const int t = e >> 8, i = (e >> 4) & 15, j = e & 15, f = f0 + i, k = c0 + 16 * t + j;
+        if (f >= n || k >= nk) continue;
+        const double s = red[0][t][i][j] + red[1][t][i][j] + red[2][t][i][j] + red[3][t][i][j];
+        if (s != 0.0) atomicAdd(out + (size_t)f * nk + k, s);
     }
 }
 
@@ -408,16 +461,18 @@ int launch_adjoint(const ModelGPU& m, const Layout& L, const FrameGPU* frames, i
     const int pb = std::max(1, std::min(64, (max_area + 255) / 256));
     TDI_HIP(hipMemsetAsync(a.loss, 0, sizeof(double) * n, s));
     if (grad) {
-        TDI_HIP(hipMemsetAsync(a.dB, 0, sizeof(double) * a.cap, s));
+        TDI_HIP(hipMemsetAsync(a.dg, 0, sizeof(double2) * a.cap, s));
+        TDI_HIP(hipMemsetAsync(a.edge, 0, sizeof(double) * n, s));
         TDI_HIP(hipMemsetAsync(a.dP0, 0, sizeof(double) * (size_t)n * m.V * 3, s));
         TDI_HIP(hipMemsetAsync(a.gpl, 0, sizeof(double) * (size_t)n * ADJ_G, s));
         if (L.nexp) TDI_HIP(hipMemsetAsync(a.gexp, 0, sizeof(double) * (size_t)n * L.nexp, s));
         if (L.nid) TDI_HIP(hipMemsetAsync(a.gid, 0, sizeof(double) * (size_t)n * L.nid, s));
     }
-    hipLaunchKernelGGL(k_adj_dB, dim3(pb, n), dim3(256), 0, s, frames, n, vis, npix, pixg, a.dB, a.loss, (int)grad);
+    hipLaunchKernelGGL(k_adj_dB, dim3(pb, n), dim3(256), 0, s, frames, n, vis, npix, pixg, a.dg, a.edge, a.loss,
+                       (int)grad);
     TDI_HIP(hipGetLastError());
     if (grad) {
-        hipLaunchKernelGGL(k_d2f, dim3(pb, n), dim3(256), 0, s, frames, n, a.dB, img);
+        hipLaunchKernelGGL(k_adj_dI, dim3(pb, n), dim3(256), 0, s, frames, n, a.dg, a.edge, img);
         TDI_HIP(hipGetLastError());
         int rc = launch_blur(frames, all_frames(n), taps, nullptr, img, tmp, blurred, max_area, s);
         if (rc) return rc;
@@ -429,17 +484,15 @@ int launch_adjoint(const ModelGPU& m, const Layout& L, const FrameGPU* frames, i
                        (int)grad);
     TDI_HIP(hipGetLastError());
     if (grad) {
-        const int rb = 64;
-        if (L.nexp) {
-            hipLaunchKernelGGL(k_adj_basis, dim3(rb, n), dim3(256), 0, s, m.V, m.exp_basis, m.exp_ld, L.nexp, n, a.dP0,
-                               a.gexp);
-            TDI_HIP(hipGetLastError());
-        }
-        if (L.nid) {
-            hipLaunchKernelGGL(k_adj_basis, dim3(rb, n), dim3(256), 0, s, m.V, m.id_basis, m.id_ld, L.nid, n, a.dP0,
-                               a.gid);
-            TDI_HIP(hipGetLastError());
-        }
+        auto coefficients = [&](const float* basis, int ld, int nk, double* out) {
+            // about three workgroups a compute unit; more only add atomic sums
+            const int ft = (n + 15) / 16, ct = (nk + 16 * BAS_TILES - 1) / (16 * BAS_TILES);
+            const int rb = std::max(16, std::min(256, 768 / (ft * ct)));
+            hipLaunchKernelGGL(k_adj_basis, dim3(rb, ft, ct), dim3(256), 0, s, m.V, basis, ld, nk, n, a.dP0, out);
+            return hipGetLastError();
+        };
+        if (L.nexp) TDI_HIP(coefficients(m.exp_basis, m.exp_ld, L.nexp, a.gexp));
+        if (L.nid) TDI_HIP(coefficients(m.id_basis, m.id_ld, L.nid, a.gid));
         hipLaunchKernelGGL(k_adj_out, dim3(std::max(1, std::min(256, (3 * m.V + 255) / 256)), n), dim3(256), 0, s, L,
                            m.V, n, gloss, a.gpl, a.gexp, a.gid, a.dP0, gtheta, gverts);
         TDI_HIP(hipGetLastError());

@@ -1073,21 +1073,23 @@ int tdi_render_loss_grad(tdi_batch* b, const float* theta, const float* dverts, 
     AdjScratch a{};
     a.cap = w.cap;
     const size_t C = (size_t)w.C;
-    const size_t nd = (grad ? (size_t)w.cap + C * V * 3 + C * 15 + C * c->L.nexp + C * c->L.nid : 0) + C;
-    double* blk = nullptr;
-    if (hipMalloc((void**)&blk, sizeof(double) * nd) != hipSuccess) {
-        set_error("tdi_render_loss_grad: scratch allocation of %zu bytes failed", sizeof(double) * nd);
-        return TDI_ERR_NOMEM;
-    }
-    double* q = blk;
-    a.loss = q; q += C;
+    Alloc blk;                 // from the context's pool, back to it once the stream is done
+    blk.pool = c->pool;
+    a.loss = blk.get<double>(C);
     if (grad) {
-        a.dB = q; q += w.cap;
-        a.dP0 = q; q += C * V * 3;
-        a.gpl = q; q += C * 15;
-        a.gexp = q; q += C * c->L.nexp;
-        a.gid = q;
+        a.dg = blk.get<double2>((size_t)w.cap);
+        a.edge = blk.get<double>(C);
+        a.dP0 = blk.get<double>(C * V * 3);
+        a.gpl = blk.get<double>(C * 15);
+        a.gexp = blk.get<double>(C * c->L.nexp);
+        a.gid = blk.get<double>(C * c->L.nid);
     }
+    for (void* p : blk.ptrs)
+        if (!p) {
+            blk.release();
+            set_error("tdi_render_loss_grad: scratch allocation failed");
+            return TDI_ERR_NOMEM;
+        }
     int rc = TDI_OK;
     for (int i0 = 0; i0 < b->n && !rc; i0 += w.C) {
         const int n = std::min(w.C, b->n - i0);
@@ -1102,7 +1104,7 @@ int tdi_render_loss_grad(tdi_batch* b, const float* theta, const float* dverts, 
     }
     const hipError_t e = hipStreamSynchronize(s);
     if (!rc && e != hipSuccess) { set_error("tdi_render_loss_grad: %s", hipGetErrorString(e)); rc = TDI_ERR_HIP; }
-    (void)hipFree(blk);
+    blk.release();
     return rc;
 }
 

@@ -492,7 +492,8 @@ int launch_shared_bounds(int Ks, long long KJ, const float* x, const float* lb, 
 
 // adjoint.hip: the render loss and its adjoint (scratch: device buffers of the caller)
 struct AdjScratch {
-    double* dB;        // [cap] dL/d(blurred render)
+    double2* dg;       // [cap] dL/d(gradient of the blurred render)
+    double* edge;      // [n] what of dL/d(blurred render) falls to pixel 0 at the crop's edge
     long long cap;
     double* dP0;       // [n][V][3] dL/d(model-space vertices)
     double* gpl;       // [n][15] pose (6) and light (9)
