@@ -114,7 +114,9 @@ __device__ __forceinline__ int ch_root(double d, double& s, double& y, F fill)
     return 12;
 }
 
-// A = L L^T in place; false (for every thread) at a pivot that is not positive.
+// A = L L^T in place; false (for every thread) at a pivot that is not positive.  *sflag: zero for every
+// thread at the start.  On false a wavefront may return while another has yet to read *sflag, so
+// neither it nor A may be written before the next barrier.
 template <typename T>
 __device__ __forceinline__ bool ch_factor(T* A, int nT, int* sflag)
 {

@@ -392,15 +392,18 @@ __global__ void __launch_bounds__(256) k_cholesky(int K, const TH* __restrict__ 
     const int f = blockIdx.x;
     if (mask && !mask[f]) return;
     extern __shared__ double dsm[];
-    __shared__ int sflag;
-    __shared__ double sb[CMAXK];                 // the residual, then the verdict
+    // a pivot that is not positive, of the FP32 and of the FP64 factorisation: two flags, as the wavefronts
+    // read the first after their last common barrier and nothing may write it from then on
+    __shared__ int sbad[2];
+    __shared__ int sdone;                        // the FP32 solution is good
+    __shared__ double sb[CMAXK];                 // the residual
     __shared__ float sx[CMAXK];
     const TH* Hf = H + (size_t)f * K * K;
     const float* gf = g + (size_t)f * K;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int nT = (K + CHB - 1) / CHB;
     const bool in0 = lane < K, in1 = lane + 64 < K;
-    if (tid == 0) sflag = 0;
+    if (tid == 0) sbad[0] = sbad[1] = sdone = 0;
     if (mode != 0) {
         float* A = (float*)dsm;
         __shared__ float sdinv[CMAXK];
@@ -411,7 +414,7 @@ __global__ void __launch_bounds__(256) k_cholesky(int K, const TH* __restrict__ 
         __syncthreads();
         ch_load<float, TH>(A, Hf, K, nT, sdinv);
         __syncthreads();
-        if (ch_factor<float>(A, nT, &sflag)) {
+        if (ch_factor<float>(A, nT, &sbad[0])) {
             float x0 = 0.f, x1 = 0.f;            // wavefront 0: the FP32 solution
             if (wave == 0) {
                 x0 = in0 ? -gf[lane] * sdinv[lane] : 0.f;
@@ -466,20 +469,17 @@ __global__ void __launch_bounds__(256) k_cholesky(int K, const TH* __restrict__ 
                     if (in1) delta[(size_t)f * K + lane + 64] = (float)((double)x1 + c1);
                     if (lane == 0) status[f] = TDI_OK;
                 }
-                if (lane == 0) sflag = good ? 2 : 0;
+                if (lane == 0) sdone = good;
             }
-        } else if (tid == 0) {
-            sflag = 0;                            // read by every thread before (ch_factor's barrier)
         }
         __syncthreads();
-        if (sflag == 2) return;
-        __syncthreads();
+        if (sdone) return;
     }
     // FP64 factorisation and solve (mode 0, and the fallback of mode 1)
     double* A = dsm;
     ch_load<double, TH>(A, Hf, K, nT, nullptr);
     __syncthreads();
-    if (!ch_factor<double>(A, nT, &sflag)) {
+    if (!ch_factor<double>(A, nT, &sbad[1])) {
         if (tid == 0) status[f] = TDI_NOT_PD;
         return;
     }

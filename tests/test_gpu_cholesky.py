@@ -53,3 +53,42 @@ def test_ill_conditioned_and_not_positive_definite(mode):
         want = -np.linalg.solve(h, g[i].astype(np.float64))
         scale = np.abs(h) @ np.abs(want) + np.abs(g[i])
         assert np.all(np.abs(h @ x + g[i]) <= 2.0 ** -23 * scale)   # FP32 rounding of the solution
+
+
+def test_fp32_pivots_that_break_down():
+    """Matrices that FP64 factors and FP32 does not: H = S L L^T S, L unit lower bidiagonal with 2 or 3 below
+    the diagonal in chains of eleven, S whole numbers; exact in FP32, condition below 2^38.  The pivots of
+    L L^T are 1 and an error in one grows by 4 to 9 a column, so FP32's turn negative or leave a correction
+    that is refused, and mode 1 ends in the FP64 factorisation: the bits of mode 0.  Every fourth matrix is
+    not positive definite in either."""
+    rng = np.random.default_rng(11)
+    n, K = 256, 94
+    c = rng.integers(2, 4, (n, K))
+    c[:, ::11] = 0
+    L = np.tile(np.eye(K), (n, 1, 1))
+    L[:, np.arange(1, K), np.arange(K - 1)] = c[:, 1:]
+    S = rng.integers(50, 201, (n, K)).astype(np.float64)
+    H = S[:, :, None] * (L @ L.transpose(0, 2, 1)) * S[:, None, :]
+    h = H.astype(np.float32)
+    assert (h == H).all()
+    # the FP32 pivots of the equilibrated matrices (tridiagonal)
+    r = np.einsum("nii->ni", h) ** np.float32(-0.5)
+    s = h * r[:, :, None] * r[:, None, :]
+    d, broke = s[:, 0, 0], np.zeros(n, bool)
+    for k in range(1, K):
+        d = s[:, k, k] - s[:, k, k - 1] ** 2 / d
+        broke |= ~(d > 0)
+        d = np.where(d > 0, d, np.float32(1))
+    assert broke.sum() > n // 2                  # the break-down is reached, whatever the last bits
+    x = rng.integers(-4, 5, (n, K))
+    g = -np.einsum("nij,nj->ni", H, x)
+    assert (g == g.astype(np.float32)).all()
+    bad = np.arange(n) % 4 == 3
+    h[bad, 50, 50] = -1.0
+    ht, gt = torch.from_numpy(h).cuda(), torch.from_numpy(g.astype(np.float32)).cuda()
+    d0, st0 = (t.cpu().numpy() for t in tdi.cholesky_solve(ht, gt, 0))
+    d1, st1 = (t.cpu().numpy() for t in tdi.cholesky_solve(ht, gt, 1))
+    assert (st0 == np.where(bad, 4, 0)).all() and (st1 == st0).all()
+    assert (d0[~bad] == d1[~bad]).all()
+    # |x| <= 4; FP64's error is about K 2^-53 times the condition
+    assert np.abs(d0[~bad] - x[~bad]).max() < 2.0 ** -8
