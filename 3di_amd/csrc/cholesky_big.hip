@@ -162,7 +162,6 @@ __global__ void __launch_bounds__(256) k_chol_update(int K, int k0, double* __re
                                                       int* __restrict__ status)
 {
     const int mtx = blockIdx.y;
-    if (status[mtx] != TDI_OK) return;
     const int r0 = k0 + CB;                        // first trailing row
     const int T = (K - r0 + CB - 1) / CB;
     int t = blockIdx.x, ti = 0;
@@ -171,8 +170,11 @@ __global__ void __launch_bounds__(256) k_chol_update(int K, int k0, double* __re
     const int tj = t;
     double* M = A + (size_t)mtx * K * K;
     __shared__ double Li[CB][CB + 1], Lj[CB][CB + 1];
+    __shared__ int sok;
     const int tid = threadIdx.x;
     const int nb = min(CB, K - k0);
+    // one read for the whole workgroup: the one that factors the next diagonal block may write it meanwhile
+    if (tid == 0) sok = status[mtx] == TDI_OK;
     {
         // every load of both slices issued before the LDS stores (256 threads, 4 entries each)
         double vi[CB * CB / 256], vj[CB * CB / 256];
@@ -193,6 +195,7 @@ __global__ void __launch_bounds__(256) k_chol_update(int K, int k0, double* __re
         }
     }
     __syncthreads();
+    if (!sok) return;
     // 256 threads x 4 entries: thread (a, b4) computes row a, columns b4..b4+3 of the tile
     const int a = tid >> 3, b4 = (tid & 7) * 4;
     double acc[4] = {0.0, 0.0, 0.0, 0.0};
