@@ -214,6 +214,7 @@ struct Workspace {
     float2* pshade = nullptr;
     uint2 *ptri = nullptr, *plist = nullptr;
     int* pstart = nullptr;
+    int nseg = 1;
     float* dI = nullptr;         // [cap][dI_stride(K)]
     float *theta = nullptr, *theta_try = nullptr, *delta = nullptr, *g = nullptr;
     double* H = nullptr;       // [C][K][K] normal matrices (FP64)
@@ -534,7 +535,8 @@ static int ws_alloc(tdi_batch* b, int C, long long cap)
     w.pshade = c->L.ntex ? A.get<float2>(cap) : nullptr;
     w.ptri = c->m.np ? A.get<uint2>(cap) : nullptr;
     w.plist = c->m.np ? A.get<uint2>(cap) : nullptr;
-    w.pstart = c->m.np ? A.get<int>((size_t)C * (c->m.np + 1)) : nullptr;
+    w.nseg = patch_segments(C, b->max_area);
+    w.pstart = c->m.np ? A.get<int>((size_t)C * w.nseg * (c->m.np + 1)) : nullptr;
     w.dI = A.get<float>((size_t)cap * dI_stride(K));
     w.theta = A.get<float>((size_t)C * K);
     w.theta_try = A.get<float>((size_t)C * K);
@@ -616,7 +618,7 @@ static int dI_area(const Workspace& w)
 
 static JacScratch jac_scratch(const Workspace& w)
 {
-    return JacScratch{w.pq, w.pshade, w.ptri, w.plist, w.pstart};
+    return JacScratch{w.pq, w.pshade, w.ptri, w.plist, w.pstart, w.nseg, mean_crop(w)};
 }
 
 static LmkArrays lmk_arrays(const Workspace& w)

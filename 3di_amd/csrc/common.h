@@ -418,17 +418,22 @@ int launch_ortho_init(const ModelGPU& m, int n, const float* lmk, const float* c
 // row stride of dI: K padded so that rows start on 16 bytes
 inline __host__ __device__ int dI_stride(int K) { return (K + 3) & ~3; }
 // per visible position: q (dI of a model-space direction e is q . e); Id and S of the shading (fitted
-// albedo only); patch and corners of its triangle; per frame the positions sorted by patch
+// albedo only); patch and corners of its triangle; per frame the positions sorted by patch, in segments
 struct JacScratch {
     float4* pq;
     float2* pshade;
     const uint2* ptri;
     uint2* plist;
-    int* pstart;           // [slots][np + 1]
+    int* pstart;           // [slots][nseg][np + 1]
+    int nseg;              // patch_segments
+    int mean_area;         // mean crop of the workspace
 };
+// Segments of a frame's positions for a workspace of so many frame slots and crops of up to max_area
+// pixels (half of them visible): enough that sorting few large frames takes the whole chip.
+int patch_segments(int frames, int max_area);
 int launch_dI(const ModelGPU& m, const Layout& L, const FrameGPU* frames, FrameList fl, const float* theta,
               const double* P0, const int4* pvert, const float2* pbary, const int* npix, const float4* pixg,
-              const JacScratch& js, float* dI, int mean_area, int max_area, hipStream_t s);
+              const JacScratch& js, float* dI, int grid_area, int max_area, hipStream_t s);
 // the light columns alone ([pixel][4]: lambda, Lintensity) of the four appended light unknowns
 int launch_dI_light(const ModelGPU& m, const Layout& L, const FrameGPU* frames, FrameList fl, const float* theta,
                     const double* P0, const int4* pvert, const float2* pbary, const int* npix, float* dIl, int max_area,

@@ -307,12 +307,15 @@ __global__ void __launch_bounds__(256) k_dI(ModelGPU m, Layout L, const FrameGPU
     }
 }
 
-// The visible positions of a frame sorted by the mesh patch of their triangle: a count, a prefix sum and
-// a scatter by one workgroup per frame, the patches' counts in LDS.  plist: (position, corners' places).
-constexpr int BIN_THREADS = 1024;
+// The visible positions of a frame sorted by the mesh patch of their triangle, in nseg segments of
+// consecutive positions: a count, a prefix sum and a scatter by one workgroup per segment, the patches'
+// counts in LDS.  plist: (position, corners' places), a segment's in its own range; pstart: per frame and
+// segment.  One workgroup takes about 2 ns a position, so with few frames a large one is cut (see
+// patch_segments; frames of fewer than BIN_PX positions per segment leave the last ones empty).
+constexpr int BIN_THREADS = 1024, BIN_PX = 8192;
 
 __global__ void __launch_bounds__(BIN_THREADS) k_patch_bin(const FrameGPU* __restrict__ frames, const int* __restrict__ act,
-                                                            int n, const int* __restrict__ npix, int np,
+                                                            int n, const int* __restrict__ npix, int np, int nseg,
                                                             const uint2* __restrict__ ptri, uint2* __restrict__ plist,
                                                             int* __restrict__ pstart)
 {
@@ -320,14 +323,15 @@ __global__ void __launch_bounds__(BIN_THREADS) k_patch_bin(const FrameGPU* __res
     __shared__ int swave[BIN_THREADS / 64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int nact = fl_count(act, n);
-    for (int yi = blockIdx.x; yi < nact; yi += gridDim.x) {
+    for (int yi = blockIdx.y; yi < nact; yi += gridDim.y) {
         const int f = fl_frame(act, yi);
         const long long base = frames[f].pix_off;
-        const int N = npix[f];
+        const int N = npix[f], seg = blockIdx.x, ns = min(nseg, max(1, (N + BIN_PX - 1) / BIN_PX));
+        const int q0 = seg < ns ? (int)((long long)N * seg / ns) : N, q1 = seg < ns ? (int)((long long)N * (seg + 1) / ns) : N;
         for (int p = tid; p < np; p += BIN_THREADS) hist[p] = 0;
         __syncthreads();
 #pragma unroll 4
-        for (int pos = tid; pos < N; pos += BIN_THREADS) atomicAdd(&hist[ptri[base + pos].x], 1);
+        for (int pos = q0 + tid; pos < q1; pos += BIN_THREADS) atomicAdd(&hist[ptri[base + pos].x], 1);
         __syncthreads();
         // exclusive prefix sum, PATCH_MAX / BIN_THREADS consecutive patches per thread
         constexpr int PER = PATCH_MAX / BIN_THREADS;
@@ -345,10 +349,10 @@ __global__ void __launch_bounds__(BIN_THREADS) k_patch_bin(const FrameGPU* __res
         }
         if (lane == 63) swave[wave] = run;
         __syncthreads();
-        int at = run - sum;
+        int at = q0 + run - sum;
 #pragma unroll
         for (int w = 0; w < BIN_THREADS / 64; ++w) at += w < wave ? swave[w] : 0;
-        int* ps = pstart + (size_t)f * (np + 1);
+        int* ps = pstart + ((size_t)f * nseg + seg) * (np + 1);
 #pragma unroll
         for (int k = 0; k < PER; ++k) {
             const int p = tid * PER + k;
@@ -358,10 +362,10 @@ __global__ void __launch_bounds__(BIN_THREADS) k_patch_bin(const FrameGPU* __res
             }
             at += c[k];
         }
-        if (tid == 0) ps[np] = N;
+        if (tid == 0) ps[np] = q1;
         __syncthreads();
 #pragma unroll 4
-        for (int pos = tid; pos < N; pos += BIN_THREADS) {
+        for (int pos = q0 + tid; pos < q1; pos += BIN_THREADS) {
             const uint2 t = ptri[base + pos];
             plist[base + atomicAdd(&hist[t.x], 1)] = make_uint2((unsigned)pos, t.y);
         }
@@ -373,15 +377,17 @@ __global__ void __launch_bounds__(BIN_THREADS) k_patch_bin(const FrameGPU* __res
 // vertices' basis rows, 2880 bytes at 80 columns: gathered per pixel that is 8 times the row it writes,
 // through L2 and beyond (159 GB of HBM traffic for 4096 frames, 7.7 TB/s, 25.8 ms).  Here a workgroup
 // holds the rows of one patch (PATCH_VERTS vertices, 120 KB of LDS) and walks the pixels that all its
-// frames have on it, so a basis row leaves HBM once per slice of the list.  A wavefront takes a
-// frame's pixels 64 at a time: their records into its own part of LDS, then four pixels per step, 16
-// lanes over the columns of each (columns 4 l .. 4 l + 3 and 64 + l of lane l).
-constexpr int PT_THREADS = 1024, PT_WAVES = PT_THREADS / 64, PT_COLS = 80;
+// frames have on it, so a basis row leaves HBM once per slice of the list.  A wavefront takes a unit's
+// pixels 64 at a time: their records into its own part of LDS, then four pixels per step, 16 lanes over
+// the columns of each (columns 4 l .. 4 l + 3 and 64 + l of lane l).  A unit is a frame, or one of its
+// segments (k_patch_bin), or, where these are fewer than the wavefronts of gridDim.y workgroups, every
+// parts-th 64 pixels of one.
+constexpr int PT_THREADS = 1024, PT_WAVES = PT_THREADS / 64, PT_COLS = 80, PT_PARTS = 16;
 constexpr size_t PT_LDS = sizeof(float) * PATCH_VERTS * 3 * PT_COLS + sizeof(float4) * 2 * 64 * PT_WAVES;
 
 __global__ void __launch_bounds__(PT_THREADS) k_dI_patch(ModelGPU m, const float* __restrict__ basis, int ld, int k0,
                                                           int nc, int off, int ldI, const FrameGPU* __restrict__ frames,
-                                                          const int* __restrict__ act, int n,
+                                                          const int* __restrict__ act, int n, int nseg,
                                                           const uint2* __restrict__ plist, const int* __restrict__ pstart,
                                                           const float4* __restrict__ pq, const float2* __restrict__ pbary,
                                                           float* __restrict__ dI)
@@ -392,11 +398,14 @@ __global__ void __launch_bounds__(PT_THREADS) k_dI_patch(ModelGPU m, const float
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = uniform(tid >> 6);
     float4* rec = spt + PATCH_VERTS * 3 * PT_COLS / 4 + 2 * 64 * wave;  // [64]: (q, al), (be, ga, position, places)
-    const int nact = fl_count(act, n);
+    const int segs = fl_count(act, n) * nseg;
+    if (segs == 0) return;
     const int p = blockIdx.x;
-    const int y0 = (int)((long long)nact * blockIdx.y / gridDim.y), y1 = (int)((long long)nact * (blockIdx.y + 1) / gridDim.y);
-    if (y0 == y1) return;
-    if (tid == 0) snext = y0;
+    const int parts = max(1, min(PT_PARTS, PT_WAVES * (int)gridDim.y / segs)), per = nseg * parts;
+    const long long units = (long long)segs * parts;
+    const int u0 = (int)(units * blockIdx.y / gridDim.y), u1 = (int)(units * (blockIdx.y + 1) / gridDim.y);
+    if (u0 == u1) return;
+    if (tid == 0) snext = u0;
     {
         const int* pv = m.patch_vert + m.patch_off[p];
         const int nv = m.patch_off[p + 1] - m.patch_off[p];
@@ -411,17 +420,23 @@ __global__ void __launch_bounds__(PT_THREADS) k_dI_patch(ModelGPU m, const float
     __syncthreads();
     const int sub = lane >> 4, l16 = lane & 15;
     const bool vec = ((off + k0) & 3) == 0;
-    // frames differ in their pixels on the patch: each wavefront takes the next one left
+    // units differ in their pixels on the patch: each wavefront takes the next one left
     for (;;) {
-        int yi = 0;
-        if (lane == 0) yi = atomicAdd(&snext, 1);
-        yi = uniform(yi);
-        if (yi >= y1) break;
+        int u = 0;
+        if (lane == 0) u = atomicAdd(&snext, 1);
+        u = uniform(u);
+        if (u >= u1) break;
+        int yi = u, seg = 0, part = 0;
+        if (per > 1) {
+            yi = u / per;
+            seg = (u - yi * per) / parts;
+            part = u - (yi * nseg + seg) * parts;
+        }
         const int f = fl_frame(act, yi);
         const long long base = frames[f].pix_off;
-        const int* ps = pstart + (size_t)f * (m.np + 1) + p;
+        const int* ps = pstart + ((size_t)f * nseg + seg) * (m.np + 1) + p;
         const int e1 = ps[1];
-        for (int e0 = ps[0]; e0 < e1; e0 += 64) {
+        for (int e0 = ps[0] + 64 * part; e0 < e1; e0 += 64 * parts) {
             const int cnt = min(64, e1 - e0);
             if (lane < cnt) {
                 const uint2 t = plist[base + e0 + lane];
@@ -1325,15 +1340,34 @@ int jtj_splits(int n, int per_frame_pixels_hint)
     return S;
 }
 
-// From this many listed frames on, the geometric columns go through mesh patches: below, too few pixels
-// share a patch to pay for loading it and for the sorting.  The whole stage by gathers against patches,
-// crops of 96 to 384 pixels: 1 frame 26 against 35 us, 4 frames 89 / 84, 8 frames 94 / 92, 12 frames
-// 93 / 71, 48 frames 418 / 219 us.
-constexpr int PATCH_MIN_FRAMES = 8;
+// Whether the geometric columns of n listed frames (mean_area crop pixels each) go through mesh patches.
+// Sorting the pixels and loading every patch cost about 25 us and the mesh's basis rows, and a patch's
+// workgroups are as busy as its share of the pixels is large: frames times patches, few columns or a few
+// thousand pixels decide.  The whole stage by gathers against patches (us; 79 columns unless stated; n
+// crops, side; 27% visible):
+//     506 patches   8, 96: 27/37     8, 192: 58/50   24, 192: 149/81   96, 192: 486/223   8, 1024: 840/568
+//      94 patches   24, 96: 38/46    8, 192: 43/53   24, 192: 91/85    96, 192: 363/203   8, 512: 173/244
+//      38 patches   24, 96: 33/47    8, 512: 160/361 24, 192: 78/88    96, 192: 339/228   48, 512: 1236/1000
+//       6 patches   48, 512: 1227/1290               24, 192: 76/86    96, 192: 322/270   448, 96: 388/245
+//     506 patches, 30 columns        8, 512: 133/127 24, 192: 87/68    94 patches, 30: 24, 192: 68/78, 96, 192: 265/190
+//       6 patches, 30 columns        96, 192: 243/264                  448, 96: 296/218
+static bool patch_path(const ModelGPU& m, const Layout& L, int n, int mean_area)
+{
+    const int cols = L.nexp + L.nid;
+    if (m.np == 0 || cols == 0 || n < 8) return false;
+    const bool few = cols < PT_COLS / 2;
+    return (n >= (few ? 128 : 64) || (long long)n * m.np >= (few ? 8192 : 2048)) &&
+           (long long)n * mean_area >= std::max(1 << 18, 512 * m.np);
+}
+
+int patch_segments(int frames, int max_area)
+{
+    return std::max(1, std::min((max_area / 2 + BIN_PX - 1) / BIN_PX, 512 / std::max(1, frames)));
+}
 
 int launch_dI(const ModelGPU& m, const Layout& L, const FrameGPU* frames, FrameList fl, const float* theta,
               const double* P0, const int4* pvert, const float2* pbary, const int* npix, const float4* pixg,
-              const JacScratch& js, float* dI, int mean_area, int max_area, hipStream_t s)
+              const JacScratch& js, float* dI, int grid_area, int max_area, hipStream_t s)
 {
     if (L.ntex > 512) {
         set_error("dI: k_tex %d > 512", L.ntex);
@@ -1344,29 +1378,30 @@ int launch_dI(const ModelGPU& m, const Layout& L, const FrameGPU* frames, FrameL
     const int px = std::max(1, std::min((max_area / 2 + 255) / 256, std::max(16, std::min(256, 8192 / std::max(1, fl.n)))));
     hipLaunchKernelGGL(k_dI_px, dim3(px, gy), dim3(256), 0, s, m, L, frames, fl.act, fl.n, theta, P0, pvert, pbary, npix,
                        pixg, js.pq, js.pshade, dI);
-    const bool patch = m.np > 0 && fl.n >= PATCH_MIN_FRAMES && L.nexp + L.nid > 0;
+    const bool patch = patch_path(m, L, fl.n, js.mean_area);
     if (patch) {
         // 155 KB of dynamic LDS, allowed once per process
         static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(k_dI_patch),
                                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)PT_LDS);
         TDI_HIP(attr);
-        hipLaunchKernelGGL(k_patch_bin, dim3(gy), dim3(BIN_THREADS), 0, s, frames, fl.act, fl.n, npix, m.np, js.ptri,
-                           js.plist, js.pstart);
-        // about 128 frames per workgroup, eight per wavefront: its patch is loaded once for them
-        const int slices = std::max(1, std::min(64, fl.n / 128));
+        hipLaunchKernelGGL(k_patch_bin, dim3(js.nseg, gy), dim3(BIN_THREADS), 0, s, frames, fl.act, fl.n, npix, m.np,
+                           js.nseg, js.ptri, js.plist, js.pstart);
+        // about 128 frames per workgroup, eight per wavefront: its patch is loaded once for them; and where
+        // the mesh has few patches, about two workgroups a compute unit (half of the patches face away)
+        const int slices = std::max(1, std::min(128, std::max(fl.n / 128, 512 / m.np)));
         for (int blk = 0; blk < 2; ++blk) {
             const int nc = blk ? L.nid : L.nexp, off = blk ? L.off_id : L.off_exp, ld = blk ? m.id_ld : m.exp_ld;
             for (int k0 = 0; k0 < nc; k0 += PT_COLS)
                 hipLaunchKernelGGL(k_dI_patch, dim3(m.np, slices), dim3(PT_THREADS), PT_LDS, s, m,
                                    blk ? m.id_basis : m.exp_basis, ld, k0, std::min(PT_COLS, nc - k0), off, dI_stride(L.K),
-                                   frames, fl.act, fl.n, js.plist, js.pstart, js.pq, pbary, dI);
+                                   frames, fl.act, fl.n, js.nseg, js.plist, js.pstart, js.pq, pbary, dI);
         }
     }
     if (!patch || L.ntex) {
         // 8 DI_PASSES strips per frame, each shared by up to nsb workgroups; one frame per grid row
-        // (sized for a quarter-visible mean crop: larger frames loop, and few workgroups of a grid
+        // (sized for a quarter-visible crop of grid_area: larger frames loop, and few workgroups of a grid
         // row find no pixels)
-        int nsb = (mean_area / 4 + 8 * DI_PASSES * DI_PX_PER_WG - 1) / (8 * DI_PASSES * DI_PX_PER_WG);
+        int nsb = (grid_area / 4 + 8 * DI_PASSES * DI_PX_PER_WG - 1) / (8 * DI_PASSES * DI_PX_PER_WG);
         if (nsb > 64) nsb = 64;
         if (nsb < 1) nsb = 1;
         hipLaunchKernelGGL(k_dI, dim3(8 * nsb, gy, DI_PASSES), dim3(256), 0, s, m, L, frames, fl.act, fl.n, theta, pvert,
