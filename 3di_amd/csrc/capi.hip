@@ -2366,9 +2366,11 @@ static int record_piece(tdi_batch* b, FitPiece piece, hipStream_t s)
     // the finetune fit's trials keep the pose (model_fitter.cu:502)
     const int hold0 = b->finetune ? c->L.off_pose : 0, hold1 = b->finetune ? c->L.off_pose + 6 : 0;
     const bool head = piece == PIECE_HEAD_STALE || piece == PIECE_HEAD_FRESH || piece == PIECE_HEAD_BOTH;
+    const int rounds = ls_rounds(o);
     auto propose = [&]() -> int {
-        const int rc = launch_ls_propose(n, c->L, o.t_min, w.st, w.theta, w.delta, w.theta_try, w.rt, w.searching,
-                                         w.evalmask, hold0, hold1, s);
+        // without a round the next evaluation reuses theta's render, with its rotations in w.rt
+        const int rc = launch_ls_propose(n, c->L, o.t_min, w.st, w.theta, w.delta, w.theta_try, rounds > 0 ? w.rt : nullptr,
+                                         w.searching, w.evalmask, hold0, hold1, s);
         return rc ? rc : launch_ls_status(n, w.st, w.evalmask, w.act_e, w.seq, b->status, s);
     };
     int rc;
@@ -2387,7 +2389,7 @@ static int record_piece(tdi_batch* b, FitPiece piece, hipStream_t s)
             return rc;
         if ((rc = launch_ls_init(n, K, w.st, w.status, w.delta, w.g, w.obj, w.searching, s))) return rc;
         if ((rc = propose())) return rc;
-        if (ls_rounds(o) == 0) return TDI_OK;
+        if (rounds == 0) return TDI_OK;
     }
     // k_ls_propose left the trials' rotations; k_ls_decide sums their objectives
     if ((rc = eval_objective(b, FrameList{w.act_e, w.C}, w.theta_try, s, nullptr, true))) return rc;

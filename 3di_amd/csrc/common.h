@@ -527,7 +527,7 @@ int launch_cholesky(int n, int K, const double* H, const float* g, float* delta,
 int launch_ls_init(int n, int K, FitState* st, const int* chol_status, const float* delta, const float* g,
                    const double* obj, int* searching, hipStream_t s);
 // unknowns [hold0, hold1) keep theta's values in the trials (hold0 == hold1: none); rt: the trials'
-// rotations and translations
+// rotations and translations, for the evaluation that follows (null: none follows)
 int launch_ls_propose(int n, const Layout& L, float t_min, FitState* st, const float* theta, const float* delta,
                       float* theta_try, double* rt, int* searching, int* evalmask, int hold0, int hold1, hipStream_t s);
 // obj: written from the barrier's value and the objective's partials (of the list act's evaluation)

@@ -528,7 +528,7 @@ __global__ void __launch_bounds__(64) k_ls_init(int n, int K, FitState* __restri
 }
 
 // Trials theta + t delta; unknowns [hold0, hold1) keep theta's value (the finetune fit's pose,
-// model_fitter.cu:502).
+// model_fitter.cu:502).  rt null: no evaluation follows, and theta's render and rotation stay.
 __global__ void k_ls_propose(int n, int K, int off_pose, float t_min, FitState* __restrict__ st,
                              const float* __restrict__ theta, const float* __restrict__ delta,
                              float* __restrict__ theta_try, double* __restrict__ rt, int* __restrict__ searching,
@@ -573,7 +573,7 @@ __global__ void k_ls_propose(int n, int K, int off_pose, float t_min, FitState* 
     }
     __syncthreads();
     // the trial's rotation and translation for the synthesis that follows
-    if (threadIdx.x == 0) {
+    if (threadIdx.x == 0 && rt) {
         double R[9];
         rodrigues_f64(pose + 3, R);
         for (int k = 0; k < 9; ++k) rt[(size_t)f * 12 + k] = R[k];
