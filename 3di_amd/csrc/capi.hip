@@ -1784,10 +1784,13 @@ int tdi_barrier_terms(tdi_batch* b, const float* theta, double* H, double* g, do
         int rc = ws_load(b, i0, n, s);
         if (rc) return rc;
         const float* th = theta + (size_t)i0 * K;
-        if ((rc = launch_synthesize(b->m, c->L, w.frames, all_frames(n), th, w.rt, w.P0, nullptr, w.vproj, s))) return rc;
+        if (c->opts.use_landmarks &&
+            (rc = launch_synthesize(b->m, c->L, w.frames, all_frames(n), th, w.rt, w.P0, nullptr, w.vproj, s)))
+            return rc;
         TDI_HIP(hipMemsetAsync(w.H, 0, sizeof(double) * (size_t)n * K * K, s));
         TDI_HIP(hipMemsetAsync(w.g, 0, sizeof(float) * (size_t)n * K, s));
-        if ((rc = barrier_objective(b, c->L, all_frames(n), th, s)))
+        if ((rc = launch_barrier_obj(c->m, c->L, w.frames, all_frames(n), th, w.rt, w.P0, w.vproj, lmk_arrays(w),
+                                     c->opts.use_landmarks, 0.f, w.obj, w.objb, nullptr, s)))
             return rc;
         if ((rc = launch_barrier(c->m, c->L, w.frames, all_frames(n), th, w.rt, w.P0, lmk_arrays(w),
                                  c->opts.use_landmarks, w.H, w.g, s)))

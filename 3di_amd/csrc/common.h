@@ -463,7 +463,8 @@ int launch_jtj_mfma(const Layout& L, const FrameGPU* frames, FrameList fl, const
 int launch_barrier_obj(const ModelGPU& m, const Layout& L, const FrameGPU* frames, FrameList fl, const float* theta,
                        const double* rt, const double* P0, const float4* vproj, const LmkArrays& lm, int use_landmarks,
                        float ref_face_size, double* obj, double* objb, int* face_ok, hipStream_t s);
-// the derivative terms, K <= 112, and at any K (D is [n][2][NLMK][K] doubles of scratch)
+// the derivative terms, K <= 112 with landmarks, and at any K (D is [n][2][NLMK][K] doubles of scratch;
+// unused without landmarks)
 int launch_barrier(const ModelGPU& m, const Layout& L, const FrameGPU* frames, FrameList fl, const float* theta,
                    const double* rt, const double* P0, const LmkArrays& lm, int use_landmarks, double* H, float* g,
                    hipStream_t s);

@@ -824,6 +824,8 @@ int launch_barrier(const ModelGPU& m, const Layout& L, const FrameGPU* frames, F
                    const double* rt, const double* P0, const LmkArrays& lm, int use_landmarks, double* H, float* g, hipStream_t s)
 {
     if (L.K > BMAXK) {
+        if (!use_landmarks)              // bounds alone: no landmark rows to hold
+            return launch_barrier_big(m, L, frames, fl, theta, rt, P0, lm, 0, nullptr, H, g, s);
         set_error("barrier: K=%d > %d (derivative terms: launch_barrier_big)", L.K, BMAXK);
         return TDI_ERR_ARG;
     }
