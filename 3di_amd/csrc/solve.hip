@@ -830,9 +830,9 @@ int launch_barrier(const ModelGPU& m, const Layout& L, const FrameGPU* frames, F
         return TDI_ERR_ARG;
     }
     const size_t lds = use_landmarks ? sizeof(double) * 2 * NLMK * ((L.K + 3) & ~3) : 0;
-    if (lds > 56 * 1024) {
-        // with the static part above the default limit: allow up to what K <= BMAXK needs (91 KB), once
-        // per process
+    if (use_landmarks) {
+        // with the static part (10 KB) above the default limit from 65 unknowns on: allow up to what K <= BMAXK
+        // needs (91 KB), once per process
         static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(k_barrier),
                                                            hipFuncAttributeMaxDynamicSharedMemorySize,
                                                            (int)(sizeof(double) * 2 * NLMK * BMAXK));
