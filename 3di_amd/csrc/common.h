@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 #include <algorithm>
+#include <atomic>
 #include <cstdint>
 #include <cstdio>
 #include <string>
@@ -333,6 +334,19 @@ void set_error(const char* fmt, ...);
 // ------------------------------------------------------------------ kernel launchers
 // All launchers take device pointers and a stream; n = frames in the call; mask selects
 // which frames take part (NULL = all).
+
+// Allows a kernel up to `bytes` of dynamic LDS on the current device (the limit belongs to the kernel on
+// one device); `done` is the kernel's own record of the devices that have it.
+inline hipError_t allow_lds(const void* kernel, size_t bytes, std::atomic<unsigned long long>& done)
+{
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    const unsigned long long bit = dev < 64 ? 1ull << dev : 0;
+    if (e != hipSuccess || (done.load(std::memory_order_relaxed) & bit)) return e;
+    e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+    if (e == hipSuccess) done.fetch_or(bit, std::memory_order_relaxed);
+    return e;
+}
 
 // Landmarks per frame, [n][6][51]: x, y (image pixels), box lx, ux, ly, uy (face-size units).
 // The frames a per-frame launch works on: every workspace slot 0..n-1 (act == nullptr), or

@@ -1380,10 +1380,8 @@ int launch_dI(const ModelGPU& m, const Layout& L, const FrameGPU* frames, FrameL
                        pixg, js.pq, js.pshade, dI);
     const bool patch = patch_path(m, L, fl.n, js.mean_area);
     if (patch) {
-        // 155 KB of dynamic LDS, allowed once per process
-        static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(k_dI_patch),
-                                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)PT_LDS);
-        TDI_HIP(attr);
+        static std::atomic<unsigned long long> done{0};
+        TDI_HIP(allow_lds(reinterpret_cast<const void*>(k_dI_patch), PT_LDS, done));   // 155 KB
         hipLaunchKernelGGL(k_patch_bin, dim3(js.nseg, gy), dim3(BIN_THREADS), 0, s, frames, fl.act, fl.n, npix, m.np,
                            js.nseg, js.ptri, js.plist, js.pstart);
         // about 128 frames per workgroup, eight per wavefront: its patch is loaded once for them; and where

@@ -832,11 +832,9 @@ int launch_barrier(const ModelGPU& m, const Layout& L, const FrameGPU* frames, F
     const size_t lds = use_landmarks ? sizeof(double) * 2 * NLMK * ((L.K + 3) & ~3) : 0;
     if (use_landmarks) {
         // with the static part (10 KB) above the default limit from 65 unknowns on: allow up to what K <= BMAXK
-        // needs (91 KB), once per process
-        static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(k_barrier),
-                                                           hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                           (int)(sizeof(double) * 2 * NLMK * BMAXK));
-        TDI_HIP(attr);
+        // needs (91 KB)
+        static std::atomic<unsigned long long> done{0};
+        TDI_HIP(allow_lds(reinterpret_cast<const void*>(k_barrier), sizeof(double) * 2 * NLMK * BMAXK, done));
     }
     hipLaunchKernelGGL(k_barrier, dim3(fl.n > 0 ? fl.n : 1), dim3(BAR_THREADS), lds, s, m, L, frames, fl.act, fl.n, theta,
                        rt, P0, lm, use_landmarks, H, g);
