@@ -431,6 +431,9 @@ int launch_ortho_init(const ModelGPU& m, int n, const float* lmk, const float* c
 
 // row stride of dI: K padded so that rows start on 16 bytes
 inline __host__ __device__ int dI_stride(int K) { return (K + 3) & ~3; }
+// byte offset of a position's row, where a frame's rows end below 2^32 bytes (not rows_far)
+inline __host__ __device__ unsigned dI_offset(int pos, int ldI) { return (unsigned)pos * (4u * (unsigned)ldI); }
+inline bool rows_far(int max_area, int K) { return (double)max_area * dI_stride(K) * 4.0 >= 4294967296.0; }
 // per visible position: q (dI of a model-space direction e is q . e); Id and S of the shading (fitted
 // albedo only); patch and corners of its triangle; per frame the positions sorted by patch, in segments
 struct JacScratch {

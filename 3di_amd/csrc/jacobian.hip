@@ -1010,7 +1010,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(T >= 7
                     if (!(rk == rk)) rk = 0.f;
                 }
                 if (!FAR) {
-                    nb.x *= 4 * ldI; nb.y *= 4 * ldI; nb.z *= 4 * ldI; nb.w *= 4 * ldI;
+                    nb.x = (int)dI_offset(nb.x, ldI); nb.y = (int)dI_offset(nb.y, ldI);
+                    nb.z = (int)dI_offset(nb.z, ldI); nb.w = (int)dI_offset(nb.w, ldI);
                 }
                 snb[tid] = nb;
                 scf[tid] = cf;
@@ -1488,7 +1489,7 @@ int launch_jtj_mfma(const Layout& L, const FrameGPU* frames, FrameList fl, const
     const int gy = grid_frames(n, 1 << 16);
     const dim3 grid(S, gy);
     const int* act = fl.act;
-    const bool far = (double)max_area * dI_stride(K) * 4.0 >= 4294967296.0;
+    const bool far = rows_far(max_area, K);
     auto launch = [&](auto near_kernel, auto far_kernel) {
         hipLaunchKernelGGL(far ? far_kernel : near_kernel, grid, dim3(256), 0, s, L, frames, act, n, npix, pnb, pcoef, pixg,
                            dI, S, nsplit, partials, gp);
