@@ -33,7 +33,7 @@ __global__ void __launch_bounds__(256) k_f32_to_f64(size_t n, const float* __res
 }
 
 // Where entry j of the row of -g (then of L^-1 (-g)) is kept: the strict upper triangle of row 0, and for
-// the last entry of row 1 (K >= 3).
+// the last entry of row 1 (K >= CHOL_BIG_MINK).
 __device__ __forceinline__ size_t rhs_at(int K, int j) { return j < K - 1 ? (size_t)j + 1 : (size_t)2 * K - 1; }
 
 // The diagonal block of the panel at k0, in r (lane i: row i, entries j <= i; rows and columns past nb
@@ -332,12 +332,22 @@ static int chol_big_run(int n, int K, double* A, const TG* g, TD* delta, int* st
     return hipGetLastError() != hipSuccess ? TDI_ERR_HIP : TDI_OK;
 }
 
-int launch_cholesky_big(int n, int K, const float* H, const float* g, float* delta, int* status, hipStream_t s)
+static int chol_big_args(int K)
 {
     if (K > CHOL_BIG_MAXK) {
         set_error("cholesky: K=%d > %d", K, CHOL_BIG_MAXK);
         return TDI_ERR_ARG;
     }
+    if (K < CHOL_BIG_MINK) {                 // rhs_at
+        set_error("cholesky (large K): K=%d < %d", K, CHOL_BIG_MINK);
+        return TDI_ERR_ARG;
+    }
+    return TDI_OK;
+}
+
+int launch_cholesky_big(int n, int K, const float* H, const float* g, float* delta, int* status, hipStream_t s)
+{
+    if (int rc = chol_big_args(K)) return rc;
     double* A = nullptr;
     const size_t nkk = (size_t)n * K * K;
     if (hipMalloc((void**)&A, sizeof(double) * nkk) != hipSuccess) {
@@ -362,10 +372,7 @@ int launch_cholesky_big(int n, int K, const float* H, const float* g, float* del
 template <typename TD>
 static int cholesky_big_f64(int n, int K, double* A, const double* g, TD* delta, int* status, hipStream_t s)
 {
-    if (K > CHOL_BIG_MAXK) {
-        set_error("cholesky: K=%d > %d", K, CHOL_BIG_MAXK);
-        return TDI_ERR_ARG;
-    }
+    if (int rc = chol_big_args(K)) return rc;
     std::vector<int> ok(n, TDI_OK);
     TDI_HIP(hipMemcpyAsync(status, ok.data(), sizeof(int) * n, hipMemcpyHostToDevice, s));
     const int rc = chol_big_run(n, K, A, g, delta, status, s);

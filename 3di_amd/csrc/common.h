@@ -489,7 +489,7 @@ int launch_barrier_big(const ModelGPU& m, const Layout& L, const FrameGPU* frame
                        const double* rt, const double* P0, const LmkArrays& lm, int use_landmarks, double* D, double* H,
                        float* g, hipStream_t s);
 // cholesky_big.hip: FP64 blocked Cholesky solve for K above what one workgroup holds in LDS
-constexpr int CHOL_BIG_MAXK = 4096;
+constexpr int CHOL_BIG_MAXK = 4096, CHOL_BIG_MINK = 3;
 int launch_cholesky_big(int n, int K, const float* H, const float* g, float* delta, int* status, hipStream_t s);
 // The same on FP64 matrices A [n][K][K] factored in place, g FP64 [n][K].
 int launch_cholesky_big_f64(int n, int K, double* A, const double* g, float* delta, int* status, hipStream_t s);
