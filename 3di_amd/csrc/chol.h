@@ -41,6 +41,15 @@ template <typename T> struct ChVec;
 template <> struct ChVec<float> { typedef ch_v4f type; };
 template <> struct ChVec<double> { typedef ch_v4d type; };
 
+// An infinite diagonal entry makes its column of the factor and its unknown zero, where ch_root and ch_div
+// would make them NaN: the largest number does it too.
+template <typename T>
+__device__ __forceinline__ T ch_finite(T x)
+{
+    const T top = sizeof(T) == 8 ? T(1.7976931348623157e308) : T(3.4028234e38);
+    return x > top ? top : x;
+}
+
 // The lower blocks of H into LDS, scaled by sdinv on both sides when given; every load of the
 // thread (one entry of each block) is issued before the stores.
 template <typename T, typename TH>
@@ -64,6 +73,7 @@ __device__ __forceinline__ void ch_load(T* A, const TH* __restrict__ Hf, int K, 
             T x = (T)v[I * (I + 1) / 2 + J];
             if (sdinv) x = x * (T)sdinv[i] * (T)sdinv[j];
             if (i >= K || j >= K) x = i == j ? T(1) : T(0);
+            if (i == j) x = ch_finite(x);
             A[ch_block(I, J) + r * CHP + c] = x;
         }
 }

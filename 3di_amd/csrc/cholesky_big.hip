@@ -280,7 +280,7 @@ __global__ void __launch_bounds__(BACK_THREADS) k_chol_back(int K, const double*
             double lc[CB];
 #pragma unroll
             for (int j = 0; j < CB; ++j) lc[j] = j > c ? sD[j][c] : 0.0;
-            const double dd = sD[c][c], rinv = 1.0 / dd;
+            const double dd = ch_finite(sD[c][c]), rinv = 1.0 / dd;
             double r = c < nb ? sy[p0 + c] : 0.0;
 #pragma unroll
             for (int j = CB - 1; j >= 0; --j) r = fma(-lc[j], lane_read(ch_div(r, dd, rinv), j), r);

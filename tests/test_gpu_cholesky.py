@@ -92,3 +92,20 @@ def test_fp32_pivots_that_break_down():
     assert (d0[~bad] == d1[~bad]).all()
     # |x| <= 4; FP64's error is about K 2^-53 times the condition
     assert np.abs(d0[~bad] - x[~bad]).max() < 2.0 ** -8
+
+
+@pytest.mark.parametrize("K,mode", [(1, 0), (5, 0), (94, 0), (94, 1), (112, 1), (200, 0)])
+def test_infinite_diagonal_entries(K, mode):
+    """An unknown whose diagonal entry is infinite (an overflowed weight) does not move, and the others are
+    solved without it, as by the plain sequence: its column of the factor is zero."""
+    H, g = _systems(1, K, K, 1e2)
+    held = sorted({0, K // 3, K - 1})
+    H[0, held, held] = np.inf
+    d, st = tdi.cholesky_solve(torch.from_numpy(H).cuda(), torch.from_numpy(g).cuda(), mode)
+    assert st.cpu().numpy().tolist() == [0]
+    x = d[0].cpu().numpy().astype(np.float64)
+    assert (x[held] == 0).all()
+    free = np.setdiff1d(np.arange(K), held)
+    h = H[0][np.ix_(free, free)].astype(np.float64)
+    scale = np.abs(h) @ np.abs(x[free])
+    assert np.all(np.abs(h @ x[free] + g[0, free]) <= 2.0 ** -23 * scale)   # FP32 rounding of the solution
