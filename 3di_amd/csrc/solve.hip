@@ -313,6 +313,7 @@ __global__ void __launch_bounds__(BAR_THREADS) k_barrier(ModelGPU m, Layout L, c
                 for (int a = 0; a < 3; ++a) dv[a] = trans && j - L.off_pose == a ? 1.0 : 0.0;
             }
             landmark_dxy(fr, B, i, dv, dx, dy);
+            if (!(exp || id || trans || rot)) dx = dy = 0.0;   // at any depth, zero included
             s += B.gx[i] * dx + B.gy[i] * dy;
             if (j < KS) {
                 sdyn[(2 * i) * KS + j] = dx * B.rx[i];

@@ -1,5 +1,5 @@
 """The barrier's FP64 terms against the oracle: the padded column counts around the launch's LDS limit, and
-more unknowns than the derivative kernel's 112 without landmarks."""
+more unknowns than the derivative kernel's 112 without landmarks; a landmark at depth zero."""
 import importlib
 
 import numpy as np
@@ -31,3 +31,21 @@ def test_barrier_terms(k_exp, light, use_landmarks):
         errors = [abs(obj[i] - ob) / abs(ob), np.linalg.norm(H[i] - Ho) / np.linalg.norm(Ho),
                   np.linalg.norm(g[i] - go) / np.linalg.norm(go)]
         assert errors[0] < 1e-12 and errors[1] < 1e-10 and errors[2] < 1e-6, errors
+
+
+def test_landmark_at_depth_zero():
+    """The rotation about z and no expression put a landmark at depth exactly zero: its derivatives are not
+    finite, but the light's, which moves no landmark, are zero still."""
+    sc = make_scene(grid=24, k_exp=10, fit_light=2, crops=(48,), noise=0.0)
+    theta = sc.init().astype(np.float32)
+    pose = sc.lay["pose"]
+    theta[0, :pose] = 0
+    z = sc.model.mean_shape.astype(np.float32).reshape(-1, 3)[sc.model.landmark_ids[20], 2]
+    theta[0, pose:pose + 6] = (3.0, 2.0, -z, 0.0, 0.0, 0.25)
+    ctx = tdi.Context(sc.model, sc.opts)
+    b = tdi.Batch(ctx, sc.frames)
+    H, g, _ = b.barrier_terms(theta)
+    b.close()
+    ctx.close()
+    light = slice(pose + 6, None)
+    assert not torch.isfinite(g[0, pose]) and (g[0, light] == 0).all() and (H[0, light, light] == 0).all()
