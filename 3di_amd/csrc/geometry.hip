@@ -14,6 +14,7 @@
 //   k_synth_tile   — [3V x K] x [K x B] on v_mfma_f64_16x16x4f64; a workgroup owns 16 vertices,
 //                    stages their basis rows in LDS and walks every frame of the list; the
 //                    epilogue fuses mean, rotation, translation and projection from registers.
+//   k_synth_one    — a single frame: a thread per vertex coordinate.
 #include "common.h"
 
 namespace tdi {
@@ -76,13 +77,13 @@ typedef double v4d __attribute__((ext_vector_type(4)));
 //
 // One group (a list of up to 16 frames, such as the last line-search rounds of any batch): nothing
 // is reused from LDS and latency is all there is, so three wavefronts take a coordinate each
-// straight from memory and the four share the epilogue.  The sums run in the same order in both
+// straight from memory and the four share the epilogue.  The sums run in the same order in all
 // forms, so a frame's vertices do not depend on the frames around it.
 //
-// Every caller takes this kernel, one frame too.  Single evaluations took a thread per vertex walking
+// Every caller of several frames takes this kernel.  Single evaluations took a thread per vertex walking
 // its own three rows before: a sector per lane and load, and the whole basis again for every frame.
 // Measured at 53,361 vertices and 79 columns, that kernel against this one: 96 frames 2493 -> 104 us,
-// 48 frames 1258 -> 55 us, one frame 19.2 -> 21.7 us.  Bound by the FP64 matrix rate (31 us of the 104)
+// 48 frames 1258 -> 55 us.  Bound by the FP64 matrix rate (31 us of the 104)
 // and the stores (40 B per vertex, 44 us).  The one-group form took the mean launch of a one-frame fit
 // from 10.2 to 6.9 us (its basis staging alone was 39 us of a launch: run-time divisors).
 constexpr int SY_VERTS = 16;               // vertices per workgroup
@@ -254,6 +255,57 @@ k_synth_tile(ModelGPU m, Layout L, const FrameGPU* __restrict__ frames, const fl
     }
 }
 
+// One frame: 15 of a tile's 16 columns would be idle, and with more than 80 columns its chunks would be
+// staged for that one, so a thread takes one row (a vertex coordinate) with its sum in the tiles' order, 64
+// vertices per workgroup.  The latency of the loads bounds it.  The whole call by a thread per vertex, by
+// tiles and by this (53,361 vertices): 79 columns 49, 53 and 44 us, 199 + 79 columns 80, 114 and 65, 200
+// columns 64, 95 and 57; two frames by tiles are faster than two of these (79 columns: 55 us).
+constexpr int ONE_VERTS = 64;
+
+__global__ void __launch_bounds__(3 * ONE_VERTS) k_synth_one(ModelGPU m, Layout L, const FrameGPU* __restrict__ frames,
+                                                             const float* __restrict__ theta, const int* __restrict__ act,
+                                                             const double* __restrict__ rt,
+                                                             const double* __restrict__ mean64, double* __restrict__ P0,
+                                                             float* __restrict__ P, float4* __restrict__ vproj)
+{
+    __shared__ double sp[3 * ONE_VERTS];
+    if (fl_count(act, 1) == 0) return;
+    const int f = fl_frame(act, 0), tid = threadIdx.x;
+    const int r0 = 3 * ONE_VERTS * blockIdx.x, r = min(r0 + tid, 3 * m.V - 1);
+    const double base = mean64 ? mean64[r] : (double)m.mean[r];
+    double s = 0.0;
+    for (int blk = 0; blk < 2; ++blk) {                    // identity columns first
+        const int nc = blk ? L.nexp : mean64 ? 0 : L.nid, ld = blk ? m.exp_ld : m.id_ld;
+        const float* row = (blk ? m.exp_basis : m.id_basis) + (size_t)r * ld;
+        const float* tb = theta + (size_t)f * L.K + (blk ? L.off_exp : L.off_id);
+#pragma unroll 2
+        for (int k0 = 0; k0 < nc; k0 += 16) {              // rows are padded to 16 columns with zeros
+            float4 e[4];
+            float c[16];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) e[q] = *(const float4*)(row + k0 + 4 * q);
+#pragma unroll
+            for (int q = 0; q < 16; ++q) c[q] = tb[min(k0 + q, nc - 1)];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                s = fma((double)e[q].x, (double)c[4 * q + 0], s);
+                s = fma((double)e[q].y, (double)c[4 * q + 1], s);
+                s = fma((double)e[q].z, (double)c[4 * q + 2], s);
+                s = fma((double)e[q].w, (double)c[4 * q + 3], s);
+            }
+        }
+    }
+    sp[tid] = base + s;
+    __syncthreads();
+    const int v = ONE_VERTS * blockIdx.x + tid;
+    if (tid >= ONE_VERTS || v >= m.V) return;
+    double R[12];
+#pragma unroll
+    for (int q = 0; q < 12; ++q) R[q] = rt[(size_t)f * 12 + q];
+    const FrameCam cam{frames[f].phix, frames[f].phiy, frames[f].cx, frames[f].cy};
+    store_vertex(cam, R, sp + 3 * tid, (size_t)f * m.V + v, P0, P, vproj);
+}
+
 } // namespace
 
 static int launch_frame_rt(const Layout& L, FrameList fl, const float* theta, double* rt, hipStream_t s)
@@ -270,7 +322,10 @@ static int synthesize(const ModelGPU& m, const Layout& L, const FrameGPU* frames
                       double* rt, const double* mean64, double* P0, float* P, float4* vproj, hipStream_t s)
 {
     const dim3 grid((m.V + SY_VERTS - 1) / SY_VERTS);
-    if ((mean64 || L.nid == 0) && L.nexp > 0 && L.nexp <= SY_KMAX)
+    if (fl.n == 1)
+        hipLaunchKernelGGL(k_synth_one, dim3((m.V + ONE_VERTS - 1) / ONE_VERTS), dim3(3 * ONE_VERTS), 0, s, m, L, frames, theta,
+                           fl.act, rt, mean64, P0, P, vproj);
+    else if ((mean64 || L.nid == 0) && L.nexp > 0 && L.nexp <= SY_KMAX)
         hipLaunchKernelGGL(k_synth_tile<true>, grid, dim3(256), 0, s, m, L, frames, theta, fl.act, fl.n, rt, mean64, P0,
                            P, vproj);
     else

@@ -45,3 +45,22 @@ def test_synthesis_matches_fp64(grid, k_id, k_exp, n):
         # FP64 rounded once: half an FP32 ulp, and 1e-12 of the operands for the FP64 roundings
         assert np.all(np.abs(xyz[i] - q) <= 2.0 ** -24 * np.abs(q) + 1e-9), i
         assert np.all(np.abs(xyp[i] - xy) <= 2.0 ** -24 * np.abs(xy) + 1e-8), i
+
+
+@pytest.mark.parametrize("grid,k_id,k_exp", [(16, 0, 1), (17, 0, 79), (20, 0, 161), (19, 81, 80), (17, 80, 7), (23, 33, 16)])
+def test_one_frame_gives_the_bits_of_a_list(grid, k_id, k_exp):
+    """A frame alone, in a list of three and in one of twenty: three forms, one order of the sums."""
+    sc = make_scene(grid=grid, k_exp=k_exp, k_id=k_id, fit_id=k_id > 0, crops=(48,), noise=0.0, seed=grid, cfg=62)
+    rng = np.random.default_rng(6)
+    theta = np.tile(sc.truths[0].theta, (20, 1))
+    theta[:, :sc.lay["pose"]] = rng.uniform(-1, 1, (20, sc.lay["pose"]))
+    theta = theta.astype(np.float32)
+    ctx = tdi.Context(sc.model, sc.opts)
+    out = {}
+    for n in (1, 3, 20):
+        b = tdi.Batch(ctx, [sc.frames[0]] * n)
+        out[n] = [t[:1].cpu().numpy() for t in b.synthesize(theta[:n])] + [b.fit_buffers(theta[:n])[0][:1].cpu().numpy()]
+        b.close()
+    ctx.close()
+    for n in (3, 20):
+        assert all((a == c).all() for a, c in zip(out[1], out[n])), n
