@@ -1785,7 +1785,7 @@ int tdi_barrier_terms(tdi_batch* b, const float* theta, double* H, double* g, do
         if (rc) return rc;
         const float* th = theta + (size_t)i0 * K;
         if (c->opts.use_landmarks &&
-            (rc = launch_synthesize(b->m, c->L, w.frames, all_frames(n), th, w.rt, w.P0, nullptr, w.vproj, s)))
+            (rc = launch_landmark_vertices(c->m, c->L, n, th, w.rt, w.P0, s)))
             return rc;
         TDI_HIP(hipMemsetAsync(w.H, 0, sizeof(double) * (size_t)n * K * K, s));
         TDI_HIP(hipMemsetAsync(w.g, 0, sizeof(float) * (size_t)n * K, s));

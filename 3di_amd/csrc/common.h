@@ -374,6 +374,9 @@ struct LmkArrays {
 // (rt_ready: rt already holds them for theta)
 int launch_synthesize(const ModelGPU& m, const Layout& L, const FrameGPU* frames, FrameList fl, const float* theta,
                       double* rt, double* P0, float* P, float4* vproj, hipStream_t s, bool rt_ready = false);
+// The landmark vertices of frames 0..n-1 in P0, with the bits of a synthesis, and rt.
+int launch_landmark_vertices(const ModelGPU& m, const Layout& L, int n, const float* theta, double* rt, double* P0,
+                             hipStream_t s);
 // Synthesis of frames that share their identity coefficients (the identity stage's evaluations):
 // the identity shape once (FP64, idshape [V][3]), then the expression MFMA tiles on it.
 int launch_synthesize_shared_id(const ModelGPU& m, const Layout& L, const FrameGPU* frames, FrameList fl,

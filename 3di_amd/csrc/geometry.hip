@@ -262,22 +262,15 @@ k_synth_tile(ModelGPU m, Layout L, const FrameGPU* __restrict__ frames, const fl
 // columns 64, 95 and 57; two frames by tiles are faster than two of these (79 columns: 55 us).
 constexpr int ONE_VERTS = 64;
 
-__global__ void __launch_bounds__(3 * ONE_VERTS) k_synth_one(ModelGPU m, Layout L, const FrameGPU* __restrict__ frames,
-                                                             const float* __restrict__ theta, const int* __restrict__ act,
-                                                             const double* __restrict__ rt,
-                                                             const double* __restrict__ mean64, double* __restrict__ P0,
-                                                             float* __restrict__ P, float4* __restrict__ vproj)
+__device__ __forceinline__ double synth_row(const ModelGPU& m, const Layout& L, const float* __restrict__ tf, int r,
+                                            const double* __restrict__ mean64)
 {
-    __shared__ double sp[3 * ONE_VERTS];
-    if (fl_count(act, 1) == 0) return;
-    const int f = fl_frame(act, 0), tid = threadIdx.x;
-    const int r0 = 3 * ONE_VERTS * blockIdx.x, r = min(r0 + tid, 3 * m.V - 1);
     const double base = mean64 ? mean64[r] : (double)m.mean[r];
     double s = 0.0;
     for (int blk = 0; blk < 2; ++blk) {                    // identity columns first
         const int nc = blk ? L.nexp : mean64 ? 0 : L.nid, ld = blk ? m.exp_ld : m.id_ld;
         const float* row = (blk ? m.exp_basis : m.id_basis) + (size_t)r * ld;
-        const float* tb = theta + (size_t)f * L.K + (blk ? L.off_exp : L.off_id);
+        const float* tb = tf + (blk ? L.off_exp : L.off_id);
 #pragma unroll 2
         for (int k0 = 0; k0 < nc; k0 += 16) {              // rows are padded to 16 columns with zeros
             float4 e[4];
@@ -295,7 +288,20 @@ __global__ void __launch_bounds__(3 * ONE_VERTS) k_synth_one(ModelGPU m, Layout 
             }
         }
     }
-    sp[tid] = base + s;
+    return base + s;
+}
+
+__global__ void __launch_bounds__(3 * ONE_VERTS) k_synth_one(ModelGPU m, Layout L, const FrameGPU* __restrict__ frames,
+                                                             const float* __restrict__ theta, const int* __restrict__ act,
+                                                             const double* __restrict__ rt,
+                                                             const double* __restrict__ mean64, double* __restrict__ P0,
+                                                             float* __restrict__ P, float4* __restrict__ vproj)
+{
+    __shared__ double sp[3 * ONE_VERTS];
+    if (fl_count(act, 1) == 0) return;
+    const int f = fl_frame(act, 0), tid = threadIdx.x;
+    const int r0 = 3 * ONE_VERTS * blockIdx.x, r = min(r0 + tid, 3 * m.V - 1);
+    sp[tid] = synth_row(m, L, theta + (size_t)f * L.K, r, mean64);
     __syncthreads();
     const int v = ONE_VERTS * blockIdx.x + tid;
     if (tid >= ONE_VERTS || v >= m.V) return;
@@ -304,6 +310,16 @@ __global__ void __launch_bounds__(3 * ONE_VERTS) k_synth_one(ModelGPU m, Layout 
     for (int q = 0; q < 12; ++q) R[q] = rt[(size_t)f * 12 + q];
     const FrameCam cam{frames[f].phix, frames[f].phiy, frames[f].cx, frames[f].cy};
     store_vertex(cam, R, sp + 3 * tid, (size_t)f * m.V + v, P0, P, vproj);
+}
+
+// The landmark vertices alone, a frame per workgroup (the rest of P0 is left as it is).
+__global__ void __launch_bounds__(192) k_landmark_vertices(ModelGPU m, Layout L, const float* __restrict__ theta,
+                                                           double* __restrict__ P0)
+{
+    const int f = blockIdx.x, tid = threadIdx.x;
+    if (tid >= 3 * NLMK) return;
+    const int r = 3 * m.lmk_ids[tid / 3] + tid % 3;
+    P0[(size_t)f * m.V * 3 + r] = synth_row(m, L, theta + (size_t)f * L.K, r, nullptr);
 }
 
 } // namespace
@@ -333,6 +349,16 @@ static int synthesize(const ModelGPU& m, const Layout& L, const FrameGPU* frames
                            P, vproj);
     TDI_HIP(hipGetLastError());
     if (m.alb && L.ntex) return launch_albedo(m, L, fl, theta, const_cast<float*>(m.alb), s);
+    return TDI_OK;
+}
+
+int launch_landmark_vertices(const ModelGPU& m, const Layout& L, int n, const float* theta, double* rt, double* P0,
+                             hipStream_t s)
+{
+    const int rc = launch_frame_rt(L, all_frames(n), theta, rt, s);
+    if (rc) return rc;
+    hipLaunchKernelGGL(k_landmark_vertices, dim3(n), dim3(192), 0, s, m, L, theta, P0);
+    TDI_HIP(hipGetLastError());
     return TDI_OK;
 }
 
