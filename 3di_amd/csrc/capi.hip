@@ -1855,11 +1855,14 @@ int tdi_batch_autotune(tdi_batch* b, const float* theta, int32_t reps, int32_t* 
     const int areas[4] = {std::max(1, a0 / 2), a0, 2 * a0, 4 * a0};
     int best_area = a0;
     float best = 1e30f;
+    // through mesh patches only the albedo columns take k_dI, whose grid the area sizes: else one timing is all four
+    const bool sized = c->L.ntex || !patch_path(b->m, c->L, n, a0);
     for (int i = 0; i < 4 && !rc; ++i) {
+        if (!sized && i > 0) { rep[i] = rep[0]; continue; }
         rc = timed([&] { return launch_dI(b->m, c->L, w.frames, all_frames(n), theta, w.P0, w.pvert, w.pbary, w.npix,
                                           w.pixg, jac_scratch(w), w.dI, areas[i], w.max_area, s); },
                    rep[i]);
-        if (!rc && rep[i] < best) { best = rep[i]; best_area = areas[i]; }
+        if (!rc && sized && rep[i] < best) { best = rep[i]; best_area = areas[i]; }
     }
     const int S0 = w.S;
     int best_S = S0;

@@ -451,6 +451,7 @@ struct JacScratch {
 // Segments of a frame's positions for a workspace of so many frame slots and crops of up to max_area
 // pixels (half of them visible): enough that sorting few large frames takes the whole chip.
 int patch_segments(int frames, int max_area);
+bool patch_path(const ModelGPU& m, const Layout& L, int n, int mean_area);
 int launch_dI(const ModelGPU& m, const Layout& L, const FrameGPU* frames, FrameList fl, const float* theta,
               const double* P0, const int4* pvert, const float2* pbary, const int* npix, const float4* pixg,
               const JacScratch& js, float* dI, int grid_area, int max_area, hipStream_t s);

@@ -1352,7 +1352,7 @@ int jtj_splits(int n, int per_frame_pixels_hint)
 //       6 patches   48, 512: 1227/1290               24, 192: 76/86    96, 192: 322/270   448, 96: 388/245
 //     506 patches, 30 columns        8, 512: 133/127 24, 192: 87/68    94 patches, 30: 24, 192: 68/78, 96, 192: 265/190
 //       6 patches, 30 columns        96, 192: 243/264                  448, 96: 296/218
-static bool patch_path(const ModelGPU& m, const Layout& L, int n, int mean_area)
+bool patch_path(const ModelGPU& m, const Layout& L, int n, int mean_area)
 {
     const int cols = L.nexp + L.nid;
     if (m.np == 0 || cols == 0 || n < 8) return false;

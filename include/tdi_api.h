@@ -396,7 +396,8 @@ int tdi_render_loss_grad(tdi_batch* b, const float* theta, const float* dverts, 
 
 /* Launch-shape autotuner (no counterpart in the reference, whose launch shapes are fixed in the
  * source): on the batch's first workspace chunk rendered at theta (DEVICE [n][K]), times the
- * per-pixel Jacobian kernel with its grid sized for 1/2, 1, 2 and 4 times the mean crop, and the
+ * per-pixel Jacobian kernel with its grid sized for 1/2, 1, 2 and 4 times the mean crop (once, for
+ * all four, where its grid does not depend on that: columns through mesh patches), and the
  * J^T J kernel with 1, 2, 4, ... splits per frame (up to twice the default), `reps` launches each,
  * and keeps the fastest of each for the batch (its captured fit schedules are rebuilt on the next
  * fit); later batches of the same shape in the process start from the same choice.  choice [4]

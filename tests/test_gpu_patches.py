@@ -55,3 +55,17 @@ def test_patches_give_the_gathers_entries(grid, k_id, k_exp, k_tex, crops, n, mi
             else:
                 a, b = a.flatten(1).double(), b.flatten(1).double()
                 assert ((a - b).norm(dim=1) <= 1e-5 * b.norm(dim=1)).all(), i
+
+
+def test_autotune_times_the_patches_once():
+    """Without albedo the patches leave nothing to the kernel whose grid is tuned: one timing stands for the
+    four areas, and the mean crop stays."""
+    sc = make_scene(grid=24, k_exp=79, fit_light=2, crops=(64,), noise=0.0)
+    ctx = tdi.Context(sc.model, sc.opts)
+    b = tdi.Batch(ctx, sc.frames * 64)
+    res = b.autotune(np.tile(sc.init(), (64, 1)).astype(np.float32), reps=1)
+    shape = b.launch_shape()
+    b.close()
+    ctx.close()
+    assert len(set(res["dI_ms"].values())) == 1 and min(res["dI_ms"].values()) > 0
+    assert shape == (res["jtj_splits"], 64 * 64)
