@@ -78,8 +78,8 @@ __device__ __forceinline__ void ch_load(T* A, const TH* __restrict__ Hf, int K, 
         }
 }
 
-// s = sqrt(d) and y = 1 / s, on the factorisation's critical path (see ch_div).  fill(i) is called after
-// each dependent step i; returns their number.
+// s = sqrt(d) and y = 1 / s to an ulp, d positive, finite and normal, on the factorisation's critical path
+// (see ch_div).  fill(i) is called after each dependent step i; returns their number.
 template <typename F>
 __device__ __forceinline__ int ch_root(float d, float& s, float& y, F fill)
 {

@@ -177,10 +177,12 @@ __device__ inline int4 pixel_nbrs(const int* __restrict__ cum, int k, long long 
     return make_int4(kl, kr, pos - 1, pos + 1);
 }
 
-// Division on a critical path: a few FMAs around a reciprocal instead of the compiler's full sequence,
-// rounded as IEEE's all the same (Markstein, "Computation of elementary functions on the IBM RISC
-// System/6000 processor", 1990): with y the rounded reciprocal of b, q = a y and one
-// fma(a - b q, y, q) give the rounded a / b.
+// Division on a critical path: a few FMAs around a reciprocal instead of the compiler's full sequence
+// (Markstein, "Computation of elementary functions on the IBM RISC System/6000 processor", 1990): with y
+// the rounded reciprocal of b, q = a y and one fma(a - b q, y, q) give the rounded a / b, as long as b is
+// finite and not zero and y, q and the residual neither overflow nor underflow.  Outside of that the
+// result differs from a / b (b infinite or zero: NaN).  With y from ch_root, which may be an ulp off, no
+// quotient and no root differed in 2.6e8 random pairs of each type over forty binades.
 template <typename T>
 __device__ __forceinline__ T ch_div(T a, T b, T y)
 {

@@ -14,8 +14,9 @@
 //   on "face too large" or a NaN barrier.
 //
 // The batched state machine keeps every per-frame decision of the reference but runs it
-// for all frames of a batch with masks, so the whole fit is a fixed launch sequence
-// (graph-capturable): frames that have accepted a step or stopped sit out later rounds.
+// for all frames of a batch with masks: frames that have accepted a step or stopped sit out later
+// rounds.  The fit is a sequence of captured pieces; k_ls_status tells the host how many frames
+// still search and whether any is active, and the host launches the pieces that some frame needs.
 #include "chol.h"
 #include "common.h"
 
@@ -372,8 +373,9 @@ __global__ void __launch_bounds__(BAR_THREADS) k_barrier(ModelGPU m, Layout L, c
 //             block), the blocks dealt to the four wavefronts; two barriers per panel;
 //   solves    wavefront 0, lane l holding entries l and l + 64, right-looking.
 // A barrier pair and an LDS round trip per column (what it replaces) took 283 us for one matrix of
-// 94 unknowns (mode 1 with the FP64 fallback) and 552 us for 448; this takes 71 and 135 us, and gives the
-// same bits (each entry takes its products in the same order; an MFMA step is four FMAs in order).
+// 94 unknowns (mode 1 with the FP64 fallback) and 552 us for 448; this takes 91 and 98 us, mode 1 without
+// the fallback 57 and 61, mode 0 36 and 39.  Each entry takes its products in the same order (an MFMA
+// step is four FMAs in order) and the root and the divisions round alike (ch_root, ch_div).
 __device__ __forceinline__ double ch_wave_sum(double v)
 {
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
@@ -707,7 +709,7 @@ __global__ void __launch_bounds__(CMP_THREADS) k_ls_status(int n, const FitState
     }
 }
 
-// The barrier's derivative terms (k_barrier mode 1) for frames with more unknowns than the
+// The barrier's derivative terms (k_barrier's) for frames with more unknowns than the
 // landmark-derivative rows fit in LDS (the identity stage): the rows go to global scratch D
 // [frame][2][NLMK][K] and the Gauss-Newton sum is formed over 32 x 32 tiles of H by a grid.
 // Same formulas, FP64 throughout.
