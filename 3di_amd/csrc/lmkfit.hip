@@ -373,11 +373,10 @@ __global__ void __launch_bounds__(LF_THREADS, 2) k_lmk_slack(ModelGPU m, Layout 
         if (gout)
             for (int j = tid; j < n; j += LF_THREADS) gout[(size_t)f * n + j] = S.g[j];
         if (Hout)
-            for (int i = tid >> 4; i < n; i += LF_THREADS / 16)
-                for (int j = tid & 15; j < n; j += 16) {
-                    const int a = max(i, j), b = min(i, j);
-                    Hout[((size_t)f * n + i) * n + j] = dyn[ch_block(a >> 4, b >> 4) + (a & 15) * CHP + (b & 15)];
-                }
+            for (int e = tid; e < n * n; e += LF_THREADS) {
+                const int a = max(e / n, e % n), b = min(e / n, e % n);
+                Hout[(size_t)f * n * n + e] = dyn[ch_block(a >> 4, b >> 4) + (a & 15) * CHP + (b & 15)];
+            }
         return;
     }
     // set_minimal_slack: s = 5 - min G at s = 0
