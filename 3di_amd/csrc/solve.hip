@@ -495,6 +495,66 @@ __global__ void __launch_bounds__(256) k_cholesky(int K, const TH* __restrict__ 
     }
 }
 
+// Up to TINY_MAXK unknowns: a thread per matrix, in registers (padded with the identity), FP64 in both
+// modes with the bits of k_cholesky's mode 0.  k_cholesky does sixteen columns whatever their number: 4096
+// matrices of 4 unknowns 29 us (mode 1: 48), of 8 the same, here 12; from 9 on it is the faster for few
+// matrices.
+constexpr int TINY_MAXK = 8, TINY_THREADS = 64;
+
+template <typename TH>
+__global__ void __launch_bounds__(TINY_THREADS) k_cholesky_tiny(int n, int K, const TH* __restrict__ H,
+                                                                const float* __restrict__ g, float* __restrict__ delta,
+                                                                int* __restrict__ status, const int* __restrict__ mask)
+{
+    const int f = blockIdx.x * TINY_THREADS + threadIdx.x;
+    if (f >= n || (mask && !mask[f])) return;
+    const TH* Hf = H + (size_t)f * K * K;
+    const float* gf = g + (size_t)f * K;
+    double A[TINY_MAXK][TINY_MAXK], b[TINY_MAXK], q[TINY_MAXK];
+#pragma unroll
+    for (int i = 0; i < TINY_MAXK; ++i) {
+#pragma unroll
+        for (int j = 0; j <= i; ++j) {
+            const double x = (double)Hf[min(i, K - 1) * K + min(j, K - 1)];
+            A[i][j] = i < K ? (i == j ? ch_finite(x) : x) : i == j ? 1.0 : 0.0;
+        }
+        const double x = -(double)gf[min(i, K - 1)];
+        b[i] = i < K ? x : 0.0;
+    }
+    bool bad = false;
+#pragma unroll
+    for (int k = 0; k < TINY_MAXK; ++k) {
+        double s, inv;
+        bad = bad || !(A[k][k] > 0.0);
+        ch_root(A[k][k], s, inv, [](int) {});
+        A[k][k] = s;
+        q[k] = 1.0 / s;
+#pragma unroll
+        for (int i = k + 1; i < TINY_MAXK; ++i) A[i][k] = ch_div(A[i][k], s, inv);
+#pragma unroll
+        for (int i = k + 1; i < TINY_MAXK; ++i)
+#pragma unroll
+            for (int j = k + 1; j <= i; ++j) A[i][j] = fma(-A[i][k], A[j][k], A[i][j]);
+    }
+    status[f] = bad ? TDI_NOT_PD : TDI_OK;
+    if (bad) return;
+#pragma unroll
+    for (int i = 0; i < TINY_MAXK; ++i) {
+        b[i] = ch_div(b[i], A[i][i], q[i]);
+#pragma unroll
+        for (int j = i + 1; j < TINY_MAXK; ++j) b[j] = fma(-A[j][i], b[i], b[j]);
+    }
+#pragma unroll
+    for (int i = TINY_MAXK - 1; i >= 0; --i) {
+        b[i] = ch_div(b[i], A[i][i], q[i]);
+#pragma unroll
+        for (int j = 0; j < i; ++j) b[j] = fma(-A[i][j], b[i], b[j]);
+    }
+#pragma unroll
+    for (int i = 0; i < TINY_MAXK; ++i)
+        if (i < K) delta[(size_t)f * K + i] = (float)b[i];
+}
+
 // ------------------------------------------------------------------ line-search state machine
 // One wavefront per frame (delta . g is a sum over its lanes in a fixed order).
 __global__ void __launch_bounds__(64) k_ls_init(int n, int K, FitState* __restrict__ st, const int* __restrict__ chol_status,
@@ -852,6 +912,12 @@ static int launch_cholesky_t(int n, int K, const TH* H, const float* g, float* d
     if (K > CMAXK) {
         set_error("cholesky: K=%d > %d", K, CMAXK);
         return TDI_ERR_ARG;
+    }
+    if (K <= TINY_MAXK) {
+        hipLaunchKernelGGL(k_cholesky_tiny<TH>, dim3((n + TINY_THREADS - 1) / TINY_THREADS), dim3(TINY_THREADS), 0, s, n, K, H,
+                           g, delta, status, mask);
+        TDI_HIP(hipGetLastError());
+        return TDI_OK;
     }
     const int nT = (K + CHB - 1) / CHB;
     // the FP64 blocks, or mode 1's FP32 blocks and 16 columns of H in FP64

@@ -109,3 +109,22 @@ def test_infinite_diagonal_entries(K, mode):
     h = H[0][np.ix_(free, free)].astype(np.float64)
     scale = np.abs(h) @ np.abs(x[free])
     assert np.all(np.abs(h @ x[free] + g[0, free]) <= 2.0 ** -23 * scale)   # FP32 rounding of the solution
+
+
+@pytest.mark.parametrize("K", [1, 2, 3, 4, 5, 6, 7, 8, 9])
+def test_few_unknowns(K):
+    """A thread per matrix up to 8 unknowns: more than two workgroups of matrices, every fifth not positive
+    definite, both modes, and mode 1 no worse than mode 0."""
+    n = 130
+    H, g = _systems(n, K, 40 + K, 1e4)
+    bad = np.arange(n) % 5 == 2
+    H[bad, K - 1, K - 1] = -1.0
+    for mode in (0, 1):
+        d, st = tdi.cholesky_solve(torch.from_numpy(H).cuda(), torch.from_numpy(g).cuda(), mode)
+        assert (st.cpu().numpy() == np.where(bad, 4, 0)).all()
+        x = d.cpu().numpy().astype(np.float64)
+        h = H.astype(np.float64)
+        res = np.abs(np.einsum("nij,nj->ni", h, x) + g)
+        scale = np.einsum("nij,nj->ni", np.abs(h), np.abs(x))
+        # FP32 rounding of the solution; mode 1 above 8 unknowns leaves (cond 2^-24)^2 beyond it
+        assert np.all((res <= (2.0 ** -23 + (1e4 * 2.0 ** -22) ** 2 * (mode and K > 8)) * scale)[~bad])
